@@ -9,10 +9,11 @@
 // weights stream from HBM with many waves in flight; the streaming kernel
 // does the same for products with many columns, one workgroup walking many
 // column blocks; the slice kernels leave the slice sums to their consumer; the
-// tiled kernel (prefill) walks the slices one after the other with both
-// operands staged in LDS, or (slice sums of 17 rows and more) a group of them
-// a workgroup.  All produce the same bits for a row, so a token's
-// projections do not depend on how many tokens share its step.
+// ring kernel (gemm_ring.h: prefill, and decode over many columns) walks the
+// slices one after the other with both operands staged in LDS, or (slice sums
+// of 17 rows and more) a group of them a workgroup; the tiled kernel does the
+// same for operands that are not 16-byte aligned.  All produce the same bits for
+// a row, so a token's projections do not depend on how many tokens share its step.
 //
 // The MFMA runs "swapped": W rows are the first operand, X rows the second,
 // so a lane ends with four consecutive n of one row m and stores them as one
@@ -26,15 +27,6 @@
 
 namespace ls {
 
-#ifndef LS_GEMM_BIG
-#define LS_GEMM_BIG 0         // from this many 128 x 128 tiles on, use them; 0: one for every CU (fewer leave CUs idle and 64 x 64 tiles win)
-#endif
-#ifndef LS_GEMM_BIG_ROWS
-#define LS_GEMM_BIG_ROWS 64   // ... and only with more rows than this: up to 64 rows half of a 128-row tile would be idle
-#endif
-#ifndef LS_GEMM_PD_BIG
-#define LS_GEMM_PD_BIG 1      // register prefetch depth (stages) of the 128 x 128 kernel (2: registers run out, a third slower)
-#endif
 #ifndef LS_GEMM_SLICES_WIDE
 #define LS_GEMM_SLICES_WIDE 1       // 0: never the wide slice kernel
 #endif
@@ -50,29 +42,14 @@ namespace ls {
 #ifndef LS_GEMM_GROUP_M
 #define LS_GEMM_GROUP_M 4     // row tiles per band of the tile numbering (0: column-major numbering)
 #endif
-#ifndef LS_GEMM_WIDE
-#define LS_GEMM_WIDE 1        // 0: never the 128 x 256 tiles of eight waves
-#endif
-#ifndef LS_GEMM_WIDE_FILL
-#define LS_GEMM_WIDE_FILL 85  // ... which need whole rounds of the CUs (one workgroup a CU): at least this share, in percent,
-#endif                        // of the last round's CUs busy, or eight rounds and more
-#ifndef LS_GEMM_PD_WIDE
-#define LS_GEMM_PD_WIDE 2     // their register prefetch depth (2 is 1 to 4 % ahead of 1)
-#endif
 #ifndef LS_GEMM_READ_AHEAD
 #define LS_GEMM_READ_AHEAD 1  // the tiled kernel reads a stage's second chunk of fragments from LDS before it multiplies the first
 #endif
 #ifndef LS_GEMM_SLICES_TILED
-#define LS_GEMM_SLICES_TILED 1      // 0: never the tiled kernel for slice sums
-#endif
-#ifndef LS_GEMM_NARROW
-#define LS_GEMM_NARROW 1      // 0: never the 64 x 32 tiles
-#endif
-#ifndef LS_GEMM_ROWS64_WIDE
-#define LS_GEMM_ROWS64_WIDE 1 // 0: never 64 x 128 tiles for products of up to 64 rows
+#define LS_GEMM_SLICES_TILED 1      // 0: never the ring kernel for slice sums
 #endif
 #ifndef LS_GEMM_PD_SMALL
-#define LS_GEMM_PD_SMALL 4    // ... and of the 64 x 64 kernel (measured 1 to 4: 4 is 2 to 10 % ahead of 2)
+#define LS_GEMM_PD_SMALL 4    // register prefetch depth (stages) of the tiled kernel (measured 1 to 4: 4 is 2 to 10 % ahead of 2)
 #endif
 
 enum Epilogue : int {
@@ -81,7 +58,7 @@ enum Epilogue : int {
   kAddF32 = 2,    // C[m][n] += total, float (residual stream)
   kSwiGLU = 3,    // W holds gate and up rows interleaved in tiles of 16 (gate rows 16t.., then up rows 16t..);
                   // C[m][16t + i] = (g * 1/(1 + exp(-g))) * u in float, stored in the compute dtype
-  kSliceSums = 4, // the tiled kernel only: C is float [slices][M][N] and gets the sums of the K slices, not their
+  kSliceSums = 4, // the ring kernel only: C is float [slices][M][N] and gets the sums of the K slices, not their
                   // total; the workgroups with blockIdx.y = y take the slices [y * out_cols, (y + 1) * out_cols)
   kXielu = 5,     // C[m][n] = xielu(total) in the compute dtype, the activation's two factors from act[0], act[1]
 };
@@ -884,33 +861,28 @@ __global__ __launch_bounds__(256) void gemm_slices_stream_kernel(const T* __rest
   }
 }
 
+}  // namespace ls
+#include "gemm_ring.h"
+namespace ls {
+
 // ---------------------------------------------------------------------------
-// Tiled kernel: BM x BN outputs per workgroup, NWM x NWN waves, each
-// (BM/NWM) x (BN/NWN).  Both operands go through LDS in stages of 128 bytes
-// of K per row, double buffered: while stage i is multiplied, stage i+1 is
-// written to the other buffer and the global loads of stage i+2 are in
-// flight.  A wave's accumulators (at most 64 x 64 outputs, twice: the slice
-// sum and the total) leave room for two waves a SIMD, which is what hides
-// the LDS and barrier latency.  Workgroups are numbered so that those that
-// share a weight tile run on the same XCD (each XCD has its own L2).
-//
-// What bounds the kernel is the rate at which a CU gets operand bytes from
-// L2 (measured: every tile shape runs at 45 to 48 GB/s a CU), so the bytes a
-// workgroup loads per MFMA decide: (BM + BN) / (BM BN).  Hence eight waves
-// with 128 x 256 outputs where that many tiles fill the CUs, and the 2 x 2
-// grids of waves below that.
+// Tiled kernel: 64 x 64 outputs per workgroup by four waves, for operands that
+// the ring kernel does not take (rows that are not 16-byte aligned, K that is
+// not whole 16-byte pieces): it loads them element by element.  Both go through
+// registers into LDS in stages of 128 bytes of K per row, double buffered.
 // ---------------------------------------------------------------------------
 constexpr int kRowBytes = 128;               // bytes of K per row per stage (two chunks)
 constexpr int kRowStride = kRowBytes + 16;   // padded LDS row
 
-template <typename T, int EPI, int BM, int BN, int PD, bool AL, int NWM = 2, int NWN = 2>
-__global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __restrict__ X, const T* __restrict__ W,
+template <typename T, int EPI>
+__global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                          void* __restrict__ C, int M, int N, int K, long ldx,
                                                          long ldc, int kslice, int vec_ok, int tiles_m, int tiles_n,
                                                          int out_cols, const float* __restrict__ act) {
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   const Factors factors = load_factors<EPI>(act);
+  constexpr int BM = 64, BN = 64, NWM = 2, NWN = 2, PD = LS_GEMM_PD_SMALL;
   constexpr int BK = kRowBytes / sizeof(T);  // elements of K per stage
   constexpr int TI = BN / (16 * NWN);        // weight tiles (16 columns) per wave
   constexpr int TJ = BM / (16 * NWM);        // row tiles per wave
@@ -959,31 +931,9 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __r
       acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-  // PD stages of global loads are in flight in registers (slot = stage % PD).
-  // AL (rows and K 16-byte aligned, K a multiple of VEC): the loads are unconditional, from addresses
-  // clamped into the matrix, and nothing reads their registers before the stage is written to LDS, so
-  // the loads of PD stages really are in flight together (a zero selected right behind a load makes the
-  // compiler wait for it there).  Rows beyond M or N then hold copies of the last row: their products
-  // land in outputs that the epilogue does not store.  Only columns from K on must read as zero, and
-  // those are cleared on the way to LDS.
+  // PD stages of global loads are in flight in registers (slot = stage % PD)
   vec_t wv[PD][WP], xv[PD][XP];
-  const T* w_src[WP];
-  const T* x_src[XP];
-  if (AL) {
-#pragma unroll
-    for (int p = 0; p < WP; ++p) w_src[p] = W + (long)min(n_base + st_row + PASS * p, N - 1) * K;
-#pragma unroll
-    for (int p = 0; p < XP; ++p) x_src[p] = X + (long)min(m_base + st_row + PASS * p, M - 1) * ldx;
-  }
   auto fetch = [&](int slot, int k0) LS_INLINED {
-    if (AL) {
-      const int k = min(k0 + st_col, K - A::VEC);
-#pragma unroll
-      for (int p = 0; p < WP; ++p) wv[slot][p] = *reinterpret_cast<const vec_t*>(w_src[p] + k);
-#pragma unroll
-      for (int p = 0; p < XP; ++p) xv[slot][p] = *reinterpret_cast<const vec_t*>(x_src[p] + k);
-      return;
-    }
 #pragma unroll
     for (int p = 0; p < WP; ++p) {
       const int r = st_row + PASS * p;
@@ -995,7 +945,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __r
       xv[slot][p] = load_vec<T>(X, m_base + r, k0 + st_col, K, ldx, m_base + r < M, false);
     }
   };
-  auto stash = [&](int slot, int buf, int k0) LS_INLINED {
+  auto stash = [&](int slot, int buf) LS_INLINED {
     unsigned char* w_lds = lds + buf * STAGE_BYTES;
     unsigned char* x_lds = w_lds + BN * kRowStride;
 #pragma unroll
@@ -1004,42 +954,16 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __r
 #pragma unroll
     for (int p = 0; p < XP; ++p)
       *reinterpret_cast<vec_t*>(&x_lds[(st_row + PASS * p) * kRowStride + st_col * sizeof(T)]) = xv[slot][p];
-    if (AL && k0 + BK > K) {  // uniform: the last stage where K is no multiple of BK; its columns from K on are cleared
-      if (k0 + st_col >= K) {
-#pragma unroll
-        for (int p = 0; p < WP; ++p)
-          *reinterpret_cast<vec_t*>(&w_lds[(st_row + PASS * p) * kRowStride + st_col * sizeof(T)]) = A::zero();
-#pragma unroll
-        for (int p = 0; p < XP; ++p)
-          *reinterpret_cast<vec_t*>(&x_lds[(st_row + PASS * p) * kRowStride + st_col * sizeof(T)]) = A::zero();
-      }
-    }
   };
 
-  // the stages of this workgroup: all of K, or (kSliceSums) those of its group of slices
-  constexpr bool SLICES = EPI == kSliceSums;
-  const int all_stages = (K + BK - 1) / BK;
-  const int first_stage = SLICES ? (int)blockIdx.y * out_cols * (kslice / BK) : 0;
-  const int stages = SLICES ? min(all_stages - first_stage, out_cols * (kslice / BK)) : all_stages;
-  auto k_of = [&](int st) LS_INLINED { return (first_stage + st) * BK; };
-  auto store_slice = [&](int slice) LS_INLINED {  // the sums of one slice to their place among the slice sums
-    float* sums = reinterpret_cast<float*>(C) + (long)slice * M * N;
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) {
-        float t[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-        epilogue4<T, kStoreF32>(sums, ldc, m_base + wm + j * 16 + row16, n_base + wn + i * 16 + g * 4, M, N, t, vec_ok);
-      }
-  };
+  const int stages = (K + BK - 1) / BK;
+  auto k_of = [&](int st) LS_INLINED { return st * BK; };
   // stage s lives in register slot s % PD until it is written to LDS buffer s % 2
   fetch(0, k_of(0));
-  stash(0, 0, k_of(0));
-  // (AL: stages past the end are fetched too, from clamped addresses: with no condition around a
-  // fetch the compiler can count which loads are still in flight when a stage goes to LDS)
+  stash(0, 0);
 #pragma unroll
   for (int u = 1; u <= PD; ++u)
-    if (AL || u < stages) fetch(u % PD, k_of(u));
+    if (u < stages) fetch(u % PD, k_of(u));
   for (int base = 0; base < stages; base += PD) {
 #pragma unroll
     for (int u = 0; u < PD; ++u) {  // unrolled so that the register slots are static
@@ -1047,7 +971,6 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __r
       if (st >= stages) break;
       const int k0 = k_of(st);
       if (st > 0 && k0 % kslice == 0) {  // a stage never straddles a slice: kslice is a multiple of BK
-        if (SLICES) store_slice(k0 / kslice - 1);
 #pragma unroll
         for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1058,9 +981,9 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __r
           }
       }
       __syncthreads();  // stage st is in its buffer; the other buffer has been read by every wave
-      if (AL || st + 1 < stages) {  // (AL: past the last stage too, into the buffer that nobody reads any more)
-        stash((u + 1) % PD, (st + 1) & 1, k_of(st + 1));
-        if (AL || st + 1 + PD < stages) fetch((u + 1) % PD, k_of(st + 1 + PD));
+      if (st + 1 < stages) {
+        stash((u + 1) % PD, (st + 1) & 1);
+        if (st + 1 + PD < stages) fetch((u + 1) % PD, k_of(st + 1 + PD));
       }
       const unsigned char* w_lds = lds + (st & 1) * STAGE_BYTES;
       const unsigned char* x_lds = w_lds + BN * kRowStride;
@@ -1088,40 +1011,138 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_tiled_kernel(const T* __r
       }
     }
   }
-  if constexpr (SLICES) {
-    if (stages > 0) store_slice(k_of(stages - 1) / kslice);
-  } else {
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int j = 0; j < TJ; ++j)
+    for (int j = 0; j < TJ; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) total[i][j][r] = total[i][j][r] + acc[i][j][r];
+      for (int r = 0; r < 4; ++r) total[i][j][r] = total[i][j][r] + acc[i][j][r];
 
-    if (EPI == kSwiGLU) {
-      // the wave's weight tiles come in pairs (gate t, up t)
+  if (EPI == kSwiGLU) {
+    // the wave's weight tiles come in pairs (gate t, up t)
 #pragma unroll
-      for (int i = 0; i < TI; i += 2)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-          float gate[4] = {total[i][j][0], total[i][j][1], total[i][j][2], total[i][j][3]};
-          float up[4] = {total[i + 1][j][0], total[i + 1][j][1], total[i + 1][j][2], total[i + 1][j][3]};
-          epilogue_swiglu4<T>(C, ldc, m_base + wm + j * 16 + row16, (n_base + wn + i * 16) / 2 + g * 4, M, out_cols,
-                              gate, up, vec_ok);
-        }
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
+    for (int i = 0; i < TI; i += 2)
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        float t[4] = {total[i][j][0], total[i][j][1], total[i][j][2], total[i][j][3]};
-        if constexpr (EPI == kXielu)
-          epilogue_xielu4<T>(C, ldc, m_base + wm + j * 16 + row16, n_base + wn + i * 16 + g * 4, M, N, t, vec_ok, factors);
-        else
-          epilogue4<T, EPI>(C, ldc, m_base + wm + j * 16 + row16, n_base + wn + i * 16 + g * 4, M, N, t, vec_ok);
+        float gate[4] = {total[i][j][0], total[i][j][1], total[i][j][2], total[i][j][3]};
+        float up[4] = {total[i + 1][j][0], total[i + 1][j][1], total[i + 1][j][2], total[i + 1][j][3]};
+        epilogue_swiglu4<T>(C, ldc, m_base + wm + j * 16 + row16, (n_base + wn + i * 16) / 2 + g * 4, M, out_cols,
+                            gate, up, vec_ok);
       }
+    return;
   }
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      float t[4] = {total[i][j][0], total[i][j][1], total[i][j][2], total[i][j][3]};
+      if constexpr (EPI == kXielu)
+        epilogue_xielu4<T>(C, ldc, m_base + wm + j * 16 + row16, n_base + wn + i * 16 + g * 4, M, N, t, vec_ok, factors);
+      else
+        epilogue4<T, EPI>(C, ldc, m_base + wm + j * 16 + row16, n_base + wn + i * 16 + g * 4, M, N, t, vec_ok);
+    }
+}
+
+// The ring kernel's tiles: rows, columns, workgroups of it that a CU holds, and the microseconds a stage takes with one
+// workgroup on every CU and with as many as it holds (bfloat16, K = 4,096, weights from HBM).  The larger the tile, the
+// fewer operand bytes a product loads; the smaller, the more CUs have one, and the fuller the last round.
+enum RingTile { kRing256x192, kRing256x128, kRing192x192, kRing128x192, kRing192x128, kRing128x128, kRing128x64, kRing64x128,
+                kRing64x64, kRingTiles };
+struct RingShape {
+  int rows, cols, a_cu;
+  float one, full;
+};
+constexpr RingShape kRingShapes[kRingTiles] = {
+    {256, 192, 1, 1.33f, 1.33f}, {256, 128, 1, 0.94f, 0.94f}, {192, 192, 1, 1.00f, 1.00f}, {128, 192, 1, 0.76f, 0.76f},
+    {192, 128, 1, 0.73f, 0.73f}, {128, 128, 1, 0.58f, 0.58f}, {128, 64, 1, 0.43f, 0.43f},  {64, 128, 2, 0.52f, 0.74f},
+    {64, 64, 2, 0.33f, 0.52f}};
+
+// The tile whose rounds of workgroups take least by that table.  (Measured over 48 to 2,048 rows and nine shapes of
+// weights: within 6 % of the best tile nearly everywhere, 15 % at worst.)  float32 has four times the matrix work a byte
+// and takes 64 x 64 tiles, three a CU, throughout (2,000 x 6,144 x 1,024 192 us, 128 x 128 tiles 204).
+template <typename T>
+static int ring_tile(int M, int N) {
+  if (sizeof(T) == 4) return kRing64x64;
+  const long cus = compute_units();
+  int best = 0;
+  float least = 0.f;
+  for (int t = 0; t < kRingTiles; ++t) {
+    const RingShape& s = kRingShapes[t];
+    const long tiles = (long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols);
+    const long rest = tiles % (cus * s.a_cu);
+    const float time = (float)(tiles / (cus * s.a_cu)) * s.full + (rest == 0 ? 0.f : rest <= cus ? s.one : s.full);
+    if (t == 0 || time < least) {
+      least = time;
+      best = t;
+    }
+  }
+  return best;
+}
+
+// Whether the ring kernel runs a product of aligned operands: more than 64 rows, or so many columns that its 64-column
+// tiles beat the kernels of a wave a slice, which read the rows of X once for 16 columns (measured, us, those kernels /
+// this one: from 8 rows on over 10,240 columns and more: 8 x 10,240 x 5,120 35 / 24, 8 x 24,576 x 4,096 43 / 38, 8 x 151,936 x
+// 1,024 67 / 57 (1 x 24,576 x 4,096 stays); over 6,144 from 17 on at K = 4,096 21.4 / 18.8 (16 rows 18.1 / 19.6), at K =
+// 1,024 from 24 on 8.0 / 7.3 (17 rows 7.0 / 7.3); over 2,048 from 48 on 7.0 / 6.9 at K = 1,024).  float32 multiplies too slowly
+// for 64 rows in place of 33 to pay (33 x 6,144 x 1,024 18 / 23, 64 x 4,096 x 1,024 18 / 23), except over the most columns.
+template <typename T>
+static bool ring_takes(int M, int N, int K) {
+  if (M > 64) return true;
+  const int blocks = (N + 63) / 64;
+  if (sizeof(T) == 4) return blocks >= 256 && M > 32;
+  return blocks >= 160 ? M >= 8 : blocks >= 96 ? M >= (K >= 2048 ? 17 : 24) : blocks >= 32 && M >= 48;
+}
+
+// Dynamic LDS beyond 64 KB has to be granted per kernel (once).
+template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS>
+static bool ring_lds_ready(int bytes) {
+  static const bool granted = [bytes] {
+    if (bytes <= 64 * 1024) return true;
+    const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    return ok;
+  }();
+  return granted;
+}
+
+// groups: workgroups along K (kSliceSums: out_cols slices each); otherwise 1.
+template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS>
+static int launch_ring_tile(const T* X, const T* W, void* C, int M, int N, int K, long ldx, long ldc, int kslice, int vec_ok,
+                            int out_cols, int groups, const float* act, hipStream_t stream) {
+  constexpr int kBytes = (WS * BN + XS * BM) * 128;
+  static_assert(kBytes <= 160 * 1024, "the rings fit the LDS of a CU");
+  if (!ring_lds_ready<T, EPI, BM, BN, NWM, NWN, WS, XS>(kBytes)) return fail("gemm: %d bytes of LDS were refused", kBytes);
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  hipLaunchKernelGGL((gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS>), dim3(tiles_m * tiles_n, groups),
+                     dim3(64 * NWM * NWN), kBytes, stream, X, W, C, M, N, K, ldx, ldc, kslice, vec_ok, tiles_m, tiles_n,
+                     out_cols, act);
+  return check_launch("gemm");
+}
+
+template <typename T, int EPI>
+static int launch_ring(int tile, const T* X, const T* W, void* C, int M, int N, int K, long ldx, long ldc, int kslice,
+                       int vec_ok, int out_cols, int groups, const float* act, hipStream_t stream) {
+#define LS_RING(...) \
+  return launch_ring_tile<T, EPI, __VA_ARGS__>(X, W, C, M, N, K, ldx, ldc, kslice, vec_ok, out_cols, groups, act, stream)
+  if constexpr (sizeof(T) == 4) {
+    LS_RING(64, 64, 2, 2, 3, 3);
+  } else if constexpr (EPI == kSliceSums) {
+    LS_RING(64, 64, 4, 2, 5, 5);
+  } else {
+    switch (tile) {
+      case kRing256x192: LS_RING(256, 192, 4, 2, 3, 2);
+      case kRing256x128: LS_RING(256, 128, 4, 2, 3, 3);
+      case kRing192x192: LS_RING(192, 192, 4, 2, 3, 3);
+      case kRing128x192: LS_RING(128, 192, 4, 2, 3, 3);
+      case kRing192x128: LS_RING(192, 128, 4, 2, 4, 4);
+      case kRing128x128: LS_RING(128, 128, 4, 2, 4, 4);
+      case kRing128x64: LS_RING(128, 64, 4, 2, 5, 5);
+      case kRing64x128: LS_RING(64, 128, 2, 4, 3, 3);
+      default: LS_RING(64, 64, 4, 2, 5, 5);
+    }
+  }
+#undef LS_RING
 }
 
 template <typename T, int EPI>
@@ -1138,17 +1159,11 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   const int vec_ok = (ldc % 4 == 0) && (reinterpret_cast<uintptr_t>(C) % (4 * out_size) == 0);
   const T* w = reinterpret_cast<const T*>(W);
   if (norm_w && M > 16) return fail("gemm: the fused norm prologue takes at most 16 rows, got %d", M);
-  // Up to 64 rows the skinny kernel; but with more than 16 rows and very many columns (the logits
-  // head) its workgroups re-read all rows of X for 16 columns each, and the tiled kernel reads less.
   const int mt_rows = (M + 15) / 16;
   const int col_blocks = (N + 16 * NT - 1) / (16 * NT);
-  // With more than 16 rows the tiled kernel does better wherever it has a workgroup for every CU (its
-  // workgroups read the rows of X once for 64 columns, through LDS, and 64 columns of weights a workgroup
-  // keep enough loads in flight): from 33 rows on always (Qwen3-8B sizes, gate and up at 64 rows: 85 -> 50
-  // us), from 17 rows on for SwiGLU, where the streaming kernel has two weight tiles a column block and
-  // holds less in flight (58 -> 46 us at 32 rows; the logits head at 24 rows: streaming 257, tiled 307 us).
-  const bool tiled_fills = !norm_w && M <= 64 && (N + 63) / 64 >= compute_units() &&
-                           (M > 32 || (M > 16 && EPI == kSwiGLU));
+  if (!norm_w && aligned && ring_takes<T>(M, N, K))
+    return launch_ring<T, EPI>(ring_tile<T>(M, N), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
+                               vec_ok, out_cols, 1, act, stream);
   const int xc = kslice / Atom<T>::KCHUNK;  // chunks per slice
   // The streaming kernel where a workgroup would get more than one column block: a CU holds 16 waves
   // of it (one per K slice), so 16 / nslices workgroups.
@@ -1157,12 +1172,9 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   const int row_groups = mt_rows <= 2 ? 1 : 2;
   const int group_tiles = mt_rows <= 2 ? mt_rows : 2;
   const size_t stream_lds = 2 * (size_t)nslices * NT * group_tiles * 256 * sizeof(float);  // two sets of slice sums
-  // (two groups read the weights twice, the second time rarely from L2 in practice: with very many
-  // columns, where the tiled kernel does well, they are not worth it)
   // (with fewer than eight slices the skinny kernel's small workgroups, several a CU, do as well or better)
-  if (!norm_w && mt_rows <= 4 && !tiled_fills && xc % 4 == 0 && xc * group_tiles <= 16 && nslices >= 8 && nslices <= 16 &&
-      col_blocks * row_groups > stream_wgs && stream_lds <= 128 * 1024 && !(row_groups > 1 && N >= 32768) &&
-      LS_GEMM_STREAM) {
+  if (!norm_w && mt_rows <= 4 && xc % 4 == 0 && xc * group_tiles <= 16 && nslices >= 8 && nslices <= 16 &&
+      col_blocks * row_groups > stream_wgs && stream_lds <= 128 * 1024 && LS_GEMM_STREAM) {
     int walkers = stream_wgs / row_groups;
     const int rounds = (col_blocks + walkers - 1) / walkers;
     walkers = (col_blocks + rounds - 1) / rounds;
@@ -1183,21 +1195,7 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
 #undef LS_STREAM
     if (launched) return check_launch("gemm");
   }
-  // 32 to 64 rows over a product that neither fills the CUs with 64-column tiles nor has a streaming kernel
-  // for its slice length (QKV of Qwen3-14B and 32B sizes: slices of 512): the skinny kernel re-reads all
-  // rows of X for 16 columns a workgroup; tiles of 64 x 32 outputs where they give most CUs a workgroup
-  // (measured at 64 rows: N = 10,240, K = 5,120 83 -> 49 us; N = 7,168 56 -> 35 us; at 17 rows no gain).
-  if constexpr (EPI != kSwiGLU) {
-    if (LS_GEMM_NARROW && !norm_w && aligned && M >= 32 && M <= 64 && !tiled_fills && N < 32768 &&
-        (N + 31) / 32 >= compute_units() * 7 / 10) {
-      const int tiles_n = (N + 31) / 32;
-      hipLaunchKernelGGL((gemm_tiled_kernel<T, EPI, 64, 32, LS_GEMM_PD_SMALL, true, 2, 2>), dim3(tiles_n), dim3(256), 0,
-                         stream, reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice, vec_ok, 1, tiles_n,
-                         out_cols, act);
-      return check_launch("gemm");
-    }
-  }
-  if (M <= 64 && !tiled_fills && !(M > 16 && N >= 32768)) {
+  if (M <= 64) {
     const int mt = (M + 15) / 16;
     // 16 waves leave 128 registers a lane: only for one or two row tiles
     const int nw = (nslices > 8 && mt * NT <= 2) ? 16 : (nslices > 4 ? 8 : 4);
@@ -1221,40 +1219,9 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
     }
 #undef LS_SKINNY
   } else {
-    // Large products take 128 x 128 tiles (least LDS traffic per MFMA); smaller ones take
-    // 64 x 64 tiles so that every CU has several workgroups, with a deeper register prefetch.
-    const long big_tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-#define LS_TILED_WAVES(BM_, BN_, PD_, AL_, NWM_, NWN_)                                                         \
-  {                                                                                                             \
-    const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = (N + BN_ - 1) / BN_;                                       \
-    hipLaunchKernelGGL((gemm_tiled_kernel<T, EPI, BM_, BN_, PD_, AL_, NWM_, NWN_>), dim3(tiles_m * tiles_n),      \
-                       dim3(64 * NWM_ * NWN_), 0, stream, reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, \
-                       kslice, vec_ok, tiles_m, tiles_n, out_cols, act);                                        \
-  }
-#define LS_TILED(BM_, BN_, PD_, AL_) LS_TILED_WAVES(BM_, BN_, PD_, AL_, 2, 2)
-    // 128 x 256 tiles load a quarter fewer operand bytes per MFMA (measured at 2,048 rows: gate and up of
-    // Qwen3-8B sizes 511 -> 446 us, down 246 -> 211 us), but a CU holds one such workgroup, so a last
-    // round that leaves CUs idle costs more than it does with the smaller tiles, two of which share a CU
-    const long wide_tiles = (long)((M + 127) / 128) * ((N + 255) / 256);
-    const long cus = compute_units();
-    const long wide_rounds = (wide_tiles + cus - 1) / cus;
-    const bool wide_fills = LS_GEMM_WIDE && sizeof(T) == 2 && M > LS_GEMM_BIG_ROWS && wide_tiles >= cus &&
-                            (wide_rounds >= 8 || wide_tiles * 100 >= wide_rounds * cus * LS_GEMM_WIDE_FILL);
-    // (operands that are not 16-byte aligned take the small tiles, element by element: every tile
-    // shape gives the same bits)
-    if (!aligned) LS_TILED(64, 64, LS_GEMM_PD_SMALL, false)
-    else if (wide_fills) {
-      if constexpr (sizeof(T) == 2) LS_TILED_WAVES(128, 256, LS_GEMM_PD_WIDE, true, 2, 4)
-    }
-    else if (big_tiles >= (LS_GEMM_BIG ? LS_GEMM_BIG : cus) && M > LS_GEMM_BIG_ROWS) LS_TILED(128, 128, LS_GEMM_PD_BIG, true)
-    // up to 64 rows over so many columns that tiles of 128 columns still give every CU a workgroup (the
-    // logits head, gate and up of 32B sizes): every workgroup reads all rows of X, so half as many
-    // workgroups halve that traffic (gate and up of 32B sizes at 64 rows 135 -> 112 us, the head 82 -> 77 us)
-    else if (LS_GEMM_ROWS64_WIDE && M <= 64 && (N + 127) / 128 >= cus)
-      LS_TILED_WAVES(64, 128, LS_GEMM_PD_SMALL, true, 2, 4)
-    else LS_TILED(64, 64, LS_GEMM_PD_SMALL, true)
-#undef LS_TILED
-#undef LS_TILED_WAVES
+    const int tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64;
+    hipLaunchKernelGGL((gemm_tiled_kernel<T, EPI>), dim3(tiles_m * tiles_n), dim3(256), 0, stream,
+                       reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice, vec_ok, tiles_m, tiles_n, out_cols, act);
   }
   return check_launch("gemm");
 }
@@ -1358,13 +1325,12 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
       (int)std::min<long>(4, (long)col_blocks * groups * std::max(row_groups, 1) / (2L * compute_units()));
   if (mt > 4 && rounds < 1) rounds = 1;  // more than 64 rows: this kernel only, if with one column block a workgroup
   // Enough rows over weights large enough that 64 x 64 tiles times groups of slices give every CU a
-  // workgroup: the tiled kernel, which stages both operands in LDS four stages ahead and so keeps twice the
-  // bytes of the wide kernel in flight (measured at 64 rows, Qwen3-8B and 32B sizes: O 18.3 -> 12.4 and
-  // 44.9 -> 27.8 us, down 42.3 -> 30.3 and 119.9 -> 68.0 us; at 256 rows O 44.5 -> 30.4 and 147.9 -> 68.1 us).
-  // A workgroup takes as many slices as give it eight stages, fewer where that leaves CUs without one.
+  // workgroup: the ring kernel, which has four stages of both operands in flight (measured against tiles staged
+  // through registers: 17 x 4,096 x 4,096 11.1 -> 9.0 us, 64 x 4,096 x 12,288 29.9 -> 26.4, 256 x 1,024 x 2,048 8.3 ->
+  // 6.5; those were ahead of the wide kernel by a third).  A workgroup takes as many slices as give it eight stages, fewer
+  // where that leaves CUs without one.
   // From 17 rows on in bfloat16 (from 8 over weights of 64 MB and more, where the kernels of a wave a slice
-  // fall to 3.7 TB/s and this one holds 4.2 to 4.6; below that and over smaller weights those are ahead),
-  // from 33 rows on in float32.
+  // fall to 3.7 TB/s; below that and over smaller weights those are ahead), from 33 rows on in float32.
   const long weight_bytes = (long)N * K * (dtype == kF32 ? 4 : 2);
   const int tiled_from = dtype == kF32 ? 33 : (weight_bytes >= (64L << 20) ? 8 : 17);
   if (LS_GEMM_SLICES_TILED && aligned && M >= tiled_from && N % 4 == 0) {
@@ -1375,13 +1341,13 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
     while (per > 1 && workgroups(per) < compute_units()) per = (per + 1) / 2;
     if (workgroups(per) >= compute_units()) {
       const int groups_y = (nslices + per - 1) / per;
-      dim3 tiled_grid(tiles_m * tiles_n, groups_y);
-#define LS_TILED_SLICES(T_)                                                                                          \
-  hipLaunchKernelGGL((gemm_tiled_kernel<T_, kSliceSums, 64, 64, LS_GEMM_PD_SMALL, true, 2, 2>), tiled_grid, dim3(256), \
-                     0, s, (const T_*)X, (const T_*)W, (void*)P, M, N, K, ldx, (long)N, kslice, 1, tiles_m, tiles_n, per, (const float*)nullptr)
-      if (dtype == kF32) { LS_TILED_SLICES(float); } else if (dtype == kBF16) { LS_TILED_SLICES(bf16_t); } else return fail("gemm_slices: unknown dtype %d", dtype);
-#undef LS_TILED_SLICES
-      return check_launch("gemm_slices");
+      if (dtype == kF32)
+        return launch_ring<float, kSliceSums>(kRing64x64, (const float*)X, (const float*)W, P, M, N, K, ldx, N, kslice, 1, per,
+                                              groups_y, nullptr, s);
+      if (dtype == kBF16)
+        return launch_ring<bf16_t, kSliceSums>(kRing64x64, (const bf16_t*)X, (const bf16_t*)W, P, M, N, K, ldx, N, kslice, 1,
+                                               per, groups_y, nullptr, s);
+      return fail("gemm_slices: unknown dtype %d", dtype);
     }
   }
   // More than 16 rows and enough columns that workgroups of 64 columns fill the GPU: the wide kernel.
@@ -1445,7 +1411,7 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
 // Whether ls_gemm_slices_folded takes this product: at most 16 rows, whole heads of a size that is a
 // multiple of four, K a multiple of the load width, at most 32 splits, the folded rows of a slice within
 // 64 KB of LDS -- and the plain slice kernel is what ls_gemm_slices itself would run for these sizes (over
-// large weights it prefers the tiled kernel from eight rows on, which reads its operand from memory).
+// large weights it prefers the ring kernel from eight rows on, which reads its operand from memory).
 extern "C" int ls_gemm_slices_folded_ok(int dtype, int M, int N, int K, int head_dim, int splits) {
   using namespace ls;
   if (dtype != kF32 && dtype != kBF16) return 0;

@@ -156,6 +156,48 @@ def test_gemm_with_many_rows_and_columns_has_the_bits_of_few_rows(dtype, k):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k", [8, 72, 328, 4424])
+@pytest.mark.parametrize("m,n", [(2041, 6152), (2041, 4091), (1501, 6139), (1003, 6139), (1501, 4088), (1003, 4096), (1003, 2044),
+                                 (64, 32700), (300, 1000), (65, 16), (130, 3)])
+def test_every_tile_of_the_products_has_the_bits_of_few_rows(dtype, k, m, n):
+    """Sizes that take each tile of the ring kernel (256 x 192 down to 64 x 64 outputs), with rows and columns that end inside
+    a tile, K of less than a stage, K that ends inside a stage and inside a slice, and columns that no vector store fits:
+    five rows at a time, which the kernels of a wave a slice compute, have the same bits."""
+    from lockstep_amd.ops import ADD_F32, STORE, STORE_F32, SWIGLU
+
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+    x[-1], w[-1] = float("inf"), float("nan")               # a row and a column must not reach another one
+    full = torch.full((m, n), 7.0, device="cuda")
+    K().gemm(x, w, full, STORE_F32)
+    stored = torch.empty(m, n, dtype=dtype, device="cuda")
+    K().gemm(x, w, stored, STORE)
+    assert torch.equal(stored[:-1, :-1], full[:-1, :-1].to(dtype))
+    base = torch.randn(m, n, generator=g, device="cuda")
+    acc = base.clone()
+    K().gemm(x, w, acc, ADD_F32)
+    assert torch.equal(acc[:-1, :-1], base[:-1, :-1] + full[:-1, :-1])
+    gated = None
+    if n % 32 == 8:                                          # as interleaved gate and up rows
+        n_gated = n - 8
+        gated = torch.empty(m, n_gated // 2, dtype=dtype, device="cuda")
+        K().gemm(x, w[:n_gated].contiguous(), gated, SWIGLU)
+    want = x[:2].double() @ w[:-1].double().T
+    assert rel_err(full[:2, :-1], want) < 2e-5
+    for first in sorted({0, m // 2, m - 7}):
+        rows = slice(first, first + 5)
+        part = torch.empty(5, n, device="cuda")
+        K().gemm(x[rows], w, part, STORE_F32)
+        assert torch.equal(part[:, :-1], full[rows, :-1]), f"rows from {first}"
+        assert torch.isnan(full[rows, -1]).all()
+        if gated is not None:
+            part = torch.empty(5, n_gated // 2, dtype=dtype, device="cuda")
+            K().gemm(x[rows], w[:n_gated].contiguous(), part, SWIGLU)
+            assert torch.equal(part, gated[rows]), f"rows from {first}, SwiGLU"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("inter,k", [(4096 + 40, 4096), (16384 + 72, 1024), (25600, 5120)])
 def test_swiglu_with_few_rows_and_many_columns_has_the_same_bits(dtype, inter, k):
     from lockstep_amd.ops import SWIGLU, interleave_gate_up
