@@ -689,6 +689,35 @@ def test_attention_row_is_the_same_alone_in_a_portion_and_in_the_whole_prompt(dt
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq,nkv,d,ps,t", [(4, 1, 128, 16, 300), (4, 2, 64, 8, 517), (6, 3, 128, 64, 260), (8, 4, 128, 32, 530),
+                                           (16, 8, 64, 16, 129), (16, 16, 128, 128, 140), (24, 24, 16, 16, 90)])
+def test_row_blocks_of_every_number_of_kv_heads_with_scales_of_either_sign_and_windows(dtype, nq, nkv, d, ps, t):
+    """How the work of a portion is numbered depends on the kv heads and on the row blocks (here odd and even
+    counts): the wide kernels against the direct one, to the bit, and against the formula.  A negative scale
+    turns the order of the scores, a zero one makes them equal; a window releases the pages behind it."""
+    n = 700
+    qkv = rand_qkv(n, nq, nkv, d, dtype, seed=nq + d)
+    case = PagedCase(dtype, nq, nkv, d, ps, n, shuffle_seed=7)
+    dev = qkv.cuda()
+    case.write(dev, 0)
+    q, k, v = split_qkv(qkv.double(), nq, nkv, d)
+    lo = n - t
+    for scale, window in ((d ** -0.5, 0), (-0.7 * d ** -0.5, 0), (0.0, 0), (d ** -0.5, 131)):
+        saved = case.table.clone()
+        if window:
+            case.table[1, :max(0, lo - window + 1) // ps] = -1
+        got = case.attend(dev[lo:], lo, scale, window=window, variant=1, force_split=False)
+        want = naive_attention(q[lo:], k, v, lo, scale, window=window or None)
+        assert rel_err(got, want) < ATT_TOL[dtype], (scale, window)
+        if K().wide_supported(d, dtype, ps):
+            for variant in (4, 5):
+                for split in (False, True):
+                    wide = case.attend(dev[lo:], lo, scale, window=window, variant=variant, force_split=split)
+                    assert torch.equal(wide, got), (scale, window, variant, split)
+        case.table.copy_(saved)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window", [1, 7, 128, 300])
 def test_attention_window(dtype, window):
     nq, nkv, d, ps, kv_len = 4, 2, 32, 16, 520
