@@ -24,6 +24,7 @@
 // tiles of a wave.
 
 #include "common.h"
+#include "ring.h"
 
 #include <type_traits>
 
@@ -572,175 +573,185 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// The same two products for tiles of 64 rows (many tokens an expert), both operands staged through LDS: a
-// workgroup takes 64 rows x 64 columns, its four waves 32 x 32 each.  A stage is 128 bytes of K for every row of
-// the operands (two chunks of the atom), copied from global memory into registers while the stage before it is
-// multiplied, then written to the other of two LDS buffers; rows of an LDS tile are 144 bytes apart, which
-// spreads the sixteen rows of a fragment read over all banks.  A row's contraction is still one chain over
-// ascending chunks from zero: the same bits as the kernels above give without a cut of K.  NB: weight matrices
-// that share the rows (gate and up: 2; down: 1).
+// The same two products for tiles of 64 rows (many tokens an expert), both operands through a ring of three stages in
+// LDS (128 bytes of K a row, written there by the loads themselves; layout, waits and barriers as gemm_ring.h describes
+// them).  A workgroup of eight waves takes 64 rows by 128 weight rows: 64 gate and the 64 up rows of the same columns, or
+// 128 columns of the down product; two workgroups share a CU.  A row's contraction is still one chain over ascending
+// chunks from zero: the same bits as the kernels above give without a cut of K.  Measured against tiles staged through
+// registers (64 x 64 by four waves; 2,048 tokens with 4 of 32 experts, width 1,024, 768 a piece): gate and up 94 -> 65
+// us (395 TFLOP/s), down 65 -> 52.  What bounds it now is the L2: 855 MB of requests in gate and up, 13 TB/s, three
+// quarters of them hits.  Four neighbouring tiles kept on one XCD, so that an expert's weights reach an L2 once, moved
+// this by no more than the runs differ (67 and 50 us): a row tile of 64 asks for too many bytes an operation.
 // ---------------------------------------------------------------------------
-constexpr int kStageBytes = 128, kLdsRow = kStageBytes + 16;
-
-template <typename T, int NB>
-struct TiledProduct {
+constexpr int kRingRows = 64, kRingWeights = 128, kRingStages = 3;
+constexpr int kRingLds = kRingStages * (kRingRows + kRingWeights) * 128;
+template <typename T, bool PAIRED>  // PAIRED: a wave's two weight tiles lie 64 rows apart (gate, up), else side by side
+struct RingProduct {
   typedef typename Atom<T>::vec_t vec_t;
-  static constexpr int VEC = Atom<T>::VEC;
-  static constexpr int kStageK = kStageBytes / (int)sizeof(T);
-  vec_t staged[1 + NB][2];
-  f32x4 acc[NB][2][2];
+  static constexpr int BK = 128 / (int)sizeof(T), S = kRingStages;
+  static constexpr int W_BYTES = kRingWeights * 128, X_BYTES = kRingRows * 128;
+  static constexpr int LOADS = 3;  // a wave's loads a stage: eight rows of X, twice eight of W
+  f32x4 acc[2][2];                 // [weight tile][row tile]
 
-  // a_row / b_row: where this thread's two pieces of a stage come from (null: zeros), for rows tid/8 and tid/8 + 32
-  __device__ __forceinline__ void request(const T* const (&a_row)[2], const T* const (&b_row)[NB][2], int k0, int K) {
-    const int seg = threadIdx.x & 7;
-    const int k = k0 + seg * VEC;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      staged[0][j] = (a_row[j] && k < K) ? *reinterpret_cast<const vec_t*>(a_row[j] + k) : Atom<T>::zero();
-#pragma unroll
-      for (int m = 0; m < NB; ++m)
-        staged[1 + m][j] = (b_row[m][j] && k < K) ? *reinterpret_cast<const vec_t*>(b_row[m][j] + k) : Atom<T>::zero();
-    }
+  // row and column of this lane's outputs acc[i][j][0..3] inside the workgroup's tile
+  static __device__ __forceinline__ int row_of(int j) { return ((threadIdx.x >> 8) & 1) * 32 + j * 16 + (threadIdx.x & 15); }
+  static __device__ __forceinline__ int weight_of(int i) {
+    const int w4 = (threadIdx.x >> 6) & 3;
+    return PAIRED ? i * 64 + w4 * 16 : w4 * 32 + i * 16;
   }
-  __device__ __forceinline__ void store(char* lds) {
-    const int row = threadIdx.x >> 3, seg = threadIdx.x & 7;
-#pragma unroll
-    for (int m = 0; m < 1 + NB; ++m)
+
+  // x_off: this lane's row of X (row wave * 8 + lane / 8 of the tile) from the start of its buffer, in bytes; w0, w1: the
+  // buffers of the first and the second 64 weight rows, rows of K elements
+  __device__ __forceinline__ void run(u32x4_t x, unsigned x_off, u32x4_t w0, u32x4_t w1, int K, unsigned char* ring) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row16 = lane & 15, g = lane >> 4;
+    const unsigned piece = ((lane & 7) ^ (lane >> 3)) * 16;
+    x_off += piece;
+    const unsigned w_off = (unsigned)((wave * 8 + (lane >> 3)) * (long)K * sizeof(T)) + piece;
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) void*)ring + wave * 1024;
+    const int stages = (K + BK - 1) / BK;
+    auto request = [&](int st, int buf) LS_INLINED {
+      buffer_to_lds16(x_off, st * 128, x, lds0 + S * W_BYTES + buf * X_BYTES);
+      buffer_to_lds16(w_off, st * 128, w0, lds0 + buf * W_BYTES);
+      buffer_to_lds16(w_off, st * 128, w1, lds0 + buf * W_BYTES + 64 * 128);
+    };
+    auto clear_past_k = [&](int buf) LS_INLINED {
+      const int first = (K % BK) / Atom<T>::VEC;  // the first piece of a row that lies past K
+      for (int idx = threadIdx.x; idx < (kRingWeights + kRingRows) * 8; idx += 512) {
+        const int row = idx >> 3;
+        if (((idx & 7) ^ (row & 7)) < first) continue;
+        unsigned char* at = row < kRingWeights ? ring + buf * W_BYTES + idx * 16
+                                               : ring + S * W_BYTES + buf * X_BYTES + (idx - kRingWeights * 8) * 16;
+        *reinterpret_cast<vec_t*>(at) = Atom<T>::zero();
+      }
+      ring_barrier();
+    };
+    const unsigned at = row16 * 128 + ((g ^ (row16 & 7)) << 4);
+    const int wm = ((wave >> 2) & 1) * 32;
+    vec_t a[2], b[2][2];
+    auto read_a = [&](int i, int buf, int c) LS_INLINED {
+      a[i] = *reinterpret_cast<const vec_t*>(ring + buf * W_BYTES + weight_of(i) * 128 + (at ^ (c * 64)));
+    };
+    auto read_b = [&](vec_t (&dst)[2], int buf, int c) LS_INLINED {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        *reinterpret_cast<vec_t*>(lds + ((m * 64) + row + 32 * j) * kLdsRow + seg * 16) = staged[m][j];
-  }
-  __device__ __forceinline__ void multiply(const char* lds) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int l16 = lane & 15, quad = lane >> 4, wr = w >> 1, wc = w & 1;
+        dst[j] = *reinterpret_cast<const vec_t*>(ring + S * W_BYTES + buf * X_BYTES + (wm + j * 16) * 128 + (at ^ (c * 64)));
+    };
+    auto multiply = [&](const vec_t (&mine)[2], vec_t (&next)[2], int buf, int c) LS_INLINED {
+      read_b(next, buf, c);
 #pragma unroll
-    for (int c = 0; c < kStageBytes / 64; ++c) {
-      vec_t a[2], b[NB][2];
+      for (int i = 0; i < 2; ++i) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        a[t] = *reinterpret_cast<const vec_t*>(lds + (wr * 32 + t * 16 + l16) * kLdsRow + c * 64 + quad * 16);
-#pragma unroll
-        for (int m = 0; m < NB; ++m)
-          b[m][t] = *reinterpret_cast<const vec_t*>(lds + ((1 + m) * 64 + wc * 32 + t * 16 + l16) * kLdsRow + c * 64 + quad * 16);
+        for (int j = 0; j < 2; ++j) Atom<T>::mma(acc[i][j], a[i], mine[j]);
+        read_a(i, buf, c);
       }
+    };
 #pragma unroll
-      for (int m = 0; m < NB; ++m)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int ct = 0; ct < 2; ++ct) Atom<T>::mma(acc[m][rt][ct], b[m][ct], a[rt]);
-    }
-  }
-  __device__ __forceinline__ void run(const T* const (&a_row)[2], const T* const (&b_row)[NB][2], int K, char* lds) {
-#pragma unroll
-    for (int m = 0; m < NB; ++m)
-#pragma unroll
-      for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) acc[m][rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int kBuffer = (1 + NB) * 64 * kLdsRow;
-    const int stages = (K + kStageK - 1) / kStageK;
-    request(a_row, b_row, 0, K);
-    store(lds);
-    __syncthreads();
-    for (int s = 0; s < stages; ++s) {
-      if (s + 1 < stages) request(a_row, b_row, (s + 1) * kStageK, K);
-      multiply(lds + (s & 1) * kBuffer);
-      if (s + 1 < stages) store(lds + ((s + 1) & 1) * kBuffer);
-      __syncthreads();
+    for (int s = 0; s < S; ++s)
+      if (s < stages) request(s, s);
+    if (stages >= S) wait_loads<(S - 1) * LOADS>(); else wait_loads<0>();
+    ring_barrier();
+    if (K % BK && stages == 1) clear_past_k(0);
+    read_b(b[0], 0, 0);
+    read_a(0, 0, 0);
+    read_a(1, 0, 0);
+    int buf = 0;
+    for (int st = 0; st < stages; ++st) {
+      multiply(b[0], b[1], buf, 1);
+      if (st + S > stages) wait_loads<0>(); else wait_loads<(S - 2) * LOADS>();  // stage st + 1 is there
+      ring_barrier();                                                            // ... for everyone, and stage st is read
+      if (st + S < stages) request(st + S, buf);
+      buf = buf + 1 == S ? 0 : buf + 1;
+      if (K % BK && st + 2 == stages) clear_past_k(buf);
+      multiply(b[1], b[0], buf, 0);
     }
   }
 };
 
 template <typename T>
-__global__ __launch_bounds__(256) void experts_gate_up_tiled_kernel(const T* __restrict__ x, long ldx,
-                                                                    const T* __restrict__ w_gate,
-                                                                    const T* __restrict__ w_up, int F, int K, int top,
-                                                                    const int* __restrict__ order,
-                                                                    const int* __restrict__ tiles, float limit, float alpha,
-                                                                    float shift, const float* __restrict__ in_weight,
-                                                                    T* __restrict__ act, long ldy, int real) {
-  __shared__ __attribute__((aligned(16))) char lds[2 * 3 * 64 * kLdsRow];
-  const int e = tiles[4 * blockIdx.x];
+__global__ __launch_bounds__(512) void experts_gate_up_ring_kernel(const T* __restrict__ x, long ldx,
+                                                                   const T* __restrict__ w_gate,
+                                                                   const T* __restrict__ w_up, int F, int K, int top,
+                                                                   const int* __restrict__ order,
+                                                                   const int* __restrict__ tiles, float limit, float alpha,
+                                                                   float shift, const float* __restrict__ in_weight,
+                                                                   T* __restrict__ act, long ldy, int real, int n_tokens) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
+  const int tile = blockIdx.y;
+  const int e = tiles[4 * tile];
   if (e < 0 || e >= real) return;
-  const int first = tiles[4 * blockIdx.x + 1], rows = tiles[4 * blockIdx.x + 2];
-  const int col0 = blockIdx.y * 64;
-  const T* a_row[2];
-  const T* b_row[2][2];
+  const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
+  const int col0 = blockIdx.x * 64;
+  const int mine = min((int)(threadIdx.x >> 3), rows - 1);  // (rows past the tile's: the last one again, not stored)
+  const long left = (long)(F - col0) * K * sizeof(T), from = ((long)e * F + col0) * K;
+  RingProduct<T, true> product;
+  product.run(buffer_of(x, ((long)(n_tokens - 1) * ldx + K) * sizeof(T)), (unsigned)((long)(order[first + mine] / top) * ldx * sizeof(T)),
+              buffer_of(w_gate + from, left), buffer_of(w_up + from, left), K, ring);
+  const int quad = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int r = (threadIdx.x >> 3) + 32 * j;
-    a_row[j] = r < rows ? x + (long)(order[first + r] / top) * ldx : nullptr;
-    b_row[0][j] = col0 + r < F ? w_gate + ((long)e * F + col0 + r) * K : nullptr;
-    b_row[1][j] = col0 + r < F ? w_up + ((long)e * F + col0 + r) * K : nullptr;
-  }
-  TiledProduct<T, 2> product;
-  product.run(a_row, b_row, K, lds);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int l16 = lane & 15, quad = lane >> 4, wr = w >> 1, wc = w & 1;
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int r = wr * 32 + rt * 16 + l16;
+    const int r = product.row_of(j);
     if (r >= rows) continue;
     T* dst = act + (long)(first + r) * ldy;
     const float wt = in_weight ? in_weight[order[first + r]] : 1.0f;
+    const int c0 = col0 + product.weight_of(0) + 4 * quad;
+    float y[4];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int i = 0; i < 4; ++i) {
+      const float g = fminf(product.acc[0][j][i] * wt, limit);
+      const float u = fminf(fmaxf(product.acc[1][j][i] * wt, -limit), limit);
+      y[i] = (g * sigmoid_e(alpha * g)) * (u + shift);
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = col0 + wc * 32 + ct * 16 + 4 * quad + i;
-        if (c < F) {
-          const float g = fminf(product.acc[0][rt][ct][i] * wt, limit);
-          const float u = fminf(fmaxf(product.acc[1][rt][ct][i] * wt, -limit), limit);
-          dst[c] = from_f32<T>((g * sigmoid_e(alpha * g)) * (u + shift));
-        }
-      }
+    for (int i = 0; i < 4; ++i)
+      if (c0 + i < F) dst[c0 + i] = from_f32<T>(y[i]);
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void experts_down_tiled_kernel(const T* __restrict__ act, long ldy,
-                                                                 const T* __restrict__ w_down, int N, int F, int top,
-                                                                 int n_tokens, const int* __restrict__ order,
-                                                                 const int* __restrict__ tiles,
-                                                                 const float* __restrict__ weight, float* __restrict__ P,
-                                                                 const T* __restrict__ x, long ldx,
-                                                                 const float* __restrict__ share, int real) {
-  __shared__ __attribute__((aligned(16))) char lds[2 * 2 * 64 * kLdsRow];
-  const int e = tiles[4 * blockIdx.x];
+__global__ __launch_bounds__(512) void experts_down_ring_kernel(const T* __restrict__ act, long ldy,
+                                                                const T* __restrict__ w_down, int N, int F, int top,
+                                                                int n_tokens, const int* __restrict__ order,
+                                                                const int* __restrict__ tiles,
+                                                                const float* __restrict__ weight, float* __restrict__ P,
+                                                                const T* __restrict__ x, long ldx,
+                                                                const float* __restrict__ share, int real) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
+  const int tile = blockIdx.y;
+  const int e = tiles[4 * tile];
   if (e < 0) return;
-  const int first = tiles[4 * blockIdx.x + 1], rows = tiles[4 * blockIdx.x + 2];
-  const int col0 = blockIdx.y * 64;
+  const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
+  const int col0 = blockIdx.x * 128;
   if (e >= real) {
-    pass_input<T>(x, ldx, share, first, rows, col0, min(N, col0 + 64), top, n_tokens, N, order, P);
+    pass_input<T>(x, ldx, share, first, rows, col0, min(N, col0 + 128), top, n_tokens, N, order, P);
     return;
   }
-  const T* a_row[2];
-  const T* b_row[1][2];
+  const int mine = min((int)(threadIdx.x >> 3), rows - 1);
+  const T* from = w_down + ((long)e * N + col0) * F;
+  const long left = (long)(N - col0) * F * sizeof(T), half = 64L * F * sizeof(T);
+  RingProduct<T, false> product;
+  product.run(buffer_of(act + (long)first * ldy, ((long)(rows - 1) * ldy + F) * sizeof(T)), (unsigned)(mine * ldy * sizeof(T)),
+              buffer_of(from, left), buffer_of(from + 64L * F, left > half ? left - half : 0), F, ring);
+  const int quad = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int r = (threadIdx.x >> 3) + 32 * j;
-    a_row[j] = r < rows ? act + (long)(first + r) * ldy : nullptr;
-    b_row[0][j] = col0 + r < N ? w_down + ((long)e * N + col0 + r) * F : nullptr;
-  }
-  TiledProduct<T, 1> product;
-  product.run(a_row, b_row, F, lds);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int l16 = lane & 15, quad = lane >> 4, wr = w >> 1, wc = w & 1;
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int r = wr * 32 + rt * 16 + l16;
+    const int r = product.row_of(j);
     if (r >= rows) continue;
     const int pair = order[first + r];
-    const float share = weight ? weight[pair] : 1.0f;
+    const float wt = weight ? weight[pair] : 1.0f;
     float* dst = P + ((long)(pair % top) * n_tokens + pair / top) * N;
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int i = 0; i < 2; ++i) {
+      const int c0 = col0 + product.weight_of(i) + 4 * quad;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = col0 + wc * 32 + ct * 16 + 4 * quad + i;
-        if (c < N) dst[c] = share * product.acc[0][rt][ct][i];
-      }
+      for (int q = 0; q < 4; ++q)
+        if (c0 + q < N) dst[c0 + q] = wt * product.acc[i][j][q];
+    }
   }
 }
 
@@ -751,6 +762,19 @@ LS_DEFINE_ERROR_API
 using namespace ls;
 
 extern "C" int ls_experts_max_top() { return kMaxTop; }
+
+// Dynamic LDS beyond 64 KB has to be granted per kernel (once).
+static bool ring_lds_ready(int dtype) {
+  auto grant = [](const void* kernel) {
+    const bool ok = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    return ok;
+  };
+  static const bool granted[2] = {
+      grant((const void*)&experts_gate_up_ring_kernel<float>) && grant((const void*)&experts_down_ring_kernel<float>),
+      grant((const void*)&experts_gate_up_ring_kernel<bf16_t>) && grant((const void*)&experts_down_ring_kernel<bf16_t>)};
+  return granted[dtype == kF32 ? 0 : 1];
+}
 
 // Tiles that the pairs of n_tokens tokens can need at most, with rows_a_tile rows each.
 extern "C" int ls_experts_tile_capacity(int n_tokens, int E, int top, int rows_a_tile) {
@@ -902,15 +926,18 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
                        (const T_*)w_down, N, F, top, n_tokens, order, tiles, out_weight, P, (const T_*)x, ldx, weight, real, \
                        shared_of((T_*)nullptr));                                                                      \
   } while (0)
-  // tiles of 64 rows go through LDS where every row of every operand starts on a 16-byte boundary
-  const bool staged = rows_a_tile == 64 && K % vec == 0 && F % vec == 0 && ldx % vec == 0 && ldy % vec == 0;
+  // tiles of 64 rows go through LDS where every row of every operand starts on a 16-byte boundary (and an offset into x
+  // fits 32 bits, and the tiles a grid's second dimension)
+  const bool staged = rows_a_tile == 64 && K % vec == 0 && F % vec == 0 && ldx % vec == 0 && ldy % vec == 0 &&
+                      (long)n_tokens * ldx < (1L << 29) && cap < 65536 && ring_lds_ready(dtype);
 #define LS_EXPERTS_STAGED(T_)                                                                                         \
   do {                                                                                                                \
-    hipLaunchKernelGGL(experts_gate_up_tiled_kernel<T_>, grid_up, dim3(256), 0, s, (const T_*)x, ldx,                 \
-                       (const T_*)w_gate, (const T_*)w_up, F, K, top, order, tiles, limit, alpha, shift, in_weight,   \
-                       (T_*)act, ldy, real);                                                                          \
-    hipLaunchKernelGGL(experts_down_tiled_kernel<T_>, grid_down, dim3(256), 0, s, (const T_*)act, ldy,                \
-                       (const T_*)w_down, N, F, top, n_tokens, order, tiles, out_weight, P, (const T_*)x, ldx, weight, real); \
+    hipLaunchKernelGGL(experts_gate_up_ring_kernel<T_>, dim3((F + 63) / 64, cap), dim3(512), kRingLds, s, (const T_*)x, \
+                       ldx, (const T_*)w_gate, (const T_*)w_up, F, K, top, order, tiles, limit, alpha, shift, in_weight, \
+                       (T_*)act, ldy, real, n_tokens);                                                                  \
+    hipLaunchKernelGGL(experts_down_ring_kernel<T_>, dim3((N + 127) / 128, cap), dim3(512), kRingLds, s,             \
+                       (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, out_weight, P,      \
+                       (const T_*)x, ldx, weight, real);                                                              \
   } while (0)
 #define LS_EXPERTS_BY_ROWS(T_)                 \
   switch (rows_a_tile) {                       \

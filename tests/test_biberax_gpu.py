@@ -305,6 +305,35 @@ def test_routing_and_the_experts_products(dtype, tokens, experts, top, width, ff
                 want[t] += s * plain.bounded_gated_unit(x[t:t + 1].double(), full, f"m.e{e}", 1.3)[0]
         assert rel_err(partials.sum(0).cpu(), want) < (2e-6 if dtype is torch.float32 else 2e-2), rows
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width, ff", [(8, 8), (64, 72), (72, 128), (136, 200), (1032, 264)])
+def test_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
+    """The products of row tiles of 64 read both operands through LDS, those of 32 rows from memory, and both are one
+    chain over K: experts with 1, 63, 64, 65 and 130 tokens and none, edges of the tile in rows and columns, contractions
+    that end inside a stage."""
+    g = torch.Generator().manual_seed(width + ff)
+    k = K()
+    sizes = [1, 63, 0, 64, 65, 130]
+    tokens, experts = sum(sizes), len(sizes)
+    owner = torch.repeat_interleave(torch.arange(experts), torch.tensor(sizes))[torch.randperm(tokens, generator=g)]
+    logits = torch.zeros(tokens, experts)
+    logits[torch.arange(tokens), owner] = 9.0
+    x = torch.randn(tokens, width, generator=g).to(dtype).cuda()
+    gate, up, down = ((torch.randn(experts, *shape, generator=g) * 0.3).to(dtype).cuda() for shape in ((ff, width), (ff, width), (width, ff)))
+    results = []
+    for rows in (32, 64):
+        cap = k.experts_tile_capacity(tokens, experts, 1, rows)
+        i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+        chosen, order, tiles, counts = i32(tokens), i32(tokens), i32(4 * cap), i32(experts)
+        share = torch.empty(tokens, device="cuda")
+        k.experts_route(logits.cuda(), torch.zeros(experts).cuda(), 1, rows, chosen, share, order, tiles, counts)
+        act = torch.full((tokens, ff), float("nan"), dtype=dtype, device="cuda")
+        partials = torch.full((1, tokens, width), float("nan"), device="cuda")
+        k.experts_apply(x, gate, up, down, 1, rows, order, tiles, share, 1.3, 1.702, act, partials)
+        results.append((act, partials))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert not torch.isnan(results[1][1]).any()
+
 
 # ---------------------------------------------------------------------------
 # one-layer models of each mechanism, then whole models
