@@ -424,96 +424,141 @@ __device__ __forceinline__ float lanes_sum(float v) {
 
 // R rows a lane, L lanes a column (R * L rows, the head size rounded up), 64 / L columns a wave.  CH: the decay is a
 // number a row of the state (decays [T][H][dp]) instead of one a head: S[r] <- g[r] S[r] first, then the rule as stated.
-template <int R, int L, bool CH>
+//
+// What bounds a long request is the instructions of one wave (a head of 128 x 128 is 32 waves, sixteen heads half of the
+// card's SIMDs), so a token carries its arithmetic and little else: operands come by buffer loads whose lane offsets
+// never change and whose scalar offset is the token's place in its block of DEPTH; a block moves the bases once; lanes
+// and columns past the state have an offset past the buffer's end, which reads as zero and is not written, in place of
+// branches; only the blocks whose requests would leave the request hold them at its last token.  beta and the decay come
+// by one vector load at the same address in every lane (as scalar loads, which return in any order, a wait for one would
+// be a wait for all, also for those of the tokens ahead).
+// DEPTH: the tokens whose operands are on their way.  2,048 tokens (16 heads over 8, 128 x 128): 270 us; with lane
+// pointers, a conditional step of each, and a branch a token it took 490.  Where requests bring a token or two, two are
+// enough and leave room for twice the waves: eight requests decoding 28 -> 13 us.
+template <int R, int L, bool CH, int DEPTH>
 __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict__ qk, const float* __restrict__ vv,
                                                         const float* __restrict__ gates, const float* __restrict__ decays,
                                                         int G, int H, int D, int DV,
                                                         const SeqMeta* __restrict__ seqs, float* __restrict__ state,
                                                         long state_stride, float* __restrict__ out, long ldo) {
+  typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
+  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
   constexpr int dp = L * R, COLS = 64 / L;
+  constexpr int kNowhere = 0x7ffffff0;  // an offset past every buffer's end
   const int seq = blockIdx.x / H, head = blockIdx.x % H;
   const SeqMeta m = seqs[seq];
-  if (m.q_len <= 0) return;
+  const int n = m.q_len;
+  if (n <= 0) return;
   const int lane = threadIdx.x, lc = lane / L, part = lane % L;
   const int col = blockIdx.y * COLS + lc;
   const bool col_ok = col < DV;
   const int row0 = part * R;
   const int kh = head / (H / G);
-  float* mine = state + (long)m.table_row * state_stride + (long)head * D * DV;
+  auto buffer = [](const float* p, int bytes) LS_INLINED {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, bytes, 0x00020000);
+  };
+  const auto mine = buffer(state + (long)m.table_row * state_stride + (long)head * D * DV, D * DV * 4);
+  int s_off[R];
   float S[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) S[r] = (row0 + r < D && col_ok) ? mine[(long)(row0 + r) * DV + col] : 0.f;
+  for (int r = 0; r < R; ++r) s_off[r] = row0 + r < D && col_ok ? ((row0 + r) * DV + col) * 4 : kNowhere;
+#pragma unroll
+  for (int r = 0; r < R; ++r) S[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(mine, s_off[r], 0, 0));
   struct Operands {
-    f32x4 q[R / 4], k[R / 4], g[CH ? R / 4 : 1];
-    float v, gate;   // gate: beta in the even lanes, the decay in the odd ones
+    u32x4_t q[R / 4], k[R / 4], g[CH ? R / 4 : 1];
+    unsigned v;
+    u32x2_t gate;  // beta, decay
   };
-  // Pointers to the operands of the token that is requested next; they move on by a token after every request and
-  // stay on the request's last token (no index arithmetic and no branch between the requests).  beta and the decay
-  // are fetched by the lanes (even: beta, odd: decay) and handed round inside the quad: a load whose address is
-  // the same in every lane would go through the scalar cache, whose loads return in any order, so that a wait for
-  // one of them waits for all, also for those of the tokens ahead.
-  const float* q_at = qk + ((long)m.q_off * 2 * G + kh) * dp + row0;
-  const float* k_at = q_at + (long)G * dp;
-  const float* v_at = vv + (long)m.q_off * H * DV + head * DV + (col_ok ? col : 0);
-  const float* g_at = gates + ((long)m.q_off * H + head) * 2 + (lane & 1);
-  const float* d_at = CH ? decays + ((long)m.q_off * H + head) * dp + row0 : nullptr;
-  int left = m.q_len - 1;   // tokens behind the one the pointers stand on
-  auto fetch = [&]() LS_INLINED {
-    Operands x;
+  // the first token of the block, and bytes from a token to the next
+  const float* qk_at = qk + ((long)m.q_off * 2 * G + kh) * dp;
+  const float* v_at = vv + (long)m.q_off * H * DV + head * DV;
+  const float* g_at = gates + ((long)m.q_off * H + head) * 2;
+  const float* d_at = CH ? decays + ((long)m.q_off * H + head) * dp : nullptr;
+  float* o_at = out + (long)m.q_off * ldo + head * DV;
+  const int qk_step = 2 * G * dp * 4, v_step = H * DV * 4, g_step = H * 8, d_step = H * dp * 4, o_step = (int)ldo * 4;
+  const int q_off = row0 * 4, k_off = (G * dp + row0) * 4, v_off = (col_ok ? col : 0) * 4;
+  const int o_off = part == 0 && col_ok ? col * 4 : kNowhere;
+  int zero = 0;
+  __asm__("" : "+v"(zero));
+  Operands ring[DEPTH];
+  auto fetch = [&](Operands& x, auto qkb, auto vb, auto gb, auto db, int t) LS_INLINED {  // the token t tokens from the block's first
 #pragma unroll
     for (int j = 0; j < R / 4; ++j) {
-      x.q[j] = *reinterpret_cast<const f32x4*>(q_at + 4 * j);
-      x.k[j] = *reinterpret_cast<const f32x4*>(k_at + 4 * j);
-      if constexpr (CH) x.g[j] = *reinterpret_cast<const f32x4*>(d_at + 4 * j);
+      x.k[j] = __builtin_amdgcn_raw_buffer_load_b128(qkb, k_off + 16 * j, t * qk_step, 0);
+      x.q[j] = __builtin_amdgcn_raw_buffer_load_b128(qkb, q_off + 16 * j, t * qk_step, 0);
+      if constexpr (CH) x.g[j] = __builtin_amdgcn_raw_buffer_load_b128(db, q_off + 16 * j, t * d_step, 0);
     }
-    x.v = *v_at;
-    x.gate = *g_at;
-    const long step = left > 0 ? 1 : 0;
-    left -= (int)step;
-    q_at += step * 2 * G * dp;
-    k_at += step * 2 * G * dp;
-    v_at += step * H * DV;
-    g_at += step * H * 2;
-    if constexpr (CH) d_at += step * H * dp;
-    return x;
+    x.v = __builtin_amdgcn_raw_buffer_load_b32(vb, v_off, t * v_step, 0);
+    x.gate = __builtin_amdgcn_raw_buffer_load_b64(gb, zero, t * g_step, 0);
   };
-  // the operands of the token DEPTH tokens on are requested before a token is worked on (a ring of registers)
-  constexpr int DEPTH = (R <= 8 && !CH) ? 8 : 4;
-  Operands ring[DEPTH];
+  float o4[4] = {};  // the lane's part of the output of the token that was worked on last
+  auto token = [&](const Operands& now) LS_INLINED {
+    auto of = [](const u32x4_t (&x)[R / 4], int r) LS_INLINED { return __uint_as_float(x[r >> 2][r & 3]); };
+    const float beta = __uint_as_float(now.gate[0]), decay = __uint_as_float(now.gate[1]);
+    // a lane's rows in four interleaved chains (rows r, r + 4, ... of each), added as (0 + 1) + (2 + 3)
+    float ks4[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (CH) {
 #pragma unroll
-  for (int j = 0; j < DEPTH; ++j) ring[j] = fetch();
-  for (int i0 = 0; i0 < m.q_len; i0 += DEPTH) {
+      for (int r = 0; r < R; ++r) S[r] = S[r] * __uint_as_float(now.g[r >> 2][r & 3]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) ks4[r & 3] = fmaf(S[r], of(now.k, r), ks4[r & 3]);
+    const float ks = lanes_sum<L>((ks4[0] + ks4[1]) + (ks4[2] + ks4[3])) * (CH ? 1.0f : decay);
+    const float u = beta * (__uint_as_float(now.v) - ks);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o4[i] = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      S[r] = fmaf(of(now.k, r), u, CH ? S[r] : decay * S[r]);
+      o4[r & 3] = fmaf(S[r], of(now.q, r), o4[r & 3]);
+    }
+  };
+  auto put = [&](auto ob, float o, int j) LS_INLINED {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), ob, o_off, j * o_step, 0);
+  };
+  {
+    const auto qkb = buffer(qk_at, kNowhere), vb = buffer(v_at, kNowhere), gb = buffer(g_at, kNowhere), db = buffer(d_at, kNowhere);
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) fetch(ring[j], qkb, vb, gb, db, min(j, n - 1));
+  }
+  auto next_block = [&]() LS_INLINED {
+    qk_at += (long)DEPTH * 2 * G * dp;
+    v_at += (long)DEPTH * H * DV;
+    g_at += (long)DEPTH * H * 2;
+    if constexpr (CH) d_at += (long)DEPTH * H * dp;
+    o_at += (long)DEPTH * ldo;
+  };
+  int i0 = 0;
+  for (; i0 + 2 * DEPTH <= n; i0 += DEPTH) {
+    const auto qkb = buffer(qk_at, kNowhere), vb = buffer(v_at, kNowhere), gb = buffer(g_at, kNowhere), db = buffer(d_at, kNowhere);
+    const auto ob = buffer(o_at, kNowhere);
+    // a token's output is added up beside the next token's products: each is a chain that waits for itself
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) {
-      const int i = i0 + j;
-      if (i >= m.q_len) break;
-      const Operands now = ring[j];
-      ring[j] = fetch();
-      const float beta = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(now.gate), 0x00, 0xF, 0xF, true));   // lane 0 of the quad
-      const float decay = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(now.gate), 0x55, 0xF, 0xF, true));  // lane 1
-      // a lane's rows in four interleaved chains (rows r, r + 4, ... of each), added as (0 + 1) + (2 + 3)
-      float ks4[4] = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (CH) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) S[r] = S[r] * now.g[r >> 2][r & 3];
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r) ks4[r & 3] = fmaf(S[r], now.k[r >> 2][r & 3], ks4[r & 3]);
-      const float ks = lanes_sum<L>((ks4[0] + ks4[1]) + (ks4[2] + ks4[3])) * (CH ? 1.0f : decay);
-      const float u = beta * (now.v - ks);
-      float o4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        S[r] = fmaf(now.k[r >> 2][r & 3], u, CH ? S[r] : decay * S[r]);
-        o4[r & 3] = fmaf(S[r], now.q[r >> 2][r & 3], o4[r & 3]);
-      }
-      const float o = lanes_sum<L>((o4[0] + o4[1]) + (o4[2] + o4[3]));
-      if (part == 0 && col_ok) out[(long)(m.q_off + i) * ldo + head * DV + col] = o;
+      const float before = (o4[0] + o4[1]) + (o4[2] + o4[3]);
+      token(ring[j]);
+      if (j > 0) put(ob, lanes_sum<L>(before), j - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(ring[j], qkb, vb, gb, db, DEPTH + j);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    put(ob, lanes_sum<L>((o4[0] + o4[1]) + (o4[2] + o4[3])), DEPTH - 1);
+    next_block();
+  }
+  for (; i0 < n; i0 += DEPTH) {
+    const auto qkb = buffer(qk_at, kNowhere), vb = buffer(v_at, kNowhere), gb = buffer(g_at, kNowhere), db = buffer(d_at, kNowhere);
+    const auto ob = buffer(o_at, kNowhere);
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) {
+      if (i0 + j >= n) break;
+      token(ring[j]);
+      put(ob, lanes_sum<L>((o4[0] + o4[1]) + (o4[2] + o4[3])), j);
+      if (i0 + DEPTH + j < n) fetch(ring[j], qkb, vb, gb, db, DEPTH + j);
+    }
+    next_block();
   }
 #pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (row0 + r < D && col_ok) mine[(long)(row0 + r) * DV + col] = S[r];
+  for (int r = 0; r < R; ++r) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[r]), mine, s_off[r], 0, 0);
 }
 
 __global__ __launch_bounds__(256) void delta_conv_state_kernel(const float* __restrict__ raw, long ld, int C, int M,
@@ -685,6 +730,7 @@ extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int
   LS_REQUIRE(raw && taps && a_log && dt_bias && tok_seq && tok_pos && seqs && state && scratch && out,
              "delta_rule: null operand");
   LS_REQUIRE(reinterpret_cast<uintptr_t>(scratch) % 16 == 0, "delta_rule: the scratch must be 16-byte aligned");
+  LS_REQUIRE(n_tokens == 1 || ldo < (1L << 26), "delta_rule: rows of the output are too far apart");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int dp = ls_delta_padded_dim(D);
   float* qk = scratch;
@@ -695,14 +741,18 @@ extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int
   hipLaunchKernelGGL(delta_prep_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, raw, ld, n_tokens, G, H, D, DV,
                      dp, M, taps, a_log, dt_bias, unit_eps, tok_seq, tok_pos, (const SeqMeta*)seqs, state, state_stride,
                      conv_at, qk, vv, gates, chan, ldc, decays);
-#define LS_DELTA(R_, L_)                                                                                              \
-  do {                                                                                                                \
-    if (chan)                                                                                                         \
-      hipLaunchKernelGGL((delta_rule_kernel<R_, L_, true>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
-                         gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo);            \
-    else                                                                                                              \
-      hipLaunchKernelGGL((delta_rule_kernel<R_, L_, false>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
-                         gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo);            \
+#define LS_DELTA_RULE(R_, L_, CH_, DEPTH_)                                                                               \
+  hipLaunchKernelGGL((delta_rule_kernel<R_, L_, CH_, DEPTH_>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
+                     gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo)
+#define LS_DELTA(R_, L_)                                                          \
+  do {                                                                            \
+    if (n_tokens <= 2 * n_seqs) {                                                 \
+      if (chan) LS_DELTA_RULE(R_, L_, true, 2); else LS_DELTA_RULE(R_, L_, false, 2); \
+    } else if (chan) {                                                            \
+      LS_DELTA_RULE(R_, L_, true, 4);                                             \
+    } else {                                                                      \
+      LS_DELTA_RULE(R_, L_, false, R_ <= 8 ? 8 : 4);                              \
+    }                                                                             \
   } while (0)
   switch (dp) {
     case 16: LS_DELTA(4, 4); break;
@@ -712,6 +762,7 @@ extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int
     default: LS_DELTA(16, 16); break;
   }
 #undef LS_DELTA
+#undef LS_DELTA_RULE
   if (M > 1)
     hipLaunchKernelGGL(delta_conv_state_kernel, dim3(n_seqs, (unsigned)((C + 255) / 256)), dim3(256), 0, s, raw, ld, (int)C,
                        M, (const SeqMeta*)seqs, state, state_stride, conv_at);

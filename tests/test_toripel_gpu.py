@@ -233,6 +233,46 @@ def test_the_delta_rule_with_its_convolutions_over_unequal_requests_in_steps(hea
         assert close(torch.cat(got[s]), want[s], torch.float32, scale=1e-2), s
 
 
+@pytest.mark.parametrize("heads, groups, d, dv", [(2, 1, 16, 17), (2, 2, 30, 5), (1, 1, 64, 64), (4, 2, 128, 20), (1, 1, 200, 9)])
+@pytest.mark.parametrize("channel_decays", [False, True])
+def test_the_delta_rule_has_the_same_bits_however_many_tokens_a_step_brings(heads, groups, d, dv, channel_decays):
+    """Requests of every length around the blocks of tokens whose operands are fetched together, all in one step, against
+    the same tokens one and two a step (which the kernel for few tokens a request takes)."""
+    lengths = [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 24, 31, 33]
+    g = torch.Generator().manual_seed(d + dv)
+    channels = 2 * groups * d + heads * dv
+    conv = (torch.randn((channels, 2), generator=g) * 0.5).cuda()
+    a_log = torch.randn(heads, generator=g).cuda()
+    dt_bias = torch.randn(heads * d if channel_decays else heads, generator=g).cuda()
+    raws = [torch.randn((n, channels + (1 if channel_decays else 2) * heads), generator=g).cuda() for n in lengths]
+    chans = [torch.randn((n, heads * d), generator=g).cuda() for n in lengths]
+    k = K()
+
+    def run(most):
+        state = torch.zeros((len(lengths), heads * d * dv + channels), dtype=torch.float32, device="cuda")
+        outs = [[] for _ in lengths]
+        for at in range(0, max(lengths), most):
+            who = [i for i, n in enumerate(lengths) if n > at]
+            counts = [min(most, lengths[i] - at) for i in who]
+            tok_seq, tok_pos, seqs = step_meta(counts, [at] * len(who), who)
+            raw = torch.cat([raws[i][at:at + n] for i, n in zip(who, counts)])
+            chan = torch.cat([chans[i][at:at + n] for i, n in zip(who, counts)]) if channel_decays else None
+            out = torch.full((raw.shape[0], heads * dv), float("nan"), dtype=torch.float32, device="cuda")
+            size = k.delta_scratch_floats(raw.shape[0], groups, heads, d, dv, channel_decays)
+            k.delta_rule(raw, groups, heads, d, dv, conv, a_log, dt_bias, 1e-6, tok_seq, tok_pos, seqs, len(who), state,
+                         torch.empty(size, dtype=torch.float32, device="cuda"), out, chan)
+            for i, part in zip(who, out.split(counts)):
+                outs[i].append(part)
+        return [torch.cat(o) for o in outs], state
+
+    whole, state = run(max(lengths))
+    assert not torch.isnan(state).any()
+    for most in (1, 2):
+        outs, after = run(most)
+        assert torch.equal(after, state), most
+        assert all(torch.equal(a, b) for a, b in zip(outs, whole)), most
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("tokens, experts, top, width, ff", [(1, 4, 2, 32, 24), (37, 7, 3, 64, 40), (300, 5, 1, 48, 16),
                                                               (700, 3, 3, 32, 8)])
