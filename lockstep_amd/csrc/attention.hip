@@ -1297,19 +1297,20 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
   long long pr_last = clock64();
   const long long pr_begin = pr_last;
 #endif
+  const int item_at = SPANS ? blockIdx.y : blockIdx.x;  // (see the launch)
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   // The item is the same for every lane: its fields go to scalar registers, so that what follows from them
   // (tile range, addresses, branch conditions) is scalar work too.
   AttnItem item;
   {
-    const int* src = reinterpret_cast<const int*>(items + blockIdx.x);
+    const int* src = reinterpret_cast<const int*>(items + item_at);
     int* dst = reinterpret_cast<int*>(&item);
 #pragma unroll
     for (int i = 0; i < 16; ++i) dst[i] = __builtin_amdgcn_readfirstlane(src[i]);
   }
   // the page ids an item of one tile brings, one a thread, requested together with the item itself
-  const int own_page = FUSE ? items[blockIdx.x].pages[threadIdx.x & 15] : 0;
+  const int own_page = FUSE ? items[item_at].pages[threadIdx.x & 15] : 0;
   if (FUSE) {
     // every other argument is requested now, while the item is on its way: left to themselves their loads
     // stand where each is first used, each with a wait of its own for memory that no cache holds yet
@@ -1318,7 +1319,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
                      "s"(fz.v_out), "s"(out), "s"(ldo), "s"(table), "s"(table_stride));
   }
   const SeqMeta sm = item.sm;
-  const int kvh = blockIdx.y;
+  const int kvh = SPANS ? blockIdx.x : blockIdx.y;
   const int rows_total = sm.q_len * G;  // <= 16, checked on the host
   const int row16 = lane & 15;
   const int g = lane >> 4;
@@ -1552,7 +1553,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
       // written when the instruction is issued).  Lanes and groups that need no operand load a spare address
       // and drop the result.
       const int vi = min(grp, n_vec - 1);
-      const float* spare = reinterpret_cast<const float*>(items + blockIdx.x);  // 128 readable bytes
+      const float* spare = reinterpret_cast<const float*>(items + item_at);  // 128 readable bytes
       const T* src = head_src(vi) + (lane_in_head ? e0_head : 0);
       const float* weight = vi < G ? fz.q_weight : vi == G ? fz.k_weight : nullptr;
       const bool weighted = weight != nullptr && lane_in_head && grp < n_vec;
@@ -1889,7 +1890,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
   if (FUSE && owner) write_new_to_cache();
 #ifdef LS_ATTN_PROBE
   if (threadIdx.x == 0 && kvh == LS_ATTN_PROBE_KVH && part_ml != nullptr) {
-    long long* dst = reinterpret_cast<long long*>(part_ml + (1 << 20)) + blockIdx.x * 32;
+    long long* dst = reinterpret_cast<long long*>(part_ml + (1 << 20)) + item_at * 32;
     for (int i = 0; i < 12; ++i) dst[i] = pr_t[i];
     dst[12] = clock64() - pr_begin;
     dst[13] = ti_hi - ti_lo;
@@ -2296,6 +2297,7 @@ static bool coop_kernel_ready() {
 // where they fit; when the grid brings at least two workgroups per CU, with
 // one buffer instead, so that two workgroups share a CU and overlap each
 // other's loads.
+constexpr int kMaxGridY = 65535;
 #ifndef LS_COOP_CROWDED_FROM
 #define LS_COOP_CROWDED_FROM 512  // from this many workgroups on: one tile buffer each, two workgroups a CU
 #endif
@@ -2310,11 +2312,20 @@ static int launch_coop_as(dim3 grid, hipStream_t s, const void* q, long ldq, con
   // (more workgroups than CUs but fewer than two a CU would be two rounds of one a CU with two buffers; with one
   // buffer they all run together: 48 requests of 8 kv heads 2.37 -> see the measurements in the planner)
   const bool crowded = (long)grid.x * grid.y >= LS_COOP_CROWDED_FROM || (long)grid.x * grid.y > compute_units() || single_tile;
+  // Items of several splits (SPANS) differ in length: the kv heads are the fast dimension of the launch, so that the items
+  // start in their order, all heads of one before the next; the host lists the longest first, and the short ones fill
+  // the CUs that the long ones leave (with the items as the fast dimension the long ones of the last head started last: 64
+  // requests of 128 to 4,096 tokens, 8 kv heads in 112 items, 70.6 -> 67 us; cut finer or coarser it is the same, 65 to
+  // 68: 4.6 TB/s of keys and values).  Items of one split keep the items as the fast dimension: an item's record is then
+  // read through one L2 (one request of 512 tokens 7.75 us, with the heads first 8.0).
 #define LS_COOP(NBUF_)                                                                                              \
-  hipLaunchKernelGGL((attention_coop_kernel<T, NBUF_, FUSE, SPANS>), grid, dim3(256), (coop_kernel_lds<T, NBUF_>()), s, \
-                     (const AttnItem*)items, (const T*)q, ldq, fz.q_weight, fz.k_weight, fz.cos_table, fz.sin_table, G, \
-                     nkv, (const T*)k_pages, (const T*)v_pages, page_size, page_shift, table, table_stride,            \
-                     (const SeqMeta*)seqs, (T*)out, ldo, part_acc, part_ml, scale, window, fz)
+  for (int first = 0, n = SPANS ? kMaxGridY : (int)grid.x; first < (int)grid.x; first += n)                         \
+    hipLaunchKernelGGL((attention_coop_kernel<T, NBUF_, FUSE, SPANS>),                                              \
+                       SPANS ? dim3(grid.y, (int)grid.x - first < n ? (int)grid.x - first : n) : grid, dim3(256),   \
+                       (coop_kernel_lds<T, NBUF_>()), s, (const AttnItem*)items + first, (const T*)q, ldq, fz.q_weight, \
+                       fz.k_weight, fz.cos_table, fz.sin_table, G, nkv, (const T*)k_pages, (const T*)v_pages, page_size, \
+                       page_shift, table, table_stride, (const SeqMeta*)seqs, (T*)out, ldo, part_acc, part_ml, scale, \
+                       window, fz)
   if (BUFS == 2 && !(crowded && coop_kernel_ready<T, 1, FUSE, SPANS>())) {
     if (!coop_kernel_ready<T, 2, FUSE, SPANS>()) return fail("attention: the cooperative kernel does not fit into LDS");
     LS_COOP(2);

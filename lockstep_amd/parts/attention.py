@@ -214,6 +214,8 @@ def plan_attention(ctx, group_size: int, nkv: int, head_dim: int, window: int, o
                 last_pos = q_start + min((block + 1) * block_rows - 1, rows - 1) // group_size
                 begin = (max(0, first_pos - window + 1) // split) if window > 0 else 0
                 target.append((i, block, begin, last_pos // split + 1, -1, 0, 0, 0))
+    if span > 1:
+        coop.sort(key=lambda it: it[2] - it[3])   # the longest items start first: they decide when the launch ends
     if ctx.fixed_shape:
         # null work (request -1 here, an item of zeros on the device) up to a size that many steps share
         null_item, null_fold = (-1, 0, 0, 0, -1, 0, 0, 0), (-1, 0, 0, 0)
@@ -223,7 +225,7 @@ def plan_attention(ctx, group_size: int, nkv: int, head_dim: int, window: int, o
         part_rows = _round_up(part_rows, buckets=(), step=PART_ROWS_STEP) if part_rows else 0
     decode_fused = (coop_ok and not items and not wide and bool((ctx.q_len == 1).all())
                     and kernels.decode_fused_supported(head_dim, dtype, page_size))
-    # the longest row blocks first: they decide when the launch ends
+    # the longest row blocks first, as above
     wide.sort(key=lambda it: it[2] - it[3])
     spans = any(it[4] >= 0 and it[3] - it[2] > 1 for it in coop)
     single_tile = bool(coop) and all((it[3] - it[2]) * split <= tile for it in coop)
