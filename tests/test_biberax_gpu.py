@@ -305,6 +305,34 @@ def test_routing_and_the_experts_products(dtype, tokens, experts, top, width, ff
                 want[t] += s * plain.bounded_gated_unit(x[t:t + 1].double(), full, f"m.e{e}", 1.3)[0]
         assert rel_err(partials.sum(0).cpu(), want) < (2e-6 if dtype is torch.float32 else 2e-2), rows
 
+@pytest.mark.parametrize("pairs", [513, 1023, 1024, 1025, 4097, 8192])
+@pytest.mark.parametrize("experts", [2, 33, 512, 600])
+def test_the_order_of_many_pairs_is_the_stable_sort_by_expert(pairs, experts):
+    """More pairs than the one-workgroup kernel takes, around the edges of the waves' shares; few, odd and the most experts
+    whose counts LDS holds, and more."""
+    g = torch.Generator().manual_seed(pairs + experts)
+    k = K()
+    table = torch.randint(0, experts, (pairs, 1), generator=g, dtype=torch.int32)
+    table[: pairs // 3] = experts - 1                                           # one expert with many, others with few or none
+    rows = 16
+    cap = k.experts_tile_capacity(pairs, experts, 1, rows)
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    chosen, order, tiles, counts = i32(pairs), i32(pairs), i32(4 * cap), i32(experts)
+    ids = torch.randperm(pairs, generator=g).to(torch.int32)
+    k.experts_route_table(ids.cuda(), table.cuda(), experts, rows, chosen, torch.empty(pairs, device="cuda"), order, tiles, counts)
+    want = table[ids.long(), 0]
+    assert torch.equal(chosen.cpu(), want)
+    assert torch.equal(order.cpu().long(), torch.argsort(want, stable=True))
+    sizes = torch.bincount(want.long(), minlength=experts)
+    assert torch.equal(counts.cpu().long(), sizes)
+    listed, at = [], 0
+    for e, n in enumerate(sizes.tolist()):
+        listed += [[e, at + i, min(rows, n - i), 0] for i in range(0, n, rows)]
+        at += n
+    listed += [[-1, 0, 0, 0]] * (cap - len(listed))
+    assert tiles.reshape(-1, 4).tolist() == listed
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width, ff", [(8, 8), (64, 72), (72, 128), (136, 200), (1032, 264)])
 def test_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
