@@ -40,7 +40,6 @@ __device__ __forceinline__ float sigmoid_e(float x) { return 1.0f / (1.0f + expf
 // k-th pick.  expert [T][top] int, weight [T][top] float.
 // ---------------------------------------------------------------------------
 constexpr int kMaxPerLane = 8;   // experts a lane holds: up to 512 experts
-constexpr int kMaxExperts = 64 * kMaxPerLane;
 
 // scoring 0: the weights are the softmax over the chosen logits; 1: each chosen expert weighs the sigmoid of its own
 // logit, and nothing is renormalised (the sigmoid grows with the logit, so the largest logits are the largest scores).
@@ -200,17 +199,17 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
 // ---------------------------------------------------------------------------
 // (2) order [P]: the pairs (token * top + choice) sorted by expert, stable.  tiles [cap][4]: expert (-1: unused),
 // first place in order, rows, 0.  A wave an expert: it counts its pairs by ballots, adds up the counts of the
-// experts before it, writes its tiles and places its pairs.  Many pairs: a workgroup an expert
-// (route_order_kernel).  Few: one workgroup that also picks the experts, with the picks and counts in LDS.
+// experts before it, writes its tiles and places its pairs.  Many pairs: two launches of a workgroup
+// an expert (count; place).  Few: one workgroup that also picks the experts, with the picks and counts in LDS.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int count_pairs(const int* expert, int P, int e, int lane) {
+__device__ __forceinline__ int count_pairs(const int* expert, int p0, int p1, int e, int lane) {
   int n = 0;
-  for (int p0 = 0; p0 < P; p0 += 256) {   // (four loads requested together)
-    int got[4];
+  for (; p0 < p1; p0 += 512) {   // (eight loads requested together)
+    int got[8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) got[u] = p0 + 64 * u + lane < P ? expert[p0 + 64 * u + lane] : -1;
+    for (int u = 0; u < 8; ++u) got[u] = p0 + 64 * u + lane < p1 ? expert[p0 + 64 * u + lane] : -1;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) n += __popcll(__ballot(got[u] == e));
+    for (int u = 0; u < 8; ++u) n += __popcll(__ballot(got[u] == e));
   }
   return n;
 }
@@ -266,48 +265,43 @@ __device__ __forceinline__ void place_pairs(const int* expert, int p0, int p1, i
   }
 }
 
-// More experts than LDS holds counts of: a wave an expert, in two launches.
-__global__ __launch_bounds__(64) void route_count_kernel(const int* __restrict__ expert, int P, int* __restrict__ counts) {
-  const int n = count_pairs(expert, P, blockIdx.x, threadIdx.x);
-  if (threadIdx.x == 0) counts[blockIdx.x] = n;
+// Many pairs: a workgroup an expert, whose sixteen waves take a sixteenth of the pairs each.  What bounds both launches is
+// the latency of reading the picks, so the reads are spread over many waves; the second counts a wave's share again,
+// because the place of a share follows from the shares before it.  8,192 pairs of 32 experts: 5.0 us to count and 5.1 to
+// place, where one wave an expert took 12.2 and 12.7.
+__device__ __forceinline__ int my_share(int P, int w, int& p1) {
+  const int share = (P + 1023) / 1024 * 64, p0 = min(w * share, P);
+  p1 = min(p0 + share, P);
+  return p0;
 }
 
-__global__ __launch_bounds__(64) void route_place_kernel(const int* __restrict__ expert, const int* __restrict__ counts,
-                                                         int P, int E, int rows_a_tile, int* __restrict__ order,
-                                                         int* __restrict__ tiles, int cap) {
-  const int at = place_tiles(counts, E, blockIdx.x, threadIdx.x, rows_a_tile, tiles, cap, true);
-  place_pairs(expert, 0, P, blockIdx.x, threadIdx.x, at, order);
-}
-
-// A workgroup an expert.  Its sixteen waves take a sixteenth of the pairs each: first they count every expert's pairs
-// into LDS and their own expert's by wave, then each wave places its share behind the shares before it.  What bounds it
-// is the latency of reading the picks twice, so the reads are spread over many waves and nothing waits for another
-// launch: 8,192 pairs of 32 experts in 4.9 us, where a wave an expert took 12.2 us to count and 12.7 us to place.
-__global__ __launch_bounds__(1024) void route_order_kernel(const int* __restrict__ expert, int* __restrict__ counts, int P, int E,
-                                                           int rows_a_tile, int* __restrict__ order, int* __restrict__ tiles,
-                                                           int cap) {
-  __shared__ int counts_s[kMaxExperts];
+__global__ __launch_bounds__(1024) void route_count_kernel(const int* __restrict__ expert, int P, int* __restrict__ counts) {
   __shared__ int mine_s[16];
-  const int e = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int share = (P + 1023) / 1024 * 64, p0 = min(w * share, P), p1 = min(p0 + share, P);
-  for (int i = threadIdx.x; i < E; i += 1024) counts_s[i] = 0;
-  __syncthreads();
-  int n = 0;
-  for (int p = p0; p < p1; p += 512) {   // (eight loads requested together)
-    int got[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) got[u] = p + 64 * u + lane < p1 ? expert[p + 64 * u + lane] : -1;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if ((unsigned)got[u] < (unsigned)E) atomicAdd(&counts_s[got[u]], 1);
-      n += __popcll(__ballot(got[u] == e));
-    }
-  }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int p1;
+  const int p0 = my_share(P, w, p1);
+  const int n = count_pairs(expert, p0, p1, blockIdx.x, lane);
   if (lane == 0) mine_s[w] = n;
   __syncthreads();
-  int at = place_tiles(counts_s, E, e, lane, rows_a_tile, tiles, cap, w == 0);
+  if (threadIdx.x == 0) {
+    int sum = 0;
+    for (int i = 0; i < 16; ++i) sum += mine_s[i];
+    counts[blockIdx.x] = sum;
+  }
+}
+
+__global__ __launch_bounds__(1024) void route_place_kernel(const int* __restrict__ expert, const int* __restrict__ counts,
+                                                           int P, int E, int rows_a_tile, int* __restrict__ order,
+                                                           int* __restrict__ tiles, int cap) {
+  __shared__ int mine_s[16];
+  const int e = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int p1;
+  const int p0 = my_share(P, w, p1);
+  const int n = count_pairs(expert, p0, p1, e, lane);
+  if (lane == 0) mine_s[w] = n;
+  int at = place_tiles(counts, E, e, lane, rows_a_tile, tiles, cap, w == 0);
+  __syncthreads();
   for (int i = 0; i < w; ++i) at += mine_s[i];
-  if (threadIdx.x == 0) counts[e] = counts_s[e];
   place_pairs(expert, p0, p1, e, lane, at, order);
 }
 
@@ -388,7 +382,7 @@ __global__ __launch_bounds__(1024) void route_small_kernel(const float* __restri
     weight[pair] = share_s[pair];
   }
   for (int e = w; e < E; e += 16) {
-    const int n = count_pairs(picks_s, P, e, lane);
+    const int n = count_pairs(picks_s, 0, P, e, lane);
     if (lane == 0) counts_s[e] = n;
   }
   lds_barrier();
@@ -855,7 +849,8 @@ extern "C" int ls_experts_route(const float* z, long ldz, const float* bias, int
   else { LS_ROUTE(kMaxPerLane) }
 #undef LS_ROUTE
   if (!(P <= kSmallPairs && E <= kSmallExperts)) {
-    hipLaunchKernelGGL(route_order_kernel, dim3(E), dim3(1024), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
+    hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(1024), 0, s, expert, P, counts);
+    hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(1024), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
   }
   return check_launch("experts_route");
 }
@@ -914,12 +909,8 @@ extern "C" int ls_experts_route_table(const int* token_ids, const int* table, in
   } else {
     hipLaunchKernelGGL(route_table_kernel, dim3((P + 255) / 256), dim3(256), 0, s, token_ids, table, n_tokens, top, expert,
                        weight);
-    if (E <= kMaxExperts) {
-      hipLaunchKernelGGL(route_order_kernel, dim3(E), dim3(1024), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
-    } else {
-      hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(64), 0, s, expert, P, counts);
-      hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(64), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
-    }
+    hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(1024), 0, s, expert, P, counts);
+    hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(1024), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
   }
   return check_launch("experts_route_table");
 }

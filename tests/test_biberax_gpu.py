@@ -308,8 +308,7 @@ def test_routing_and_the_experts_products(dtype, tokens, experts, top, width, ff
 @pytest.mark.parametrize("pairs", [513, 1023, 1024, 1025, 4097, 8192])
 @pytest.mark.parametrize("experts", [2, 33, 512, 600])
 def test_the_order_of_many_pairs_is_the_stable_sort_by_expert(pairs, experts):
-    """More pairs than the one-workgroup kernel takes, around the edges of the waves' shares; few, odd and the most experts
-    whose counts LDS holds, and more."""
+    """More pairs than the one-workgroup kernel takes, around the edges of the waves' shares; few, odd and many experts."""
     g = torch.Generator().manual_seed(pairs + experts)
     k = K()
     table = torch.randint(0, experts, (pairs, 1), generator=g, dtype=torch.int32)
