@@ -11,8 +11,7 @@
 // kTileKeys, and in splits of kSplitKeys anchored at multiples of kSplitKeys,
 // whatever the step's first position is.  Inside a split the tiles are walked
 // in ascending order with the online softmax
-//     m' = max(m, rowmax(s)); a = exp(m - m'); p = exp(s - m') (s = -inf if masked, so p = 0;
-//                                                               ScoreScale says how each type computes it);
+//     m' = max(m, rowmax(s)); a = exp(m - m'); p = exp(s - m') (s = -inf if masked, so p = 0);
 //     l = l*a + sum(p); acc = acc*a + round(p) . V
 // (sum(p): a lane adds its four keys of a 16-key block as (p0+p1)+(p2+p3),
 // the eight blocks in ascending order, then the four lanes of the row)
@@ -174,18 +173,6 @@ __device__ __forceinline__ f32x4 mask_keys(f32x4 v, int n_lo, int n_hi) {
   return v;
 }
 
-// The query's sign turned where the scale is negative and the softmax wants a positive factor (bfloat16).
-template <typename T, int N>
-__device__ __forceinline__ void flip_rows(typename Atom<T>::vec_t (&q)[N], float scale) {
-  if constexpr (sizeof(T) == 2) {
-    if (scale < 0.f) {
-      typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-#pragma unroll
-      for (int c = 0; c < N; ++c) q[c] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, q[c]) ^ 0x80008000u);
-    }
-  }
-}
-
 // All bits set in every element (the operand of mask_keys that turns it into a mask), and the bitwise AND.
 template <typename T> __device__ __forceinline__ typename Atom<T>::vec_t ones_vec();
 template <> __device__ __forceinline__ bf16x8 ones_vec<bf16_t>() {
@@ -293,8 +280,6 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
 #pragma unroll
   for (int c = 0; c < NC; ++c)
     qv[c] = load_vec<T>(q + (long)head * D, sm.q_off + qi, c * A::KCHUNK + g * A::VEC, D, ldq, row_ok, true);
-  flip_rows<T>(qv, scale);
-  const ScoreScale<T> score(scale);
 
   RowState run;
   run.reset();
@@ -336,7 +321,7 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            s[kb][e] = score.kept(s[kb][e]);
+            s[kb][e] = s[kb][e] * scale;
             tile_max = fmaxf(tile_max, s[kb][e]);
           }
       } else {
@@ -345,19 +330,19 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-            const float v = ((key <= key_hi) & (key >= key_lo)) ? score.kept(s[kb][e]) : kMasked;
+            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * scale : kMasked;
             s[kb][e] = v;
             tile_max = fmaxf(tile_max, v);
           }
       }
       tile_max = quad16_max(tile_max);
-      const float m_new = fmaxf(cur.m, score.top(tile_max));
+      const float m_new = fmaxf(cur.m, tile_max);
       const float alpha = softmax_exp<T>(cur.m - m_new);
       float p_sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[kb][e] = score.probability(s[kb][e], m_new);  // masked: exp(-inf) = 0
+        for (int e = 0; e < 4; ++e) s[kb][e] = softmax_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
         p_sum = p_sum + ((s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]));
       }
       p_sum = quad16_sum(p_sum);
@@ -498,8 +483,6 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 #pragma unroll
   for (int c = 0; c < NC; ++c)
     qv[c] = load_vec<T>(q + (long)head * D, sm.q_off + qi, c * A::KCHUNK + g * A::VEC, D, ldq, row_ok, true);
-  flip_rows<T>(qv, scale);
-  const ScoreScale<T> score(scale);
 
   // tiles this workgroup walks: a contiguous range
   int ti_lo = item.split_begin * TILES_PER_SPLIT;
@@ -665,7 +648,7 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            s[kb][e] = score.kept(s[kb][e]);
+            s[kb][e] = s[kb][e] * scale;
             tile_max = fmaxf(tile_max, s[kb][e]);
           }
       } else {
@@ -674,19 +657,19 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-            const float v = ((key <= key_hi) & (key >= key_lo)) ? score.kept(s[kb][e]) : kMasked;
+            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * scale : kMasked;
             s[kb][e] = v;
             tile_max = fmaxf(tile_max, v);
           }
       }
       tile_max = quad16_max(tile_max);
-      const float m_new = fmaxf(cur.m, score.top(tile_max));
+      const float m_new = fmaxf(cur.m, tile_max);
       const float alpha = softmax_exp<T>(cur.m - m_new);
       float p_sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[kb][e] = score.probability(s[kb][e], m_new);  // masked: exp(-inf) = 0
+        for (int e = 0; e < 4; ++e) s[kb][e] = softmax_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
         p_sum = p_sum + ((s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]));
       }
       p_sum = quad16_sum(p_sum);
@@ -790,16 +773,11 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 // row is the instruction sequence of the other variants, so the bits are the
 // same.
 //
-// What bounds it: the vector unit (two instructions a score for the
-// exponentials, plus the maximum and the conversion) with the matrix cores
-// behind it, at one workgroup of eight waves a CU; for prompts from position 0
-// also the last row blocks, which walk the most tiles.  Measured (bfloat16,
-// D = 128): one 2,048-token prompt with 32 heads over 8 kv heads 115 -> 73 us, with
-// 16 heads over 8 61 -> 57, portions of 2,048 up to position 9,000 138 -> 124 and
-// the last 808 tokens in 4-wave workgroups 213 -> 205.  Of the 42 us, 36 come
-// from the kv heads' numbering over the XCDs, the rest from the two phases and
-// the base-2 exponentials.  Deeper operand rings (six or eight in place of
-// four) changed nothing.
+// What bounds it: the vector unit (scaling, exponentials, maximum and conversion)
+// with the matrix cores behind it, at one workgroup of eight waves a CU; for
+// prompts from position 0 also the last row blocks, which walk the most tiles.
+// Measured (bfloat16, D = 128, 2,048 tokens): 32 heads over 8 kv heads 116 -> 74 us,
+// from the kv heads' numbering over the XCDs; 16 heads over 8 60.5 -> 60.
 template <typename T, int NW>
 __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
@@ -880,8 +858,6 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
 #pragma unroll
   for (int c = 0; c < NC; ++c)
     qv[c] = load_vec<T>(q + (long)head * D, sm.q_off + qi, c * A::KCHUNK + g * VEC, D, ldq, row_ok, true);
-  flip_rows<T>(qv, scale);
-  const ScoreScale<T> score(scale);
 
   int ti_lo = item.split_begin;
   if (window > 0) ti_lo = max(ti_lo, max(0, block_first_pos - window + 1) / kTileKeys);
@@ -1001,7 +977,7 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   auto scale_block = [&](int kb) LS_INLINED {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      s[kb][e] = score.kept(s[kb][e]);
+      s[kb][e] = s[kb][e] * scale;
       tile_max = fmaxf(tile_max, s[kb][e]);
     }
   };
@@ -1015,7 +991,7 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int key = key_of_row<T>(kb, e);
-        const float v = ((key <= hi) & (key >= lo)) ? score.kept(s[kb][e]) : kMasked;
+        const float v = ((key <= hi) & (key >= lo)) ? s[kb][e] * scale : kMasked;
         s[kb][e] = v;
         tile_max = fmaxf(tile_max, v);
       }
@@ -1031,7 +1007,7 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   auto prob_block = [&](int kb, float m) LS_INLINED {
     f32x4 p;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = score.probability(s[kb][e], m);  // masked: exp(-inf) = 0
+    for (int e = 0; e < 4; ++e) p[e] = softmax_exp<T>(s[kb][e] - m);  // masked: exp(-inf) = 0
     p_sum = p_sum + ((p[0] + p[1]) + (p[2] + p[3]));
 #pragma unroll
     for (int e = 0; e < 4; ++e) prob[kb][e] = from_f32<T>(p[e]);
@@ -1179,7 +1155,7 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
       const float b = any ? softmax_exp<T>(cur_m - m_new) : -0.f;
       run.l = any ? run.l * a + cur_l * b : run.l;
       run.m = m_new;
-      cur_m = fmaxf(kNegSentinel, score.top(tile_max));
+      cur_m = fmaxf(kNegSentinel, tile_max);
       if (next) probabilities(k_next, std::true_type{}, cur_m, a, b);
       else probabilities(k_next, std::false_type{}, cur_m, a, b);
       cur_l = p_sum;
@@ -1652,8 +1628,6 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
 #pragma unroll
     for (int c = 0; c < NC; ++c) __asm__ volatile("" ::"v"(qv[c]));
   }
-  flip_rows<T>(qv, scale);
-  const ScoreScale<T> score(scale);
   PROBE(3)
   for (int ti = ti_lo; ti < ti_hi; ++ti) {
     const int t0 = ti * kTileKeys;
@@ -1726,7 +1700,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-          const float v = ((key <= key_hi) & (key >= key_lo)) ? score.kept(s[j][e]) : kMasked;
+          const float v = ((key <= key_hi) & (key >= key_lo)) ? s[j][e] * scale : kMasked;
           s[j][e] = v;
           my_max = fmaxf(my_max, v);
         }
@@ -1739,13 +1713,13 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     PROBE(8)
     if (NBUF == 1 && ahead) issue_k(ti + 1);  // every wave has its scores: the K half of the buffer is free
     const float tile_max = fmaxf(fmaxf(wmax[row16], wmax[16 + row16]), fmaxf(wmax[32 + row16], wmax[48 + row16]));
-    const float m_new = fmaxf(cur_m, score.top(tile_max));
+    const float m_new = fmaxf(cur_m, tile_max);
     const float alpha = softmax_exp<T>(cur_m - m_new);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int kb = 2 * wave + j;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[j][e] = score.probability(s[j][e], m_new);  // masked: exp(-inf) = 0
+      for (int e = 0; e < 4; ++e) s[j][e] = softmax_exp<T>(s[j][e] - m_new);  // masked: exp(-inf) = 0
       psum[kb * 64 + lane] = (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
       prob[kb * 64 + lane] = s[j];
     }

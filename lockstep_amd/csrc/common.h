@@ -107,36 +107,11 @@ __device__ __forceinline__ typename Atom<T>::vec_t load_vec(const T* __restrict_
 
 namespace ls {
 
-// The exponential of the softmax of the other attention kernels and of the fold over attention splits: the library
-// routine on the 32-bit path, the hardware's on the bfloat16 path.  One definition for every kernel that folds.
+// The exponential of the softmax and of the fold over attention splits: the library routine on the
+// 32-bit path, the hardware's on the bfloat16 path.  One definition for every kernel that folds.
 template <typename T> __device__ __forceinline__ float softmax_exp(float x);
 template <> __device__ __forceinline__ float softmax_exp<float>(float x) { return expf(x); }
 template <> __device__ __forceinline__ float softmax_exp<bf16_t>(float x) { return __expf(x); }
-
-// The softmax of the paged attention.  float32: scores times the scale, exponentials of their distance to the maximum.
-// bfloat16: the scores stay as the products leave them and a probability is 2^(score * c - maximum * log2(e)), c = scale
-// * log2(e), by one fused multiply-add and the hardware's exponential: two instructions a score, where scaling,
-// subtracting and the base change took four, and fewer roundings in the exponent.  Maxima are kept scaled in both, so a
-// split's sums mean the same to whoever folds them.  (A negative scale turns the query's sign, see flip_rows: c is
-// positive, and above zero, so that a masked score stays minus infinity.)
-constexpr float kLog2E = 1.44269504088896340736f;
-template <typename T> struct ScoreScale;
-template <> struct ScoreScale<float> {
-  float scale;
-  __device__ __forceinline__ explicit ScoreScale(float s) : scale(s) {}
-  __device__ __forceinline__ float kept(float s) const { return s * scale; }
-  __device__ __forceinline__ float top(float m) const { return m; }
-  __device__ __forceinline__ float probability(float s, float m) const { return expf(s - m); }
-};
-template <> struct ScoreScale<bf16_t> {
-  float scale, c;
-  __device__ __forceinline__ explicit ScoreScale(float s) : scale(fmaxf(fabsf(s), 1e-37f)), c(scale * kLog2E) {}
-  __device__ __forceinline__ float kept(float s) const { return s; }
-  __device__ __forceinline__ float top(float m) const { return m * scale; }
-  __device__ __forceinline__ float probability(float s, float m) const {
-    return __builtin_amdgcn_exp2f(fmaf(s, c, -(m * kLog2E)));
-  }
-};
 
 // Sum / max over the four lanes {l, l^16, l^32, l^48}; every lane of the
 // four ends with the same bits because each step adds a pair commutatively.

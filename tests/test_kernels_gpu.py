@@ -750,6 +750,34 @@ def test_attention_window(dtype, window):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq,nkv,d,ps", [(4, 2, 64, 16), (16, 8, 128, 16), (6, 2, 48, 8)])
+@pytest.mark.parametrize("scale", [0.13, -0.13])
+def test_scores_of_great_size_leave_finite_results(dtype, nq, nkv, d, ps, scale):
+    """Queries and keys of +-2^20 and scores up to 10^13: the largest probability of a row is exp(0) whatever its score, so
+    nothing overflows.  Products and sums are whole multiples of 2^40 below 2^47 and exact in every order, so equal scores tie
+    exactly, and a step between two scores (2^41 times the scale) leaves the lower one nothing."""
+    n = 700
+    g = torch.Generator().manual_seed(d)
+    qkv = torch.randn(n, (nq + 2 * nkv) * d, generator=g)
+    signs = torch.randint(0, 2, (n, (nq + nkv) * d), generator=g).float() * 2 - 1
+    qkv[:, : (nq + nkv) * d] = signs * 2.0 ** 20
+    qkv = qkv.to(dtype)
+    case = PagedCase(dtype, nq, nkv, d, ps, n, shuffle_seed=2)
+    dev = qkv.cuda()
+    case.write(dev, 0)
+    q, k, v = split_qkv(qkv.double(), nq, nkv, d)
+    want = naive_attention(q, k, v, 0, scale)
+    for variant in (0, 1) + ((4, 5) if K().wide_supported(d, dtype, ps) else ()):
+        got = case.attend(dev, 0, scale, variant=variant, force_split=False)
+        assert torch.isfinite(got).all(), variant
+        assert rel_err(got, want) < ATT_TOL[dtype], variant
+    for p in (5, 127, 128, n - 1):
+        for split in (False, True):
+            one = case.attend(dev[p:p + 1], p, scale, variant=3, force_split=split)
+            assert torch.isfinite(one).all() and rel_err(one, want[p:p + 1]) < ATT_TOL[dtype], (p, split)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_norm_rotation_and_cache_write(dtype):
     nq, nkv, d, ps, t, start = 6, 3, 32, 8, 21, 5
     rot = 32
