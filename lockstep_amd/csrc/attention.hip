@@ -106,13 +106,6 @@ __device__ __forceinline__ void load_to_lds16(const void* src, __attribute__((ad
   __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory", "m0");
 }
 
-// The same with an address that all lanes share and a lane's distance from it in bytes.
-__device__ __forceinline__ void load_to_lds16(unsigned lane_bytes, const void* base, unsigned lds_wave_base) {
-  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_bytes), "s"(base),
-                   "s"(lds_wave_base)
-                   : "memory", "m0");
-}
-
 // Sixteen bytes into registers by an instruction the compiler does not know to be a load: it places no wait for
 // it, so the kernel can keep it in flight across other loads and wait with a count of its own (wait_for_loads,
 // which also ties the registers, so that no use moves above the wait).
@@ -756,28 +749,27 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 
 
 // Variant 4, "wide": prompt portions.  A workgroup of NW waves owns 16*NW rows
-// and walks the key tiles with two LDS buffers for keys and two for values.
-// The tiles go from global memory straight into LDS (no registers in between):
-// a load instruction of a wave fills 64 consecutive 16-byte pieces of LDS, and
-// each lane chooses the source of its piece, so a key's pieces arrive in the
-// slots slot_of names and the V tile as [8 or 4 keys][column][16 bytes].  Keys
-// outside the held range need no zeroing in K (their scores are replaced by
-// -inf), and the V tile of a boundary tile is cleaned in LDS before use.
-//
-// A tile has two phases, and the matrix cores have work in both: while a
-// tile's probabilities are computed (the vector unit's phase) the products of
-// the next tile's scores run between them and the tile before is folded; while
-// the probabilities meet the values, the maxima of the next tile's scores are
-// taken.  The barrier behind a phase frees the buffer it read, whose next tile
-// is asked for at once, so keys arrive a whole tile ahead.  The arithmetic of a
-// row is the instruction sequence of the other variants, so the bits are the
-// same.
+// and walks the key tiles with two LDS buffers.  The tiles go from global
+// memory straight into LDS (no registers in between): a load instruction of a
+// wave fills 64 consecutive 16-byte pieces of LDS, and each lane chooses the
+// source of its piece, so the K tile arrives in the rotated layout of the
+// staged kernel and the V tile as [8 or 4 keys][column][16 bytes].  While a
+// tile is multiplied the next one is in flight.  Keys outside the held range
+// need no zeroing in K (their scores are replaced by -inf), and the V tile of
+// a boundary tile is cleaned in LDS before use.  The arithmetic of a row is
+// the instruction sequence of the other variants, so the bits are the same.
 //
 // What bounds it: the vector unit (scaling, exponentials, maximum and conversion)
-// with the matrix cores behind it, at one workgroup of eight waves a CU; for
-// prompts from position 0 also the last row blocks, which walk the most tiles.
-// Measured (bfloat16, D = 128, 2,048 tokens): 32 heads over 8 kv heads 116 -> 74 us,
-// from the kv heads' numbering over the XCDs; 16 heads over 8 60.5 -> 60.
+// in turn with the matrix cores, at one workgroup of eight waves a CU (bfloat16,
+// D = 128); for prompts from position 0 also the last row blocks, which walk the
+// most tiles.  Measured, 2,048 tokens, row blocks going round the XCDs / a kv
+// head's blocks on one: 32 heads over 8 kv heads 116 / 74 us (D = 128), 75 / 46
+// (64), 117 / 70 (112), 168 / 101 (144); 16 over 8 60.5 / 60.5.
+// Not kept: the score products of the next tile between the exponentials and its
+// maxima between the value products (a second set of scores and sums alive): at D
+// = 128 and eight waves the same times, everywhere else slower (16 over 8 heads,
+// D = 112 60 / 101 us, D = 144 88 / 175: registers spill; portions of 512 tokens
+// in blocks of 64 rows, D = 128 16.6 / 18.6).
 template <typename T, int NW>
 __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
@@ -796,24 +788,16 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   constexpr int TOTAL = kTileKeys * KPIECES;  // pieces of the K tile == pieces of the V tile
   constexpr int PER = (TOTAL + NT - 1) / NT;
   constexpr int TILE_BYTES = TOTAL * 16;
+  constexpr int BUF_BYTES = 2 * TILE_BYTES;
+  constexpr int TILES_PER_SPLIT = kSplitKeys / kTileKeys;
+  typedef const __attribute__((address_space(1))) void* gptr_t;
   typedef __attribute__((address_space(3))) void* lptr_t;
-  // Which slot of its row in the LDS tile holds a key's piece: exclusive-or with the row where a row has a power of two
-  // of pieces (the sixteen lanes that LDS serves together, four runs of four from both ends of two rows' lanes, then
-  // start in sixteen different slots; with a rotation by the row two of them met, a third of LDS's time), else a rotation.
-  constexpr bool XOR_SLOTS = (KPIECES & (KPIECES - 1)) == 0;
-  auto slot_of = [](int row, int piece) LS_INLINED -> int {
-    return XOR_SLOTS ? piece ^ (row_rotation<T>(row) & (KPIECES - 1)) : (piece + row_rotation<T>(row)) % KPIECES;
-  };
-  auto piece_in = [](int row, int slot) LS_INLINED -> int {
-    return XOR_SLOTS ? slot ^ (row_rotation<T>(row) & (KPIECES - 1)) : (slot - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
-  };
-  static_assert(kSplitKeys == kTileKeys, "a tile is a split: its sums start from nothing and are folded as they are");
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // K tiles 0 and 1, V tiles 0 and 1
-  int* tile_pages = reinterpret_cast<int*>(lds + 4 * TILE_BYTES);      // [2 windows][kPageWindow][16]
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  int* tile_pages = reinterpret_cast<int*>(lds + 2 * BUF_BYTES);  // [kPageWindow][16]
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = threadIdx.x >> 6;
   // Workgroup ids go round the eight XCDs.  All row blocks of a kv head walk the same keys and values: they are given to
   // one XCD (8, 16, ... kv heads; fewer heads: to as many XCDs as share one), whose L2 then answers most of them.  With
   // the row blocks going round instead, every XCD reads every head from beyond its L2: that bound the whole kernel.
@@ -859,268 +843,92 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   for (int c = 0; c < NC; ++c)
     qv[c] = load_vec<T>(q + (long)head * D, sm.q_off + qi, c * A::KCHUNK + g * VEC, D, ldq, row_ok, true);
 
-  int ti_lo = item.split_begin;
+  int ti_lo = item.split_begin * TILES_PER_SPLIT;
   if (window > 0) ti_lo = max(ti_lo, max(0, block_first_pos - window + 1) / kTileKeys);
-  const int ti_hi = min(item.split_end, block_last_pos / kTileKeys + 1);
+  const int ti_hi = min(item.split_end * TILES_PER_SPLIT, block_last_pos / kTileKeys + 1);
 
-  // Start the loads of a tile's keys or values into their buffer.  Keys past the request's end need no clamp of
-  // their own: the page id of their page is that of the last held page, so the loads stay inside the cache, and what
-  // they bring is masked.
-  const long page_stride = (long)nkv * page_size * D;  // elements of one page, K or V
-  // Heads of 64 and 128 elements in bfloat16: the 64 pieces of a wave's load lie in one page, so the page id is a scalar
-  // load, the page's address scalar arithmetic, and a lane keeps its place inside a page for all of them: what a load of
-  // the thread adds to that is the same for every lane (its rows start at multiples of kStep keys).
-  constexpr bool kScalarPages = SZ == 2 && D % 64 == 0 && 64 % KPIECES == 0 && NT % D == 0 && PER * NT == TOTAL;
-  constexpr int kStep = NT / KPIECES > 0 ? NT / KPIECES : 1;  // key rows between two loads of a thread; values: the same
-  constexpr int kPlaces = kStep >= 32 ? 1 : 32 / kStep;       // the rotation of a key row repeats every 32 rows
-  // Other heads: a place a load, and the page ids of two windows of kPageWindow tiles in LDS: the one that is walked and
-  // the next, which is filled (by ordinary loads, for which the compiler waits, tile loads included) when the walk
-  // enters a window.
-  constexpr int K_PLACES = kScalarPages ? kPlaces : PER, V_PLACES = kScalarPages ? 1 : PER;
-  int k_off[K_PLACES], v_off[V_PLACES];
-#pragma unroll
-  for (int i = 0; i < K_PLACES; ++i) {
-    const int p = i * NT + (int)threadIdx.x;
-    const int row = p / KPIECES;
-    const int slot = p % KPIECES;
-    const int piece = piece_in(row, slot);
-    const int in_page = (kScalarPages ? (int)threadIdx.x / KPIECES : row) & (page_size - 1);
-    k_off[i] = (kvh * page_size + in_page) * D + piece * VEC;
-    if (kScalarPages) k_off[i] *= SZ;  // bytes
-  }
-#pragma unroll
-  for (int i = 0; i < V_PLACES; ++i) {
-    const int p = i * NT + (int)threadIdx.x;
-    v_off[i] = ((kvh * D + p % D) << page_shift) + ((p / D * VEC) & (page_size - 1));
-    if (kScalarPages) v_off[i] *= SZ;
-  }
-  auto fill_pages = [&](int win) LS_INLINED {
+  // The page ids of kPageWindow tiles at a time go into LDS, by ordinary loads, while no tile load is in
+  // flight (the compiler's waits for ordinary loads do not know of the tile loads and would wait for them too).
+  auto fill_pages = [&](int first_tile) LS_INLINED {
     for (int idx = threadIdx.x; idx < kPageWindow * 16; idx += NT) {
-      const int t = ti_lo + win * kPageWindow + idx / 16;
+      const int t = first_tile + idx / 16;
       const int pg = idx % 16;
       if (t < ti_hi && pg < pages_per_tile) {
         const int key = min(t * kTileKeys + (pg << page_shift), sm.kv_len - 1);
-        tile_pages[(win & 1) * kPageWindow * 16 + idx] = tbl[key >> page_shift];
+        tile_pages[idx] = tbl[key >> page_shift];
       }
     }
   };
-  // the pages that a thread's loads of tile ti come from (kScalarPages), asked for a tile ahead
-  auto pages_of = [&](int ti, bool keys, int (&page)[PER]) LS_INLINED {
+  auto window_start = [&](int ti) LS_INLINED -> bool { return (ti - ti_lo) % kPageWindow == 0; };  // tile ti opens a window of ids
+  // Start the loads of a tile into its buffer.  What does not depend on the
+  // tile is computed once: the offset of each of the thread's pieces inside
+  // its page.  Keys past the request's end need no clamp of their own: the
+  // page id of their page is that of the last held page (fill_pages clamps),
+  // so the loads stay inside the cache, and what they bring is masked.
+  const long page_stride = (long)nkv * page_size * D;  // elements of one page, K or V
+  int k_off[PER], v_off[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int first = keys ? (i * NT + wave * 64) / KPIECES : (i * NT + wave * 64) / D * VEC;
-      page[i] = tbl[__builtin_amdgcn_readfirstlane(min(ti * kTileKeys + first, sm.kv_len - 1) >> page_shift)];
-    }
-  };
-  auto request = [&](int ti, const T* pool, bool keys, const int (&asked)[PER]) LS_INLINED {
-    unsigned char* buf = lds + ((keys ? 0 : 2) + (ti & 1)) * TILE_BYTES;
-    if constexpr (kScalarPages) {
-      const unsigned at = (unsigned)(unsigned long)(lptr_t)buf + wave * 1024;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int in_page = (i * kStep) & (page_size - 1);
-        const T* base = pool + (long)max(asked[i], 0) * page_stride + (keys ? in_page * D : in_page);
-        load_to_lds16(keys ? k_off[i % K_PLACES] : v_off[0], base, at + i * NT * 16);
-      }
-      return;
-    }
-    const int* pages = tile_pages + ((ti - ti_lo) % (2 * kPageWindow)) * 16;
-    int page[PER];
+  for (int i = 0; i < PER; ++i) {
+    const int p = i * NT + (int)threadIdx.x;
+    const int row = p / KPIECES;
+    const int slot = p % KPIECES;
+    const int piece = (slot - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
+    k_off[i] = (kvh * page_size + (row & (page_size - 1))) * D + piece * VEC;
+    const int c = p / D;
+    const int d = p % D;
+    v_off[i] = ((kvh * D + d) << page_shift) + ((c * VEC) & (page_size - 1));
+  }
+  auto issue = [&](int ti) LS_INLINED {
+    const int* pages = tile_pages + ((ti - ti_lo) % kPageWindow) * 16;
+    unsigned char* k_buf = lds + (ti & 1) * BUF_BYTES;
+    unsigned char* v_buf = k_buf + TILE_BYTES;
+    int k_page[PER], v_page[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {  // all page ids first: their LDS reads overlap
       const int p = i * NT + (int)threadIdx.x;
-      page[i] = pages[min((keys ? p / KPIECES : (p / D) * VEC) >> page_shift, 15)];
+      k_page[i] = pages[min((p / KPIECES) >> page_shift, 15)];
+      v_page[i] = pages[min(((p / D) * VEC) >> page_shift, 15)];
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       if (PER * NT != TOTAL && i * NT + wave * 64 >= TOTAL) break;  // uniform for the wave
-      load_to_lds16(pool + (long)max(page[i], 0) * page_stride + (keys ? k_off[i % K_PLACES] : v_off[i % V_PLACES]),
-                    (lptr_t)(buf + (i * NT + wave * 64) * 16));
+      const T* k_src = k_pages + (long)max(k_page[i], 0) * page_stride + k_off[i];
+      load_to_lds16(k_src, (lptr_t)(k_buf + (i * NT + wave * 64) * 16));
+      const T* v_src = v_pages + (long)max(v_page[i], 0) * page_stride + v_off[i];
+      load_to_lds16(v_src, (lptr_t)(v_buf + (i * NT + wave * 64) * 16));
     }
-  };
-  auto mine = [&](int ti) LS_INLINED -> bool {  // whether a row of the wave sees a key of the tile
-    const int t0 = ti * kTileKeys;
-    return ti < ti_hi && wave_active && t0 <= wave_last_pos && !(window > 0 && t0 + kTileKeys <= wave_first_pos - window + 1);
   };
 
-  // ---- the pieces of a tile's work --------------------------------------
-  constexpr int NS = NB * NC;
-  constexpr int KR = NS < 4 ? NS : 4;
-  f32x4 s[NB];   // scores of the tile that comes next, masked
-  vec_t kr[KR];  // operand reads in flight ahead of the products
-  auto k_read = [&](const unsigned char* k_lds, int idx) LS_INLINED -> vec_t {
-    const int row = key_of_row<T>(idx / NC, row16);
-    const int piece = (idx % NC) * 4 + g;
-    const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
-    vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + slot_of(row, pc) * 16);
-    if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
-    return kv;
-  };
-  auto k_start = [&](const unsigned char* k_lds) LS_INLINED {
-#pragma unroll
-    for (int i = 0; i < KR; ++i) kr[i] = k_read(k_lds, i);
-  };
-  auto k_block = [&](const unsigned char* k_lds, int kb) LS_INLINED {  // S^T = K . Q^T of sixteen keys
-    s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int idx = kb * NC + c;
-      A::mma(s[kb], kr[idx % KR], qv[c]);
-      if (idx + KR < NS) kr[idx % KR] = k_read(k_lds, idx + KR);
-    }
-  };
-  float tile_max = kNegSentinel, cur_m = kNegSentinel, cur_l = 0.f;
-  auto all_visible = [&](int ti) LS_INLINED -> bool {
-    const int t0 = ti * kTileKeys;
-    return t0 + kTileKeys - 1 <= wave_first_pos && r0 + 15 < rows_total && (window <= 0 || wave_last_pos - t0 < window);
-  };
-  auto scale_block = [&](int kb) LS_INLINED {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      s[kb][e] = s[kb][e] * scale;
-      tile_max = fmaxf(tile_max, s[kb][e]);
-    }
-  };
-  auto scale_masked = [&](int ti) LS_INLINED {
-    // the row's first and last key, counted from the first key that the lane holds: the others are constants away
-    // (opaque, or the compiler keeps a register a key through the whole walk)
-    int lo = key_lo - ti * kTileKeys - key_of_row<T>(0, 4 * g), hi = key_hi - ti * kTileKeys - key_of_row<T>(0, 4 * g);
-    __asm__ volatile("" : "+v"(lo), "+v"(hi));
-#pragma unroll
-    for (int kb = 0; kb < NB; ++kb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = key_of_row<T>(kb, e);
-        const float v = ((key <= hi) & (key >= lo)) ? s[kb][e] * scale : kMasked;
-        s[kb][e] = v;
-        tile_max = fmaxf(tile_max, v);
-      }
-  };
-  RowState run;
+  RowState run, cur;
   run.reset();
-  f32x4 acc[DB];  // the sums of the tile before, folded into `run` while the next one's scores are multiplied
-#pragma unroll
-  for (int blk = 0; blk < DB; ++blk) acc[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
-  typedef __attribute__((ext_vector_type(4))) T four_t;
-  four_t prob[NB];
-  float p_sum = 0.f;
-  auto prob_block = [&](int kb, float m) LS_INLINED {
-    f32x4 p;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = softmax_exp<T>(s[kb][e] - m);  // masked: exp(-inf) = 0
-    p_sum = p_sum + ((p[0] + p[1]) + (p[2] + p[3]));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) prob[kb][e] = from_f32<T>(p[e]);
-  };
-  // O^T = V^T . P^T; SCALE: the scores of the next tile are scaled between the products
-  constexpr int KB16 = VEC / 4;
-  constexpr int NP = (NB / KB16) * DB;
-  constexpr int VR = NP < 4 ? NP : 4;
-  auto values = [&](const unsigned char* v_lds, auto also) LS_INLINED {
-    constexpr bool SCALE = decltype(also)::value;
-    auto v_read = [&](int idx) LS_INLINED -> vec_t {
-      const int kb = (idx / DB) * KB16;
-      const int d = (idx % DB) * 16 + row16;
-      vec_t vv;
-#pragma unroll
-      for (int h = 0; h < KB16; ++h) {
-        const int key = key_of_row<T>(kb + h, 4 * g);  // the lane's four keys inside the tile
-        const four_t four = *reinterpret_cast<const four_t*>(v_lds + ((key / VEC) * D + d) * 16 + (key % VEC) * SZ);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) vv[h * 4 + e] = four[e];
-      }
-      return vv;
-    };
-    vec_t vr[VR];
-#pragma unroll
-    for (int i = 0; i < VR; ++i) vr[i] = v_read(i);
-#pragma unroll
-    for (int blk = 0; blk < DB; ++blk) acc[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
-    vec_t pv;
-#pragma unroll
-    for (int idx = 0; idx < NP; ++idx) {
-      if (idx % DB == 0) {
-        const int kb = (idx / DB) * KB16;
-#pragma unroll
-        for (int h = 0; h < KB16; ++h)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) pv[h * 4 + e] = prob[kb + h][e];
-      }
-      A::mma(acc[idx % DB], vr[idx % VR], pv);
-      if (idx + VR < NP) vr[idx % VR] = v_read(idx + VR);
-      // the blocks of the next tile's scores are spread over the products
-      if (SCALE) {
-#pragma unroll
-        for (int kb = idx * NB / NP; kb < (idx + 1) * NB / NP; ++kb) scale_block(kb);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  // A tile's probabilities; between them the next tile's score products (NEXT) and the fold of the tile before.  The
-  // fold is fold_split's: a row that has nothing to fold (its sums are zeros, see below) keeps what it has, to the bit,
-  // since x * 1 + 0 * -0 = x for every x.
-  auto probabilities = [&](const unsigned char* k_lds, auto next, float m, float a, float b) LS_INLINED {
-    constexpr bool NEXT = decltype(next)::value;
-    if (NEXT) k_start(k_lds);
-    p_sum = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < NB; ++kb) {
-      prob_block(kb, m);
-      if (NEXT) k_block(k_lds, kb);
-#pragma unroll
-      for (int blk = kb * DB / NB; blk < (kb + 1) * DB / NB; ++blk)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) run.acc[blk][e] = run.acc[blk][e] * a + acc[blk][e] * b;
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    p_sum = quad16_sum(p_sum);
-  };
+  cur.reset();
 
-  int k_asked[PER] = {}, v_asked[PER] = {};
   if (ti_lo < ti_hi) {
-    int k_first[PER] = {};
-    if constexpr (kScalarPages) {
-      pages_of(ti_lo, true, k_first);
-      pages_of(ti_lo, false, v_asked);
-      pages_of(ti_lo + 1, true, k_asked);
-    } else {
-      fill_pages(0);
-      fill_pages(1);
-      __syncthreads();
-    }
-    request(ti_lo, k_pages, true, k_first);
-    request(ti_lo, v_pages, false, v_asked);
-    if (ti_lo + 1 < ti_hi) request(ti_lo + 1, k_pages, true, k_asked);
-    if constexpr (kScalarPages) {
-      pages_of(ti_lo + 1, false, v_asked);
-      pages_of(ti_lo + 2, true, k_asked);
-    }
+    fill_pages(ti_lo);
+    __syncthreads();
+    issue(ti_lo);
   }
+#ifdef LS_ATTN_PROBE
+  long long pr_t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  long long pr_last = clock64();
+  const long long pr_begin = pr_last;
+#endif
 #pragma unroll
   for (int c = 0; c < NC; ++c) __asm__ volatile("" ::"v"(qv[c]));  // the query rows are awaited here, not inside the loop
-  bool have = mine(ti_lo);  // the wave's scores of tile ti are in s
-  if (ti_lo < ti_hi) {
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
-    if (have) {
-      k_start(lds + (ti_lo & 1) * TILE_BYTES);
-#pragma unroll
-      for (int kb = 0; kb < NB; ++kb) k_block(lds + (ti_lo & 1) * TILE_BYTES, kb);
-      if (all_visible(ti_lo)) {
-#pragma unroll
-        for (int kb = 0; kb < NB; ++kb) scale_block(kb);
-      } else {
-        scale_masked(ti_lo);
-      }
-      tile_max = quad16_max(tile_max);
-    }
-  }
   for (int ti = ti_lo; ti < ti_hi; ++ti) {
     const int t0 = ti * kTileKeys;
-    unsigned char* v_lds = lds + (2 + (ti & 1)) * TILE_BYTES;
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's pieces of V(ti) and K(ti + 1) have landed
-    lds_barrier();  // both tiles are complete; K(ti) and V(ti - 1) have been read by every wave
-    if (!kScalarPages && ti != ti_lo && (ti - ti_lo) % kPageWindow == 0) fill_pages((ti - ti_lo) / kPageWindow + 1);
+    const unsigned char* k_lds = lds + (ti & 1) * BUF_BYTES;
+    unsigned char* v_lds = lds + (ti & 1) * BUF_BYTES + TILE_BYTES;
+    if (ti != ti_lo && window_start(ti)) {  // nothing is in flight: the previous tile did not request this one
+      lds_barrier();
+      fill_pages(ti);
+      lds_barrier();
+      issue(ti);
+    }
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's pieces of the tile have landed
+    PROBE(0)
+    lds_barrier();  // the tile is complete, and the other buffer has been read by every wave
+    PROBE(1)
     if (t0 + kTileKeys > sm.kv_len || t0 < lo_valid) {  // uniform: clean the values of keys that are not held
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
@@ -1132,63 +940,147 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
       }
       lds_barrier();
     }
-    if (ti + 2 < ti_hi) request(ti + 2, k_pages, true, k_asked);
-    if (ti + 1 < ti_hi) request(ti + 1, v_pages, false, v_asked);
-    if constexpr (kScalarPages) {  // (past the last tile: ids of the last held page, not used)
-      pages_of(ti + 3, true, k_asked);
-      pages_of(ti + 2, false, v_asked);
-    }
+    if (ti + 1 < ti_hi && !window_start(ti + 1)) issue(ti + 1);  // a tile that opens a window of page ids waits for them
 
-    const bool next = mine(ti + 1);
-    const unsigned char* k_next = lds + ((ti + 1) & 1) * TILE_BYTES;
-    if (have) {
-      // what is left of the tile before: its sums under (cur_m, cur_l)
-      const bool any = cur_l > 0.f;
-      if (!__all(any)) {
+    PROBE(2)
+    const bool mine = wave_active && t0 <= wave_last_pos &&
+                      !(window > 0 && t0 + kTileKeys <= wave_first_pos - window + 1);
+    if (mine) {
+      // ---- S^T = K . Q^T ---------------------------------------------------
+      f32x4 s[NB];
+      {
+        constexpr int NS = NB * NC;
+        constexpr int RING = NS < kRing ? NS : kRing;
+        auto k_read = [&](int idx) LS_INLINED -> vec_t {
+          const int row = key_of_row<T>(idx / NC, row16);
+          const int piece = (idx % NC) * 4 + g;
+          const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
+          vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + ((pc + row_rotation<T>(row)) % KPIECES) * 16);
+          if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
+          return kv;
+        };
+        vec_t ring[RING];
 #pragma unroll
-        for (int blk = 0; blk < DB; ++blk)
+        for (int i = 0; i < RING; ++i) ring[i] = k_read(i);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[blk][e] = any ? acc[blk][e] : 0.f;  // (a value that is no number stays out)
+        for (int idx = 0; idx < NS; ++idx) {
+          if (idx % NC == 0) s[idx / NC] = f32x4{0.f, 0.f, 0.f, 0.f};
+          A::mma(s[idx / NC], ring[idx % RING], qv[idx % NC]);
+          if (idx + RING < NS) ring[idx % RING] = k_read(idx + RING);
+        }
       }
-      const float m_new = any ? fmaxf(run.m, cur_m) : run.m;
-      const float a = any ? softmax_exp<T>(run.m - m_new) : 1.f;
-      const float b = any ? softmax_exp<T>(cur_m - m_new) : -0.f;
-      run.l = any ? run.l * a + cur_l * b : run.l;
-      run.m = m_new;
-      cur_m = fmaxf(kNegSentinel, tile_max);
-      if (next) probabilities(k_next, std::true_type{}, cur_m, a, b);
-      else probabilities(k_next, std::false_type{}, cur_m, a, b);
-      cur_l = p_sum;
-      tile_max = kNegSentinel;
-      if (next && all_visible(ti + 1)) {
-        values(v_lds, std::true_type{});
+      PROBE(3)
+      // ---- scale, mask, online softmax --------------------------------------
+      const bool all_visible = t0 + kTileKeys - 1 <= wave_first_pos && r0 + 15 < rows_total &&
+                               (window <= 0 || wave_last_pos - t0 < window);
+      float tile_max = kNegSentinel;
+      if (all_visible) {
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            s[kb][e] = s[kb][e] * scale;
+            tile_max = fmaxf(tile_max, s[kb][e]);
+          }
       } else {
-        if (next) scale_masked(ti + 1);
-        values(v_lds, std::false_type{});
-      }
-      if (next) tile_max = quad16_max(tile_max);
-    } else if (next) {
-      k_start(k_next);
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb) k_block(k_next, kb);
-      scale_masked(ti + 1);
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = t0 + key_of_row<T>(kb, 4 * g + e);
+            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * scale : kMasked;
+            s[kb][e] = v;
+            tile_max = fmaxf(tile_max, v);
+          }
+      }
       tile_max = quad16_max(tile_max);
+      const float m_new = fmaxf(cur.m, tile_max);
+      const float alpha = softmax_exp<T>(cur.m - m_new);
+      float p_sum = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < NB; ++kb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[kb][e] = softmax_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
+        p_sum = p_sum + ((s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]));
+      }
+      p_sum = quad16_sum(p_sum);
+      cur.l = cur.l * alpha + p_sum;
+      cur.m = m_new;
+#pragma unroll
+      for (int blk = 0; blk < DB; ++blk)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cur.acc[blk][e] = cur.acc[blk][e] * alpha;
+      PROBE(4)
+      // ---- O^T += V^T . P^T --------------------------------------------------
+      constexpr int KB16 = VEC / 4;
+      {
+        constexpr int NP = (NB / KB16) * DB;
+        constexpr int RING = NP < kRing ? NP : kRing;
+        auto v_read = [&](int idx) LS_INLINED -> vec_t {
+          const int kb = (idx / DB) * KB16;
+          const int d = (idx % DB) * 16 + row16;
+          vec_t vv;
+#pragma unroll
+          for (int h = 0; h < KB16; ++h) {
+            const int key = key_of_row<T>(kb + h, 4 * g);  // the lane's four keys inside the tile
+            const unsigned char* src = v_lds + ((key / VEC) * D + d) * 16 + (key % VEC) * SZ;
+            if (SZ == 2) {
+              bf16x4 four = *reinterpret_cast<const bf16x4*>(src);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) vv[h * 4 + e] = four[e];
+            } else {
+              f32x4 four = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) vv[h * 4 + e] = four[e];
+            }
+          }
+          return vv;
+        };
+        vec_t ring[RING];
+#pragma unroll
+        for (int i = 0; i < RING; ++i) ring[i] = v_read(i);
+        vec_t pv;
+#pragma unroll
+        for (int idx = 0; idx < NP; ++idx) {
+          if (idx % DB == 0) {
+            const int kb = (idx / DB) * KB16;
+#pragma unroll
+            for (int h = 0; h < KB16; ++h)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) pv[h * 4 + e] = from_f32<T>(s[kb + h][e]);
+          }
+          A::mma(cur.acc[idx % DB], ring[idx % RING], pv);
+          if (idx + RING < NP) ring[idx % RING] = v_read(idx + RING);
+        }
+      }
     }
-    have = next;
+    PROBE(5)
+    if (direct && ((ti + 1) % TILES_PER_SPLIT == 0 || ti + 1 == ti_hi)) {
+      fold_split<T>(run, cur.acc, cur.m, cur.l);
+      cur.reset();
+    }
   }
+
+#ifdef LS_ATTN_PROBE
+  if ((threadIdx.x == 0 || threadIdx.x == 64 * (NW - 1)) && kvh == 0 && part_ml != nullptr) {
+    long long* dst = reinterpret_cast<long long*>(part_ml + (1 << 20)) + (blockIdx.x * 2 + (threadIdx.x ? 1 : 0)) * 10;
+    for (int i = 0; i < 8; ++i) dst[i] = pr_t[i];
+    dst[8] = clock64() - pr_begin;
+    dst[9] = ti_hi - ti_lo;
+  }
+#endif
   if (!row_ok) return;
   if (direct) {
-    fold_split<T>(run, acc, cur_m, cur_l);
     store_output<T>(run, out + (long)(sm.q_off + qi) * ldo + (long)head * D, g);
   } else {
     const int split = item.split_begin;
     const long pr = item.part_base + ((long)kvh * rows_total + r) * item.n_splits + (split - item.split_lo);
     float* pa = part_acc + pr * D;
 #pragma unroll
-    for (int blk = 0; blk < DB; ++blk) *reinterpret_cast<f32x4*>(pa + blk * 16 + 4 * g) = acc[blk];
+    for (int blk = 0; blk < DB; ++blk) *reinterpret_cast<f32x4*>(pa + blk * 16 + 4 * g) = cur.acc[blk];
     if (g == 0) {
-      part_ml[pr * 2] = cur_m;
-      part_ml[pr * 2 + 1] = cur_l;
+      part_ml[pr * 2] = cur.m;
+      part_ml[pr * 2 + 1] = cur.l;
     }
   }
 }
@@ -2405,9 +2297,7 @@ extern "C" int ls_attention_decode(int dtype, const void* qkv, long ld, void* k_
 // 128) or, for steps with so few rows that 128-row blocks would leave CUs without work, four (blocks of 64).
 constexpr int kWideWaves = 8;
 constexpr int kNarrowWaves = 4;
-static size_t wide_lds_bytes(int dtype) {
-  return 4 * (size_t)kTileKeys * D * (dtype == kF32 ? 4 : 2) + 2 * kPageWindow * 16 * sizeof(int);
-}
+static size_t wide_lds_bytes(int dtype) { return 4 * (size_t)kTileKeys * D * (dtype == kF32 ? 4 : 2) + kPageWindow * 16 * sizeof(int); }
 template <typename T, int NW>
 static bool wide_kernel_ready(size_t bytes) {
   static int state = 0;  // 0 unknown, 1 granted, -1 refused
