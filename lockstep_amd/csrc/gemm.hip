@@ -1093,6 +1093,10 @@ static bool ring_takes(int M, int N, int K) {
   return blocks >= 160 ? M >= 8 : blocks >= 96 ? M >= (K >= 2048 ? 17 : 24) : blocks >= 32 && M >= 48;
 }
 
+// Whether the ring kernel's 32-bit byte offsets inside a tile reach every operand: the rows of the largest tile, and what
+// the last stage reads behind the last row.  (Rows further apart go to the other kernels, which form 64-bit addresses.)
+static bool ring_reaches(long ldx, long K, long size) { return (256 * std::max(ldx, K) + 128) * size <= 0xffffffffL; }
+
 // Dynamic LDS beyond 64 KB has to be granted per kernel (once).
 template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS>
 static bool ring_lds_ready(int bytes) {
@@ -1161,7 +1165,7 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   if (norm_w && M > 16) return fail("gemm: the fused norm prologue takes at most 16 rows, got %d", M);
   const int mt_rows = (M + 15) / 16;
   const int col_blocks = (N + 16 * NT - 1) / (16 * NT);
-  if (!norm_w && aligned && ring_takes<T>(M, N, K))
+  if (!norm_w && aligned && ring_reaches(ldx, K, sizeof(T)) && ring_takes<T>(M, N, K))
     return launch_ring<T, EPI>(ring_tile<T>(M, N), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
                                vec_ok, out_cols, 1, act, stream);
   const int xc = kslice / Atom<T>::KCHUNK;  // chunks per slice
@@ -1333,7 +1337,7 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
   // fall to 3.7 TB/s; below that and over smaller weights those are ahead), from 33 rows on in float32.
   const long weight_bytes = (long)N * K * (dtype == kF32 ? 4 : 2);
   const int tiled_from = dtype == kF32 ? 33 : (weight_bytes >= (64L << 20) ? 8 : 17);
-  if (LS_GEMM_SLICES_TILED && aligned && M >= tiled_from && N % 4 == 0) {
+  if (LS_GEMM_SLICES_TILED && aligned && ring_reaches(ldx, K, dtype == kF32 ? 4 : 2) && M >= tiled_from && N % 4 == 0) {
     const int stages_a_slice = kslice / (128 / (dtype == kF32 ? 4 : 2));
     int per = std::min(nslices, std::max(1, (8 + stages_a_slice - 1) / stages_a_slice));
     const int tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64;

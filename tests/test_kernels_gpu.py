@@ -198,6 +198,31 @@ def test_every_tile_of_the_products_has_the_bits_of_few_rows(dtype, k, m, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_of_x_further_apart_than_offsets_of_32_bits_reach(dtype):
+    """64 rows of X that span 4 GiB and more (a view into a wide buffer): the product and its slice sums have the bits of the
+    same rows side by side."""
+    from lockstep_amd.ops import STORE_F32
+
+    size = torch.finfo(dtype).bits // 8
+    ldx, k = (1 << 26) // size + 16, 1024
+    g = torch.Generator(device="cuda").manual_seed(size)
+    near = torch.randn(65, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(4096, k, generator=g, device="cuda") * 0.1).to(dtype)
+    far = torch.empty(64 * ldx + k, dtype=dtype, device="cuda").as_strided((65, k), (ldx, 1))
+    far.copy_(near)
+    out, want = (torch.empty(65, 4096, device="cuda") for _ in range(2))
+    K().gemm(far, w, out, STORE_F32)
+    K().gemm(near, w, want, STORE_F32)
+    assert torch.equal(out, want)
+    sums, expected = (torch.empty(K().gemm_slices_count(k), 64, 4096, device="cuda") for _ in range(2))
+    K().gemm_slices(far[:64], w, sums)
+    K().gemm_slices(near[:64], w, expected)
+    assert torch.equal(sums, expected)
+    del far
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("inter,k", [(4096 + 40, 4096), (16384 + 72, 1024), (25600, 5120)])
 def test_swiglu_with_few_rows_and_many_columns_has_the_same_bits(dtype, inter, k):
     from lockstep_amd.ops import SWIGLU, interleave_gate_up
