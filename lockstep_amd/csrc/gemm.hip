@@ -40,8 +40,9 @@ namespace ls {
 #define LS_GEMM_STREAM 1      // 0: never the streaming kernel
 #endif
 #ifndef LS_GEMM_GROUP_M
-#define LS_GEMM_GROUP_M 4     // row tiles per band of the tile numbering (0: column-major numbering)
+#define LS_GEMM_GROUP_M 4     // row tiles per band of the tile numbering
 #endif
+static_assert(LS_GEMM_GROUP_M > 0, "a band of the tile numbering has a row of tiles at least");
 #ifndef LS_GEMM_READ_AHEAD
 #define LS_GEMM_READ_AHEAD 1  // the tiled kernel reads a stage's second chunk of fragments from LDS before it multiplies the first
 #endif
@@ -897,7 +898,6 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ X
   int id = blockIdx.x;
   const int total_tiles = tiles_m * tiles_n;
   if (total_tiles % 8 == 0) id = (id % 8) * (total_tiles / 8) + id / 8;
-#if LS_GEMM_GROUP_M > 0
   // ... and inside bands of LS_GEMM_GROUP_M row tiles, so that the workgroups that run together on an XCD
   // form a block of tiles with few distinct operand tiles (those stay in the XCD's L2)
   const int band = id / (LS_GEMM_GROUP_M * tiles_n);
@@ -905,10 +905,6 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ X
   const int band_rows = min(LS_GEMM_GROUP_M, tiles_m - band * LS_GEMM_GROUP_M);
   const int tile_m = band * LS_GEMM_GROUP_M + in_band % band_rows;
   const int tile_n = in_band / band_rows;
-#else
-  const int tile_m = id % tiles_m;
-  const int tile_n = id / tiles_m;
-#endif
   const int m_base = tile_m * BM;
   const int n_base = tile_n * BN;
 

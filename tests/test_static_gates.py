@@ -52,3 +52,19 @@ def test_engine_does_not_import_tests_or_working_files():
         code = path.read_text()
         assert "_work" not in code, path
         assert not re.search(r"^\s*(from|import)\s+(tests|plain)\b", code, flags=re.M), path
+
+
+def test_the_products_tile_numbering_refuses_a_band_of_no_rows():
+    """A tuning macro of 0 would be a division by zero in device code."""
+    import shutil
+    import subprocess
+
+    import pytest
+
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).is_file():
+        pytest.skip("no hipcc")
+    check = [hipcc, "--offload-arch=gfx950", "--offload-host-only", "-fsyntax-only", "-std=c++17", str(CSRC / "gemm.hip")]
+    assert subprocess.run(check, capture_output=True).returncode == 0
+    refused = subprocess.run(check + ["-DLS_GEMM_GROUP_M=0"], capture_output=True, text=True)
+    assert refused.returncode != 0 and "static assertion failed" in refused.stderr
