@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ X
 // workgroup on every CU and with as many as it holds (bfloat16, K = 4,096, weights from HBM).  The larger the tile, the
 // fewer operand bytes a product loads; the smaller, the more CUs have one, and the fuller the last round.
 enum RingTile { kRing256x192, kRing256x128, kRing192x192, kRing128x192, kRing192x128, kRing128x128, kRing128x64, kRing64x128,
-                kRing64x64, kRingTiles };
+                kRing64x64, kRingTiles, kRing64x32 = kRingTiles };
 struct RingShape {
   int rows, cols, a_cu;
   float one, full;
@@ -1053,12 +1053,16 @@ constexpr RingShape kRingShapes[kRingTiles] = {
     {192, 128, 1, 0.73f, 0.73f}, {128, 128, 1, 0.58f, 0.58f}, {128, 64, 1, 0.43f, 0.43f},  {64, 128, 2, 0.52f, 0.74f},
     {64, 64, 2, 0.33f, 0.52f}};
 
-// The tile whose rounds of workgroups take least by that table.  (Measured over 48 to 2,048 rows and nine shapes of
-// weights: within 6 % of the best tile nearly everywhere, 15 % at worst.)  float32 has four times the matrix work a byte
-// and takes 64 x 64 tiles, three a CU, throughout (2,000 x 6,144 x 1,024 192 us, 128 x 128 tiles 204).
-template <typename T>
-static int ring_tile(int M, int N) {
-  if (sizeof(T) == 4) return kRing64x64;
+// The tile whose rounds of workgroups take least by that table.  (Every tile forced in turn over 65 to 2,048 rows and nine
+// shapes of weights: within 2 % of the best one everywhere.)  Two rules stand in front of it: up to 64 rows whose rows of
+// weights lie a multiple of 4 KB apart take 64 x 64 tiles (128 such rows asked for together meet in few memory channels: 16 x
+// 32,768 x 4,096 62.6 -> 55.1 us, 16 x 24,576 x 4,096 49.2 -> 45.5; other K 0.9 to 1.05 times as long).  float32 has four times
+// the matrix work a byte and takes 64 x 64 tiles, three a CU (2,000 x 6,144 x 1,024 192 us, 128 x 128 tiles 204), and for up
+// to 64 rows 64 x 32 tiles where every CU gets at most one (64 x 6,144 x 1,024 15.5, 64 x 64 tiles 23.8).
+template <typename T, int EPI>
+static int ring_tile(int M, int N, int K) {
+  if (sizeof(T) == 4) return EPI != kSwiGLU && M <= 64 && (N + 31) / 32 <= compute_units() ? kRing64x32 : kRing64x64;
+  if (M <= 64 && K % 2048 == 0) return kRing64x64;
   const long cus = compute_units();
   int best = 0;
   float least = 0.f;
@@ -1076,17 +1080,38 @@ static int ring_tile(int M, int N) {
 }
 
 // Whether the ring kernel runs a product of aligned operands: more than 64 rows, or so many columns that its 64-column
-// tiles beat the kernels of a wave a slice, which read the rows of X once for 16 columns (measured, us, those kernels /
-// this one: from 8 rows on over 10,240 columns and more: 8 x 10,240 x 5,120 35 / 24, 8 x 24,576 x 4,096 43 / 38, 8 x 151,936 x
-// 1,024 67 / 57 (1 x 24,576 x 4,096 stays); over 6,144 from 17 on at K = 4,096 21.4 / 18.8 (16 rows 18.1 / 19.6), at K =
-// 1,024 from 24 on 8.0 / 7.3 (17 rows 7.0 / 7.3); over 2,048 from 48 on 7.0 / 6.9 at K = 1,024).  float32 multiplies too slowly
-// for 64 rows in place of 33 to pay (33 x 6,144 x 1,024 18 / 23, 64 x 4,096 x 1,024 18 / 23), except over the most columns.
-template <typename T>
+// tiles beat the kernels of a wave a slice, which read the rows of X once for 16 columns.  A stage costs the ring kernel the
+// same at any number of rows, so the line is a number of rows, lower the more columns there are (and for SwiGLU, where a wave
+// of the other kernels holds two weight tiles).  Measured on both sides, us, those kernels / this one:
+//   10,240 columns and more  8 x 10,240 x 5,120 36 / 28, SwiGLU 8 x 24,576 x 4,096 48 / 43, 8 x 151,936 x 1,024 66 / 58
+//   5,057 and more           17 x 6,144 x 5,120 29 / 25, 20 x 6,144 x 1,024 7.9 / 7.6 (17 rows 7.5 / 7.5), 40 x 5,696 x 5,120
+//                            42 / 26; SwiGLU 24 x 8,192 x 4,096 24 / 22, 32 x 6,144 x 1,024 7.6 / 8.0, 40 rows 8.8 / 8.0
+//   1,985 and more           48 x 2,048 x 5,120 25 / 27, 56 rows 27.7 / 27.8, 64 rows 29.5 / 28.3; SwiGLU 48 x 2,048 x 4,096 25 / 21
+// Below 768 of K there are few stages behind the first, which everybody waits for; up to 320 they are all asked for at once:
+//   K = 520                  16 x 10,240 4.9 / 6.0, 32 rows 8.1 / 6.2, 17 x 16,384 8.8 / 7.1, 64 x 5,696 6.0 / 6.4; SwiGLU 17 x
+//                            10,240 6.4 / 6.2, 48 x 6,144 6.2 / 6.3, 56 rows 6.9 / 6.3, 8 x 32,768 12.8 / 11.0
+//   K = 264                  17 x 16,384 6.9 / 5.3, 16 rows 4.3 / 5.2, 48 x 2,048 4.8 / 4.5, 8 x 65,536 12.5 / 11.0; SwiGLU 17 x
+//                            2,048 5.1 / 4.5, 16 rows 4.2 / 4.5
+// float32 multiplies too slowly for 64 rows in place of 32 to pay while the other kernels have a block of 16 columns for every
+// CU and no more (33 x 4,096 x 1,024 12.9 / 15.2); beyond that they take a second round (32 x 5,120 x 1,024 18.1 / 15.3, 64 x
+// 10,240 x 5,120 203 / 103; K = 264: 32 x 10,240 7.8 / 9.3, 33 rows 16.5 / 9.4), for SwiGLU and for 17 to 31 rows later (SwiGLU
+// 33 x 16,384 x 1,024 31 / 26, 17 x 32,768 x 1,024 53 / 39).
+template <typename T, int EPI>
 static bool ring_takes(int M, int N, int K) {
   if (M > 64) return true;
   const int blocks = (N + 63) / 64;
-  if (sizeof(T) == 4) return blocks >= 256 && M > 32;
-  return blocks >= 160 ? M >= 8 : blocks >= 96 ? M >= (K >= 2048 ? 17 : 24) : blocks >= 32 && M >= 48;
+  constexpr bool GATED = EPI == kSwiGLU;
+  if (sizeof(T) == 4) {
+    if (GATED) return blocks >= 256 && M > 32;
+    return M >= (K >= 512 ? 32 : 33) ? (N + 15) / 16 > compute_units() : M > 16 && blocks >= 512;
+  }
+  if (K < 768) {
+    if (GATED) return blocks >= 32 && M >= (blocks >= 512 ? 8 : K <= 320 || blocks >= 160 ? 17 : 56);
+    return blocks >= 256 ? M >= (blocks >= 1024 ? 8 : 17) : blocks >= 90 ? M >= 32 : blocks >= 32 && K <= 320 && M >= 48;
+  }
+  if (blocks >= 160) return M >= 8;
+  if (blocks >= 80) return M >= (GATED ? (K >= 2048 ? 24 : 40) : K >= 2048 ? 17 : 20);
+  return blocks >= 32 && M >= (GATED ? 48 : 56);
 }
 
 // Whether the ring kernel's 32-bit byte offsets inside a tile reach every operand: the rows of the largest tile, and what
@@ -1126,6 +1151,8 @@ static int launch_ring(int tile, const T* X, const T* W, void* C, int M, int N, 
 #define LS_RING(...) \
   return launch_ring_tile<T, EPI, __VA_ARGS__>(X, W, C, M, N, K, ldx, ldc, kslice, vec_ok, out_cols, groups, act, stream)
   if constexpr (sizeof(T) == 4) {
+    if constexpr (EPI != kSwiGLU && EPI != kSliceSums)
+      if (tile == kRing64x32) LS_RING(64, 32, 2, 2, 5, 5);
     LS_RING(64, 64, 2, 2, 3, 3);
   } else if constexpr (EPI == kSliceSums) {
     LS_RING(64, 64, 4, 2, 5, 5);
@@ -1161,9 +1188,14 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   if (norm_w && M > 16) return fail("gemm: the fused norm prologue takes at most 16 rows, got %d", M);
   const int mt_rows = (M + 15) / 16;
   const int col_blocks = (N + 16 * NT - 1) / (16 * NT);
-  if (!norm_w && aligned && ring_reaches(ldx, K, sizeof(T)) && ring_takes<T>(M, N, K))
-    return launch_ring<T, EPI>(ring_tile<T>(M, N), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
+  const bool ring = aligned && ring_reaches(ldx, K, sizeof(T));
+  if (!norm_w && ring && ring_takes<T, EPI>(M, N, K))
+    return launch_ring<T, EPI>(ring_tile<T, EPI>(M, N, K), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
                                vec_ok, out_cols, 1, act, stream);
+  // What the ring kernel cannot take goes to the tiled kernel from 33 rows on (SwiGLU from 17) where its tiles give every CU a
+  // workgroup, and from 17 on over the most columns (operands off 16 bytes, the kernels of a wave a slice / tiles, us: 17 x
+  // 32,800 x 1,024 151 / 87, 64 x 32,800 x 1,024 336 / 111).
+  const bool tiles = !ring && ((N + 63) / 64 >= compute_units() && (M > 32 || (M > 16 && EPI == kSwiGLU)));
   const int xc = kslice / Atom<T>::KCHUNK;  // chunks per slice
   // The streaming kernel where a workgroup would get more than one column block: a CU holds 16 waves
   // of it (one per K slice), so 16 / nslices workgroups.
@@ -1173,7 +1205,7 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   const int group_tiles = mt_rows <= 2 ? mt_rows : 2;
   const size_t stream_lds = 2 * (size_t)nslices * NT * group_tiles * 256 * sizeof(float);  // two sets of slice sums
   // (with fewer than eight slices the skinny kernel's small workgroups, several a CU, do as well or better)
-  if (!norm_w && mt_rows <= 4 && xc % 4 == 0 && xc * group_tiles <= 16 && nslices >= 8 && nslices <= 16 &&
+  if (!norm_w && mt_rows <= 4 && !tiles && xc % 4 == 0 && xc * group_tiles <= 16 && nslices >= 8 && nslices <= 16 &&
       col_blocks * row_groups > stream_wgs && stream_lds <= 128 * 1024 && LS_GEMM_STREAM) {
     int walkers = stream_wgs / row_groups;
     const int rounds = (col_blocks + walkers - 1) / walkers;
@@ -1195,7 +1227,7 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
 #undef LS_STREAM
     if (launched) return check_launch("gemm");
   }
-  if (M <= 64) {
+  if (M <= 64 && !tiles && (ring || M <= 16 || N < 32768)) {
     const int mt = (M + 15) / 16;
     // 16 waves leave 128 registers a lane: only for one or two row tiles
     const int nw = (nslices > 8 && mt * NT <= 2) ? 16 : (nslices > 4 ? 8 : 4);
@@ -1274,6 +1306,15 @@ extern "C" int ls_gemm_xielu(int dtype, const void* X, const void* W, void* C, i
 }
 
 extern "C" int ls_gemm_kslice(int K) { return ls::kslice_for(K); }
+
+// The tile (enum RingTile) that ls_gemm gives the ring kernel for a product of aligned operands; -1: another kernel's.
+extern "C" int ls_gemm_ring_tile(int dtype, int epilogue, int M, int N, int K) {
+  using namespace ls;
+#define LS_TILE(T_, EPI_) (ring_takes<T_, EPI_>(M, N, K) ? ring_tile<T_, EPI_>(M, N, K) : -1)
+  if (dtype == kF32) return epilogue == kSwiGLU ? LS_TILE(float, kSwiGLU) : LS_TILE(float, kStore);
+  return epilogue == kSwiGLU ? LS_TILE(bf16_t, kSwiGLU) : LS_TILE(bf16_t, kStore);
+#undef LS_TILE
+}
 
 // Number of K slices of a product over K (the first dimension of the partial sums of ls_gemm_slices).
 extern "C" int ls_gemm_slices_count(int K) {

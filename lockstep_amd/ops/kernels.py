@@ -258,6 +258,11 @@ class Kernels:
             c_int(DTYPE_CODE[w.dtype]), _ptr(x), _ptr(w), _ptr(out), c_int(m), c_int(n), c_int(k), c_long(x.stride(0)),
             c_long(out.stride(0)), _ptr(act), _stream()))
 
+    def gemm_ring_tile(self, dtype: torch.dtype, epilogue: int, m: int, n: int, k: int) -> int:
+        """Which tile of the ring kernel a product of these sizes (and of 16-byte aligned operands) takes: its place in
+        ``RingTile`` of gemm.hip, -1 where another kernel computes it."""
+        return int(self.core.ls_gemm_ring_tile(c_int(DTYPE_CODE[dtype]), c_int(epilogue), c_int(m), c_int(n), c_int(k)))
+
     def gemm_slices_count(self, k: int) -> int:
         """K slices of a product over ``k`` (first dimension of ``gemm_slices``'s output)."""
         return self._memo(("slices", k), lambda: int(self.core.ls_gemm_slices_count(c_int(k))))

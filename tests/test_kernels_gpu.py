@@ -222,6 +222,96 @@ def test_rows_of_x_further_apart_than_offsets_of_32_bits_reach(dtype):
     torch.cuda.empty_cache()
 
 
+# (rows, columns) that take each tile of the ring kernel, in the order of RingTile, with both ending inside a tile
+RING_TILE_SIZES = [(2041, 4448), (1003, 6176), (1501, 5408), (1003, 5408), (700, 5408), (500, 4128), (130, 5472), (300, 5472), (97, 96)]
+
+
+@pytest.mark.parametrize("k", [72, 328])
+@pytest.mark.parametrize("m,n", RING_TILE_SIZES)
+def test_every_ring_tile_with_every_epilogue_has_the_bits_of_few_rows(m, n, k):
+    """Each tile by the name that the dispatch gives it, K that ends inside the second stage and inside a slice."""
+    from lockstep_amd.ops import ADD_F32, STORE, STORE_F32, SWIGLU
+
+    dtype = torch.bfloat16
+    tile = RING_TILE_SIZES.index((m, n))
+    assert [K().gemm_ring_tile(dtype, e, m, n, k) for e in (STORE, STORE_F32, ADD_F32, SWIGLU)] == [tile] * 4
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+    base = torch.randn(m, n, generator=g, device="cuda")
+    act = torch.tensor([0.8, 0.3], device="cuda")
+
+    def run(epilogue, rows):
+        out = (base[rows].clone() if epilogue == ADD_F32 else
+               torch.empty(rows.stop - rows.start, n // 2 if epilogue == SWIGLU else n, device="cuda",
+                           dtype=torch.float32 if epilogue == STORE_F32 else dtype))
+        if epilogue == "xielu":
+            K().gemm_xielu(x[rows], w, out, act)
+        else:
+            K().gemm(x[rows], w, out, epilogue)
+        return out
+
+    for epilogue in (STORE, STORE_F32, ADD_F32, SWIGLU, "xielu"):
+        full = run(epilogue, slice(0, m))
+        for first in (0, m // 2, m - 5):
+            rows = slice(first, first + 5)
+            assert torch.equal(run(epilogue, rows), full[rows]), (epilogue, first)
+
+
+# (rows, columns, K, whether SwiGLU) on both sides of the lines between the ring kernel and the others, and the tile it takes
+RING_LINES = {
+    torch.float32: [(33, 4096, 72, False, -1), (33, 4112, 72, False, 9), (32, 4112, 508, False, -1), (32, 4112, 512, False, 9), (31, 4112, 512, False, -1),
+                    (64, 8192, 264, False, 9), (64, 8193, 264, False, 8),
+                    (32, 32704, 72, False, -1), (17, 32705, 72, False, 8), (16, 32768, 72, False, -1), (32, 16384, 72, True, -1),
+                    (33, 16352, 72, True, 8), (33, 16320, 72, True, -1)],
+    torch.bfloat16: [(47, 1985, 320, False, -1), (48, 1985, 320, False, 8), (64, 1985, 328, False, -1), (31, 5697, 520, False, -1),
+                     (32, 5697, 520, False, 8), (16, 16321, 520, False, -1), (17, 16321, 520, False, 8), (7, 65473, 72, False, -1),
+                     (8, 65473, 72, False, 7), (16, 2016, 72, True, -1), (17, 2016, 72, True, 8), (16, 10208, 520, True, -1),
+                     (17, 10208, 520, True, 8), (55, 5088, 520, True, -1), (56, 5088, 520, True, 8), (7, 32736, 520, True, -1),
+                     (8, 32736, 520, True, 7), (7, 10240, 768, False, -1), (8, 10240, 768, False, 8), (19, 5057, 768, False, -1),
+                     (20, 5057, 768, False, 8), (16, 5057, 2048, False, -1), (17, 5057, 2048, False, 8), (55, 1985, 768, False, -1),
+                     (56, 1985, 768, False, 8), (23, 5088, 2048, True, -1), (24, 5088, 2048, True, 8), (39, 5088, 1024, True, -1),
+                     (40, 5088, 1024, True, 8), (47, 2016, 768, True, -1), (48, 2016, 768, True, 8), (64, 32768, 1024, False, 7),
+                     (64, 32768, 2048, False, 8)],
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_products_on_both_sides_of_the_lines_between_the_kernels_have_the_same_bits(dtype):
+    from lockstep_amd.ops import STORE_F32, SWIGLU
+
+    for m, n, k, gated, tile in RING_LINES[dtype]:
+        epilogue = SWIGLU if gated else STORE_F32
+        assert K().gemm_ring_tile(dtype, epilogue, m, n, k) == tile, (m, n, k, gated)
+        g = torch.Generator(device="cuda").manual_seed(m + n + k)
+        x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+        w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+        out = torch.empty(m, n // 2 if gated else n, dtype=dtype if gated else torch.float32, device="cuda")
+        K().gemm(x, w, out, epilogue)
+        for first in range(0, m, 5):
+            part = torch.empty_like(out[first:first + 5])
+            K().gemm(x[first:first + 5], w, part, epilogue)
+            assert torch.equal(part, out[first:first + 5]), (m, n, k, gated, first)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,k,gated", [(16352, 200, False), (16352, 200, True), (32768 + 40, 96, False), (32768, 72, True)])
+def test_products_off_a_16_byte_boundary_with_few_rows_have_the_bits_of_aligned_ones(dtype, n, k, gated):
+    """Weights one element behind a 16-byte boundary: 17 to 64 rows over so many columns go to tiles, fewer to a wave a slice."""
+    from lockstep_amd.ops import STORE_F32, SWIGLU
+
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    x = torch.randn(64, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+    off = torch.empty(n * k + 8, dtype=dtype, device="cuda")[1:1 + n * k].view(n, k)
+    off.copy_(w)
+    for m in (5, 16, 17, 32, 33, 64):
+        a, b = (torch.empty(m, n // 2 if gated else n, dtype=dtype if gated else torch.float32, device="cuda") for _ in range(2))
+        K().gemm(x[:m], w, a, SWIGLU if gated else STORE_F32)
+        K().gemm(x[:m], off, b, SWIGLU if gated else STORE_F32)
+        assert torch.equal(a, b), m
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("inter,k", [(4096 + 40, 4096), (16384 + 72, 1024), (25600, 5120)])
 def test_swiglu_with_few_rows_and_many_columns_has_the_same_bits(dtype, inter, k):
