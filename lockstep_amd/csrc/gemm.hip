@@ -1131,13 +1131,16 @@ static bool ring_lds_ready(int bytes) {
   return granted;
 }
 
+constexpr int kNotLaunched = 1;  // the LDS was refused: the caller has another kernel
+constexpr int kMutantNoRing = 16;  // bit of the controls' mask (common.h): that refusal, as a test wants it
+
 // groups: workgroups along K (kSliceSums: out_cols slices each); otherwise 1.
 template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS>
 static int launch_ring_tile(const T* X, const T* W, void* C, int M, int N, int K, long ldx, long ldc, int kslice, int vec_ok,
                             int out_cols, int groups, const float* act, hipStream_t stream) {
   constexpr int kBytes = (WS * BN + XS * BM) * 128;
   static_assert(kBytes <= 160 * 1024, "the rings fit the LDS of a CU");
-  if (!ring_lds_ready<T, EPI, BM, BN, NWM, NWN, WS, XS>(kBytes)) return fail("gemm: %d bytes of LDS were refused", kBytes);
+  if (LS_MUTANT_HOST(kMutantNoRing) || !ring_lds_ready<T, EPI, BM, BN, NWM, NWN, WS, XS>(kBytes)) return kNotLaunched;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   hipLaunchKernelGGL((gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS>), dim3(tiles_m * tiles_n, groups),
                      dim3(64 * NWM * NWN), kBytes, stream, X, W, C, M, N, K, ldx, ldc, kslice, vec_ok, tiles_m, tiles_n,
@@ -1188,10 +1191,13 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   if (norm_w && M > 16) return fail("gemm: the fused norm prologue takes at most 16 rows, got %d", M);
   const int mt_rows = (M + 15) / 16;
   const int col_blocks = (N + 16 * NT - 1) / (16 * NT);
-  const bool ring = aligned && ring_reaches(ldx, K, sizeof(T));
-  if (!norm_w && ring && ring_takes<T, EPI>(M, N, K))
-    return launch_ring<T, EPI>(ring_tile<T, EPI>(M, N, K), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
-                               vec_ok, out_cols, 1, act, stream);
+  bool ring = aligned && ring_reaches(ldx, K, sizeof(T));
+  if (!norm_w && ring && ring_takes<T, EPI>(M, N, K)) {
+    const int rc = launch_ring<T, EPI>(ring_tile<T, EPI>(M, N, K), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
+                                       vec_ok, out_cols, 1, act, stream);
+    if (rc != kNotLaunched) return rc;
+    ring = false;
+  }
   // What the ring kernel cannot take goes to the tiled kernel from 33 rows on (SwiGLU from 17) where its tiles give every CU a
   // workgroup, and from 17 on over the most columns (operands off 16 bytes, the kernels of a wave a slice / tiles, us: 17 x
   // 32,800 x 1,024 151 / 87, 64 x 32,800 x 1,024 336 / 111).
@@ -1382,13 +1388,16 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
     while (per > 1 && workgroups(per) < compute_units()) per = (per + 1) / 2;
     if (workgroups(per) >= compute_units()) {
       const int groups_y = (nslices + per - 1) / per;
+      int rc;
       if (dtype == kF32)
-        return launch_ring<float, kSliceSums>(kRing64x64, (const float*)X, (const float*)W, P, M, N, K, ldx, N, kslice, 1, per,
-                                              groups_y, nullptr, s);
-      if (dtype == kBF16)
-        return launch_ring<bf16_t, kSliceSums>(kRing64x64, (const bf16_t*)X, (const bf16_t*)W, P, M, N, K, ldx, N, kslice, 1,
-                                               per, groups_y, nullptr, s);
-      return fail("gemm_slices: unknown dtype %d", dtype);
+        rc = launch_ring<float, kSliceSums>(kRing64x64, (const float*)X, (const float*)W, P, M, N, K, ldx, N, kslice, 1, per,
+                                            groups_y, nullptr, s);
+      else if (dtype == kBF16)
+        rc = launch_ring<bf16_t, kSliceSums>(kRing64x64, (const bf16_t*)X, (const bf16_t*)W, P, M, N, K, ldx, N, kslice, 1,
+                                             per, groups_y, nullptr, s);
+      else
+        return fail("gemm_slices: unknown dtype %d", dtype);
+      if (rc != kNotLaunched) return rc;
     }
   }
   // More than 16 rows and enough columns that workgroups of 64 columns fill the GPU: the wide kernel.

@@ -150,7 +150,7 @@ class Kernels:
 
     #: bits of ``set_mutants`` (csrc/common.h)
     MUTANT_KSLICE_BY_ROWS, MUTANT_NORM_BY_ROWS, MUTANT_SAMPLE_CHUNKS_BY_ROWS = 1, 2, 4      # core library
-    MUTANT_REVERSED_FOLD_IN_PRODUCT = 8
+    MUTANT_REVERSED_FOLD_IN_PRODUCT, MUTANT_NO_RING = 8, 16
     MUTANT_REVERSED_FOLD = 1                               # attention libraries
 
     def set_mutants(self, core: int = 0, attention: int = 0) -> None:

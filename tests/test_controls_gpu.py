@@ -87,6 +87,26 @@ def test_k_blocking_that_depends_on_the_rows_of_a_launch_is_caught(control_kerne
         assert (product(40) - full[:40]).abs().max() < 1e-2          # another order of the same sum, nothing else
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_products_whose_rings_get_no_lds_go_to_the_other_kernels(control_kernels, dtype):
+    from lockstep_amd.ops import STORE_F32
+
+    k = control_kernels
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(200, 1024, generator=g).to(dtype).cuda()
+    for n in (272, 4096, 32768):
+        w = torch.randn(n, 1024, generator=g).to(dtype).cuda()
+        for rows in (17, 33, 64, 200):
+            with_ring, without = (torch.empty(rows, n, device="cuda") for _ in range(2))
+            sums, sums_without = (torch.empty(k.gemm_slices_count(1024), rows, n, device="cuda") for _ in range(2))
+            k.gemm(x[:rows], w, with_ring, STORE_F32)
+            k.gemm_slices(x[:rows], w, sums)
+            with mutant(k, core=k.MUTANT_NO_RING):
+                k.gemm(x[:rows], w, without, STORE_F32)
+                k.gemm_slices(x[:rows], w, sums_without)
+            assert torch.equal(without, with_ring) and torch.equal(sums_without, sums), (n, rows)
+
+
 def test_a_norm_whose_order_depends_on_the_rows_of_a_launch_is_caught(control_kernels):
     k = control_kernels
     g = torch.Generator().manual_seed(4)
