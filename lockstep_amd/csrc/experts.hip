@@ -507,13 +507,13 @@ __global__ __launch_bounds__(256) void experts_gate_up_kernel(const T* __restric
 }
 
 // A tile of an expert that returns its input: P[choice][token][c] = share * x[token][c] for the columns [c0, c1), the
-// routing weight multiplying the input or the output alike.
-template <typename T>
+// routing weight multiplying the input or the output alike.  THREADS: those of the workgroup, each element one thread's.
+template <typename T, int THREADS>
 __device__ __forceinline__ void pass_input(const T* __restrict__ x, long ldx, const float* __restrict__ share, int first, int rows,
                                            int c0, int c1, int top, int n_tokens, int N, const int* __restrict__ order,
                                            float* __restrict__ P) {
   const int width = c1 - c0;
-  for (int i = threadIdx.x; i < rows * width; i += 256) {
+  for (int i = threadIdx.x; i < rows * width; i += THREADS) {
     const int pair = order[first + i / width], c = c0 + i % width;
     P[((long)(pair % top) * n_tokens + pair / top) * N + c] = share[pair] * to_f32(x[(long)(pair / top) * ldx + c]);
   }
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
   }
   if (e >= real) {   // (the whole workgroup)
     constexpr int kCols = KS == 1 ? 64 : 16;
-    pass_input<T>(x, ldx, share, first, rows, blockIdx.y * kCols, min(N, (int)(blockIdx.y + 1) * kCols), top, n_tokens, N, order, P);
+    pass_input<T, 256>(x, ldx, share, first, rows, blockIdx.y * kCols, min(N, (int)(blockIdx.y + 1) * kCols), top, n_tokens, N, order, P);
     return;
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -764,7 +764,7 @@ __global__ __launch_bounds__(512) void experts_down_ring_kernel(const T* __restr
   const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
   const int col0 = blockIdx.x * 128;
   if (e >= real) {
-    pass_input<T>(x, ldx, share, first, rows, col0, min(N, col0 + 128), top, n_tokens, N, order, P);
+    pass_input<T, 512>(x, ldx, share, first, rows, col0, min(N, col0 + 128), top, n_tokens, N, order, P);
     return;
   }
   const int mine = min((int)(threadIdx.x >> 3), rows - 1);

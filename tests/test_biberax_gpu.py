@@ -333,6 +333,37 @@ def test_the_order_of_many_pairs_is_the_stable_sort_by_expert(pairs, experts):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width, ff", [(8, 8), (64, 72), (136, 200), (1032, 264)])
+def test_experts_that_return_their_input_in_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
+    """Experts without weights beside one with weights, with 1, 64, 65 and 200 tokens, columns that end inside a tile:
+    every element of their outputs is written."""
+    g = torch.Generator().manual_seed(width)
+    k = K()
+    sizes = [70, 1, 64, 65, 200]
+    tokens, experts = sum(sizes), len(sizes)
+    owner = torch.repeat_interleave(torch.arange(experts), torch.tensor(sizes))[torch.randperm(tokens, generator=g)]
+    logits = torch.randn(tokens, experts, generator=g)
+    logits[torch.arange(tokens), owner] = 9.0
+    x = torch.randn(tokens, width, generator=g).to(dtype).cuda()
+    gate, up, down = ((torch.randn(1, *shape, generator=g) * 0.3).to(dtype).cuda() for shape in ((ff, width), (ff, width), (width, ff)))
+    results = []
+    for rows in (32, 64):
+        cap = k.experts_tile_capacity(tokens, experts, 2, rows)
+        i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+        chosen, order, tiles, counts = i32(2 * tokens), i32(2 * tokens), i32(4 * cap), i32(experts)
+        share = torch.empty(2 * tokens, device="cuda")
+        k.experts_route(logits.cuda(), torch.zeros(experts).cuda(), 2, rows, chosen, share, order, tiles, counts)
+        act = torch.full((2 * tokens, ff), float("nan"), dtype=dtype, device="cuda")
+        partials = torch.full((2, tokens, width), float("nan"), device="cuda")
+        k.experts_apply(x, gate, up, down, 2, rows, order, tiles, share, 1.3, 1.702, act, partials, identity=experts - 1)
+        results.append(partials)
+        back = chosen.view(tokens, 2) > 0
+        want = share.view(tokens, 2)[..., None] * x.float()[:, None]
+        assert torch.equal(partials.transpose(0, 1)[back], want[back])
+    assert torch.equal(results[0], results[1]) and not torch.isnan(results[1]).any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width, ff", [(8, 8), (64, 72), (72, 128), (136, 200), (1032, 264)])
 def test_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
     """The products of row tiles of 64 read both operands through LDS, those of 32 rows from memory, and both are one
