@@ -265,15 +265,19 @@ __device__ __forceinline__ void place_pairs(const int* expert, int p0, int p1, i
   }
 }
 
-// Many pairs: a workgroup an expert, whose sixteen waves take a sixteenth of the pairs each.  What bounds both launches is
-// the latency of reading the picks, so the reads are spread over many waves; the second counts a wave's share again,
+// Many pairs: a workgroup an expert, whose waves take equal shares of the pairs.  What bounds both launches is the
+// latency of reading the picks, so the reads are spread over up to sixteen waves; the second counts a wave's share again,
 // because the place of a share follows from the shares before it.  8,192 pairs of 32 experts: 5.0 us to count and 5.1 to
 // place, where one wave an expert took 12.2 and 12.7.
 __device__ __forceinline__ int my_share(int P, int w, int& p1) {
-  const int share = (P + 1023) / 1024 * 64, p0 = min(w * share, P);
+  const int group = blockDim.x;  // 64 pairs a wave
+  const int share = (P + group - 1) / group * 64, p0 = min(w * share, P);
   p1 = min(p0 + share, P);
   return p0;
 }
+// Waves an expert: one for every 256 pairs.  (Sixteen from 513 pairs on crowd the card where there are many experts: the whole
+// routing of 520 pairs by 512 experts took 17.4 us, one wave an expert 14.8, so 14.7; of 1,024 pairs by 64 experts 9.7, 10.0, 9.4.)
+static int route_waves(int P) { return P >= 16 * 256 ? 16 : (P + 255) / 256; }
 
 __global__ __launch_bounds__(1024) void route_count_kernel(const int* __restrict__ expert, int P, int* __restrict__ counts) {
   __shared__ int mine_s[16];
@@ -285,7 +289,7 @@ __global__ __launch_bounds__(1024) void route_count_kernel(const int* __restrict
   __syncthreads();
   if (threadIdx.x == 0) {
     int sum = 0;
-    for (int i = 0; i < 16; ++i) sum += mine_s[i];
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) sum += mine_s[i];
     counts[blockIdx.x] = sum;
   }
 }
@@ -849,8 +853,8 @@ extern "C" int ls_experts_route(const float* z, long ldz, const float* bias, int
   else { LS_ROUTE(kMaxPerLane) }
 #undef LS_ROUTE
   if (!(P <= kSmallPairs && E <= kSmallExperts)) {
-    hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(1024), 0, s, expert, P, counts);
-    hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(1024), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
+    hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(64 * route_waves(P)), 0, s, expert, P, counts);
+    hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(64 * route_waves(P)), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
   }
   return check_launch("experts_route");
 }
@@ -909,8 +913,8 @@ extern "C" int ls_experts_route_table(const int* token_ids, const int* table, in
   } else {
     hipLaunchKernelGGL(route_table_kernel, dim3((P + 255) / 256), dim3(256), 0, s, token_ids, table, n_tokens, top, expert,
                        weight);
-    hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(1024), 0, s, expert, P, counts);
-    hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(1024), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
+    hipLaunchKernelGGL(route_count_kernel, dim3(E), dim3(64 * route_waves(P)), 0, s, expert, P, counts);
+    hipLaunchKernelGGL(route_place_kernel, dim3(E), dim3(64 * route_waves(P)), 0, s, expert, counts, P, E, rows_a_tile, order, tiles, cap);
   }
   return check_launch("experts_route_table");
 }

@@ -332,6 +332,28 @@ def test_the_order_of_many_pairs_is_the_stable_sort_by_expert(pairs, experts):
     assert tiles.reshape(-1, 4).tolist() == listed
 
 
+@pytest.mark.parametrize("experts, top, tokens", [(512, 2, 257), (64, 1, 1023), (64, 1, 1024), (64, 1, 1025), (7, 3, 1365), (9, 1, 4095),
+                                                   (9, 1, 4097), (300, 8, 1000)])
+def test_the_order_of_pairs_with_every_number_of_waves_an_expert(experts, top, tokens):
+    """514 pairs (three waves) to 8,000 (sixteen): the pairs sorted by expert, in their order within one, and the tiles."""
+    g = torch.Generator().manual_seed(tokens)
+    k = K()
+    logits = torch.randn(tokens, experts, generator=g)
+    pairs, cap = tokens * top, k.experts_tile_capacity(tokens, experts, top, 16)
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    chosen, order, tiles, counts = i32(pairs), i32(pairs), i32(4 * cap), i32(experts)
+    k.experts_route(logits.cuda(), None, top, 16, chosen, torch.empty(pairs, device="cuda"), order, tiles, counts)
+    assert torch.equal(chosen.view(tokens, top).cpu().long(), logits.topk(top, dim=1).indices)
+    assert torch.equal(order.long(), torch.sort(chosen.long(), stable=True).indices)
+    assert torch.equal(counts.long(), torch.bincount(chosen.long(), minlength=experts))
+    want, at = [], 0
+    for e, n in enumerate(counts.tolist()):
+        want += [[e, at + i, min(16, n - i), 0] for i in range(0, n, 16)]
+        at += n
+    got = tiles.view(cap, 4).tolist()
+    assert got[:len(want)] == want and all(row[0] == -1 for row in got[len(want):])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width, ff", [(8, 8), (64, 72), (136, 200), (1032, 264)])
 def test_experts_that_return_their_input_in_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
