@@ -467,7 +467,7 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
   struct Operands {
     u32x4_t q[R / 4], k[R / 4], g[CH ? R / 4 : 1];
     unsigned v;
-    u32x2_t gate;  // beta, decay
+    u32x2_t gate;  // beta, decay (CH: beta alone, see fetch)
   };
   // the first token of the block, and bytes from a token to the next
   const float* qk_at = qk + ((long)m.q_off * 2 * G + kh) * dp;
@@ -489,12 +489,15 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
       if constexpr (CH) x.g[j] = __builtin_amdgcn_raw_buffer_load_b128(db, q_off + 16 * j, t * d_step, 0);
     }
     x.v = __builtin_amdgcn_raw_buffer_load_b32(vb, v_off, t * v_step, 0);
-    x.gate = __builtin_amdgcn_raw_buffer_load_b64(gb, zero, t * g_step, 0);
+    // (a second word that nobody reads would be a register the compiler uses for something else while the load is still on
+    // its way to it, behind a wait for every load in flight)
+    if constexpr (CH) x.gate[0] = __builtin_amdgcn_raw_buffer_load_b32(gb, zero, t * g_step, 0);
+    else x.gate = __builtin_amdgcn_raw_buffer_load_b64(gb, zero, t * g_step, 0);
   };
   float o4[4] = {};  // the lane's part of the output of the token that was worked on last
   auto token = [&](const Operands& now) LS_INLINED {
     auto of = [](const u32x4_t (&x)[R / 4], int r) LS_INLINED { return __uint_as_float(x[r >> 2][r & 3]); };
-    const float beta = __uint_as_float(now.gate[0]), decay = __uint_as_float(now.gate[1]);
+    const float beta = __uint_as_float(now.gate[0]), decay = CH ? 1.0f : __uint_as_float(now.gate[1]);
     // a lane's rows in four interleaved chains (rows r, r + 4, ... of each), added as (0 + 1) + (2 + 3)
     float ks4[4] = {0.f, 0.f, 0.f, 0.f};
     if constexpr (CH) {

@@ -24,6 +24,8 @@ WIDE_MAY_SPILL = {"attention_wide_kernelIfLi8E": {80: 160, 96: 312, 112: 472, 12
                   "attention_wide_kernelIfLi4E": {144: 216}, "attention_wide_kernelIDF16bLi8E": {144: 192}}
 # ... and registers a lane with which two workgroups of eight waves share a CU
 WIDE_REGISTERS = {"attention_wide_kernelIDF16bLi8E": {16: 128, 32: 128}}
+# recurrences of one wave a workgroup, whose registers let two waves share a SIMD
+TWO_WAVES = ("delta_rule_kernel",)
 MAY_SPILL_AT_HEAD_256 = ("attention_",)               # every float instance at a head size of 256, and some bfloat16
 # sink attention with keys of more than 256 or values of more than 128 elements (a library of such a shape is built when a
 # model first asks for it): correct, not fast, or the instances of four row tiles, which only measurements use
@@ -85,6 +87,8 @@ def test_no_kernel_calls_a_function_and_only_known_ones_spill():
             name = kernel[".name"]
             assert not kernel.get(".uses_dynamic_stack", False), f"{lib.name}: {name} calls a function"
             scratch = kernel.get(".private_segment_fixed_size", 0)
+            if any(part in name for part in TWO_WAVES):
+                assert kernel[".vgpr_count"] <= 256, f"{lib.name}: {name}"
             for part, limits in WIDE_REGISTERS.items():
                 if part in name:
                     assert kernel[".vgpr_count"] <= limits.get(head, 512), f"{lib.name}: {name}"
