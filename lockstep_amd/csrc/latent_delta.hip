@@ -433,8 +433,10 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // by one vector load at the same address in every lane (as scalar loads, which return in any order, a wait for one would
 // be a wait for all, also for those of the tokens ahead).
 // DEPTH: the tokens whose operands are on their way.  2,048 tokens (16 heads over 8, 128 x 128): 270 us; with lane
-// pointers, a conditional step of each, and a branch a token it took 490.  Where requests bring a token or two, two are
-// enough and leave room for twice the waves: eight requests decoding 28 -> 13 us.
+// pointers, a conditional step of each, and a branch a token it took 490.  Where the longest request brings a token or two,
+// two are enough and leave room for twice the waves: eight requests decoding 28 -> 13 us.  Where most requests decode beside
+// a longer one, the longest's chain counts as much as the room: four (63 requests of one token and one of 64, two / four / eight
+// ahead, convolution included: 64 x 64 48 / 39 / 38 us, 128 x 128 114 / 113 / 130, 192 x 128 143 / 95 / 100).
 template <int R, int L, bool CH, int DEPTH>
 __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict__ qk, const float* __restrict__ vv,
                                                         const float* __restrict__ gates, const float* __restrict__ decays,
@@ -716,11 +718,12 @@ extern "C" long ls_delta_scratch_floats_channel(int n_tokens, int G, int H, int 
   return ls_delta_scratch_floats(n_tokens, G, H, D, DV) + (long)n_tokens * H * ls_delta_padded_dim(D);
 }
 
-extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int H, int D, int DV, int M,
-                             const float* taps, const float* a_log, const float* dt_bias, float unit_eps,
-                             const int* tok_seq, const int* tok_pos, const void* seqs, int n_seqs, float* state,
-                             long state_stride, float* scratch, float* out, long ldo, const float* chan, long ldc,
-                             void* stream) {
+// longest: the most tokens that one request brings, 0 if the caller does not know (it decides the time, not the result).
+extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, int G, int H, int D, int DV, int M,
+                                     const float* taps, const float* a_log, const float* dt_bias, float unit_eps,
+                                     const int* tok_seq, const int* tok_pos, const void* seqs, int n_seqs, float* state,
+                                     long state_stride, float* scratch, float* out, long ldo, const float* chan, long ldc,
+                                     int longest, void* stream) {
   // chan [T][ldc] (or null): the logits of a decay a head and key channel, H * D a token; dt_bias then has H * D
   // entries, raw needs no `a` columns, and the scratch is that of ls_delta_scratch_floats_channel.
   LS_REQUIRE(!chan || ldc >= (long)H * D, "delta_rule: the channel decays' rows are too short");
@@ -744,15 +747,18 @@ extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int
   hipLaunchKernelGGL(delta_prep_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, raw, ld, n_tokens, G, H, D, DV,
                      dp, M, taps, a_log, dt_bias, unit_eps, tok_seq, tok_pos, (const SeqMeta*)seqs, state, state_stride,
                      conv_at, qk, vv, gates, chan, ldc, decays);
+  const int most = longest > 0 ? longest : n_tokens;
 #define LS_DELTA_RULE(R_, L_, CH_, DEPTH_)                                                                               \
   hipLaunchKernelGGL((delta_rule_kernel<R_, L_, CH_, DEPTH_>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
                      gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo)
 #define LS_DELTA(R_, L_)                                                          \
   do {                                                                            \
-    if (n_tokens <= 2 * n_seqs) {                                                 \
+    if (most <= 2) {                                                              \
       if (chan) LS_DELTA_RULE(R_, L_, true, 2); else LS_DELTA_RULE(R_, L_, false, 2); \
     } else if (chan) {                                                            \
       LS_DELTA_RULE(R_, L_, true, 4);                                             \
+    } else if (n_tokens <= 2 * n_seqs) {                                          \
+      LS_DELTA_RULE(R_, L_, false, 4);                                            \
     } else {                                                                      \
       LS_DELTA_RULE(R_, L_, false, R_ <= 8 ? 8 : 4);                              \
     }                                                                             \
@@ -770,4 +776,13 @@ extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int
     hipLaunchKernelGGL(delta_conv_state_kernel, dim3(n_seqs, (unsigned)((C + 255) / 256)), dim3(256), 0, s, raw, ld, (int)C,
                        M, (const SeqMeta*)seqs, state, state_stride, conv_at);
   return check_launch("delta_rule");
+}
+
+extern "C" int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int H, int D, int DV, int M,
+                             const float* taps, const float* a_log, const float* dt_bias, float unit_eps,
+                             const int* tok_seq, const int* tok_pos, const void* seqs, int n_seqs, float* state,
+                             long state_stride, float* scratch, float* out, long ldo, const float* chan, long ldc,
+                             void* stream) {
+  return ls_delta_rule_longest(raw, ld, n_tokens, G, H, D, DV, M, taps, a_log, dt_bias, unit_eps, tok_seq, tok_pos, seqs, n_seqs,
+                               state, state_stride, scratch, out, ldo, chan, ldc, 0, stream);
 }

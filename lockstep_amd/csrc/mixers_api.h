@@ -118,6 +118,12 @@ int ls_delta_rule(const float* raw, long ld, int n_tokens, int G, int H, int D, 
                   const float* a_log, const float* dt_bias, float unit_eps, const int* tok_seq, const int* tok_pos,
                   const void* seqs, int n_seqs, float* state, long state_stride, float* scratch, float* out, long ldo,
                   const float* chan, long ldc, void* stream);
+// The same by a caller that knows the most tokens that one request brings (0: it does not): `longest` decides how many
+// tokens' operands are asked for ahead, not the result.
+int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, int G, int H, int D, int DV, int M, const float* taps,
+                          const float* a_log, const float* dt_bias, float unit_eps, const int* tok_seq, const int* tok_pos,
+                          const void* seqs, int n_seqs, float* state, long state_stride, float* scratch, float* out, long ldo,
+                          const float* chan, long ldc, int longest, void* stream);
 
 // Between two sublayers of a residual stream X [.][width] float (see sublayers.hip): y = P[0][row] + P[1][row] + ...;
 // x = X[row] + norm(y) (post_w null: + y); results[keep][row] = x (results [.][r_rows][width] or null); x = the sum of

@@ -1443,7 +1443,7 @@ class Kernels:
 
     def delta_rule(self, raw: torch.Tensor, kv_heads: int, heads: int, dim: int, vdim: int, taps: torch.Tensor, a_log,
                    dt_bias, unit_eps: float, tok_seq, tok_pos, seqs, n_seqs: int, state: torch.Tensor,
-                   scratch: torch.Tensor, out: torch.Tensor, channel_decay: torch.Tensor | None = None) -> None:
+                   scratch: torch.Tensor, out: torch.Tensor, channel_decay: torch.Tensor | None = None, longest: int = 0) -> None:
         """The gated delta rule over the tokens of every request of the step.  ``raw`` float32 holds the
         projections ``q | k`` (``kv_heads`` heads of ``dim``) ``| v`` (``heads`` of ``vdim``) ``| b | a``
         (``heads`` each); every channel of q, k and v passes a causal convolution with ``taps [channels, M]``
@@ -1453,7 +1453,8 @@ class Kernels:
         float32 ``[slots, heads*dim*vdim + (M-1)*channels]``: the matrices, then the convolutions' last inputs;
         read and left for the next step.  ``out`` float32 ``[T, heads*vdim]``.  ``channel_decay`` (float32 rows of
         ``heads*dim`` logits): a decay for every head and key channel instead, ``g = exp(-exp(a_log_h) softplus(logit +
-        dt_bias))`` with ``dt_bias [heads*dim]``, which multiplies the rows of ``S``; ``raw`` then ends with ``b``."""
+        dt_bias))`` with ``dt_bias [heads*dim]``, which multiplies the rows of ``S``; ``raw`` then ends with ``b``.
+        ``longest``: the most tokens that one request brings, if the caller knows (a hint: it decides the time)."""
         _rows_ok(raw, "delta_rule raw"); _rows_ok(out, "delta_rule out")
         t = raw.shape[0]
         channels = 2 * kv_heads * dim + heads * vdim
@@ -1487,11 +1488,11 @@ class Kernels:
         if n_seqs == 0 or t == 0:
             return
         lib = self.mixers_lib()
-        self._launch(lib, lib.ls_delta_rule, (
+        self._launch(lib, lib.ls_delta_rule_longest, (
             _ptr(raw), c_long(raw.stride(0)), c_int(t), c_int(kv_heads), c_int(heads), c_int(dim), c_int(vdim), c_int(m),
             _ptr(taps), _ptr(a_log), _ptr(dt_bias), c_float(unit_eps), _ptr(tok_seq), _ptr(tok_pos), _ptr(seqs),
             c_int(n_seqs), _ptr(state), c_long(state.stride(0)), _ptr(scratch), _ptr(out), c_long(out.stride(0)),
-            _ptr(channel_decay), c_long(ldc), _stream()))
+            _ptr(channel_decay), c_long(ldc), c_int(longest), _stream()))
 
     # -- an embedding with a table of token pairs, and the shift of a sublayer's input by a token -------------
     def embed_pair(self, tokens: torch.Tensor, tok_seq, tok_pos, seqs, table: torch.Tensor, pairs: torch.Tensor,

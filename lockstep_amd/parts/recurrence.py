@@ -294,7 +294,8 @@ class GatedDelta(Mixer):
             gate = ctx.buf("delta.gate_f32", (t, n * dv), torch.float32)
             k.gemm(low[:, self.low_gate_at:], self.w_g2, gate, STORE_F32)
         k.delta_rule(raw, g, n, d, dv, self.conv, self.a_log, self.dt_bias, self.unit_eps, ctx.tok_seq, ctx.tok_pos,
-                     ctx.seqs, ctx.n_seqs, ctx.cache.unit_state(run.cache), scratch, o, channel_decay=decay_logits)
+                     ctx.seqs, ctx.n_seqs, ctx.cache.unit_state(run.cache), scratch, o, channel_decay=decay_logits,
+                     longest=int(ctx.q_len.max()))
         gated = ctx.buf("delta.normed", (t, n * dv), rt.dtype)
         k.head_norm_gate(o, n, dv, self.norm, gate, self.eps, gated, gate_act=self.gate_act)
         return project_out(ctx, gated, self.w_o, out, accumulate, defer, "delta.out_slices")

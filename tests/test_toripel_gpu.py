@@ -273,6 +273,38 @@ def test_the_delta_rule_has_the_same_bits_however_many_tokens_a_step_brings(head
         assert all(torch.equal(a, b) for a, b in zip(outs, whole)), most
 
 
+@pytest.mark.parametrize("heads, groups, d, dv", [(2, 1, 16, 17), (2, 2, 30, 5), (1, 1, 64, 64), (4, 2, 128, 20), (1, 1, 200, 9)])
+@pytest.mark.parametrize("channel_decays", [False, True])
+def test_the_delta_rule_has_the_same_bits_whatever_it_is_told_of_the_longest_request(heads, groups, d, dv, channel_decays):
+    """Many requests of one token beside a longer one: two, four or eight tokens ahead, as the caller names the longest request
+    or not; each against the longer request alone."""
+    g = torch.Generator().manual_seed(d + dv)
+    channels = 2 * groups * d + heads * dv
+    conv = (torch.randn((channels, 2), generator=g) * 0.5).cuda()
+    a_log = torch.randn(heads, generator=g).cuda()
+    dt_bias = torch.randn(heads * d if channel_decays else heads, generator=g).cuda()
+    k = K()
+
+    def run(counts, raw, chan, longest):
+        state = torch.zeros((len(counts), heads * d * dv + channels), dtype=torch.float32, device="cuda")
+        tok_seq, tok_pos, seqs = step_meta(counts, [0] * len(counts), list(range(len(counts))))
+        out = torch.full((sum(counts), heads * dv), float("nan"), dtype=torch.float32, device="cuda")
+        size = k.delta_scratch_floats(sum(counts), groups, heads, d, dv, channel_decays)
+        k.delta_rule(raw, groups, heads, d, dv, conv, a_log, dt_bias, 1e-6, tok_seq, tok_pos, seqs, len(counts), state,
+                     torch.empty(size, dtype=torch.float32, device="cuda"), out, chan, longest)
+        return out, state
+
+    for long in (2, 3, 5, 9, 13):
+        counts = [1] * 13 + [long]
+        n = sum(counts)
+        raw = torch.randn((n, channels + (1 if channel_decays else 2) * heads), generator=g).cuda()
+        chan = torch.randn((n, heads * d), generator=g).cuda() if channel_decays else None
+        alone, after = run([long], raw[13:], chan[13:] if channel_decays else None, long)
+        for told in (0, 1, long, 1000):
+            out, state = run(counts, raw, chan, told)
+            assert torch.equal(out[13:], alone) and torch.equal(state[13], after[0]), (long, told)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("tokens, experts, top, width, ff", [(1, 4, 2, 32, 24), (37, 7, 3, 64, 40), (300, 5, 1, 48, 16),
                                                               (700, 3, 3, 32, 8)])
