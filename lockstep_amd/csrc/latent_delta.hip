@@ -477,7 +477,7 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
   const float* g_at = gates + ((long)m.q_off * H + head) * 2;
   const float* d_at = CH ? decays + ((long)m.q_off * H + head) * dp : nullptr;
   float* o_at = out + (long)m.q_off * ldo + head * DV;
-  const int qk_step = 2 * G * dp * 4, v_step = H * DV * 4, g_step = H * 8, d_step = H * dp * 4, o_step = (int)ldo * 4;
+  const int qk_step = 2 * G * dp * 4, v_step = H * DV * 4, g_step = H * 8, d_step = H * dp * 4, o_step = DEPTH > 1 ? (int)ldo * 4 : 0;
   const int q_off = row0 * 4, k_off = (G * dp + row0) * 4, v_off = (col_ok ? col : 0) * 4;
   const int o_off = part == 0 && col_ok ? col * 4 : kNowhere;
   int zero = 0;
@@ -736,7 +736,6 @@ extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, in
   LS_REQUIRE(raw && taps && a_log && dt_bias && tok_seq && tok_pos && seqs && state && scratch && out,
              "delta_rule: null operand");
   LS_REQUIRE(reinterpret_cast<uintptr_t>(scratch) % 16 == 0, "delta_rule: the scratch must be 16-byte aligned");
-  LS_REQUIRE(n_tokens == 1 || ldo < (1L << 26), "delta_rule: rows of the output are too far apart");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int dp = ls_delta_padded_dim(D);
   float* qk = scratch;
@@ -748,12 +747,15 @@ extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, in
                      dp, M, taps, a_log, dt_bias, unit_eps, tok_seq, tok_pos, (const SeqMeta*)seqs, state, state_stride,
                      conv_at, qk, vv, gates, chan, ldc, decays);
   const int most = longest > 0 ? longest : n_tokens;
+  const bool far = ldo >= (1L << 26);  // output rows that a block's 32-bit offsets do not reach: a block of one token
 #define LS_DELTA_RULE(R_, L_, CH_, DEPTH_)                                                                               \
   hipLaunchKernelGGL((delta_rule_kernel<R_, L_, CH_, DEPTH_>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
                      gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo)
 #define LS_DELTA(R_, L_)                                                          \
   do {                                                                            \
-    if (most <= 2) {                                                              \
+    if (far) {                                                                    \
+      if (chan) LS_DELTA_RULE(R_, L_, true, 1); else LS_DELTA_RULE(R_, L_, false, 1); \
+    } else if (most <= 2) {                                                       \
       if (chan) LS_DELTA_RULE(R_, L_, true, 2); else LS_DELTA_RULE(R_, L_, false, 2); \
     } else if (chan) {                                                            \
       LS_DELTA_RULE(R_, L_, true, 4);                                             \

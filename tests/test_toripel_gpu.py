@@ -305,6 +305,31 @@ def test_the_delta_rule_has_the_same_bits_whatever_it_is_told_of_the_longest_req
             assert torch.equal(out[13:], alone) and torch.equal(state[13], after[0]), (long, told)
 
 
+@pytest.mark.parametrize("channel_decays", [False, True])
+def test_the_delta_rule_writes_rows_any_distance_apart(channel_decays):
+    """Output rows 256 MiB apart (a view into a wide buffer) get the bits of rows side by side."""
+    heads, groups, d, dv, counts = 2, 1, 30, 5, [4, 1]
+    g = torch.Generator().manual_seed(7)
+    channels = 2 * groups * d + heads * dv
+    conv = (torch.randn((channels, 2), generator=g) * 0.5).cuda()
+    a_log = torch.randn(heads, generator=g).cuda()
+    dt_bias = torch.randn(heads * d if channel_decays else heads, generator=g).cuda()
+    raw = torch.randn((5, channels + (1 if channel_decays else 2) * heads), generator=g).cuda()
+    chan = torch.randn((5, heads * d), generator=g).cuda() if channel_decays else None
+    tok_seq, tok_pos, seqs = step_meta(counts, [0, 0], [0, 1])
+    k = K()
+    results = []
+    for stride in (heads * dv, (1 << 26) + 2):
+        out = torch.empty(4 * stride + heads * dv, device="cuda").as_strided((5, heads * dv), (stride, 1))
+        state = torch.zeros((2, heads * d * dv + channels), device="cuda")
+        scratch = torch.empty(k.delta_scratch_floats(5, groups, heads, d, dv, channel_decays), device="cuda")
+        k.delta_rule(raw, groups, heads, d, dv, conv, a_log, dt_bias, 1e-6, tok_seq, tok_pos, seqs, 2, state, scratch, out, chan)
+        results.append((out.clone(memory_format=torch.contiguous_format), state))
+        del out
+    torch.cuda.empty_cache()
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("tokens, experts, top, width, ff", [(1, 4, 2, 32, 24), (37, 7, 3, 64, 40), (300, 5, 1, 48, 16),
                                                               (700, 3, 3, 32, 8)])
