@@ -32,8 +32,8 @@ TOL = {torch.float32: 2e-5, torch.bfloat16: 1.5e-2}
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (1, 1000, 96), (5, 48, 200), (16, 100, 64), (17, 33, 72),
                                    (64, 256, 1024), (65, 130, 260), (37, 3072, 1024), (200, 96, 4100),
                                    (130, 1000, 8), (3, 40, 12),
-                                   # 128 x 128 tiles with rows, columns and K that end inside a tile (operand
-                                   # loads from clamped addresses), and the same with K not 16-byte aligned
+                                   # tiles of 192 x 128 with rows, columns and K that end inside a tile, and the same
+                                   # with K not 16-byte aligned
                                    (2050, 2100, 264), (2050, 2100, 260),
                                    # an odd K: no operand row is 16-byte aligned, in either precision
                                    (200, 90, 101), (9, 50, 37)])
@@ -60,11 +60,11 @@ def test_gemm_matches_linear(dtype, m, n, k):
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_row_does_not_depend_on_the_batch(dtype):
     """Row i alone, in a 16-row batch, in a 64-row batch and in a 300-row batch:
-    same bits (the skinny and the tiled kernel share one summation order)."""
+    same bits (the kernels of few and of many rows share one summation order)."""
     from lockstep_amd.ops import STORE_F32
 
     g = torch.Generator().manual_seed(7)
-    # the last shape has so many columns that 17 to 64 rows already take the tiled kernel
+    # the last shape has so many columns that 17 to 64 rows already take the ring kernel
     for k, n in ((1024, 272), (3072, 96), (200, 130), (5000, 64), (96, 32768 + 40)):
         x = torch.randn(300, k, generator=g).to(dtype).cuda()
         w = torch.randn(n, k, generator=g).to(dtype).cuda()
@@ -82,10 +82,10 @@ def test_gemm_row_does_not_depend_on_the_batch(dtype):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("k,n", [(4096, 4096 + 24), (1000, 16384 + 24), (5120, 4096 + 104), (260, 32768 + 40),
-                                 # slices of 512 and some 7,000 columns: from 32 rows on tiles of 64 x 32 outputs
+                                 # slices of 512 and some 7,000 columns: tiles of 64 x 64 outputs (float32 64 x 32) from 17 and 32 rows on
                                  (5120, 7168 + 24), (1000, 6144 + 8),
                                  (2048, 8192 + 8), (96, 65536 + 48),
-                                 # K of 5,120 over so many columns that tiles of 64 x 128 give every CU one
+                                 # K of 5,120 over so many columns that tiles of 64 x 128 give every CU one (bfloat16)
                                  (5120, 36864 + 72)])
 def test_gemm_with_few_rows_and_many_columns_has_the_same_bits(dtype, k, n):
     """With up to 64 rows and more column blocks than the GPU holds workgroups, a workgroup walks
@@ -120,8 +120,8 @@ def test_gemm_with_few_rows_and_many_columns_has_the_same_bits(dtype, k, n):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("k", [264, 1088])
 def test_gemm_with_many_rows_and_columns_has_the_bits_of_few_rows(dtype, k):
-    """2,050 rows by 3,740 columns: 17 x 15 tiles of 128 x 256 outputs fill one round of 256 CUs, so
-    bfloat16 takes the workgroups of eight waves; rows, columns and (with 264) K end inside a tile.
+    """2,050 rows by 3,740 columns: 11 x 20 tiles of 192 x 192 outputs fit one round of 256 CUs, so
+    bfloat16 takes those (float32 64 x 64 tiles); rows, columns and (with 264) K end inside a tile.
     Every epilogue; rows from all over the product have the bits they have in a product of 40 rows,
     which the skinny kernel computes."""
     from lockstep_amd.ops import ADD_F32, STORE, STORE_F32, SWIGLU, interleave_gate_up
@@ -160,8 +160,8 @@ def test_gemm_with_many_rows_and_columns_has_the_bits_of_few_rows(dtype, k):
 @pytest.mark.parametrize("m,n", [(2041, 6152), (2041, 4091), (1501, 6139), (1003, 6139), (1501, 4088), (1003, 4096), (1003, 2044),
                                  (64, 32700), (300, 1000), (65, 16), (130, 3)])
 def test_every_tile_of_the_products_has_the_bits_of_few_rows(dtype, k, m, n):
-    """Sizes that take each tile of the ring kernel (256 x 192 down to 64 x 64 outputs), with rows and columns that end inside
-    a tile, K of less than a stage, K that ends inside a stage and inside a slice, and columns that no vector store fits:
+    """Sizes over the tiles of the ring kernel (bfloat16: all but 256 x 192 with a plain epilogue, see the test of every tile by
+    name; float32: 64 x 64), with rows and columns that end inside a tile, K of less than a stage, K that ends inside a stage and inside a slice, and columns that no vector store fits:
     five rows at a time, which the kernels of a wave a slice compute, have the same bits."""
     from lockstep_amd.ops import ADD_F32, STORE, STORE_F32, SWIGLU
 
@@ -335,7 +335,7 @@ def test_swiglu_with_few_rows_and_many_columns_has_the_same_bits(dtype, inter, k
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("k", [1024, 4096, 5120])
 def test_the_full_vocabulary_head_against_double_precision(dtype, k):
-    """151,936 columns (the streaming kernel for few rows, tiles of 64 x 128 up to 64 rows, large tiles
+    """151,936 columns (the streaming kernel for few rows, tiles of 64 rows up to 64 rows, larger ones
     beyond) at 1, 8, 64 and 200 rows: every row equals the double-precision product and has the
     same bits at every number of rows."""
     from lockstep_amd.ops import STORE_F32
