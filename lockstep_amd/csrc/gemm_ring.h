@@ -1,12 +1,12 @@
 // The tiled product of gemm.hip: BM x BN outputs a workgroup, both operands through LDS, and a ring of
 // stages that the memory writes into LDS by itself (buffer loads with LDS as their target), so that a stage
-// takes no register and no instruction of its own on its way and up to three stages are in flight.
+// takes no register and no instruction of its own on its way; a ring of n stages has n - 1 of them in flight.
 //
 // What bounds it: a workgroup's stage (128 bytes of K of all its rows) has to arrive before anyone may
 // multiply it, and takes 1 to 2 us from the memory side; a CU's 160 KB of LDS hold two to five stages, so the
-// larger the tile, the more multiplications stand behind a byte in flight.  Counters (256 x 128 tiles, 2,048 x
-// 24,576 x 4,096): the matrix pipe is busy 47 % of the time, LDS 24 %, no bank conflicts; the clock falls to 1.9
-// GHz under this load.  Measured against the register-staged kernel that was here before (bfloat16, weights from
+// larger the tile, the more multiplications stand behind a byte in flight.  Counters (256 x 192 tiles, 2,048 x
+// 24,576 x 4,096): of the cycles that a CU is busy the matrix pipe is busy 56 %, LDS 24 %, no bank conflicts; the clock falls
+// to 1.9 GHz under this load.  Measured against the register-staged kernel that was here before (bfloat16, weights from
 // HBM, us): 2,048 x 24,576 x 4,096 471 -> 341 (1,210 TFLOP/s), 2,048 x 6,144 x 4,096 142 -> 86, 2,048 x 4,096 x
 // 12,288 218 -> 164 (1,255), 999 x 4,096 x 4,096 64 -> 38, 97 x 4,096 x 1,024 10.0 -> 7.0; float32 2,000 x
 // 1,024 x 2,048 90 -> 71 (118 TFLOP/s).

@@ -19,6 +19,9 @@ __device__ __forceinline__ u32x4_t buffer_of(const void* p, long bytes) {
   return r;
 }
 
+// (Naming m0 keeps the compiler from relying on a value of its own there; that it warns of the name is all the diagnostic says.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 // Sixteen bytes a lane from buffer + lane_off + off straight into LDS: the wave's 64 pieces land at lds_base + 16 *
 // lane.  The instruction itself, because the compiler would wait for the compiler's own form of it in front of every
 // later LDS read.  The whole offset goes through the vector register: the buffer's bound counts that one for certain.
@@ -29,6 +32,7 @@ __device__ __forceinline__ void buffer_to_lds16(unsigned lane_off, unsigned off,
                    : "v"(lane_off), "s"(off), "s"(buffer), "s"(lds_base)
                    : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 template <int YOUNGER>  // loads issued after those that are waited for
 __device__ __forceinline__ void wait_loads() {
