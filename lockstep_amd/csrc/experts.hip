@@ -26,6 +26,7 @@
 #include "common.h"
 #include "ring.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace ls {
@@ -966,10 +967,12 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
                        (const T_*)w_down, N, F, top, n_tokens, order, tiles, out_weight, P, (const T_*)x, ldx, weight, real, \
                        shared_of((T_*)nullptr));                                                                      \
   } while (0)
-  // tiles of 64 rows go through LDS where every row of every operand starts on a 16-byte boundary (and an offset into x
-  // fits 32 bits, and the tiles a grid's second dimension)
+  // tiles of 64 rows go through LDS where every row of every operand starts on a 16-byte boundary, 32-bit offsets reach the
+  // rows (all of x, whose rows are picked; 64 of the weights and of act) and what the last stage reads behind them, and the
+  // tiles fit a grid's second dimension.  Rows further apart go to the kernel that forms 64-bit addresses.
+  const long across = 64 * std::max({(long)K, (long)F, ldy}), all_of_x = (n_tokens - 1) * ldx + K;
   const bool staged = rows_a_tile == 64 && K % vec == 0 && F % vec == 0 && ldx % vec == 0 && ldy % vec == 0 &&
-                      (long)n_tokens * ldx < (1L << 29) && cap < 65536 && ring_lds_ready(dtype);
+                      std::max(across, all_of_x) * (16 / vec) + 128 <= 0xffffffffL && cap < 65536 && ring_lds_ready(dtype);
 #define LS_EXPERTS_STAGED(T_)                                                                                         \
   do {                                                                                                                \
     hipLaunchKernelGGL(experts_gate_up_ring_kernel<T_>, dim3((F + 63) / 64, cap), dim3(512), kRingLds, s, (const T_*)x, \

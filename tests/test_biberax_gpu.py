@@ -386,6 +386,39 @@ def test_experts_that_return_their_input_in_tiles_of_64_rows_have_the_bits_of_ti
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("far_rows", ["x", "act"])
+def test_rows_of_experts_further_apart_than_offsets_of_32_bits_reach(dtype, far_rows):
+    """64 rows of the input, or of the activations, that span 4 GiB and more (views into wide buffers), in tiles of 64 rows:
+    the bits of rows side by side."""
+    tokens, width, ff, size = 65, 136, 72, torch.finfo(dtype).bits // 8
+    g = torch.Generator().manual_seed(size)
+    k = K()
+    stride = (1 << 26) // size + 16
+    wide = torch.empty(64 * stride + width, dtype=dtype, device="cuda")
+    near = torch.randn(tokens, width, generator=g).to(dtype).cuda()
+    gate, up, down = ((torch.randn(1, *shape, generator=g) * 0.3).to(dtype).cuda() for shape in ((ff, width), (ff, width), (width, ff)))
+    cap = k.experts_tile_capacity(tokens, 1, 1, 64)
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    chosen, order, tiles, counts, share = i32(tokens), i32(tokens), i32(4 * cap), i32(1), torch.empty(tokens, device="cuda")
+    k.experts_route(torch.zeros(tokens, 1).cuda(), None, 1, 64, chosen, share, order, tiles, counts)
+    results = []
+    for far in (False, True):
+        x, act = near, torch.full((tokens, ff), float("nan"), dtype=dtype, device="cuda")
+        if far and far_rows == "x":
+            x = wide.as_strided((tokens, width), (stride, 1))
+            x.copy_(near)
+        elif far:
+            act = wide.as_strided((tokens, ff), (stride, 1))
+        partials = torch.full((1, tokens, width), float("nan"), device="cuda")
+        k.experts_apply(x, gate, up, down, 1, 64, order, tiles, share, 1.3, 1.702, act, partials)
+        results.append(partials)
+        del x, act
+    del wide
+    torch.cuda.empty_cache()
+    assert torch.equal(results[0], results[1]) and not torch.isnan(results[0]).any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width, ff", [(8, 8), (64, 72), (72, 128), (136, 200), (1032, 264)])
 def test_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
     """The products of row tiles of 64 read both operands through LDS, those of 32 rows from memory, and both are one
