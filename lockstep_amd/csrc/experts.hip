@@ -617,28 +617,31 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
 // The same two products for tiles of 64 rows (many tokens an expert), both operands through a ring of three stages in
 // LDS (128 bytes of K a row, written there by the loads themselves; layout, waits and barriers as gemm_ring.h describes
 // them).  A workgroup of eight waves takes 64 rows by 128 weight rows: 64 gate and the 64 up rows of the same columns, or
-// 128 columns of the down product; two workgroups share a CU.  A row's contraction is still one chain over ascending
+// 128 columns of the down product (float32: 64); two workgroups share a CU.  A row's contraction is still one chain over ascending
 // chunks from zero: the same bits as the kernels above give without a cut of K.  Measured against tiles staged through
 // registers (64 x 64 by four waves; 2,048 tokens with 4 of 32 experts, width 1,024, 768 a piece): gate and up 94 -> 65
 // us (395 TFLOP/s), down 65 -> 52.  What bounds it now is the L2: 855 MB of requests in gate and up, 13 TB/s, three
 // quarters of them hits.  Four neighbouring tiles kept on one XCD, so that an expert's weights reach an L2 once, moved
 // this by no more than the runs differ (67 and 50 us): a row tile of 64 asks for too many bytes an operation.
 // ---------------------------------------------------------------------------
-constexpr int kRingRows = 64, kRingWeights = 128, kRingStages = 3;
-constexpr int kRingLds = kRingStages * (kRingRows + kRingWeights) * 128;
-template <typename T, bool PAIRED>  // PAIRED: a wave's two weight tiles lie 64 rows apart (gate, up), else side by side
+constexpr int kRingRows = 64, kRingStages = 3;
+constexpr int ring_lds(int weights) { return kRingStages * (kRingRows + weights) * 128; }
+// WEIGHTS: weight rows, 128 or 64 (two tiles a wave or one).  PAIRED: a wave's two weight tiles lie 64 rows apart (gate,
+// up), else side by side.
+template <typename T, int WEIGHTS, bool PAIRED>
 struct RingProduct {
   typedef typename Atom<T>::vec_t vec_t;
   static constexpr int BK = 128 / (int)sizeof(T), S = kRingStages;
-  static constexpr int W_BYTES = kRingWeights * 128, X_BYTES = kRingRows * 128;
-  static constexpr int LOADS = 3;  // a wave's loads a stage: eight rows of X, twice eight of W
-  f32x4 acc[2][2];                 // [weight tile][row tile]
+  static constexpr int W_BYTES = WEIGHTS * 128, X_BYTES = kRingRows * 128;
+  static constexpr int TI = WEIGHTS / 64;  // weight tiles a wave
+  static constexpr int LOADS = 1 + TI;     // a wave's loads a stage: eight rows of X, TI times eight of W
+  f32x4 acc[TI][2];                        // [weight tile][row tile]
 
   // row and column of this lane's outputs acc[i][j][0..3] inside the workgroup's tile
   static __device__ __forceinline__ int row_of(int j) { return ((threadIdx.x >> 8) & 1) * 32 + j * 16 + (threadIdx.x & 15); }
   static __device__ __forceinline__ int weight_of(int i) {
     const int w4 = (threadIdx.x >> 6) & 3;
-    return PAIRED ? i * 64 + w4 * 16 : w4 * 32 + i * 16;
+    return PAIRED ? i * 64 + w4 * 16 : w4 * 16 * TI + i * 16;
   }
 
   // x_off: this lane's row of X (row wave * 8 + lane / 8 of the tile) from the start of its buffer, in bytes; w0, w1: the
@@ -655,22 +658,22 @@ struct RingProduct {
     auto request = [&](int st, int buf) LS_INLINED {
       buffer_to_lds16(x_off, st * 128, x, lds0 + S * W_BYTES + buf * X_BYTES);
       buffer_to_lds16(w_off, st * 128, w0, lds0 + buf * W_BYTES);
-      buffer_to_lds16(w_off, st * 128, w1, lds0 + buf * W_BYTES + 64 * 128);
+      if constexpr (TI == 2) buffer_to_lds16(w_off, st * 128, w1, lds0 + buf * W_BYTES + 64 * 128);
     };
     auto clear_past_k = [&](int buf) LS_INLINED {
       const int first = (K % BK) / Atom<T>::VEC;  // the first piece of a row that lies past K
-      for (int idx = threadIdx.x; idx < (kRingWeights + kRingRows) * 8; idx += 512) {
+      for (int idx = threadIdx.x; idx < (WEIGHTS + kRingRows) * 8; idx += 512) {
         const int row = idx >> 3;
         if (((idx & 7) ^ (row & 7)) < first) continue;
-        unsigned char* at = row < kRingWeights ? ring + buf * W_BYTES + idx * 16
-                                               : ring + S * W_BYTES + buf * X_BYTES + (idx - kRingWeights * 8) * 16;
+        unsigned char* at = row < WEIGHTS ? ring + buf * W_BYTES + idx * 16
+                                               : ring + S * W_BYTES + buf * X_BYTES + (idx - WEIGHTS * 8) * 16;
         *reinterpret_cast<vec_t*>(at) = Atom<T>::zero();
       }
       ring_barrier();
     };
     const unsigned at = row16 * 128 + ((g ^ (row16 & 7)) << 4);
     const int wm = ((wave >> 2) & 1) * 32;
-    vec_t a[2], b[2][2];
+    vec_t a[TI], b[2][2];
     auto read_a = [&](int i, int buf, int c) LS_INLINED {
       a[i] = *reinterpret_cast<const vec_t*>(ring + buf * W_BYTES + weight_of(i) * 128 + (at ^ (c * 64)));
     };
@@ -682,14 +685,14 @@ struct RingProduct {
     auto multiply = [&](const vec_t (&mine)[2], vec_t (&next)[2], int buf, int c) LS_INLINED {
       read_b(next, buf, c);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < TI; ++i) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) Atom<T>::mma(acc[i][j], a[i], mine[j]);
         read_a(i, buf, c);
       }
     };
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -699,8 +702,8 @@ struct RingProduct {
     ring_barrier();
     if (K % BK && stages == 1) clear_past_k(0);
     read_b(b[0], 0, 0);
-    read_a(0, 0, 0);
-    read_a(1, 0, 0);
+#pragma unroll
+    for (int i = 0; i < TI; ++i) read_a(i, 0, 0);
     int buf = 0;
     for (int st = 0; st < stages; ++st) {
       multiply(b[0], b[1], buf, 1);
@@ -730,7 +733,7 @@ __global__ __launch_bounds__(512) void experts_gate_up_ring_kernel(const T* __re
   const int col0 = blockIdx.x * 64;
   const int mine = min((int)(threadIdx.x >> 3), rows - 1);  // (rows past the tile's: the last one again, not stored)
   const long left = (long)(F - col0) * K * sizeof(T), from = ((long)e * F + col0) * K;
-  RingProduct<T, true> product;
+  RingProduct<T, 128, true> product;
   product.run(buffer_of(x, ((long)(n_tokens - 1) * ldx + K) * sizeof(T)), (unsigned)((long)(order[first + mine] / top) * ldx * sizeof(T)),
               buffer_of(w_gate + from, left), buffer_of(w_up + from, left), K, ring);
   const int quad = (threadIdx.x & 63) >> 4;
@@ -754,6 +757,13 @@ __global__ __launch_bounds__(512) void experts_gate_up_ring_kernel(const T* __re
   }
 }
 
+// Columns of the down product a workgroup.  float32 is bound by the matrix cores of the CUs that have a workgroup, so narrow
+// tiles, of which there are more, are never slower (gate and up included, us, 64 / 128 columns: 700 tokens of one expert, width
+// 1,024, 2,048 a piece 112 / 144; 2,048 tokens with 4 of 32 experts, 1,024 and 768 367 / 379; staged through registers 140 and
+// 487).  bfloat16 is bound by the operands that a tile asks for (2,048 tokens of 4,096 and 1,536 a piece 646 / 610).
+template <typename T>
+constexpr int kDownCols = sizeof(T) == 4 ? 64 : 128;
+
 template <typename T>
 __global__ __launch_bounds__(512) void experts_down_ring_kernel(const T* __restrict__ act, long ldy,
                                                                 const T* __restrict__ w_down, int N, int F, int top,
@@ -763,19 +773,20 @@ __global__ __launch_bounds__(512) void experts_down_ring_kernel(const T* __restr
                                                                 const T* __restrict__ x, long ldx,
                                                                 const float* __restrict__ share, int real) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
+  constexpr int COLS = kDownCols<T>;
   const int tile = blockIdx.y;
   const int e = tiles[4 * tile];
   if (e < 0) return;
   const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
-  const int col0 = blockIdx.x * 128;
+  const int col0 = blockIdx.x * COLS;
   if (e >= real) {
-    pass_input<T, 512>(x, ldx, share, first, rows, col0, min(N, col0 + 128), top, n_tokens, N, order, P);
+    pass_input<T, 512>(x, ldx, share, first, rows, col0, min(N, col0 + COLS), top, n_tokens, N, order, P);
     return;
   }
   const int mine = min((int)(threadIdx.x >> 3), rows - 1);
   const T* from = w_down + ((long)e * N + col0) * F;
   const long left = (long)(N - col0) * F * sizeof(T), half = 64L * F * sizeof(T);
-  RingProduct<T, false> product;
+  RingProduct<T, COLS, false> product;
   product.run(buffer_of(act + (long)first * ldy, ((long)(rows - 1) * ldy + F) * sizeof(T)), (unsigned)(mine * ldy * sizeof(T)),
               buffer_of(from, left), buffer_of(from + 64L * F, left > half ? left - half : 0), F, ring);
   const int quad = (threadIdx.x & 63) >> 4;
@@ -787,7 +798,7 @@ __global__ __launch_bounds__(512) void experts_down_ring_kernel(const T* __restr
     const float wt = weight ? weight[pair] : 1.0f;
     float* dst = P + ((long)(pair % top) * n_tokens + pair / top) * N;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < product.TI; ++i) {
       const int c0 = col0 + product.weight_of(i) + 4 * quad;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -807,7 +818,7 @@ extern "C" int ls_experts_max_top() { return kMaxTop; }
 // Dynamic LDS beyond 64 KB has to be granted per kernel (once).
 static bool ring_lds_ready(int dtype) {
   auto grant = [](const void* kernel) {
-    const bool ok = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds) == hipSuccess;
+    const bool ok = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, ring_lds(128)) == hipSuccess;
     if (!ok) (void)hipGetLastError();
     return ok;
   };
@@ -975,12 +986,12 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
                       std::max(across, all_of_x) * (16 / vec) + 128 <= 0xffffffffL && cap < 65536 && ring_lds_ready(dtype);
 #define LS_EXPERTS_STAGED(T_)                                                                                         \
   do {                                                                                                                \
-    hipLaunchKernelGGL(experts_gate_up_ring_kernel<T_>, dim3((F + 63) / 64, cap), dim3(512), kRingLds, s, (const T_*)x, \
+    hipLaunchKernelGGL(experts_gate_up_ring_kernel<T_>, dim3((F + 63) / 64, cap), dim3(512), ring_lds(128), s, (const T_*)x, \
                        ldx, (const T_*)w_gate, (const T_*)w_up, F, K, top, order, tiles, limit, alpha, shift, in_weight, \
                        (T_*)act, ldy, real, n_tokens);                                                                  \
-    hipLaunchKernelGGL(experts_down_ring_kernel<T_>, dim3((N + 127) / 128, cap), dim3(512), kRingLds, s,             \
-                       (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, out_weight, P,      \
-                       (const T_*)x, ldx, weight, real);                                                              \
+    hipLaunchKernelGGL(experts_down_ring_kernel<T_>, dim3((N + kDownCols<T_> - 1) / kDownCols<T_>, cap), dim3(512),  \
+                       ring_lds(kDownCols<T_>), s, (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, \
+                       out_weight, P, (const T_*)x, ldx, weight, real);                                                \
   } while (0)
 #define LS_EXPERTS_BY_ROWS(T_)                 \
   switch (rows_a_tile) {                       \
