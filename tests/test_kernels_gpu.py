@@ -864,6 +864,16 @@ def test_attention_window(dtype, window):
         assert torch.equal(wide, out[lo:p + 1]), f"rows {lo}..{p}, wide kernel"
 
 
+def test_more_row_blocks_than_a_grid_numbers_in_its_second_dimension():
+    """The same three row blocks 22,000 times over (65,535 a launch): all are worked on, the last launch's too."""
+    n, nq, nkv, d = 70, 4, 2, 16
+    qkv = rand_qkv(n, nq, nkv, d, torch.bfloat16, seed=1)
+    case = PagedCase(torch.bfloat16, nq, nkv, d, 16, n, shuffle_seed=7)
+    case.write(qkv.cuda(), 0)
+    want = case.attend(qkv.cuda(), 0, 0.25, variant=1, force_split=False)
+    assert torch.equal(case.attend(qkv.cuda(), 0, 0.25, variant=5, force_split=False, repeat=22000), want)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nq,nkv,d,ps", [(4, 2, 64, 16), (16, 8, 128, 16), (6, 2, 48, 8)])
 @pytest.mark.parametrize("scale", [0.13, -0.13])
