@@ -436,7 +436,9 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // pointers, a conditional step of each, and a branch a token it took 490.  Where the longest request brings a token or two,
 // two are enough and leave room for twice the waves: eight requests decoding 28 -> 13 us.  Where most requests decode beside
 // a longer one, the longest's chain counts as much as the room: four (63 requests of one token and one of 64, two / four / eight
-// ahead, convolution included: 64 x 64 48 / 39 / 38 us, 128 x 128 114 / 113 / 130, 192 x 128 143 / 95 / 100).
+// ahead, convolution included: 64 x 64 48 / 39 / 38 us, 128 x 128 114 / 113 / 130, 192 x 128 143 / 95 / 100).  Else eight, with
+// sixteen rows a lane four (1,024 tokens, 192 x 128 231 us, eight 240), or two where the waves are more than two a SIMD, as
+// many as four leave room for (16 requests of one token and four of 256 98 us, four 165).
 template <int R, int L, bool CH, int DEPTH>
 __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict__ qk, const float* __restrict__ vv,
                                                         const float* __restrict__ gates, const float* __restrict__ decays,
@@ -521,6 +523,16 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
   auto put = [&](auto ob, float o, int j) LS_INLINED {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), ob, o_off, j * o_step, 0);
   };
+  // ... in a whole block every GROUP tokens at once, lane i of a column the i-th of them: a store whose lanes mostly have nothing
+  // to write holds up the loads behind it (four requests of 512 tokens, 16 heads of 128 x 128, with a store a token 231 us, so 212)
+  constexpr int GROUP = L < DEPTH ? L : DEPTH;
+  const int group_off = part < GROUP && col_ok ? part * o_step + col * 4 : kNowhere;
+  float kept = 0.f;
+  auto put_grouped = [&](auto ob, float o, int j) LS_INLINED {
+    kept = part == j % GROUP ? o : kept;
+    if (j % GROUP == GROUP - 1)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(kept), ob, group_off, (j - (GROUP - 1)) * o_step, 0);
+  };
   {
     const auto qkb = buffer(qk_at, kNowhere), vb = buffer(v_at, kNowhere), gb = buffer(g_at, kNowhere), db = buffer(d_at, kNowhere);
 #pragma unroll
@@ -542,12 +554,12 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
     for (int j = 0; j < DEPTH; ++j) {
       const float before = (o4[0] + o4[1]) + (o4[2] + o4[3]);
       token(ring[j]);
-      if (j > 0) put(ob, lanes_sum<L>(before), j - 1);
+      if (j > 0) put_grouped(ob, lanes_sum<L>(before), j - 1);
       __builtin_amdgcn_sched_barrier(0);
       fetch(ring[j], qkb, vb, gb, db, DEPTH + j);
       __builtin_amdgcn_sched_barrier(0);
     }
-    put(ob, lanes_sum<L>((o4[0] + o4[1]) + (o4[2] + o4[3])), DEPTH - 1);
+    put_grouped(ob, lanes_sum<L>((o4[0] + o4[1]) + (o4[2] + o4[3])), DEPTH - 1);
     next_block();
   }
   for (; i0 < n; i0 += DEPTH) {
@@ -747,6 +759,7 @@ extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, in
                      dp, M, taps, a_log, dt_bias, unit_eps, tok_seq, tok_pos, (const SeqMeta*)seqs, state, state_stride,
                      conv_at, qk, vv, gates, chan, ldc, decays);
   const int most = longest > 0 ? longest : n_tokens;
+  const bool mixed = n_tokens <= 2 * n_seqs;  // (and a longer request among them)
   const bool far = ldo >= (1L << 26);  // output rows that a block's 32-bit offsets do not reach: a block of one token
 #define LS_DELTA_RULE(R_, L_, CH_, DEPTH_)                                                                               \
   hipLaunchKernelGGL((delta_rule_kernel<R_, L_, CH_, DEPTH_>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
@@ -755,14 +768,12 @@ extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, in
   do {                                                                            \
     if (far) {                                                                    \
       if (chan) LS_DELTA_RULE(R_, L_, true, 1); else LS_DELTA_RULE(R_, L_, false, 1); \
-    } else if (most <= 2) {                                                       \
+    } else if (most <= 2 || (R_ > 8 && !mixed && (long)n_seqs * H * ((DV * L_ + 63) / 64) > 8L * compute_units())) { \
       if (chan) LS_DELTA_RULE(R_, L_, true, 2); else LS_DELTA_RULE(R_, L_, false, 2); \
-    } else if (chan) {                                                            \
-      LS_DELTA_RULE(R_, L_, true, 4);                                             \
-    } else if (n_tokens <= 2 * n_seqs) {                                          \
-      LS_DELTA_RULE(R_, L_, false, 4);                                            \
+    } else if (mixed) {                                                           \
+      if (chan) LS_DELTA_RULE(R_, L_, true, 4); else LS_DELTA_RULE(R_, L_, false, 4); \
     } else {                                                                      \
-      LS_DELTA_RULE(R_, L_, false, R_ <= 8 ? 8 : 4);                              \
+      if (chan) LS_DELTA_RULE(R_, L_, true, R_ <= 8 ? 8 : 4); else LS_DELTA_RULE(R_, L_, false, R_ <= 8 ? 8 : 4); \
     }                                                                             \
   } while (0)
   switch (dp) {

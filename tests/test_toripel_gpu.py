@@ -306,6 +306,41 @@ def test_the_delta_rule_has_the_same_bits_whatever_it_is_told_of_the_longest_req
 
 
 @pytest.mark.parametrize("channel_decays", [False, True])
+def test_the_delta_rule_of_more_waves_than_fit_has_the_bits_of_one_token_a_step(channel_decays):
+    """Keys of more than 128 (sixteen rows a lane) and more than two waves a SIMD: blocks of two tokens, requests of 1 to 9."""
+    heads, groups, d, dv, k = 4, 2, 200, 68, K()
+    n = 8 * k.compute_units() // (heads * 17) + 1  # requests: a wave works on four columns of a head
+    lengths = [1 + i % 9 for i in range(n)]
+    g = torch.Generator().manual_seed(n)
+    channels = 2 * groups * d + heads * dv
+    conv = (torch.randn((channels, 2), generator=g) * 0.5).cuda()
+    a_log = torch.randn(heads, generator=g).cuda()
+    dt_bias = torch.randn(heads * d if channel_decays else heads, generator=g).cuda()
+    raws = [torch.randn((m, channels + (1 if channel_decays else 2) * heads), generator=g).cuda() for m in lengths]
+    chans = [torch.randn((m, heads * d), generator=g).cuda() for m in lengths]
+
+    def run(most):
+        state = torch.zeros((n, heads * d * dv + channels), dtype=torch.float32, device="cuda")
+        outs = [[] for _ in lengths]
+        for at in range(0, max(lengths), most):
+            who = [i for i, m in enumerate(lengths) if m > at]
+            counts = [min(most, lengths[i] - at) for i in who]
+            tok_seq, tok_pos, seqs = step_meta(counts, [at] * len(who), who)
+            raw = torch.cat([raws[i][at:at + m] for i, m in zip(who, counts)])
+            chan = torch.cat([chans[i][at:at + m] for i, m in zip(who, counts)]) if channel_decays else None
+            out = torch.full((raw.shape[0], heads * dv), float("nan"), dtype=torch.float32, device="cuda")
+            size = k.delta_scratch_floats(raw.shape[0], groups, heads, d, dv, channel_decays)
+            k.delta_rule(raw, groups, heads, d, dv, conv, a_log, dt_bias, 1e-6, tok_seq, tok_pos, seqs, len(who), state,
+                         torch.empty(size, dtype=torch.float32, device="cuda"), out, chan, max(counts))
+            for i, part in zip(who, out.split(counts)):
+                outs[i].append(part)
+        return torch.cat([torch.cat(o) for o in outs]), state
+
+    (whole, state), (single, after) = run(9), run(1)
+    assert not torch.isnan(whole).any() and torch.equal(whole, single) and torch.equal(state, after)
+
+
+@pytest.mark.parametrize("channel_decays", [False, True])
 def test_the_delta_rule_writes_rows_any_distance_apart(channel_decays):
     """Output rows 256 MiB apart (a view into a wide buffer) get the bits of rows side by side."""
     heads, groups, d, dv, counts = 2, 1, 30, 5, [4, 1]
