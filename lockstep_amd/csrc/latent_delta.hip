@@ -432,8 +432,8 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // branches; only the blocks whose requests would leave the request hold them at its last token.  beta and the decay come
 // by one vector load at the same address in every lane (as scalar loads, which return in any order, a wait for one would
 // be a wait for all, also for those of the tokens ahead).
-// DEPTH: the tokens whose operands are on their way.  2,048 tokens (16 heads over 8, 128 x 128): 270 us; with lane
-// pointers, a conditional step of each, and a branch a token it took 490.  Where the longest request brings a token or two,
+// DEPTH: the tokens whose operands are on their way.  2,048 tokens (16 heads over 8, 128 x 128): 258 us, 281 with a decay
+// a channel; with lane pointers, a conditional step of each, and a branch a token it took 490.  Where the longest request brings a token or two,
 // two are enough and leave room for twice the waves: eight requests decoding 28 -> 13 us.  Where most requests decode beside
 // a longer one, the longest's chain counts as much as the room: four (63 requests of one token and one of 64, two / four / eight
 // ahead, convolution included: 64 x 64 48 / 39 / 38 us, 128 x 128 114 / 113 / 130, 192 x 128 143 / 95 / 100).  Else eight, with
