@@ -36,6 +36,8 @@
 //                      consecutive keys of one column are one load), second:
 //                      the probabilities exactly as S^T left them in the lane.
 
+#include <type_traits>
+
 #include "common.h"
 
 #ifndef LS_HEAD_DIM
@@ -59,6 +61,7 @@ constexpr int kSplitKeys = 128;
 #define LS_ATTN_RING 8
 #endif
 constexpr int kRing = LS_ATTN_RING;  // LDS operand reads kept in flight ahead of the MFMAs
+constexpr int kWideRing = 4;         // the same in the wide kernel, whose order the compiler keeps (8: the times of 4, sixteen registers more)
 constexpr int kPageWindow = 32;      // tiles whose page ids a workgroup of the streaming kernels holds in LDS at a time
 #ifdef LS_ATTN_PROBE
 #define PROBE(i) { long long now_ = clock64(); pr_t[i] += now_ - pr_last; pr_last = now_; }
@@ -107,6 +110,12 @@ __device__ __forceinline__ void load_to_lds16(const void* src, __attribute__((ad
   const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long)lds_wave_base);
   __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory", "m0");
 }
+// The same with the address in two parts: a base that the wave shares, in scalar registers, and a lane's 32-bit offset.
+__device__ __forceinline__ void load_to_lds16_from(unsigned long long base, unsigned offset, unsigned lds_wave_base) {
+  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base),
+                   "s"(lds_wave_base)
+                   : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // Sixteen bytes into registers by an instruction the compiler does not know to be a load: it places no wait for
@@ -150,6 +159,20 @@ __device__ __forceinline__ constexpr int key_of_row(int kb, int r) {
 template <typename T>
 __device__ __forceinline__ constexpr int row_rotation(int row) {
   return sizeof(T) == 2 ? (row & 3) + 4 * ((row >> 3) & 3) : row;
+}
+
+// The slot of a key row's 16-byte piece, and the other way round.  Rows of a multiple of 256 bytes all start at bank 0
+// (64 banks of 4 bytes): exclusive-or in place of the rotation.
+template <typename T>
+__device__ __forceinline__ constexpr int slot_of_piece(int row, int piece) {
+  constexpr int KPIECES = D * (int)sizeof(T) / 16;
+  return KPIECES % 16 == 0 ? piece ^ (row_rotation<T>(row) & 15) : (piece + row_rotation<T>(row)) % KPIECES;
+}
+template <typename T>
+__device__ __forceinline__ constexpr int piece_of_slot(int row, int slot) {
+  constexpr int KPIECES = D * (int)sizeof(T) / 16;
+  return KPIECES % 16 == 0 ? slot ^ (row_rotation<T>(row) & 15)
+                           : (slot - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
 }
 
 // Keep elements n_lo <= e < n_hi of a vector of VEC consecutive keys, zero the others.
@@ -552,7 +575,7 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
       const int piece = p % KPIECES;
       const int key = t0 + kt;
       const bool k_ok = key < sm.kv_len && key >= lo_valid && kpage_held[i] >= 0;
-      *reinterpret_cast<vec_t*>(k_lds + kt * KROW + ((piece + row_rotation<T>(kt)) % KPIECES) * 16) =
+      *reinterpret_cast<vec_t*>(k_lds + kt * KROW + slot_of_piece<T>(kt, piece) * 16) =
           k_ok ? kreg[j] : A::zero();
       const int q1 = p >> vshift;
       const int kp = p & ((1 << vshift) - 1);
@@ -620,7 +643,7 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
           const int row = key_of_row<T>(idx / NC, row16);
           const int piece = (idx % NC) * 4 + g;
           const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
-          vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + ((pc + row_rotation<T>(row)) % KPIECES) * 16);
+          vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + slot_of_piece<T>(row, pc) * 16);
           if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
           return kv;
         };
@@ -752,30 +775,34 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 }
 
 
-// Variant 4, "wide": prompt portions.  A workgroup of NW waves owns 16*NW rows
-// and walks the key tiles with two LDS buffers.  The tiles go from global
+// Variants 4 and 5, "wide": prompt portions.  A workgroup of NW waves owns 16*NW rows
+// and walks the key tiles with one LDS buffer, K and V.  The tiles go from global
 // memory straight into LDS (no registers in between): a load instruction of a
 // wave fills 64 consecutive 16-byte pieces of LDS, and each lane chooses the
-// source of its piece, so the K tile arrives in the rotated layout of the
-// staged kernel and the V tile as [8 or 4 keys][column][16 bytes].  While a
-// tile is multiplied the next one is in flight.  Keys outside the held range
+// source of its piece, so the K tile arrives in the swizzled layout of the
+// staged kernel and the V tile as [8 or 4 keys][column][16 bytes].  A tile's V is
+// asked for among its score products and the next tile's K among the exponentials:
+// a CU takes 64 bytes of such loads a clock, and a wave that issues them in a row
+// stands still meanwhile (16 loads: 1,100 of a tile's cycles).  Keys outside the held range
 // need no zeroing in K (their scores are replaced by -inf), and the V tile of
 // a boundary tile is cleaned in LDS before use.  The arithmetic of a row is
-// the instruction sequence of the other variants, so the bits are the same.
+// that of the other variants, value for value, so the bits are the same.
 //
-// What bounds it: the vector unit (scaling, exponentials, maximum and conversion)
-// in turn with the matrix cores, at one workgroup of eight waves a CU (bfloat16,
-// D = 128); for prompts from position 0 also the last row blocks, which walk the
-// most tiles.  Measured, 2,048 tokens, row blocks going round the XCDs / a kv
-// head's blocks on one: 32 heads over 8 kv heads 116 / 74 us (D = 128), 75 / 46
-// (64), 117 / 70 (112), 168 / 101 (144); 16 over 8 60.5 / 60.5.
-// Not kept: the score products of the next tile between the exponentials and its
-// maxima between the value products (a second set of scores and sums alive): at D
-// = 128 and eight waves the same times, everywhere else slower (16 over 8 heads,
-// D = 112 60 / 101 us, D = 144 88 / 175: registers spill; portions of 512 tokens
-// in blocks of 64 rows, D = 128 16.6 / 18.6).
+// Why four waves and one buffer: two such workgroups share a CU (66 KB of LDS each at D = 128), and one's
+// matrix products run under the other's exponentials and waits; with two buffers one workgroup of eight
+// waves had the CU, its waves in step, and LDS, vector unit and matrix cores took turns.  Raised priority during the
+// products lets a wave that has operands go first (2,048 tokens, 32 over 8 heads: 64.7 -> 57.7 us).
+// What bounds it: LDS (a tile's 64 KB are written once and read by each of the four waves: 2,600 of some 3,400 cycles a
+// workgroup's tile) and the vector unit (1,600 a wave).  Measured, bfloat16, D = 128, us, two buffers / now: 2,048 tokens from
+// position 0, 16 over 8 heads 59.6 / 42, 32 over 8 66 / 58; from 6,144 207 / 168; 808 tokens from 8,192 195 / 152;
+// D = 64 38 / 31, 43 / 41, 133 / 111, 131 / 115; D = 256 (which did not fit two buffers) 738 / 70 against the staged
+// kernel; float32 D = 128 the same 495 / 178.
+// Not kept: 32 rows a wave (half the LDS reads; one wave a SIMD then waits for itself: 63 us for the first of these).
+// Whether two workgroups' K and V tiles (and the page ids, 2 KB each) fit into a CU's LDS.
+constexpr bool wide_shares_cu(int element_bytes) { return 2 * (2 * kTileKeys * D * element_bytes + kPageWindow * 64) <= 160 * 1024; }
+
 template <typename T, int NW>
-__global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
+__global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void attention_wide_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, int page_shift, const int* __restrict__ table, int table_stride,
     const SeqMeta* __restrict__ seqs, const AttnItem* __restrict__ items, T* __restrict__ out, long ldo,
@@ -792,21 +819,24 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   constexpr int TOTAL = kTileKeys * KPIECES;  // pieces of the K tile == pieces of the V tile
   constexpr int PER = (TOTAL + NT - 1) / NT;
   constexpr int TILE_BYTES = TOTAL * 16;
-  constexpr int BUF_BYTES = 2 * TILE_BYTES;
-  constexpr int TILES_PER_SPLIT = kSplitKeys / kTileKeys;
+  // a wave's 64 pieces of K are whole rows of one page, and its 64 pieces of V columns of one page (pages are of 8 keys at least)
+  constexpr bool ONE_PAGE = 64 % KPIECES == 0 && 64 / KPIECES <= 8 && D % 64 == 0 && TOTAL % NT == 0;
+  static_assert(kSplitKeys == kTileKeys, "a tile is folded into the running sums as a split of its own");
   typedef const __attribute__((address_space(1))) void* gptr_t;
   typedef __attribute__((address_space(3))) void* lptr_t;
 
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  int* tile_pages = reinterpret_cast<int*>(lds + 2 * BUF_BYTES);  // [kPageWindow][16]
+  unsigned char* k_lds = lds;
+  unsigned char* v_lds = lds + TILE_BYTES;
+  int* tile_pages = reinterpret_cast<int*>(lds + 2 * TILE_BYTES);  // [kPageWindow][16]
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const AttnItem item = items[blockIdx.y];
   const int kvh = blockIdx.x;  // (see the launch)
   const SeqMeta sm = item.sm;
   const int rows_total = sm.q_len * G;
-  const int block_r0 = item.row_block * ROWS;
+  const int block_r0 = (item.row_block * (int)gridDim.z + (int)blockIdx.z) * ROWS;  // (an item's block may be two workgroups')
   if (block_r0 >= rows_total) return;  // uniform for the workgroup
   const int block_first_pos = sm.q_start + block_r0 / G;
   const int block_last_pos = sm.q_start + min(block_r0 + ROWS - 1, rows_total - 1) / G;
@@ -834,9 +864,9 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   for (int c = 0; c < NC; ++c)
     qv[c] = load_vec<T>(q + (long)head * D, sm.q_off + qi, c * A::KCHUNK + g * VEC, D, ldq, row_ok, true);
 
-  int ti_lo = item.split_begin * TILES_PER_SPLIT;
+  int ti_lo = item.split_begin;
   if (window > 0) ti_lo = max(ti_lo, max(0, block_first_pos - window + 1) / kTileKeys);
-  const int ti_hi = min(item.split_end * TILES_PER_SPLIT, block_last_pos / kTileKeys + 1);
+  const int ti_hi = min(item.split_end, block_last_pos / kTileKeys + 1);
 
   // The page ids of kPageWindow tiles at a time go into LDS, by ordinary loads, while no tile load is in
   // flight (the compiler's waits for ordinary loads do not know of the tile loads and would wait for them too).
@@ -851,53 +881,88 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
     }
   };
   auto window_start = [&](int ti) LS_INLINED -> bool { return (ti - ti_lo) % kPageWindow == 0; };  // tile ti opens a window of ids
-  // Start the loads of a tile into its buffer.  What does not depend on the
-  // tile is computed once: the offset of each of the thread's pieces inside
+  // What does not depend on the tile is computed once: the offset of each of the thread's pieces inside
   // its page.  Keys past the request's end need no clamp of their own: the
   // page id of their page is that of the last held page (fill_pages clamps),
   // so the loads stay inside the cache, and what they bring is masked.
   const long page_stride = (long)nkv * page_size * D;  // elements of one page, K or V
-  int k_off[PER], v_off[PER];
+  // (K rows of a load: the rotation repeats every PERIOD rows, so KV lane offsets serve all loads)
+  constexpr int RPI = NT / KPIECES, PERIOD = SZ == 2 ? 32 : KPIECES;
+  constexpr int KV = !ONE_PAGE ? PER : RPI % PERIOD == 0 ? 1 : PERIOD % RPI == 0 && PERIOD / RPI < PER ? PERIOD / RPI : PER;
+  constexpr int VV = ONE_PAGE ? 1 : PER;
+  int k_off[KV], v_off[VV];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
+  for (int i = 0; i < KV; ++i) {
     const int p = i * NT + (int)threadIdx.x;
     const int row = p / KPIECES;
-    const int slot = p % KPIECES;
-    const int piece = (slot - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
-    k_off[i] = (kvh * page_size + (row & (page_size - 1))) * D + piece * VEC;
-    const int c = p / D;
-    const int d = p % D;
-    v_off[i] = ((kvh * D + d) << page_shift) + ((c * VEC) & (page_size - 1));
+    const int piece = piece_of_slot<T>(row, p % KPIECES);
+    k_off[i] = ONE_PAGE ? (kvh * page_size + lane / KPIECES) * D + piece * VEC
+                        : (kvh * page_size + (row & (page_size - 1))) * D + piece * VEC;
   }
-  auto issue = [&](int ti) LS_INLINED {
-    const int* pages = tile_pages + ((ti - ti_lo) % kPageWindow) * 16;
-    unsigned char* k_buf = lds + (ti & 1) * BUF_BYTES;
-    unsigned char* v_buf = k_buf + TILE_BYTES;
-    int k_page[PER], v_page[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {  // all page ids first: their LDS reads overlap
-      const int p = i * NT + (int)threadIdx.x;
-      k_page[i] = pages[min((p / KPIECES) >> page_shift, 15)];
-      v_page[i] = pages[min(((p / D) * VEC) >> page_shift, 15)];
-    }
+  for (int i = 0; i < VV; ++i) {
+    const int p = i * NT + (int)threadIdx.x;
+    v_off[i] = ((kvh * D + p % D) << page_shift) + (ONE_PAGE ? 0 : (p / D * VEC) & (page_size - 1));
+  }
+  // With ONE_PAGE a wave's load has its address in scalar registers: lane i of `from` holds where the wave's K load i
+  // starts, lane 32 + i where its V load i does.
+  static_assert(!ONE_PAGE || PER <= 32, "a lane for every load");
+  const int my_at = ((lane & 31) < PER ? lane & 31 : 0) * NT + wave * 64;
+  const int my_key = lane < 32 ? my_at / KPIECES : my_at / D * VEC;
+  const char* my_base = reinterpret_cast<const char*>(lane < 32 ? k_pages : v_pages) +
+                        (my_key & (page_size - 1)) * (lane < 32 ? KROW : SZ);
+  auto loads_of = [&](int ti) LS_INLINED -> unsigned long long {
+    const int id = max(tile_pages[((ti - ti_lo) % kPageWindow) * 16 + (my_key >> page_shift)], 0);
+    return (unsigned long long)my_base + (unsigned long long)id * (unsigned long long)(page_stride * SZ);
+  };
+  const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long)(lptr_t)lds) + wave * 1024;
+  auto load_at = [&](unsigned long long from, int index) LS_INLINED -> unsigned long long {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)from, index) |
+           (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(from >> 32), index) << 32;
+  };
+  auto load_k = [&](unsigned long long from, int i) LS_INLINED {
+    load_to_lds16_from(load_at(from, i), k_off[i % KV] * SZ, lds_base + i * NT * 16);
+  };
+  auto load_v = [&](unsigned long long from, int i) LS_INLINED {
+    load_to_lds16_from(load_at(from, 32 + i), v_off[0] * SZ, lds_base + TILE_BYTES + i * NT * 16);
+  };
+  // All of a tile's K (or V) loads.
+  auto issue = [&](int ti, auto values) LS_INLINED {
+    constexpr bool V = decltype(values)::value;
+    if constexpr (ONE_PAGE) {
+      const unsigned long long from = loads_of(ti);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      if (PER * NT != TOTAL && i * NT + wave * 64 >= TOTAL) break;  // uniform for the wave
-      const T* k_src = k_pages + (long)max(k_page[i], 0) * page_stride + k_off[i];
-      load_to_lds16(k_src, (lptr_t)(k_buf + (i * NT + wave * 64) * 16));
-      const T* v_src = v_pages + (long)max(v_page[i], 0) * page_stride + v_off[i];
-      load_to_lds16(v_src, (lptr_t)(v_buf + (i * NT + wave * 64) * 16));
+      for (int i = 0; i < PER; ++i) {
+        if (V) load_v(from, i);
+        else load_k(from, i);
+      }
+    } else {
+      const int* pages = tile_pages + ((ti - ti_lo) % kPageWindow) * 16;
+      int page[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {  // all page ids first: their LDS reads overlap
+        const int p = i * NT + (int)threadIdx.x;
+        page[i] = pages[min((V ? p / D * VEC : p / KPIECES) >> page_shift, 15)];
+      }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        if (PER * NT != TOTAL && i * NT + wave * 64 >= TOTAL) break;  // uniform for the wave
+        const T* src = (V ? v_pages : k_pages) + (long)max(page[i], 0) * page_stride + (V ? v_off[i % VV] : k_off[i % KV]);
+        load_to_lds16(src, (lptr_t)((V ? v_lds : k_lds) + (i * NT + wave * 64) * 16));
+      }
     }
   };
+  constexpr std::false_type keys{};
+  constexpr std::true_type values{};
 
-  RowState run, cur;
+  RowState run;
   run.reset();
-  cur.reset();
 
   if (ti_lo < ti_hi) {
     fill_pages(ti_lo);
     __syncthreads();
-    issue(ti_lo);
+    issue(ti_lo, keys);
+    issue(ti_lo, values);
   }
 #ifdef LS_ATTN_PROBE
   long long pr_t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -908,60 +973,80 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   for (int c = 0; c < NC; ++c) __asm__ volatile("" ::"v"(qv[c]));  // the query rows are awaited here, not inside the loop
   for (int ti = ti_lo; ti < ti_hi; ++ti) {
     const int t0 = ti * kTileKeys;
-    const unsigned char* k_lds = lds + (ti & 1) * BUF_BYTES;
-    unsigned char* v_lds = lds + (ti & 1) * BUF_BYTES + TILE_BYTES;
-    if (ti != ti_lo && window_start(ti)) {  // nothing is in flight: the previous tile did not request this one
+    const bool opens = window_start(ti);  // its page ids were not there when the tile before ran: its loads are made at once
+    if (ti != ti_lo && opens) {
       lds_barrier();
       fill_pages(ti);
       lds_barrier();
-      issue(ti);
+      issue(ti, keys);
+      issue(ti, values);
     }
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's pieces of the tile have landed
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's pieces of K (and of V, where they were asked for) have landed
     PROBE(0)
-    lds_barrier();  // the tile is complete, and the other buffer has been read by every wave
+    lds_barrier();  // K is complete, and every wave has read the V before
     PROBE(1)
-    if (t0 + kTileKeys > sm.kv_len || t0 < lo_valid) {  // uniform: clean the values of keys that are not held
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int p = i * NT + (int)threadIdx.x;
-        if (PER * NT != TOTAL && p >= TOTAL) break;
-        const int key0 = t0 + (p / D) * VEC;
-        vec_t* at = reinterpret_cast<vec_t*>(v_lds + p * 16);
-        *at = mask_keys(*at, lo_valid - key0, sm.kv_len - key0);
-      }
-      lds_barrier();
-    }
-    if (ti + 1 < ti_hi && !window_start(ti + 1)) issue(ti + 1);  // a tile that opens a window of page ids waits for them
-
-    PROBE(2)
     const bool mine = wave_active && t0 <= wave_last_pos &&
                       !(window > 0 && t0 + kTileKeys <= wave_first_pos - window + 1);
-    if (mine) {
-      // ---- S^T = K . Q^T ---------------------------------------------------
-      f32x4 s[NB];
-      {
-        constexpr int NS = NB * NC;
-        constexpr int RING = NS < kRing ? NS : kRing;
-        auto k_read = [&](int idx) LS_INLINED -> vec_t {
-          const int row = key_of_row<T>(idx / NC, row16);
-          const int piece = (idx % NC) * 4 + g;
-          const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
-          vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + ((pc + row_rotation<T>(row)) % KPIECES) * 16);
-          if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
-          return kv;
-        };
-        vec_t ring[RING];
+    if (!opens && !(ONE_PAGE && mine)) issue(ti, values);
+    // ---- S^T = K . Q^T, two blocks of sixteen keys in turn, so that no product waits for the one before; with the
+    // loads of V between the products, so that the wave does not stand still until they are taken -------------------
+    f32x4 s[NB];
+    auto score_products = [&](auto with_loads) LS_INLINED {
+      constexpr int NS = NB * NC;
+      constexpr int RING = NS < kWideRing ? NS : kWideRing;
+      constexpr int EVERY = NS / PER > 0 ? NS / PER : 1;   // products a load
+      constexpr int LOADS = (PER * EVERY + NS - 1) / NS;   // loads at such a place
+      auto block_of = [](int idx) constexpr { return 2 * (idx / (2 * NC)) + idx % 2; };
+      auto chunk_of = [](int idx) constexpr { return idx / 2 % NC; };
+      auto k_read = [&](int idx) LS_INLINED -> vec_t {
+        const int row = key_of_row<T>(block_of(idx), row16);
+        const int piece = chunk_of(idx) * 4 + g;
+        const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
+        vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + slot_of_piece<T>(row, pc) * 16);
+        if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
+        return kv;
+      };
+      unsigned long long from = 0;
+      if constexpr (decltype(with_loads)::value) from = loads_of(ti);
+      vec_t ring[RING];
 #pragma unroll
-        for (int i = 0; i < RING; ++i) ring[i] = k_read(i);
+      for (int i = 0; i < RING; ++i) ring[i] = k_read(i);
+      __builtin_amdgcn_sched_barrier(0);  // (left to itself the compiler reads an operand when it is needed)
 #pragma unroll
-        for (int idx = 0; idx < NS; ++idx) {
-          if (idx % NC == 0) s[idx / NC] = f32x4{0.f, 0.f, 0.f, 0.f};
-          A::mma(s[idx / NC], ring[idx % RING], qv[idx % NC]);
-          if (idx + RING < NS) ring[idx % RING] = k_read(idx + RING);
+      for (int idx = 0; idx < NS; ++idx) {
+        const int kb = block_of(idx), c = chunk_of(idx);
+        if (c == 0) s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        A::mma(s[kb], ring[idx % RING], qv[c]);
+        if (idx + RING < NS) ring[idx % RING] = k_read(idx + RING);
+        if constexpr (decltype(with_loads)::value) {
+          if (idx % EVERY == 0) {
+#pragma unroll
+            for (int n = idx / EVERY * LOADS; n < (idx / EVERY + 1) * LOADS && n < PER; ++n) load_v(from, n);
+          }
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      PROBE(3)
-      // ---- scale, mask, online softmax --------------------------------------
+    };
+    __builtin_amdgcn_s_setprio(1);
+    if (mine) {
+      if (ONE_PAGE && !opens) score_products(std::bool_constant<ONE_PAGE>{});
+      else score_products(std::false_type{});
+    }
+    __builtin_amdgcn_s_setprio(0);
+    PROBE(2)
+    lds_barrier();  // every wave has read this K
+    PROBE(3)
+    const bool ahead = ti + 1 < ti_hi && !window_start(ti + 1);  // (a tile that opens a window of page ids waits for them)
+    if (ahead && !(ONE_PAGE && mine)) issue(ti + 1, keys);
+    constexpr int KB16 = VEC / 4;
+    constexpr int NK = NB / KB16;  // value products an output block takes
+    vec_t pv[NK];
+    float keep = 1.f, take = 0.f;  // the factors of the row's sums so far and of the tile's
+    bool some = false;             // the row sees a key of the tile (else its sums stay)
+    if (mine) {
+      unsigned long long from = 0;
+      if (ONE_PAGE && ahead) from = loads_of(ti + 1);
+      // ---- scale, mask, softmax; the next K's loads among it ---------------------------------------------------
       const bool all_visible = t0 + kTileKeys - 1 <= wave_first_pos && r0 + 15 < rows_total &&
                                (window <= 0 || wave_last_pos - t0 < window);
       float tile_max = kNegSentinel;
@@ -984,72 +1069,96 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
             tile_max = fmaxf(tile_max, v);
           }
       }
-      tile_max = quad16_max(tile_max);
-      const float m_new = fmaxf(cur.m, tile_max);
-      const float alpha = softmax_exp<T>(cur.m - m_new);
+      const float m = quad16_max(tile_max);
       float p_sum = 0.f;
+      auto probabilities = [&](auto with_loads) LS_INLINED {
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb) {
+        for (int kb = 0; kb < NB; ++kb) {
+          float pr[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[kb][e] = softmax_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
-        p_sum = p_sum + ((s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]));
-      }
-      p_sum = quad16_sum(p_sum);
-      cur.l = cur.l * alpha + p_sum;
-      cur.m = m_new;
-#pragma unroll
-      for (int blk = 0; blk < DB; ++blk)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) cur.acc[blk][e] = cur.acc[blk][e] * alpha;
-      PROBE(4)
-      // ---- O^T += V^T . P^T --------------------------------------------------
-      constexpr int KB16 = VEC / 4;
-      {
-        constexpr int NP = (NB / KB16) * DB;
-        constexpr int RING = NP < kRing ? NP : kRing;
-        auto v_read = [&](int idx) LS_INLINED -> vec_t {
-          const int kb = (idx / DB) * KB16;
-          const int d = (idx % DB) * 16 + row16;
-          vec_t vv;
-#pragma unroll
-          for (int h = 0; h < KB16; ++h) {
-            const int key = key_of_row<T>(kb + h, 4 * g);  // the lane's four keys inside the tile
-            const unsigned char* src = v_lds + ((key / VEC) * D + d) * 16 + (key % VEC) * SZ;
-            if (SZ == 2) {
-              bf16x4 four = *reinterpret_cast<const bf16x4*>(src);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) vv[h * 4 + e] = four[e];
-            } else {
-              f32x4 four = *reinterpret_cast<const f32x4*>(src);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) vv[h * 4 + e] = four[e];
-            }
+          for (int e = 0; e < 4; ++e) {
+            pr[e] = softmax_exp<T>(s[kb][e] - m);  // masked: exp(-inf) = 0
+            pv[kb / KB16][kb % KB16 * 4 + e] = from_f32<T>(pr[e]);
           }
-          return vv;
+          p_sum = p_sum + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
+          if constexpr (decltype(with_loads)::value) {
+#pragma unroll
+            for (int n = kb * PER / NB; n < (kb + 1) * PER / NB; ++n) load_k(from, n);
+          }
+        }
+      };
+      if (ONE_PAGE && ahead) probabilities(std::bool_constant<ONE_PAGE>{});
+      else probabilities(std::false_type{});
+      const float l = quad16_sum(p_sum);
+      some = l > 0.f;
+      // the tile's sums are a split's: folded into the row's as fold_split does, with the factors `keep` and `take`
+      const float m_new = fmaxf(run.m, m);
+      keep = softmax_exp<T>(run.m - m_new);
+      take = softmax_exp<T>(m - m_new);
+      run.l = some ? run.l * keep + l * take : run.l;
+      run.m = some ? m_new : run.m;
+    }
+    PROBE(4)
+    // V has landed; the next K, asked for after it, is still on its way
+    if (ONE_PAGE && ahead) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+    else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (t0 + kTileKeys > sm.kv_len || t0 < lo_valid) {  // uniform: clean the values of keys that are not held
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int p = i * NT + (int)threadIdx.x;
+        if (PER * NT != TOTAL && p >= TOTAL) break;
+        const int key0 = t0 + (p / D) * VEC;
+        vec_t* at = reinterpret_cast<vec_t*>(v_lds + p * 16);
+        *at = mask_keys(*at, lo_valid - key0, sm.kv_len - key0);
+      }
+      lds_barrier();
+    }
+    if (mine) {
+      // ---- O^T = O^T * keep + (V^T . P^T) * take -------------------------------------------------------------
+      // Two output blocks' products, then their fold, under the next two's: the tile's sums live in a few registers.
+      auto value_products = [&](auto all_held) LS_INLINED {
+        constexpr int NP = NK * DB;
+        constexpr int RING = NP < kWideRing ? NP : kWideRing;
+        constexpr int PAIR = DB % 2 == 0 ? 2 : 1;  // blocks whose products alternate
+        constexpr int STEPS = PAIR * NK, PARTS = PAIR * 4;   // products of such a set of blocks, and its sums a lane
+        auto v_read = [&](int idx) LS_INLINED -> vec_t {
+          const int kb = (idx / PAIR % NK) * KB16;
+          const int d = (PAIR * (idx / STEPS) + idx % PAIR) * 16 + row16;
+          const int key = key_of_row<T>(kb, 4 * g);  // the lane's first key inside the tile (its others follow)
+          return *reinterpret_cast<const vec_t*>(v_lds + ((key / VEC) * D + d) * 16);
         };
         vec_t ring[RING];
 #pragma unroll
         for (int i = 0; i < RING; ++i) ring[i] = v_read(i);
-        vec_t pv;
+        f32x4 acc[2][PAIR];  // the set whose products run, and the set before, which is being folded
+        auto fold = [&](int set, int from, int to) LS_INLINED {
+#pragma unroll
+          for (int n = from; n < to; ++n) {
+            const int at = n / 4, e = n % 4;
+            const float before = run.acc[set * PAIR + at][e];
+            const float folded = before * keep + acc[set % 2][at][e] * take;
+            run.acc[set * PAIR + at][e] = decltype(all_held)::value || some ? folded : before;
+          }
+        };
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int idx = 0; idx < NP; ++idx) {
-          if (idx % DB == 0) {
-            const int kb = (idx / DB) * KB16;
-#pragma unroll
-            for (int h = 0; h < KB16; ++h)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) pv[h * 4 + e] = from_f32<T>(s[kb + h][e]);
-          }
-          A::mma(cur.acc[idx % DB], ring[idx % RING], pv);
+          const int at = idx % PAIR, k = idx / PAIR % NK, set = idx / STEPS, step = idx % STEPS;
+          if (k == 0) acc[set % 2][at] = f32x4{0.f, 0.f, 0.f, 0.f};
+          A::mma(acc[set % 2][at], ring[idx % RING], pv[k]);
           if (idx + RING < NP) ring[idx % RING] = v_read(idx + RING);
+          if (set > 0) fold(set - 1, PARTS * step / STEPS, PARTS * (step + 1) / STEPS);
+          __builtin_amdgcn_sched_barrier(0);
         }
-      }
+        fold(DB / PAIR - 1, 0, PARTS);
+      };
+      __builtin_amdgcn_s_setprio(1);
+      if (__all(some)) value_products(std::true_type{});
+      else value_products(std::false_type{});
+      __builtin_amdgcn_s_setprio(0);
     }
     PROBE(5)
-    if (direct && ((ti + 1) % TILES_PER_SPLIT == 0 || ti + 1 == ti_hi)) {
-      fold_split<T>(run, cur.acc, cur.m, cur.l);
-      cur.reset();
-    }
   }
 
 #ifdef LS_ATTN_PROBE
@@ -1063,15 +1172,15 @@ __global__ __launch_bounds__(64 * NW) void attention_wide_kernel(
   if (!row_ok) return;
   if (direct) {
     store_output<T>(run, out + (long)(sm.q_off + qi) * ldo + (long)head * D, g);
-  } else {
+  } else {  // one tile, whose fold into empty sums left them as they are
     const int split = item.split_begin;
     const long pr = item.part_base + ((long)kvh * rows_total + r) * item.n_splits + (split - item.split_lo);
     float* pa = part_acc + pr * D;
 #pragma unroll
-    for (int blk = 0; blk < DB; ++blk) *reinterpret_cast<f32x4*>(pa + blk * 16 + 4 * g) = cur.acc[blk];
+    for (int blk = 0; blk < DB; ++blk) *reinterpret_cast<f32x4*>(pa + blk * 16 + 4 * g) = run.acc[blk];
     if (g == 0) {
-      part_ml[pr * 2] = cur.m;
-      part_ml[pr * 2 + 1] = cur.l;
+      part_ml[pr * 2] = run.m;
+      part_ml[pr * 2 + 1] = run.l;
     }
   }
 }
@@ -1237,7 +1346,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
       const int p = i * NT + (int)threadIdx.x;
       const int row = p / KPIECES;
       const int slot = p % KPIECES;
-      const int piece = (slot - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
+      const int piece = piece_of_slot<T>(row, slot);
       k_off[i] = (kvh * page_size + (row & (page_size - 1))) * D + piece * VEC;
       const int c = p / D;
       const int d = p % D;
@@ -1547,7 +1656,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
         const int p = i * NT + (int)threadIdx.x;
         const int row = p / KPIECES;
         if (t0 + row == p_new) {
-          const int piece = (p % KPIECES - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
+          const int piece = piece_of_slot<T>(row, p % KPIECES);
           *reinterpret_cast<vec_t*>(const_cast<unsigned char*>(k_lds) + p * 16) =
               *reinterpret_cast<const vec_t*>(knew + piece * VEC);
         }
@@ -1569,7 +1678,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
         for (int c = 0; c < NC; ++c) {
           const int piece = c * 4 + g;
           const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
-          vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + ((pc + row_rotation<T>(row)) % KPIECES) * 16);
+          vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + slot_of_piece<T>(row, pc) * 16);
           if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
           kop[j][c] = kv;
         }
@@ -2284,11 +2393,14 @@ extern "C" int ls_attention_decode(int dtype, const void* qkv, long ld, void* k_
   return check_launch("attention (decode, fused)");
 }
 
-// The wide kernel: two buffers of a K and a V tile, and two rows of page ids.  Eight waves (row blocks of
-// 128) or, for steps with so few rows that 128-row blocks would leave CUs without work, four (blocks of 64).
-constexpr int kWideWaves = 8;
-constexpr int kNarrowWaves = 4;
-static size_t wide_lds_bytes(int dtype) { return 4 * (size_t)kTileKeys * D * (dtype == kF32 ? 4 : 2) + kPageWindow * 16 * sizeof(int); }
+// The wide kernel: a K and a V tile, and the page ids.  Four waves (64 rows) where two workgroups share a CU:
+// never slower there than eight waves (128 rows; 2,048 tokens, D = 128, 16 over 8 heads 42 / 49 us, 32 over 8 58 / 58).  Where
+// one workgroup has the CU, eight waves fill it once there are more blocks of 128 rows than CUs (float32, D = 128: 2,048 tokens, 32
+// over 8 heads 309 us against 354 by four; bfloat16, D = 256, 2,048 tokens from 6,144 638 / 769; but float32, 16 over 8 heads, a block a
+// CU, 281 / 178), unless their loads need addresses of their own (float32, D = 80: 286 / 262, registers spill).
+constexpr int kLargeBlock = 128, kSmallBlock = 64;   // rows of variant 4's and variant 5's row blocks
+constexpr bool wide_has_eight_waves(int element_bytes) { return !wide_shares_cu(element_bytes) && D % 64 == 0; }
+static size_t wide_lds_bytes(int dtype) { return 2 * (size_t)kTileKeys * D * (dtype == kF32 ? 4 : 2) + kPageWindow * 16 * sizeof(int); }
 template <typename T, int NW>
 static bool wide_kernel_ready(size_t bytes) {
   static int state = 0;  // 0 unknown, 1 granted, -1 refused
@@ -2300,18 +2412,50 @@ static bool wide_kernel_ready(size_t bytes) {
   }
   return state == 1;
 }
+template <typename T>
+static bool wide_ready(size_t bytes) {
+  if constexpr (wide_has_eight_waves(sizeof(T)))
+    if (!wide_kernel_ready<T, 8>(bytes)) return false;
+  return wide_kernel_ready<T, 4>(bytes);
+}
 static bool wide_supported(int dtype) {
   const size_t bytes = wide_lds_bytes(dtype);
   if (bytes > kLdsLimit) return false;
   if (bytes <= 64 * 1024) return true;
-  return dtype == kF32 ? (wide_kernel_ready<float, kWideWaves>(bytes) && wide_kernel_ready<float, kNarrowWaves>(bytes))
-                       : (wide_kernel_ready<bf16_t, kWideWaves>(bytes) && wide_kernel_ready<bf16_t, kNarrowWaves>(bytes));
+  return dtype == kF32 ? wide_ready<float>(bytes) : wide_ready<bf16_t>(bytes);
 }
 // 1 if the wide kernel (variants 4 and 5) can run for this dtype.
 extern "C" int ls_attn_wide_supported(int dtype) { return wide_supported(dtype) ? 1 : 0; }
+// 1 if variant 4's row blocks have a workgroup of eight waves each (else two of variant 5's workgroups).
+extern "C" int ls_attn_wide_eight_waves(int dtype) { return wide_has_eight_waves(dtype == kF32 ? 4 : 2) ? 1 : 0; }
 // Rows of one work item's row block: AttnItem.row_block counts blocks of this many rows.
 extern "C" int ls_attn_block_rows(int variant) {
-  return variant == 4 ? 16 * kWideWaves : variant == 5 ? 16 * kNarrowWaves : 64;
+  return variant == 4 ? kLargeBlock : variant == 5 ? kSmallBlock : 64;
+}
+template <typename T>
+static void launch_wide(int variant, hipStream_t s, const void* q, long ldq, const void* k_pages, const void* v_pages, int nkv,
+                        int page_size, int page_shift, const int* table, int table_stride, const void* seqs, const void* items,
+                        int n_items, void* out, long ldo, float* part_acc, float* part_ml, int G, float scale, int window) {
+  const size_t bytes = wide_lds_bytes(sizeof(T) == 4 ? kF32 : kBF16);
+  // Workgroup ids go round the eight XCDs, and all row blocks of a kv head walk the same keys and values.  With the kv heads
+  // as the fast dimension a head's blocks meet on one XCD (8, 16, ... heads; fewer: on as many XCDs as share one), whose L2
+  // then answers most of their loads; with the row blocks as the fast dimension every XCD reads every head from beyond
+  // its L2, which bound the whole kernel.  (Numbered so inside the kernel instead, an item's record waits for the
+  // divisions: 97 tokens, 2 kv heads of 64, 7.3 us in place of 7.1.)
+  for (int first = 0; first < n_items; first += kMaxGridY) {
+    const int n = n_items - first < kMaxGridY ? n_items - first : kMaxGridY;
+    auto launch = [&](auto kernel, int waves, int halves) {
+      hipLaunchKernelGGL(kernel, dim3(nkv, n, halves), dim3(64 * waves), bytes, s, (const T*)q, ldq, (const T*)k_pages,
+                         (const T*)v_pages, nkv, page_size, page_shift, table, table_stride, (const SeqMeta*)seqs,
+                         (const AttnItem*)items + first, (T*)out, ldo, part_acc, part_ml, G, scale, window);
+    };
+    if (variant == 4) {
+      if constexpr (wide_has_eight_waves(sizeof(T))) launch(attention_wide_kernel<T, 8>, 8, 1);
+      else launch(attention_wide_kernel<T, 4>, 4, 2);
+    } else {
+      launch(attention_wide_kernel<T, 4>, 4, 1);
+    }
+  }
 }
 
 // variant: 4 and 5 run the wide kernel (row blocks of ls_attn_block_rows(variant) rows: 128 and 64);
@@ -2362,24 +2506,12 @@ extern "C" int ls_attention(int dtype, const void* q, long ldq, const void* k_pa
     LS_REQUIRE(wide_supported(dtype), "attention: the wide variant does not fit into LDS for this head size");
     LS_REQUIRE(page_size >= 8, "attention: the wide variant needs pages of at least 8 keys, got %d", page_size);
     LS_REQUIRE(dtype == kF32 || dtype == kBF16, "attention: unknown dtype %d", dtype);
-    const size_t bytes = wide_lds_bytes(dtype);
-    // Workgroup ids go round the eight XCDs, and all row blocks of a kv head walk the same keys and values.  With the kv heads
-    // as the fast dimension a head's blocks meet on one XCD (8, 16, ... heads; fewer: on as many XCDs as share one), whose L2
-    // then answers most of their loads; with the row blocks as the fast dimension every XCD reads every head from beyond
-    // its L2, which bound the whole kernel.  (Numbered so inside the kernel instead, an item's record waits for the
-    // divisions: 97 tokens, 2 kv heads of 64, 7.3 us in place of 7.1.)
-#define LS_WIDE(T_, NW_)                                                                                          \
-  for (int first = 0; first < n_items; first += kMaxGridY)                                                         \
-    hipLaunchKernelGGL((attention_wide_kernel<T_, NW_>), dim3(nkv, n_items - first < kMaxGridY ? n_items - first : kMaxGridY), \
-                       dim3(64 * NW_), bytes, s, (const T_*)q, ldq, (const T_*)k_pages, (const T_*)v_pages, nkv, page_size, \
-                       page_shift, table, table_stride, (const SeqMeta*)seqs, (const AttnItem*)items + first, (T_*)out, ldo, \
-                       part_acc, part_ml, G, scale, window)
-    if (dtype == kF32) {
-      if (variant == 4) LS_WIDE(float, kWideWaves); else LS_WIDE(float, kNarrowWaves);
-    } else {
-      if (variant == 4) LS_WIDE(bf16_t, kWideWaves); else LS_WIDE(bf16_t, kNarrowWaves);
-    }
-#undef LS_WIDE
+    if (dtype == kF32)
+      launch_wide<float>(variant, s, q, ldq, k_pages, v_pages, nkv, page_size, page_shift, table, table_stride, seqs, items, n_items,
+                         out, ldo, part_acc, part_ml, G, scale, window);
+    else
+      launch_wide<bf16_t>(variant, s, q, ldq, k_pages, v_pages, nkv, page_size, page_shift, table, table_stride, seqs, items, n_items,
+                          out, ldo, part_acc, part_ml, G, scale, window);
     return check_launch("attention (wide)");
   }
   const bool staged = variant != 1 && staged_fits(dtype, lds_bytes);

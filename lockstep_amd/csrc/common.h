@@ -113,17 +113,32 @@ template <typename T> __device__ __forceinline__ float softmax_exp(float x);
 template <> __device__ __forceinline__ float softmax_exp<float>(float x) { return expf(x); }
 template <> __device__ __forceinline__ float softmax_exp<bf16_t>(float x) { return __expf(x); }
 
+// A lane's value and that of lane l^16, or l^32, as two values in an order that is the same in both lanes, by an
+// exchange of registers (an LDS permute waits some 120 cycles for its answer).
+__device__ __forceinline__ void with_lane_xor16(float v, float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  a = __builtin_bit_cast(float, (unsigned)r[0]);
+  b = __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ void with_lane_xor32(float v, float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  a = __builtin_bit_cast(float, (unsigned)r[0]);
+  b = __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
 // Sum / max over the four lanes {l, l^16, l^32, l^48}; every lane of the
 // four ends with the same bits because each step adds a pair commutatively.
 __device__ __forceinline__ float quad16_sum(float v) {
-  v = v + __shfl_xor(v, 16, kWave);
-  v = v + __shfl_xor(v, 32, kWave);
-  return v;
+  float a, b;
+  with_lane_xor16(v, a, b);
+  with_lane_xor32(a + b, a, b);
+  return a + b;
 }
 __device__ __forceinline__ float quad16_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  v = fmaxf(v, __shfl_xor(v, 32, kWave));
-  return v;
+  float a, b;
+  with_lane_xor16(v, a, b);
+  with_lane_xor32(fmaxf(a, b), a, b);
+  return fmaxf(a, b);
 }
 
 // Butterfly sum over all 64 lanes, same bits in every lane.

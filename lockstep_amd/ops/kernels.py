@@ -189,6 +189,12 @@ class Kernels:
         return self._memo(("wide", head_dim, dtype, page_size), lambda: page_size >= 8 and bool(
             self.attention_lib(head_dim).ls_attn_wide_supported(c_int(DTYPE_CODE[dtype]))))
 
+    def wide_eight_waves(self, head_dim: int, dtype: torch.dtype) -> bool:
+        """Whether variant 4's row blocks of the wide attention kernel are workgroups of their own size (else two of
+        variant 5's)."""
+        return self._memo(("wide_eight_waves", head_dim, dtype), lambda: bool(
+            self.attention_lib(head_dim).ls_attn_wide_eight_waves(c_int(DTYPE_CODE[dtype]))))
+
     def attention_block_rows(self, head_dim: int, variant: int) -> int:
         """Rows of the row blocks that work items of this variant count in."""
         return self._memo(("block_rows", head_dim, variant),
@@ -597,7 +603,7 @@ class Kernels:
         ``variant``: 0 staged through LDS where it fits, 1 direct from global memory, 2 staged or
         error, 3 cooperative (every item has at most 16 rows; ``max_rows`` states the largest),
         4 wide (prompt portions; items count row blocks of ``attention_block_rows``), 5 the same
-        with half the rows a block (for steps with few rows).  ``spans`` (cooperative only): items
+        with half the rows a block (where two of its workgroups share a compute unit, and for steps with few rows).  ``spans`` (cooperative only): items
         that leave partial results may hold several splits each.  ``single_tile`` (cooperative only): every
         item holds one key tile (a hint: such a launch needs one tile buffer a workgroup, not two)."""
         lib = self.attention_lib(d)

@@ -131,9 +131,10 @@ def plan_attention(ctx, group_size: int, nkv: int, head_dim: int, window: int, o
     wide_ok = kernels.wide_supported(head_dim, dtype, page_size)
     wide_variant, wide_rows = 4, kernels.attention_block_rows(head_dim, 4)
     if wide_ok:
-        # so few rows that the large row blocks would leave half of the CUs without a workgroup: smaller blocks
+        # large row blocks where a workgroup of eight waves takes one and there are more of them than CUs (figures beside
+        # kLargeBlock in attention.hip)
         blocks = sum(-(-(int(q) * group_size) // wide_rows) for q in ctx.q_len if int(q) * group_size > 64)
-        if 0 < blocks * nkv <= kernels.compute_units() // 2:
+        if not kernels.wide_eight_waves(head_dim, dtype) or blocks * nkv <= kernels.compute_units():
             wide_variant, wide_rows = 5, kernels.attention_block_rows(head_dim, 5)
 
     # splits every request has (when the step's last token of the horizon is in): first, count

@@ -767,6 +767,27 @@ def test_attention_over_more_keys_than_one_window_of_page_ids(dtype, nq, nkv, d,
         assert torch.equal(crowd, full[n - 1:]), "decoded token, crowded launch"
 
 
+@pytest.mark.parametrize("dtype,nq,nkv,d,ps", [(torch.bfloat16, 4, 2, 256, 16), (torch.bfloat16, 4, 2, 128, 8),
+                                               (torch.float32, 4, 2, 128, 8), (torch.float32, 2, 1, 80, 16)])
+def test_wide_attention_at_the_edges_of_its_row_blocks_and_page_windows(dtype, nq, nkv, d, ps):
+    """Portions whose rows end beside a wave's, a workgroup's and a large block's edge, over contexts that end beside a
+    tile's edge and beside a window of page ids': the bits of the kernel that loads straight from global memory."""
+    starts, lengths = (0, 127, 4000), (31, 32, 33, 63, 64, 65, 95, 96, 97, 130)
+    n = max(starts) + max(lengths)
+    qkv = rand_qkv(n, nq, nkv, d, dtype, seed=d + ps)
+    case = PagedCase(dtype, nq, nkv, d, ps, n, shuffle_seed=7)
+    dev = qkv.cuda()
+    case.write(dev, 0)
+    assert K().wide_supported(d, dtype, ps)
+    for start in starts:
+        for length in lengths:
+            rows = dev[start:start + length]
+            want = case.attend(rows, start, d ** -0.5, variant=1, force_split=False)
+            for variant in (4, 5):
+                got = case.attend(rows, start, d ** -0.5, variant=variant, force_split=False)
+                assert torch.equal(got, want), (start, length, variant)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nq,nkv,d,ps", [(16, 8, 128, 16), (6, 3, 32, 8), (8, 1, 64, 16)])
 def test_attention_row_is_the_same_alone_in_a_portion_and_in_the_whole_prompt(dtype, nq, nkv, d, ps):
