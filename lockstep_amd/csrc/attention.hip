@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "ring.h"
 
 #ifndef LS_HEAD_DIM
 #error "compile with -DLS_HEAD_DIM=<head size, a multiple of 16>"
@@ -97,27 +98,6 @@ static_assert(sizeof(AttnItem) == 128, "the host packs 32 ints an item");
 // "m" never becomes infinite and no difference of infinities can arise.
 constexpr float kMasked = -__builtin_huge_valf();
 
-// One 16-byte piece per lane from global memory straight into LDS: the wave's 64 pieces land at
-// `lds_wave_base` + 16 * lane, each lane names its own source.  Written as the instruction itself
-// (M0 holds the wave's LDS address): after the compiler's own form of it
-// (__builtin_amdgcn_global_load_lds) every later LDS read and every barrier waits for all such
-// loads in flight, because they might be reading what the loads write, and the loads of the next
-// tile could not overlap the work on this one.  The kernels wait for a tile's loads themselves
-// (s_waitcnt vmcnt) before the barrier after which the tile is read.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // (it warns of the name m0, which keeps the compiler from relying on it)
-__device__ __forceinline__ void load_to_lds16(const void* src, __attribute__((address_space(3))) void* lds_wave_base) {
-  const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long)lds_wave_base);
-  __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory", "m0");
-}
-// The same with the address in two parts: a base that the wave shares, in scalar registers, and a lane's 32-bit offset.
-__device__ __forceinline__ void load_to_lds16_from(unsigned long long base, unsigned offset, unsigned lds_wave_base) {
-  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base),
-                   "s"(lds_wave_base)
-                   : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 // Sixteen bytes into registers by an instruction the compiler does not know to be a load: it places no wait for
 // it, so the kernel can keep it in flight across other loads and wait with a count of its own (wait_for_loads,
 // which also ties the registers, so that no use moves above the wait).
@@ -135,12 +115,6 @@ __device__ __forceinline__ void wait_for_loads(f32x4& a, f32x4& b, f32x4& c, f32
                    : "n"(YOUNGER)
                    : "memory");
 }
-
-// A workgroup barrier that makes the waves' own LDS writes visible and nothing else.  __syncthreads() also
-// waits for every load that is still writing into LDS (global_load_lds), which would end the overlap of the
-// next tile's loads with the work on this one; where a tile has to be complete, the kernel waits for its own
-// loads explicitly (s_waitcnt vmcnt) before the barrier.
-__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Which key of a tile row r (0..15) of the score block kb stands for.  The score MFMA leaves a lane with rows
 // 4g..4g+3 of each 16-key block, and the value MFMA of two such blocks (bfloat16: 32 keys an atom) wants the
@@ -975,15 +949,15 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
     const int t0 = ti * kTileKeys;
     const bool opens = window_start(ti);  // its page ids were not there when the tile before ran: its loads are made at once
     if (ti != ti_lo && opens) {
-      lds_barrier();
+      ring_barrier();
       fill_pages(ti);
-      lds_barrier();
+      ring_barrier();
       issue(ti, keys);
       issue(ti, values);
     }
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's pieces of K (and of V, where they were asked for) have landed
     PROBE(0)
-    lds_barrier();  // K is complete, and every wave has read the V before
+    ring_barrier();  // K is complete, and every wave has read the V before
     PROBE(1)
     const bool mine = wave_active && t0 <= wave_last_pos &&
                       !(window > 0 && t0 + kTileKeys <= wave_first_pos - window + 1);
@@ -1034,7 +1008,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
     }
     __builtin_amdgcn_s_setprio(0);
     PROBE(2)
-    lds_barrier();  // every wave has read this K
+    ring_barrier();  // every wave has read this K
     PROBE(3)
     const bool ahead = ti + 1 < ti_hi && !window_start(ti + 1);  // (a tile that opens a window of page ids waits for them)
     if (ahead && !(ONE_PAGE && mine)) issue(ti + 1, keys);
@@ -1102,7 +1076,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
     // V has landed; the next K, asked for after it, is still on its way
     if (ONE_PAGE && ahead) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
     else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
+    ring_barrier();
     if (t0 + kTileKeys > sm.kv_len || t0 < lo_valid) {  // uniform: clean the values of keys that are not held
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
@@ -1112,7 +1086,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
         vec_t* at = reinterpret_cast<vec_t*>(v_lds + p * 16);
         *at = mask_keys(*at, lo_valid - key0, sm.kv_len - key0);
       }
-      lds_barrier();
+      ring_barrier();
     }
     if (mine) {
       // ---- O^T = O^T * keep + (V^T . P^T) * take -------------------------------------------------------------
@@ -1608,7 +1582,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
   if (FUSE) {
     if (n_vec <= 16 && grp < n_vec) finish_head(grp);  // (more heads than groups: done above, before the tile loads)
     PROBE(14)
-    lds_barrier();
+    ring_barrier();
     PROBE(15)
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -1628,9 +1602,9 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     // the next tile is requested ahead unless it opens a new window of page ids
     const bool ahead = ti + 1 < ti_hi && !window_start(ti + 1);
     if (ti != ti_lo && window_start(ti)) {  // nothing is in flight: the previous tile did not request this one
-      lds_barrier();
+      ring_barrier();
       fill_pages(ti);
-      lds_barrier();
+      ring_barrier();
       issue_tile(ti);
     }
     if (NBUF == 2) {
@@ -1646,7 +1620,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
       __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
     }
     PROBE(4)
-    lds_barrier();  // the tile (one buffer: its K half) is complete (and the other buffer has been read by every wave)
+    ring_barrier();  // the tile (one buffer: its K half) is complete (and the other buffer has been read by every wave)
     PROBE(5)
     const bool patch = owner && ti == tile_new;  // the new key and value go into this tile
     const bool clean = t0 + kTileKeys > sm.kv_len || t0 < lo_valid || patch;  // uniform
@@ -1661,7 +1635,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
               *reinterpret_cast<const vec_t*>(knew + piece * VEC);
         }
       }
-      lds_barrier();
+      ring_barrier();
     }
     if (NBUF == 2 && ahead && !(primed && ti == ti_lo)) issue(ti + 1);
 
@@ -1701,7 +1675,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     my_max = quad16_max(my_max);
     if (g == 0) wmax[wave * 16 + row16] = my_max;
     PROBE(7)
-    lds_barrier();
+    ring_barrier();
     PROBE(8)
     if (NBUF == 1 && ahead) issue_k(ti + 1);  // every wave has its scores: the K half of the buffer is free
     const float tile_max = fmaxf(fmaxf(wmax[row16], wmax[16 + row16]), fmaxf(wmax[32 + row16], wmax[48 + row16]));
@@ -1789,7 +1763,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
       __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     PROBE(9)
-    lds_barrier();
+    ring_barrier();
     PROBE(10)
     if (NBUF == 1) {
       read_values();
@@ -1848,7 +1822,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
       cur_l = 0.f;
     }
     if (NBUF == 1 && ti + 1 < ti_hi) {
-      lds_barrier();  // every wave is done with the V half of the buffer
+      ring_barrier();  // every wave is done with the V half of the buffer
       if (ahead) issue_v(ti + 1);
     }
   }

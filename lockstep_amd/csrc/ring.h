@@ -1,5 +1,6 @@
-// What a ring of stages in LDS is made of: loads that the memory writes into LDS by itself, the waits for them, and a
-// barrier that leaves them in flight.  The kernels that use it: gemm_ring.h (which says how the steps interlock), experts.hip.
+// What stages and tiles in LDS are made of: loads that the memory writes into LDS by itself, the waits for them, and a
+// barrier that leaves them in flight.  The kernels that use it: gemm_ring.h (which says how the steps interlock), experts.hip,
+// attention.hip, sink_attention.hip.
 #pragma once
 
 #include "common.h"
@@ -32,6 +33,23 @@ __device__ __forceinline__ void buffer_to_lds16(unsigned lane_off, unsigned off,
                    : "v"(lane_off), "s"(off), "s"(buffer), "s"(lds_base)
                    : "memory", "m0");
 }
+// One 16-byte piece per lane from global memory straight into LDS: the wave's 64 pieces land at
+// `lds_wave_base` + 16 * lane, each lane names its own source.  Written as the instruction itself
+// (M0 holds the wave's LDS address): after the compiler's own form of it
+// (__builtin_amdgcn_global_load_lds) every later LDS read and every barrier waits for all such
+// loads in flight, because they might be reading what the loads write, and the loads of the next
+// tile could not overlap the work on this one.  The kernels wait for a tile's loads themselves
+// (s_waitcnt vmcnt) before the barrier after which the tile is read.
+__device__ __forceinline__ void load_to_lds16(const void* src, __attribute__((address_space(3))) void* lds_wave_base) {
+  const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long)lds_wave_base);
+  __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory", "m0");
+}
+// The same with the address in two parts: a base that the wave shares, in scalar registers, and a lane's 32-bit offset.
+__device__ __forceinline__ void load_to_lds16_from(unsigned long long base, unsigned offset, unsigned lds_wave_base) {
+  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base),
+                   "s"(lds_wave_base)
+                   : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 template <int YOUNGER>  // loads issued after those that are waited for
@@ -41,6 +59,7 @@ __device__ __forceinline__ void wait_loads() {
 }
 
 // A barrier behind the waves' own LDS reads and writes; loads into LDS stay in flight (wait_loads waits for those).
+// (__syncthreads() would wait for them too, which would end the overlap of the next tile's loads with the work on this one.)
 __device__ __forceinline__ void ring_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 }  // namespace ls

@@ -31,6 +31,7 @@
 // zeros and are masked; their values are replaced by zeros before the product.
 
 #include "common.h"
+#include "ring.h"
 
 #include <type_traits>
 
@@ -389,43 +390,80 @@ __global__ __launch_bounds__(64 * (DEC ? 1 : kMaxWaves)) void sink_attention_ker
 // ---------------------------------------------------------------------------
 // Prompt portions, key and value tiles staged in LDS.  The kernel above spends some 25 vector instructions on
 // every MFMA: addresses and selects for each fragment it takes from global memory, and the row statistics of a
-// tile of only 32 keys.  Here a workgroup of four waves copies a tile of kStagedKeys keys (128 bytes of keys a
-// value column: 64 in bfloat16, 32 in float) into LDS once, with a few 16-byte pieces a thread, and every wave
-// reads its fragments from there at constant offsets.  A wave owns 32 rows of one head; the waves of a workgroup
+// tile of only 32 keys.  Here a workgroup of four waves has a tile of kKeys keys (128 bytes of keys a
+// value column: 64 in bfloat16, 32 in float) loaded straight into LDS, and every wave
+// reads its fragments from there.  A wave owns 32 rows of one head; the waves of a workgroup
 // are min(GS, 4) query heads of the key/value head times 4 / min(GS, 4) groups of 32 rows, so a work item names a
-// block of 32, 64 or 128 rows.  The next tile is requested into registers while a tile is worked on.  The
-// arithmetic of a row (scores, statistics, sums) is that of the kernel above with larger tiles.
+// block of 32, 64 or 128 rows.  A tile's values are asked for among its score products, the next tile's keys among
+// the exponentials.  The arithmetic of a row (scores, statistics, sums) is that of the kernel above with larger tiles.
+//
+// Layout: the 16-byte piece `piece` of key row r lies in slot slot_of_piece(r, piece) of the row; the values lie as [VEC
+// keys][column][16 bytes].  In bfloat16 the rows of a pair of 16-key score blocks are dealt (key_of_row) so that the eight
+// probabilities a lane ends with belong to eight consecutive keys, which is one read of the values.
+//
+// ONE_PAGE (rows of a multiple of 128 bytes, 64, 128, ... value columns, pages of 8 keys at least): the 64 pieces of a
+// wave's load lie in one page, whose address is a scalar; else every lane looks its piece's page up.
+//
+// What bounds it: the vector unit (scales, maxima, exponentials: 1,200 of a wave's cycles a tile of 64 keys) in turn with the
+// matrix cores (1,280 at keys of 192 and values of 128 elements), two workgroups a CU.  Measured with its fold, us, tiles through
+// registers with one workgroup a CU / now, 16 heads: 2,048 tokens, keys of 192 and values of 128, one key/value head 132 / 64, keys of
+// 128 and eight of them 121 / 55; 700 from 1,500 on in a window of 600 45 / 34; 2,048 from 6,000 on 434 / 129.
 // ---------------------------------------------------------------------------
 template <typename T> struct Staged {
   static constexpr int kKeys = 128 / (int)sizeof(T);                 // keys of a tile
-  static constexpr int kKeyRow = D * (int)sizeof(T) + 16;            // bytes from a key to the next in LDS
-  static constexpr int kValueRow = 128 + 16;                         // bytes from a value column to the next
-  static constexpr int kBytes = kKeys * kKeyRow + DV * kValueRow;
+  static constexpr int kKeyPieces = D * (int)sizeof(T) / 16;         // 16-byte pieces of a key
+  static constexpr int kKeyBytes = kKeys * kKeyPieces * 16;          // of the tile's keys
+  static constexpr int kValueBytes = (8 * DV + 63) / 64 * 1024;      // and of its values (whole loads of a wave)
+  static constexpr int kWindow = 32;                                 // tiles whose page ids a workgroup holds
+  static constexpr int kTilePages = 16;                              // page ids of a tile, at most
+  static constexpr int kBytes = kKeyBytes + kValueBytes + kWindow * kTilePages * 4;
   static constexpr bool kFits = kBytes <= 64 * 1024 && D % Atom<T>::VEC == 0;
+  static constexpr bool kOnePage = kKeyPieces % 8 == 0 && DV % 64 == 0;
 };
 
+// Which key of a tile row r (0..15) of the score block kb stands for.
 template <typename T>
-__global__ __launch_bounds__(256) void sink_attention_staged_kernel(
+__device__ __forceinline__ constexpr int key_of_row(int kb, int r) {
+  return sizeof(T) == 2 ? 32 * (kb >> 1) + 8 * (r >> 2) + 4 * (kb & 1) + (r & 3) : 16 * kb + r;
+}
+// The slot of a piece in its key's row (and the piece in a slot: each of these is its own inverse).  `l` is the row's place among
+// the sixteen that a read takes together; of those LDS serves 0-3 and 12-15 at one piece with 4-11 at the piece beside it.
+template <typename T>
+__device__ __forceinline__ constexpr int slot_at(int l, int piece) {
+  constexpr int P = Staged<T>::kKeyPieces;
+  if (P % 16 == 0) return (piece & ~15) + ((piece & 15) ^ l);
+  if (P % 8 == 0) return (piece & ~7) + ((piece & 7) ^ (l >> 1));
+  if (P % 4 == 0) return (piece & ~3) + ((piece & 3) ^ (((l >> 1) & 2) ^ ((l >> 3) * 3)));
+  return piece;
+}
+template <typename T>
+__device__ __forceinline__ constexpr int slot_of_piece(int key, int piece) {
+  return slot_at<T>(sizeof(T) == 2 ? (key & 3) + 4 * ((key >> 3) & 3) : key & 15, piece);
+}
+
+template <typename T, bool ONE_PAGE>
+__global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int page_size,
     const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs, const int* __restrict__ items,
     int H, int G, float scale, int window, int chunk, int keep_first, const float* __restrict__ sink,
     const float* __restrict__ dist_bias, int n_dist, const float* __restrict__ gate, long ldg, T* __restrict__ out,
     long ldo, float* __restrict__ part, int part_rows) {
-  typedef typename Atom<T>::vec_t vec_t;
-  typedef typename std::conditional<sizeof(T) == 2, bf16x4, f32x4>::type v4_t;
-  constexpr int VEC = Atom<T>::VEC, KC = Atom<T>::KCHUNK;
+  typedef Atom<T> A;
+  typedef typename A::vec_t vec_t;
+  typedef Staged<T> S;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  constexpr int SZ = sizeof(T), VEC = A::VEC, KC = A::KCHUNK;
   constexpr int KCH = D / KC + (D % KC ? 1 : 0);
-  constexpr int TK = Staged<T>::kKeys, NG = TK / 16;              // groups of 16 keys in a tile
-  constexpr int kKeyRow = Staged<T>::kKeyRow, kValueRow = Staged<T>::kValueRow;
-  constexpr int kKeyPieces = TK * (D / VEC), kValuePieces = DV * (TK / VEC);
-  constexpr int KP = (kKeyPieces + 255) / 256, VP = (kValuePieces + 255) / 256;
-  __shared__ __attribute__((aligned(16))) char lds[Staged<T>::kFits ? Staged<T>::kBytes : 16];
-  char* const k_lds = lds;
-  char* const v_lds = lds + TK * kKeyRow;
-  // the page ids of a tile and of the next one: looked up by a few threads two tiles ahead, so that no thread waits
-  // for the block table before it can ask for its pieces
-  constexpr int kTilePages = 16;
-  __shared__ int page_s[2][kTilePages];
+  constexpr int TK = S::kKeys, NG = TK / 16;                       // keys of a tile, and groups of 16 of them
+  constexpr int KP = S::kKeyPieces > 0 ? S::kKeyPieces : 1;
+  constexpr int K_TOTAL = TK * KP, V_TOTAL = 8 * DV;               // pieces of a tile
+  constexpr int KPER = (K_TOTAL + 255) / 256, VPER = (V_TOTAL + 255) / 256;
+  constexpr int NC = sizeof(T) == 2 ? NG / 2 : NG;                 // chunks of keys of the value product
+  static_assert(!ONE_PAGE || (K_TOTAL % 256 == 0 && V_TOTAL % 256 == 0 && KPER <= 32 && VPER <= 32), "whole loads");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[S::kFits ? S::kBytes : 16];
+  unsigned char* const k_lds = lds;
+  unsigned char* const v_lds = lds + S::kKeyBytes;
+  int* const tile_pages = reinterpret_cast<int*>(lds + S::kKeyBytes + S::kValueBytes);  // [kWindow][kTilePages]
 
   const int seq = items[4 * blockIdx.x], rb = items[4 * blockIdx.x + 1];
   const int run = items[4 * blockIdx.x + 2], n_runs = max(1, items[4 * blockIdx.x + 3]);
@@ -433,7 +471,7 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
   const int GS = H / G, g = blockIdx.y;
   const int HW = GS < 4 ? GS : 4, RG = 4 / HW;                     // heads and groups of 32 rows a workgroup
   const int block_rows = 32 * RG;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, quad = lane >> 4;
   const int row0 = rb * block_rows;
   if (row0 >= m.q_len) return;                                      // (the whole workgroup)
@@ -449,7 +487,7 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
   const int my_head = g * GS + (in_group < GS ? in_group : 0);
   const int wave_first = p_first + min(wave_row0, nrows - 1), wave_last = p_first + min(wave_row0 + 31, nrows - 1);
   bool row_ok[2];
-  int my_pos[2], my_lo[2];
+  int my_pos[2], my_lo[2], seen_to[2];
   vec_t qv[2][KCH];
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
@@ -457,6 +495,7 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
     row_ok[r] = active && row < nrows;
     my_pos[r] = p_first + (row_ok[r] ? row : 0);
     my_lo[r] = first_seen(my_pos[r], window, chunk);
+    seen_to[r] = row_ok[r] ? my_pos[r] : -1;
     const T* q_row = q + (long)(m.q_off + row0 + (row_ok[r] ? row : 0)) * ldq + (long)my_head * D;
 #pragma unroll
     for (int c = 0; c < KCH; ++c) {
@@ -477,7 +516,8 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
     for (int b = 0; b < VB; ++b) acc[r][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  const int lo_tile = first_seen(p_first, window, chunk) / TK;
+  const int block_lo = first_seen(p_first, window, chunk);           // no row of the block sees a key in front of it (but kept ones)
+  const int lo_tile = block_lo / TK;
   const int hi_tile = p_last / TK;
   const int kept_tiles = min((keep_first + TK - 1) / TK, lo_tile);   // tiles of kept first tokens below the window's
   const int n_tiles = kept_tiles + hi_tile - lo_tile + 1;
@@ -485,135 +525,215 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
   const int per_run = (n_tiles + n_runs - 1) / n_runs;
   const int step_begin = run * per_run, step_end = min(n_tiles, (run + 1) * per_run);
 
-  // a thread's pieces of a tile: 16 bytes of a key, and of a value column (VEC consecutive keys, inside one page)
-  vec_t k_piece[KP], v_piece[VP];
-  // (pages of at least a tile's keys: one page a tile)
-  const int tile_pages = max(1, TK >> page_shift);
-  auto look_up = [&](int step) LS_INLINED {       // thread i: the page of the tile's i-th run of keys, -1 beyond the block
-    const int key0 = tile_at(step) * TK;
-    const int key = max(key0, ((key0 >> page_shift) + (int)threadIdx.x) << page_shift);
-    const bool in = (int)threadIdx.x < tile_pages && step < step_end && key <= p_last;
-    return in ? my_table[key >> page_shift] : -1;
-  };
-  auto request = [&](int step) LS_INLINED {
-    const int key0 = tile_at(step) * TK;
-    const int* pages = page_s[step & 1];
-    const int first_page = key0 >> page_shift;
-#pragma unroll
-    for (int j = 0; j < KP; ++j) {
-      const int p = threadIdx.x + 256 * j;
-      const int key = key0 + p / (D / VEC), seg = p % (D / VEC);
-      const bool in = p < kKeyPieces && key <= p_last;
-      const int page = in ? pages[(key >> page_shift) - first_page] : -1;
-      const long at = (((long)(page >= 0 ? page : 0) * G + g) << page_shift) + (page >= 0 ? key & page_mask : 0);
-      k_piece[j] = load_or_zero<T>(k_pages + at * D + seg * VEC, page >= 0);
-    }
-#pragma unroll
-    for (int j = 0; j < VP; ++j) {
-      const int p = threadIdx.x + 256 * j;
-      const int col = p / (TK / VEC), key = key0 + (p % (TK / VEC)) * VEC;
-      const bool in = p < kValuePieces && key <= p_last;
-      const int page = in ? pages[(key >> page_shift) - first_page] : -1;
-      const long at = ((((long)(page >= 0 ? page : 0) * G + g) * DV + (in ? col : 0)) << page_shift) + (page >= 0 ? key & page_mask : 0);
-      vec_t v = load_or_zero<T>(v_pages + at, page >= 0);
-      if (key0 + TK - 1 > p_last) {                                  // (only the tile that holds the block's last row:
-#pragma unroll
-        for (int i = 0; i < VEC; ++i)                                //  what lies beyond that row is not held)
-          if (key + i > p_last) v[i] = (T)0.f;
+  // The page ids of kWindow tiles at a time, by ordinary loads while no tile's load is in flight.  Keys behind the block's last row have the
+  // page of that row, pages that were given back page 0: what is loaded from there is masked, or cleared in LDS.
+  auto fill_pages = [&](int first_step) LS_INLINED {
+    for (int idx = threadIdx.x; idx < S::kWindow * S::kTilePages; idx += 256) {
+      const int step = first_step + idx / S::kTilePages;
+      if (step < step_end) {
+        const int key = min(((tile_at(step) * TK >> page_shift) + idx % S::kTilePages) << page_shift, p_last);
+        tile_pages[idx] = max(my_table[key >> page_shift], 0);
       }
-      v_piece[j] = v;
     }
   };
-  auto store = [&]() LS_INLINED {
-#pragma unroll
-    for (int j = 0; j < KP; ++j) {
-      const int p = threadIdx.x + 256 * j;
-      if (p < kKeyPieces) *reinterpret_cast<vec_t*>(k_lds + (p / (D / VEC)) * kKeyRow + (p % (D / VEC)) * 16) = k_piece[j];
-    }
-#pragma unroll
-    for (int j = 0; j < VP; ++j) {
-      const int p = threadIdx.x + 256 * j;
-      if (p < kValuePieces) *reinterpret_cast<vec_t*>(v_lds + (p / (TK / VEC)) * kValueRow + (p % (TK / VEC)) * 16) = v_piece[j];
-    }
-  };
+  auto opens = [&](int step) LS_INLINED { return (step - step_begin) % S::kWindow == 0; };
 
-  if (threadIdx.x < kTilePages) {
-    page_s[step_begin & 1][threadIdx.x] = look_up(step_begin);
-    page_s[(step_begin + 1) & 1][threadIdx.x] = look_up(step_begin + 1);
+  // Loads.  Piece p of the keys is slot p % KP of key p / KP; piece p of the values is VEC keys (p / DV) of column p % DV.
+  // ONE_PAGE: lane i of `from` holds where the wave's key load i starts, lane 32 + i where its value load i does, and a
+  // lane's offset from there is the same for every tile.
+  constexpr int KO = ONE_PAGE ? KPER : 1;
+  unsigned k_off[KO];
+  const unsigned v_off = ONE_PAGE ? (unsigned)((((w * 64 + lane) % DV) << page_shift) * SZ) : 0u;
+  auto group_of = [&](int load) LS_INLINED { return (load * 256 + w * 64) / (8 * KP) * 8; };   // first of the eight keys a load lies in
+#pragma unroll
+  for (int i = 0; i < KO; ++i) {
+    const int p = i * 256 + (int)threadIdx.x, key = p / KP;
+    k_off[i] = (unsigned)(((key - group_of(i)) * D + slot_of_piece<T>(key, p % KP) * VEC) * SZ);
   }
-  __syncthreads();
-  if (step_begin < step_end) {
-    request(step_begin);
-    store();
-  }
-  __syncthreads();
+  const bool values_lane = lane >= 32;
+  const int my_load = lane & 31;
+  const int my_key = values_lane ? (my_load < VPER ? (my_load * 256 + w * 64) / DV * VEC : 0) : (my_load < KPER ? group_of(my_load) : 0);
+  auto loads_of = [&](int step) LS_INLINED -> unsigned long long {
+    const int key = tile_at(step) * TK + my_key;
+    const int id = tile_pages[(step - step_begin) % S::kWindow * S::kTilePages + (key >> page_shift) - (tile_at(step) * TK >> page_shift)];
+    const long page = (long)id * G + g;
+    return values_lane ? (unsigned long long)(v_pages + ((page * DV) << page_shift) + (key & page_mask))
+                       : (unsigned long long)(k_pages + ((page << page_shift) + (key & page_mask)) * D);
+  };
+  auto load_at = [&](unsigned long long from, int index) LS_INLINED -> unsigned long long {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)from, index) |
+           (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(from >> 32), index) << 32;
+  };
+  const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long)(lptr_t)lds) + w * 1024;
+  auto load_k = [&](unsigned long long from, int i) LS_INLINED {
+    load_to_lds16_from(load_at(from, i), k_off[i % KO], lds_base + i * 4096);
+  };
+  auto load_v = [&](unsigned long long from, int i) LS_INLINED {
+    load_to_lds16_from(load_at(from, 32 + i), v_off, lds_base + S::kKeyBytes + i * 4096);
+  };
+  auto request = [&](int step, auto values) LS_INLINED {              // all of a tile's keys, or values
+    constexpr bool V = decltype(values)::value;
+    if constexpr (ONE_PAGE) {
+      const unsigned long long from = loads_of(step);
+#pragma unroll
+      for (int i = 0; i < (V ? VPER : KPER); ++i) {
+        if (V) load_v(from, i);
+        else load_k(from, i);
+      }
+    } else {
+      const int key0 = tile_at(step) * TK;
+      const int* pages = tile_pages + (step - step_begin) % S::kWindow * S::kTilePages;
+#pragma unroll
+      for (int i = 0; i < (V ? VPER : KPER); ++i) {
+        if (i * 256 + w * 64 >= (V ? V_TOTAL : K_TOTAL)) break;       // uniform for the wave
+        const int p = min(i * 256 + (int)threadIdx.x, (V ? V_TOTAL : K_TOTAL) - 1);
+        const int key = V ? p / DV * VEC : p / KP;
+        const long page = (long)pages[((key0 + key) >> page_shift) - (key0 >> page_shift)] * G + g;
+        const int slot = (key0 + key) & page_mask;
+        const T* src = V ? v_pages + ((page * DV + p % DV) << page_shift) + slot
+                         : k_pages + ((page << page_shift) + slot) * D + slot_of_piece<T>(key, p % KP) * VEC;
+        load_to_lds16(src, (lptr_t)((V ? v_lds : k_lds) + (i * 256 + w * 64) * 16));
+      }
+    }
+  };
+  constexpr std::false_type keys{};
+  constexpr std::true_type values{};
+  // where a lane's fragment of chunk c lies, but for a constant: the swizzle repeats every PERIOD chunks
+  constexpr int PERIOD = KP % 16 == 0 ? 4 : KP % 8 == 0 ? 2 : 1;
+  const unsigned char* k_at[PERIOD];
+#pragma unroll
+  for (int c = 0; c < PERIOD; ++c) k_at[c] = k_lds + (key_of_row<T>(0, l16) * KP + slot_at<T>(l16, 4 * c + quad)) * 16;
+
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) __asm__ volatile("" ::"v"(qv[r][c]));  // the query rows are awaited here, not inside the loop
   for (int step = step_begin; step < step_end; ++step) {
     const int key0 = tile_at(step) * TK;
-    const int page_after = threadIdx.x < kTilePages ? look_up(step + 2) : -1;   // (on its way during the tile)
-    if (step + 1 < step_end) request(step + 1);
-    if (active && key0 <= wave_last) {
-      // -- 1. transposed scores of the tile's groups of 16 keys ----------------------------------
-      f32x4 s[2][NG];
+    const bool fresh = opens(step);          // the tile's page ids were not there when the tile before ran
+    if (fresh) {
+      ring_barrier();
+      fill_pages(step);
+      __syncthreads();
+      request(step, keys);
+      request(step, values);
+    }
+    wait_loads<0>();
+    ring_barrier();                          // the keys are there, and every wave has read the values before
+    const bool mine = active && key0 <= wave_last;
+    if (!fresh && !(ONE_PAGE && mine)) request(step, values);
+    // -- 1. transposed scores of the tile's groups of 16 keys; two groups in turn, the values' loads between ------
+    f32x4 s[2][NG];
+    auto score_products = [&](auto with_loads) LS_INLINED {
+      constexpr int N = NG * KCH, RING = N < 4 ? N : 4;
+      constexpr int PLACES = N < VPER ? 1 : N / VPER;                 // products a load
+      constexpr int AT_ONCE = N < VPER ? (VPER + N - 1) / N : 1;      // loads at such a place
+      auto group = [](int idx) constexpr { return 2 * (idx / (2 * KCH)) + idx % 2; };
+      auto chunk_of = [](int idx) constexpr { return idx / 2 % KCH; };
+      auto k_read = [&](int idx) LS_INLINED -> vec_t {
+        const int c = chunk_of(idx);
+        const unsigned char* src = k_at[c % PERIOD] + (key_of_row<T>(group(idx), 0) * KP + (c - c % PERIOD) * 4) * 16;
+        const bool in = KP % 4 == 0 || c * 4 + quad < KP;
+        vec_t kf = *reinterpret_cast<const vec_t*>(in ? src : k_lds);
+        return in ? kf : A::zero();
+      };
+      unsigned long long from = 0;
+      if constexpr (decltype(with_loads)::value) from = loads_of(step);
+      vec_t ring[RING];
 #pragma unroll
-      for (int ng = 0; ng < NG; ++ng) {
+      for (int i = 0; i < RING; ++i) ring[i] = k_read(i);
+      __builtin_amdgcn_sched_barrier(0);     // (left to itself the compiler reads an operand when it is needed)
 #pragma unroll
-        for (int r = 0; r < 2; ++r) s[r][ng] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int idx = 0; idx < N; ++idx) {
 #pragma unroll
-        for (int c = 0; c < KCH; ++c) {
-          const bool in = c * KC + VEC * quad + VEC <= D;
-          vec_t kf = *reinterpret_cast<const vec_t*>(k_lds + (ng * 16 + l16) * kKeyRow + (in ? c * 64 + quad * 16 : 0));
-          if (!in) kf = Atom<T>::zero();
-#pragma unroll
-          for (int r = 0; r < 2; ++r) Atom<T>::mma(s[r][ng], kf, qv[r][c]);
+        for (int r = 0; r < 2; ++r) {
+          if (chunk_of(idx) == 0) s[r][group(idx)] = f32x4{0.f, 0.f, 0.f, 0.f};
+          A::mma(s[r][group(idx)], ring[idx % RING], qv[r][chunk_of(idx)]);
         }
+        if (idx + RING < N) ring[idx % RING] = k_read(idx + RING);
+        if constexpr (decltype(with_loads)::value) {
+          if (idx % PLACES == 0) {
+#pragma unroll
+            for (int n = idx / PLACES * AT_ONCE; n < (idx / PLACES + 1) * AT_ONCE && n < VPER; ++n) load_v(from, n);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // -- 2. scale, bias, mask, online softmax -----------------------------------------------------
+    };
+    __builtin_amdgcn_s_setprio(1);
+    if (mine) {
+      if (ONE_PAGE && !fresh) score_products(std::bool_constant<ONE_PAGE>{});
+      else score_products(std::false_type{});
+    }
+    __builtin_amdgcn_s_setprio(0);
+    ring_barrier();                          // every wave has read these keys
+    const bool ahead = step + 1 < step_end && !opens(step + 1);
+    if (ahead && !(ONE_PAGE && mine)) request(step + 1, keys);
+    vec_t pb[2][NC];
+    if (mine) {
+      // -- 2. scale, bias, mask, online softmax; the next keys' loads among it --------------------------------
       float shrink[2];
       bool moved = false;
-      auto softmax_tile = [&](auto whole, auto biased) LS_INLINED {
+      unsigned long long from = 0;
+      if (ONE_PAGE && ahead) from = loads_of(step + 1);
+      auto softmax_tile = [&](auto whole, auto biased, auto with_loads) LS_INLINED {
         constexpr bool kWhole = decltype(whole)::value, kBiased = decltype(biased)::value;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-          bool see[NG][4];
           float top = kNegSentinel;
 #pragma unroll
           for (int ng = 0; ng < NG; ++ng)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const int key = key0 + 16 * ng + 4 * quad + i;
-              see[ng][i] = kWhole || (row_ok[r] && key <= my_pos[r] && (key >= my_lo[r] || key < keep_first));
+              const int key = key0 + key_of_row<T>(ng, 4 * quad + i);
+              const bool see = kWhole || ((key <= seen_to[r]) & ((key >= my_lo[r]) | (key < keep_first)));
               float v = s[r][ng][i] * scale;
               if constexpr (kBiased) v = v + my_bias[min(max(my_pos[r] - key, 0), n_dist - 1)];
+              v = see ? v : -__builtin_huge_valf();                   // (its weight is then exp(-inf) = 0)
               s[r][ng][i] = v;
-              top = fmaxf(top, see[ng][i] ? v : kNegSentinel);
+              top = fmaxf(top, v);
+              if constexpr (kBiased) {       // (four biases at a time: the registers of all would not be there)
+                if (i == 3) __builtin_amdgcn_sched_barrier(0);
+              }
             }
           top = quad16_max(top);
           const float m_new = fmaxf(m_run[r], top);
           shrink[r] = softmax_exp<T>(m_run[r] - m_new);
           float sum = 0.f;
 #pragma unroll
-          for (int ng = 0; ng < NG; ++ng)
+          for (int ng = 0; ng < NG; ++ng) {
+            float p[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              s[r][ng][i] = see[ng][i] ? softmax_exp<T>(s[r][ng][i] - m_new) : 0.f;
-              sum = sum + s[r][ng][i];
+              p[i] = softmax_exp<T>(s[r][ng][i] - m_new);
+              pb[r][ng * NC / NG][(sizeof(T) == 2 ? ng % 2 * 4 : 0) + i] = from_f32<T>(p[i]);
             }
+            sum = sum + ((p[0] + p[1]) + (p[2] + p[3]));
+            if constexpr (decltype(with_loads)::value) {
+              constexpr int PLACES = 2 * NG;
+#pragma unroll
+              for (int n = (r * NG + ng) * KPER / PLACES; n < (r * NG + ng + 1) * KPER / PLACES; ++n) load_k(from, n);
+            }
+          }
           sum = quad16_sum(sum);
           l_run[r] = l_run[r] * shrink[r] + sum;
           m_run[r] = m_new;
           moved = moved || shrink[r] != 1.0f;
         }
       };
-      const bool whole_tile = key0 + TK - 1 <= wave_first && (key0 >= wave_lo_last || key0 + TK <= keep_first);
-      if (my_bias) {
-        if (whole_tile) softmax_tile(std::true_type{}, std::true_type{});
-        else softmax_tile(std::false_type{}, std::true_type{});
+      const bool whole_tile = key0 + TK - 1 <= wave_first && (key0 >= wave_lo_last || key0 + TK <= keep_first) && wave_row0 + 31 < nrows;
+      auto softmax_of = [&](auto biased, auto with_loads) LS_INLINED {
+        if (whole_tile) softmax_tile(std::true_type{}, biased, with_loads);
+        else softmax_tile(std::false_type{}, biased, with_loads);
+      };
+      if (my_bias) {                         // (its loads are ordinary ones, whose waits would be for the keys' too)
+        if (ONE_PAGE && ahead) request(step + 1, keys);
+        softmax_of(std::true_type{}, std::false_type{});
       } else {
-        if (whole_tile) softmax_tile(std::true_type{}, std::false_type{});
-        else softmax_tile(std::false_type{}, std::false_type{});
+        if (ONE_PAGE && ahead) softmax_of(std::false_type{}, std::bool_constant<ONE_PAGE>{});
+        else softmax_of(std::false_type{}, std::false_type{});
       }
-      // -- 3. values ---------------------------------------------------------------------------
-      if (__all(!moved) == 0) {
+      if (__any(moved)) {
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -621,60 +741,72 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[r][b][i] = acc[r][b][i] * shrink[r];
       }
-      constexpr int NC = sizeof(T) == 2 ? NG / 2 : NG;   // chunks of keys of the value product
-      vec_t pb[2][NC];
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          if constexpr (sizeof(T) == 2) {
-            typedef __attribute__((ext_vector_type(8))) float f32x8;
-            const f32x8 both = __builtin_shufflevector(s[r][2 * c], s[r][2 * c + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-            pb[r][c] = __builtin_convertvector(both, bf16x8);
-          } else {
-            pb[r][c] = s[r][c];
-          }
-        }
-#pragma unroll
-      for (int b = 0; b < VB; ++b) {
-        const bool col_ok = 16 * b + l16 < DV;
-        const char* column = v_lds + (col_ok ? 16 * b + l16 : 0) * kValueRow;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          vec_t a;
-          if constexpr (sizeof(T) == 2) {
-            const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(column + ((2 * c) * 16 + 4 * quad) * 2);
-            const bf16x4 v1 = *reinterpret_cast<const bf16x4*>(column + ((2 * c + 1) * 16 + 4 * quad) * 2);
-            a = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-          } else {
-            a = *reinterpret_cast<const f32x4*>(column + (c * 16 + 4 * quad) * 4);
-          }
-          if constexpr (DV % 16 != 0) {
-            if (!col_ok) a = Atom<T>::zero();
-          }
-#pragma unroll
-          for (int r = 0; r < 2; ++r) Atom<T>::mma(acc[r][b], a, pb[r][c]);
-        }
-      }
     }
-    __syncthreads();                       // every wave has read this tile
-    if (step + 1 < step_end) store();
-    if (threadIdx.x < kTilePages) page_s[step & 1][threadIdx.x] = page_after;   // (this tile's ids are no longer read)
-    __syncthreads();
+    // the values have landed; the next keys, asked for after them, are still on their way
+    if (ONE_PAGE && ahead) wait_loads<ONE_PAGE ? KPER : 0>();
+    else wait_loads<0>();
+    ring_barrier();
+    if (key0 + TK - 1 > p_last || (key0 < block_lo && key0 + TK > keep_first)) {   // uniform: clear the values of keys that are not held
+#pragma unroll
+      for (int i = 0; i < VPER; ++i) {
+        const int p = i * 256 + (int)threadIdx.x;
+        if (p >= V_TOTAL) break;
+        vec_t* at = reinterpret_cast<vec_t*>(v_lds + p * 16);
+        vec_t v = *at;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const int key = key0 + p / DV * VEC + e;
+          if (!(key <= p_last && (key >= block_lo || key < keep_first))) v[e] = (T)0.f;
+        }
+        *at = v;
+      }
+      ring_barrier();
+    }
+    if (mine) {
+      // -- 3. values ---------------------------------------------------------------------------
+      constexpr int N = VB * NC, RING = N < 4 ? N : 4;
+      auto v_read = [&](int idx) LS_INLINED -> vec_t {
+        const int col = 16 * (idx / NC) + l16;
+        const bool in = DV % 16 == 0 || col < DV;
+        vec_t a = *reinterpret_cast<const vec_t*>(v_lds + ((4 * (idx % NC) + quad) * DV + (in ? col : 0)) * 16);
+        return in ? a : A::zero();
+      };
+      __builtin_amdgcn_s_setprio(1);
+      vec_t ring[RING];
+#pragma unroll
+      for (int i = 0; i < RING; ++i) ring[i] = v_read(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int idx = 0; idx < N; ++idx) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) A::mma(acc[r][idx / NC], ring[idx % RING], pb[r][idx % NC]);
+        if (idx + RING < N) ring[idx % RING] = v_read(idx + RING);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
   }
 
   if (!active) return;
+  const bool vec_ok = DV % 16 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * SZ) == 0;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     if (!row_ok[r]) continue;
     const int row = wave_row0 + 16 * r + l16;
     if (n_runs > 1) {
+      typedef __attribute__((ext_vector_type(2))) float f32x2;
       float* dst = part + (((long)blockIdx.x * part_rows + row) * H + my_head) * (DV + 2);
 #pragma unroll
-      for (int b = 0; b < VB; ++b)
+      for (int b = 0; b < VB; ++b) {
+        if constexpr (DV % 16 == 0) {        // (rows of an even number of floats)
+          *reinterpret_cast<f32x2*>(dst + 16 * b + 4 * quad) = f32x2{acc[r][b][0], acc[r][b][1]};
+          *reinterpret_cast<f32x2*>(dst + 16 * b + 4 * quad + 2) = f32x2{acc[r][b][2], acc[r][b][3]};
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (16 * b + 4 * quad + i < DV) dst[16 * b + 4 * quad + i] = acc[r][b][i];
+          for (int i = 0; i < 4; ++i)
+            if (16 * b + 4 * quad + i < DV) dst[16 * b + 4 * quad + i] = acc[r][b][i];
+        }
+      }
       if (quad == 0) {
         dst[DV] = m_run[r];
         dst[DV + 1] = l_run[r];
@@ -692,16 +824,19 @@ __global__ __launch_bounds__(256) void sink_attention_staged_kernel(
     T* dst = out + (long)(m.q_off + row0 + row) * ldo + (long)my_head * DV;
     const float* g_row = gate ? gate + (long)(m.q_off + row0 + row) * ldg + (long)my_head * DV : nullptr;
 #pragma unroll
-    for (int b = 0; b < VB; ++b)
+    for (int b = 0; b < VB; ++b) {
+      typedef typename std::conditional<sizeof(T) == 2, bf16x4, f32x4>::type v4_t;
+      v4_t o;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int c = 16 * b + 4 * quad + i;
-        if (c < DV) {
-          float v = acc[r][b][i] * inv;
-          if (g_row) v = v * sigmoid_f(g_row[c]);
-          dst[c] = from_f32<T>(v);
-        }
+        float v = acc[r][b][i] * inv;
+        if (g_row && c < DV) v = v * sigmoid_f(g_row[c]);
+        o[i] = from_f32<T>(v);
+        if (!vec_ok && c < DV) dst[c] = o[i];
       }
+      if (vec_ok) *reinterpret_cast<v4_t*>(dst + 16 * b + 4 * quad) = o;
+    }
   }
 }
 
@@ -818,11 +953,14 @@ extern "C" int ls_sink_attention(int dtype, const void* q, long ldq, const void*
                      (const T_*)k_pages, (const T_*)v_pages, page_size, table, table_stride, (const SeqMeta*)seqs,     \
                      items, H, G, scale, window, chunk, keep_first, sink, dist_bias, n_dist, gate, ldg, (T_*)out, ldo, \
                      part, part_rows)
-#define LS_SINK_STAGED(T_)                                                                                             \
-  hipLaunchKernelGGL(sink_attention_staged_kernel<T_>, dim3(n_items, G, (GS + 3) / 4), dim3(256), 0, s, (const T_*)q,  \
-                     ldq, (const T_*)k_pages, (const T_*)v_pages, page_size, table, table_stride,                      \
+#define LS_SINK_STAGED_AS(T_, ONE_PAGE_)                                                                               \
+  hipLaunchKernelGGL((sink_attention_staged_kernel<T_, ONE_PAGE_>), dim3(n_items, G, (GS + 3) / 4), dim3(256), 0, s,   \
+                     (const T_*)q, ldq, (const T_*)k_pages, (const T_*)v_pages, page_size, table, table_stride,        \
                      (const SeqMeta*)seqs, items, H, G, scale, window, chunk, keep_first, sink, dist_bias, n_dist,     \
                      gate, ldg, (T_*)out, ldo, part, part_rows)
+#define LS_SINK_STAGED(T_)                                                                                             \
+  if (Staged<T_>::kOnePage && page_size >= 8) LS_SINK_STAGED_AS(T_, Staged<T_>::kOnePage);                             \
+  else LS_SINK_STAGED_AS(T_, false)
 #define LS_SINK_BY_ROWS(T_)                       \
   switch (row_tiles) {                            \
     case 0: LS_SINK_LAUNCH(T_, 1, true); break;   \
@@ -844,6 +982,7 @@ extern "C" int ls_sink_attention(int dtype, const void* q, long ldq, const void*
   }
 #undef LS_SINK_BY_ROWS
 #undef LS_SINK_STAGED
+#undef LS_SINK_STAGED_AS
 #undef LS_SINK_LAUNCH
   return check_launch("sink_attention");
 }

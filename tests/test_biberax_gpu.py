@@ -247,6 +247,20 @@ def test_attention_kernel_with_every_mask_sink_bias_and_gate(dtype, heads, group
             assert rel_err(got, want) < bound, (label, row_tiles, runs)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, groups, d, dv, page", [(2, 1, 192, 128, 16), (2, 2, 128, 128, 8), (4, 1, 128, 128, 128), (2, 1, 40, 40, 8)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_staged_attention_over_more_tiles_than_one_window_of_page_ids(dtype, heads, groups, d, dv, page, window):
+    """A workgroup holds the page ids of 32 tiles at a time (2,048 keys in bfloat16, 1,024 in float32) and asks for a tile's
+    values and the next one's keys while it multiplies: one run over more tiles than that, and block edges."""
+    bound = 6e-6 if dtype is torch.float32 else 2e-2      # (as above)
+    start = 2100 if dtype is torch.bfloat16 else 1050
+    for runs, lengths, starts in ((1, [33, 65], [start, 63]), (2, [64], [start - 17])):
+        got, want = run_attention_kernel(dtype, heads, groups, d, dv, lengths, starts, page, 8, runs, 0.1, window, 0,
+                                         torch.ones(heads), None, False, seed=d + page + runs)
+        assert rel_err(got, want) < bound, (runs, lengths)
+
+
 def test_a_sink_left_out_or_a_chunk_one_off_shows_in_the_kernel_test():
     """Controls of the test above: the same inputs against a plain result without the sink, or with the
     chunk one larger, differ by many times the bound."""
