@@ -221,14 +221,8 @@ __device__ __forceinline__ int place_tiles(const int* counts, int E, int e, int 
   int base = 0, tile = 0;
   for (int j0 = 0; j0 < e; j0 += 64) {   // (sums of whole numbers: any order)
     const int c = j0 + lane < e ? counts[j0 + lane] : 0;
-    int b = c, t = (c + rows_a_tile - 1) / rows_a_tile;
-#pragma unroll
-    for (int step = 1; step < 64; step <<= 1) {
-      b += __shfl_xor(b, step, kWave);
-      t += __shfl_xor(t, step, kWave);
-    }
-    base += b;
-    tile += t;
+    base += wave_sum(c);
+    tile += wave_sum((c + rows_a_tile - 1) / rows_a_tile);
   }
   if (!write) return base;
   const int n = counts[e];

@@ -10,6 +10,7 @@
 // request was cut into steps or on what else is in the batch.
 
 #include "common.h"
+#include "ring.h"
 #include "mixers_api.h"
 
 namespace ls {
@@ -60,7 +61,10 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int e, int W
 }
 
 // (N, the number of copies, is a template parameter: every copy's load stands in straight-line code, so all of a
-// thread's loads are on their way before the first is used)
+// thread's loads are on their way before the first is used.)  What bounds it at few rows is the chain of answers from memory, so a
+// thread's first run of four elements, the slices' sums, the mixing factors and the weights are asked for together, in front of the
+// first barrier, and what a run was read as stays in registers (rows of up to 1,024 elements are one run): requests of one
+// token through four copies of 1,024 (28 layers, all kernels) 2,633 -> 2,574 us a step
 template <typename T, int N>
 __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X, long ldx, int W,
                                                            const float* __restrict__ P, int slices, long p_stride,
@@ -71,30 +75,47 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
   __shared__ float mix_s[N * N], gain_s[N], take_s[N], scratch[4], sums_s[4];
   const int r_out = blockIdx.x;
   const long row = rows ? rows[r_out] : r_out;
-  if (threadIdx.x < N * N) mix_s[threadIdx.x] = P ? mix[threadIdx.x] : 0.f;
-  if (threadIdx.x < N) {
-    gain_s[threadIdx.x] = P ? gain[threadIdx.x] : 0.f;
-    take_s[threadIdx.x] = take ? take[threadIdx.x] : 1.0f;
-  }
-  __syncthreads();
   float* x = X + row * ldx;
   // rows of whole vectors of four: a copy's elements and a slice's move as 16 bytes
   const bool vec_ok = W % 4 == 0 && ldx % 4 == 0;
   extern __shared__ float u_s[];   // what the row's read gave, until the row's sum of squares is known (a thread's own elements)
-  float part = 0.f;
+  const int e_first = 4 * (int)threadIdx.x;
   constexpr int BATCH = 8;         // slice sums requested together
-#pragma unroll 1
-  for (int e = 4 * (int)threadIdx.x; e < W; e += 1024) {
-    f32x4 copy[N];
+  f32x4 copy[N], got[BATCH], w_first = {0.f, 0.f, 0.f, 0.f}, b_first = w_first;
+  const float* p = P ? P + row * W : nullptr;
+  auto load_run = [&](int e) LS_INLINED {
 #pragma unroll
     for (int s = 0; s < N; ++s) copy[s] = load4(x + (long)s * W, e, W, vec_ok);
+  };
+  auto load_sums = [&](int e, int s0) LS_INLINED {
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) got[u] = load4(p + (long)min(s0 + u, slices - 1) * p_stride, e, W, vec_ok);   // (clamped: no branch between the loads)
+  };
+  const int i_mix = min((int)threadIdx.x, N * N - 1), i_copy = min((int)threadIdx.x, N - 1);
+  const float my_mix = P ? mix[i_mix] : 0.f, my_gain = P ? gain[i_copy] : 0.f, my_take = take ? take[i_copy] : 1.0f;
+  if (e_first < W) {
+    load_run(e_first);
+    if (P) load_sums(e_first, 0);
+    if (out) {
+      w_first = load4(weight, e_first, W, vec_ok);
+      if (bias) b_first = load4(bias, e_first, W, vec_ok);
+    }
+  }
+  if (threadIdx.x < N * N) mix_s[threadIdx.x] = my_mix;
+  if (threadIdx.x < N) {
+    gain_s[threadIdx.x] = my_gain;
+    take_s[threadIdx.x] = my_take;
+  }
+  ring_barrier();                  // (the factors are there; loads from memory stay on their way)
+  float part = 0.f;
+  f32x4 u_first = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int e = e_first; e < W; e += 1024) {
+    if (e != e_first) load_run(e);
     if (P) {
-      const float* p = P + row * W;
       f32x4 y = {0.f, 0.f, 0.f, 0.f};
       for (int s0 = 0; s0 < slices; s0 += BATCH) {
-        f32x4 got[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) got[u] = load4(p + (long)min(s0 + u, slices - 1) * p_stride, e, W, vec_ok);   // (clamped: no branch between the loads)
+        if (s0 > 0 || e != e_first) load_sums(e, s0);
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
           if (s0 + u < slices) y = y + got[u];
@@ -122,18 +143,26 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < N; ++t) sum = sum + take_s[t] * copy[t];
-    if (out) *reinterpret_cast<f32x4*>(u_s + e) = sum;
+    if (e == e_first) u_first = sum;
+    else if (out) *reinterpret_cast<f32x4*>(u_s + e) = sum;
 #pragma unroll
     for (int i = 0; i < 4; ++i) part = part + (centred ? sum[i] : sum[i] * sum[i]);   // (elements beyond W are zeros)
   }
   if (!out) return;
+  // (what a thread reads of u_s it wrote itself; the barriers of the sums are for LDS alone)
+  auto row_sum = [&](float v, float* sums) LS_INLINED -> float {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = v;
+    ring_barrier();
+    return ((sums[0] + sums[1]) + sums[2]) + sums[3];
+  };
   float mean = 0.f;
   if (centred) {   // (the same for the whole launch)
-    mean = block_sum4(part, sums_s) / (float)W;
+    mean = row_sum(part, sums_s) / (float)W;
     part = 0.f;
 #pragma unroll 1
-    for (int e = 4 * (int)threadIdx.x; e < W; e += 1024) {
-      const f32x4 u = *reinterpret_cast<const f32x4*>(u_s + e);
+    for (int e = e_first; e < W; e += 1024) {
+      const f32x4 u = e == e_first ? u_first : *reinterpret_cast<const f32x4*>(u_s + e);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float d = e + i < W ? u[i] - mean : 0.f;
@@ -141,22 +170,27 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
       }
     }
   }
-  const float scale = 1.0f / sqrtf(block_sum4(part, scratch) / (float)W + eps);
+  const float scale = 1.0f / sqrtf(row_sum(part, scratch) / (float)W + eps);
+  const bool vec_out = vec_ok && ld_out % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(T)) == 0;
 #pragma unroll 1
-  for (int e0 = 4 * (int)threadIdx.x; e0 < W; e0 += 1024) {
-    const f32x4 u = *reinterpret_cast<const f32x4*>(u_s + e0);
-    if (vec_ok) {
-      const f32x4 w = *reinterpret_cast<const f32x4*>(weight + e0);
-      f32x4 b = {0.f, 0.f, 0.f, 0.f};
-      if (bias) b = *reinterpret_cast<const f32x4*>(bias + e0);
-      T* dst = out + (long)r_out * ld_out + e0;
+  for (int e0 = e_first; e0 < W; e0 += 1024) {
+    f32x4 u = u_first, w = w_first, b = b_first;
+    if (e0 != e_first) {
+      u = *reinterpret_cast<const f32x4*>(u_s + e0);
+      w = load4(weight, e0, W, vec_ok);
+      if (bias) b = load4(bias, e0, W, vec_ok);
+    }
+    typedef __attribute__((ext_vector_type(4))) T t4;
+    t4 o;
+    T* dst = out + (long)r_out * ld_out + e0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) dst[i] = from_f32<T>(((u[i] - mean) * scale) * w[i] + b[i]);
+    for (int i = 0; i < 4; ++i) o[i] = from_f32<T>(((u[i] - mean) * scale) * w[i] + b[i]);
+    if (vec_out) {
+      *reinterpret_cast<t4*>(dst) = o;
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (e0 + i < W)
-          out[(long)r_out * ld_out + e0 + i] = from_f32<T>(((u[i] - mean) * scale) * weight[e0 + i] + (bias ? bias[e0 + i] : 0.f));
+        if (e0 + i < W) dst[i] = o[i];
     }
   }
 }

@@ -859,19 +859,16 @@ __global__ __launch_bounds__(64) void sink_combine_kernel(const float* __restric
     const int k_mine = threadIdx.x;
     const float m_k = k_mine < n_runs ? mine[k_mine * stride + DV] : kNegSentinel;
     const float l_k = k_mine < n_runs ? mine[k_mine * stride + DV + 1] : 0.f;
-    float top = sink ? sink[h] : kNegSentinel;
-#pragma unroll
-    for (int step = 1; step < 64; step <<= 1) top = fmaxf(top, __shfl_xor(top, step, kWave));
-    float top_runs = m_k;
-#pragma unroll
-    for (int step = 1; step < 64; step <<= 1) top_runs = fmaxf(top_runs, __shfl_xor(top_runs, step, kWave));
-    top = fmaxf(top, top_runs);
+    const float sink_h = sink ? sink[h] : kNegSentinel;
+    const float top = fmaxf(sink_h, wave_max(m_k));
     const float f_k = k_mine < n_runs ? softmax_exp<T>(m_k - top) : 0.f;
     __syncthreads();
     factor_s[k_mine] = f_k;
     float total = 0.f;
-    for (int k = 0; k < n_runs; ++k) total = total + __shfl(l_k, k, kWave) * __shfl(f_k, k, kWave);   // ascending
-    if (sink) total = total + softmax_exp<T>(sink[h] - top);
+    for (int k = 0; k < n_runs; ++k)   // ascending
+      total = total + __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, l_k), k)) *
+                          __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f_k), k));
+    if (sink) total = total + softmax_exp<T>(sink_h - top);
     const float inv = 1.0f / total;
     __syncthreads();
     for (int c = threadIdx.x; c < DV; c += 64) {
