@@ -414,8 +414,9 @@ template <typename T> struct Staged {
   static constexpr int kKeyPieces = D * (int)sizeof(T) / 16;         // 16-byte pieces of a key
   static constexpr int kKeyBytes = kKeys * kKeyPieces * 16;          // of the tile's keys
   static constexpr int kValueBytes = (8 * DV + 63) / 64 * 1024;      // and of its values (whole loads of a wave)
-  static constexpr int kWindow = 32;                                 // tiles whose page ids a workgroup holds
   static constexpr int kTilePages = 16;                              // page ids of a tile, at most
+  static constexpr int kWindow =                                     // tiles whose page ids a workgroup holds
+      kKeyBytes + kValueBytes + 32 * kTilePages * 4 <= 64 * 1024 ? 32 : 8;
   static constexpr int kBytes = kKeyBytes + kValueBytes + kWindow * kTilePages * 4;
   static constexpr bool kFits = kBytes <= 64 * 1024 && D % Atom<T>::VEC == 0;
   static constexpr bool kOnePage = kKeyPieces % 8 == 0 && DV % 64 == 0;
