@@ -185,6 +185,34 @@ def test_the_passes_around_attention_over_a_latent(dtype):
     assert float(got[:, :, kv_rank + rot_dim:].float().abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, dim, rot_dim, rot, kv_rank, dk", [(3, 8, 12, 6, 12, 28), (16, 128, 64, 64, 128, 192), (5, 4, 4, 4, 4, 8),
+                                                                   (7, 12, 8, 2, 8, 16), (3, 8, 10, 6, 12, 24)])
+def test_latent_queries_by_whole_vectors_and_one_by_one(dtype, heads, dim, rot_dim, rot, kv_rank, dk):
+    """Sizes of whole vectors of four take four elements a thread (rotated pairs that end inside a vector among them), others, and rows off a
+    vector's boundary, one: the same bits, and the plain rotation."""
+    t = 9
+    g = torch.Generator().manual_seed(heads + dk)
+    qf = torch.randn((t, heads * (dim + rot_dim)), generator=g)
+    tok_pos = torch.randint(0, 30, (t,), generator=g).to(torch.int32).cuda()
+    f = 50.0 ** (-torch.arange(rot // 2, dtype=torch.float64) * 2.0 / rot)
+    angle = torch.arange(32, dtype=torch.float64)[:, None] * f
+    cos, sin = angle.cos().float().cuda(), angle.sin().float().cuda()
+    results = []
+    for offset in (0, 1):
+        plain_buf = torch.full((t * heads * dim + offset,), float("nan"), dtype=dtype, device="cuda")
+        plain_out = plain_buf[offset:].view(t, heads * dim)
+        q = torch.full((t, heads * dk), float("nan"), dtype=dtype, device="cuda")
+        K().latent_query(qf.cuda(), t, heads, dim, rot_dim, kv_rank, dk, cos, sin, rot, 31, tok_pos, plain_out, q)
+        results.append((plain_out.clone(), q.view(t, heads, dk)[:, :, kv_rank:].clone()))
+        assert bool(torch.isnan(q.view(t, heads, dk)[:, :, :kv_rank]).all())     # (another product's place)
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    per_head = qf.double().view(t, heads, dim + rot_dim)
+    assert close(results[0][0].view(t, heads, dim), per_head[:, :, :dim], dtype)
+    assert float(results[0][1][:, :, rot_dim:].float().abs().max() if dk > kv_rank + rot_dim else 0.0) == 0.0
+    assert close(results[0][1][:, :, :rot_dim], plain.rotate_pairs(per_head[:, :, dim:], tok_pos.cpu().long(), f, 1.0), dtype)
+
+
 @pytest.mark.parametrize("heads, groups, d, dv, taps", [(4, 2, 24, 16, 3), (1, 1, 16, 70, 5), (3, 1, 8, 8, 1), (2, 2, 130, 20, 2),
                                                         (2, 1, 64, 33, 4)])
 def test_the_delta_rule_with_its_convolutions_over_unequal_requests_in_steps(heads, groups, d, dv, taps):
