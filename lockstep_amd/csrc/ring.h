@@ -45,8 +45,11 @@ __device__ __forceinline__ void load_to_lds16(const void* src, __attribute__((ad
   __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory", "m0");
 }
 // The same with the address in two parts: a base that the wave shares, in scalar registers, and a lane's 32-bit offset.
+// The base may come from a vector instruction (v_readlane) right in front of this.  A memory instruction may read such a scalar
+// register five wait states later at the earliest, the hardware does not check it, and the compiler, which sees to it for loads of
+// its own, does not look in here: the s_mov is one of the five, the s_nop four.
 __device__ __forceinline__ void load_to_lds16_from(unsigned long long base, unsigned offset, unsigned lds_wave_base) {
-  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base),
+  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base),
                    "s"(lds_wave_base)
                    : "memory", "m0");
 }

@@ -5,13 +5,16 @@ instances of the fused decode attention once took 75 us a launch that way instea
 So: no kernel may need a stack whose size is only known at run time (that is what a call leaves), and beyond a
 few words (a small object the compiler keeps in memory: the products' kernels have up to 48 bytes) only the
 kernels listed here may use scratch memory (true register spills, known and measured), the wide attention kernels
-no more of it than is listed for their head size."""
+no more of it than is listed for their head size.  And from the code itself: the distance that the hardware asks for
+between a vector instruction that writes a scalar register and a memory instruction that reads it."""
 
 from __future__ import annotations
 
+import concurrent.futures
 import pathlib
 import re
 import struct
+import subprocess
 
 import pytest
 
@@ -65,6 +68,46 @@ def code_object_notes(blob: bytes):
         at += 4
 
 
+def code_objects(blob: bytes):
+    """The AMDGPU code objects bundled in a library, each an ELF file of its own."""
+    at = blob.find(b"\x7fELF")
+    while at >= 0:
+        shoff, = struct.unpack_from("<Q", blob, at + 0x28)
+        shentsize, shnum = struct.unpack_from("<HH", blob, at + 0x3A)
+        if struct.unpack_from("<H", blob, at + 0x12)[0] == 224:
+            yield blob[at: at + shoff + shentsize * shnum]
+        at = blob.find(b"\x7fELF", at + 4)
+
+
+def scalar_registers(operands: str) -> set:
+    """The numbers of the scalar registers that an instruction's operands name."""
+    found = set()
+    for first, last, one in re.findall(r"\bs\[(\d+):(\d+)\]|\bs(\d+)\b", operands):
+        found |= {int(one)} if one else set(range(int(first), int(last) + 1))
+    return found
+
+
+def early_scalar_reads(listing: str):
+    """(function, instruction) of the memory instructions that read a scalar register fewer than five wait states after a
+    vector instruction wrote it (v_readlane, v_readfirstlane, a comparison), in the order of the listing."""
+    function, age = "", {}                                    # age: wait states since a register was written so
+    for line in listing.splitlines():
+        if line.endswith(">:"):
+            function, age = line, {}
+            continue
+        op, _, operands = line.split("//")[0].strip().partition(" ")
+        if op.startswith(("global_", "buffer_", "flat_", "scratch_")) and scalar_registers(operands) & age.keys():
+            yield function, line.strip()
+        passed = int(operands.strip(), 0) + 1 if op == "s_nop" else 1
+        age = {reg: n + passed for reg, n in age.items() if n + passed < 5}
+        written = scalar_registers(operands.split(",")[0])
+        if op.startswith(("v_readlane", "v_readfirstlane", "v_cmp")):
+            age.update(dict.fromkeys(written, 0))
+        elif op.startswith("s_") and "cmp" not in op:         # (the scalar unit's own writes need no distance)
+            for reg in written:
+                age.pop(reg, None)
+
+
 def kernels_of(path: pathlib.Path):
     for note in code_object_notes(path.read_bytes()):
         for kernel in note.get("amdhsa.kernels", []):
@@ -98,3 +141,36 @@ def test_no_kernel_calls_a_function_and_only_known_ones_spill():
             if scratch > SMALL and not any(part in name for part in allowed):
                 pytest.fail(f"{lib.name}: {name} uses {scratch} bytes of scratch memory a lane")
     assert seen > 100, "the libraries' metadata was not found"
+
+
+def test_early_reads_of_scalar_registers_are_seen():
+    listing = "0000 <f>:\n\tv_readlane_b32 s8, v1, 3\n\ts_mov_b32 m0, s5\n\t{}\n\tglobal_load_lds_dwordx4 v2, s[8:9]  // 00"
+    assert len(list(early_scalar_reads(listing.format("s_nop 0")))) == 1
+    assert len(list(early_scalar_reads(listing.format("s_nop 2")))) == 1
+    assert not list(early_scalar_reads(listing.format("s_nop 3")))
+    assert not list(early_scalar_reads(listing.format("s_mov_b32 s8, s6")))
+
+
+@pytest.mark.skipif(not LIBS, reason="no library has been built in the tree")
+def test_memory_instructions_leave_scalar_registers_their_wait_states(tmp_path):
+    """A memory instruction that reads a scalar register which a vector instruction has just written gets the old value,
+    unless five wait states lie between: the compiler sees to it, but not inside inline assembly."""
+    objdump = pathlib.Path("/opt/rocm/llvm/bin/llvm-objdump")
+    if not objdump.is_file():
+        pytest.skip("no llvm-objdump")
+
+    def early(lib):
+        found = []
+        for i, code in enumerate(code_objects(lib.read_bytes())):
+            path = tmp_path / f"{lib.name}.{i}.o"
+            path.write_bytes(code)
+            listing = subprocess.run([str(objdump), "-d", "--no-show-raw-insn", "--no-leading-addr", str(path)], capture_output=True,
+                                     text=True, check=True).stdout
+            path.unlink()
+            assert "s_endpgm" in listing, lib.name
+            found += [(lib.name, *where) for where in early_scalar_reads(listing)]
+        return found
+
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        found = [hit for hits in pool.map(early, LIBS) for hit in hits]
+    assert not found, (len(found), found[:4])
