@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
   // lane's offset from there is the same for every tile.
   constexpr int KO = ONE_PAGE ? KPER : 1;
   unsigned k_off[KO];
-  const unsigned v_off = ONE_PAGE ? (unsigned)((((w * 64 + lane) % DV) << page_shift) * SZ) : 0u;
+  const unsigned v_off = ONE_PAGE ? (unsigned)((lane << page_shift) * SZ) : 0u;   // (64 columns from the load's first)
   auto group_of = [&](int load) LS_INLINED { return (load * 256 + w * 64) / (8 * KP) * 8; };   // first of the eight keys a load lies in
 #pragma unroll
   for (int i = 0; i < KO; ++i) {
@@ -553,12 +553,13 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
   }
   const bool values_lane = lane >= 32;
   const int my_load = lane & 31;
-  const int my_key = values_lane ? (my_load < VPER ? (my_load * 256 + w * 64) / DV * VEC : 0) : (my_load < KPER ? group_of(my_load) : 0);
+  const int my_piece = values_lane && my_load < VPER ? my_load * 256 + w * 64 : 0, my_col = my_piece % DV;   // (the waves' first columns differ where DV does not divide 256)
+  const int my_key = values_lane ? my_piece / DV * VEC : (my_load < KPER ? group_of(my_load) : 0);
   auto loads_of = [&](int step) LS_INLINED -> unsigned long long {
     const int key = tile_at(step) * TK + my_key;
     const int id = tile_pages[(step - step_begin) % S::kWindow * S::kTilePages + (key >> page_shift) - (tile_at(step) * TK >> page_shift)];
     const long page = (long)id * G + g;
-    return values_lane ? (unsigned long long)(v_pages + ((page * DV) << page_shift) + (key & page_mask))
+    return values_lane ? (unsigned long long)(v_pages + ((page * DV + my_col) << page_shift) + (key & page_mask))
                        : (unsigned long long)(k_pages + ((page << page_shift) + (key & page_mask)) * D);
   };
   auto load_at = [&](unsigned long long from, int index) LS_INLINED -> unsigned long long {

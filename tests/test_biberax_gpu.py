@@ -261,6 +261,20 @@ def test_staged_attention_over_more_tiles_than_one_window_of_page_ids(dtype, hea
         assert rel_err(got, want) < bound, (runs, lengths)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, groups, d, dv, page", [(2, 1, 64, 192, 16), (4, 2, 64, 320, 8), (1, 1, 64, 192, 128)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_staged_attention_with_value_rows_that_do_not_divide_a_load_of_the_workgroup(dtype, heads, groups, d, dv, page, window):
+    """A workgroup's four waves load 256 pieces of values at a time: with 192 or 320 columns a wave's loads start at
+    another column each, over several tiles and in one run or two."""
+    bound = 6e-6 if dtype is torch.float32 else 2e-2      # (as above)
+    assert K().sink_staged_keys(d, dv, dtype)
+    for runs, lengths, starts in ((1, [33, 65], [200, 63]), (2, [64], [150])):
+        got, want = run_attention_kernel(dtype, heads, groups, d, dv, lengths, starts, page, 8, runs, 0.1, window, 0,
+                                         torch.ones(heads), None, False, seed=d + page + runs)
+        assert rel_err(got, want) < bound, (runs, lengths)
+
+
 def test_a_sink_left_out_or_a_chunk_one_off_shows_in_the_kernel_test():
     """Controls of the test above: the same inputs against a plain result without the sink, or with the
     chunk one larger, differ by many times the bound."""
