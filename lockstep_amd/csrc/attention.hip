@@ -132,7 +132,7 @@ __device__ __forceinline__ constexpr int key_of_row(int kb, int r) {
 // the wide kernel at a head size of 128 show bank conflicts in 31 % of LDS's active cycles.)
 template <typename T>
 __device__ __forceinline__ constexpr int row_rotation(int row) {
-  return sizeof(T) == 2 ? (row & 3) + 4 * ((row >> 3) & 3) : row;
+  return sizeof(T) == 2 ? (row & 3) + 4 * ((row >> 3) & 3) : row & 15;
 }
 
 // The slot of a key row's 16-byte piece, and the other way round.  Rows of a multiple of 256 bytes all start at bank 0
@@ -140,12 +140,12 @@ __device__ __forceinline__ constexpr int row_rotation(int row) {
 template <typename T>
 __device__ __forceinline__ constexpr int slot_of_piece(int row, int piece) {
   constexpr int KPIECES = D * (int)sizeof(T) / 16;
-  return KPIECES % 16 == 0 ? piece ^ (row_rotation<T>(row) & 15) : (piece + row_rotation<T>(row)) % KPIECES;
+  return KPIECES % 16 == 0 ? piece ^ row_rotation<T>(row) : (piece + row_rotation<T>(row)) % KPIECES;
 }
 template <typename T>
 __device__ __forceinline__ constexpr int piece_of_slot(int row, int slot) {
   constexpr int KPIECES = D * (int)sizeof(T) / 16;
-  return KPIECES % 16 == 0 ? slot ^ (row_rotation<T>(row) & 15)
+  return KPIECES % 16 == 0 ? slot ^ row_rotation<T>(row)
                            : (slot - row_rotation<T>(row) % KPIECES + KPIECES) % KPIECES;
 }
 
@@ -767,10 +767,18 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 // waves had the CU, its waves in step, and LDS, vector unit and matrix cores took turns.  Raised priority during the
 // products lets a wave that has operands go first (2,048 tokens, 32 over 8 heads: 64.7 -> 57.7 us).
 // What bounds it: LDS (a tile's 64 KB are written once and read by each of the four waves: 2,600 of some 3,400 cycles a
-// workgroup's tile) and the vector unit (1,600 a wave).  Measured, bfloat16, D = 128, us, two buffers / now: 2,048 tokens from
-// position 0, 16 over 8 heads 59.6 / 42, 32 over 8 66 / 58; from 6,144 207 / 168; 808 tokens from 8,192 195 / 152;
-// D = 64 38 / 31, 43 / 41, 133 / 111, 131 / 115; D = 256 (which did not fit two buffers) 738 / 70 against the staged
-// kernel; float32 D = 128 the same 495 / 178.
+// workgroup's tile) and the vector unit (1,600 a wave).  Measured, bfloat16, us, two buffers / now, for 2,048 tokens from
+// position 0 of 16 over 8 heads, the same of 32 over 8, 2,048 tokens of 16 over 8 from 6,144, 808 from 8,192:
+//   D = 128  62 / 46    71 / 59   211 / 171   196 / 158        D = 64   40 / 34   45 / 43   134 / 116   133 / 120
+//   D = 112  61 / 51    69 / 67   211 / 186   187 / 180        D = 80   51 / 43   58 / 57   181 / 157   155 / 155
+//   D = 144  89 / 60   101 / 79   311 / 225   235 / 216        D = 32   33 / 28   38 / 32   110 / 99    101 / 103
+// (D = 32, 2,048 tokens of 32 over 8 heads from 6,144, 164 / 173, is the one that two buffers took more than a few per cent
+// faster); sizes that did not fit two buffers, against the staged kernel: D = 192 239 / 77, D = 256 734 / 77, float32
+// D = 128 496 / 184, D = 144 592 / 219 for the first of these.
+// Registers: two workgroups share a CU while a lane needs 256 at most, and a spilled register costs more than its instruction,
+// because the wait for it is a wait for every load in flight (D = 144 with 86 of them: 131 us in place of 60, 2,048 from 6,144 769
+// in place of 225).  So what can be worked out again for a tile is not kept from one to the next: operand addresses are a lane's
+// base and constants, page ids four bits a load, 64-bit sources are formed at the load (333 registers -> 256 at D = 144, none spilled).
 // Not kept: 32 rows a wave (half the LDS reads; one wave a SIMD then waits for itself: 63 us for the first of these).
 // Whether two workgroups' K and V tiles (and the page ids, 2 KB each) fit into a CU's LDS.
 constexpr bool wide_shares_cu(int element_bytes) { return 2 * (2 * kTileKeys * D * element_bytes + kPageWindow * 64) <= 160 * 1024; }
@@ -861,7 +869,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
   // so the loads stay inside the cache, and what they bring is masked.
   const long page_stride = (long)nkv * page_size * D;  // elements of one page, K or V
   // (K rows of a load: the rotation repeats every PERIOD rows, so KV lane offsets serve all loads)
-  constexpr int RPI = NT / KPIECES, PERIOD = SZ == 2 ? 32 : KPIECES;
+  constexpr int RPI = NT / KPIECES, PERIOD = SZ == 2 ? 32 : 16;
   constexpr int KV = !ONE_PAGE ? PER : RPI % PERIOD == 0 ? 1 : PERIOD % RPI == 0 && PERIOD / RPI < PER ? PERIOD / RPI : PER;
   constexpr int VV = ONE_PAGE ? 1 : PER;
   int k_off[KV], v_off[VV];
@@ -877,6 +885,17 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
   for (int i = 0; i < VV; ++i) {
     const int p = i * NT + (int)threadIdx.x;
     v_off[i] = ((kvh * D + p % D) << page_shift) + (ONE_PAGE ? 0 : (p / D * VEC) & (page_size - 1));
+  }
+  // Otherwise every lane looks its piece's page up: which of the tile's sixteen ids, four bits a load.
+  constexpr int IDS = ONE_PAGE ? 1 : (PER + 7) / 8;
+  unsigned k_ids[IDS], v_ids[IDS];
+#pragma unroll
+  for (int i = 0; i < IDS; ++i) k_ids[i] = v_ids[i] = 0;
+#pragma unroll
+  for (int i = 0; i < (ONE_PAGE ? 0 : PER); ++i) {
+    const int p = i * NT + (int)threadIdx.x;
+    k_ids[i / 8] |= (unsigned)min((p / KPIECES) >> page_shift, 15) << (4 * (i % 8));
+    v_ids[i / 8] |= (unsigned)min((p / D * VEC) >> page_shift, 15) << (4 * (i % 8));
   }
   // With ONE_PAGE a wave's load has its address in scalar registers: lane i of `from` holds where the wave's K load i
   // starts, lane 32 + i where its V load i does.
@@ -915,19 +934,30 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
       int page[PER];
 #pragma unroll
       for (int i = 0; i < PER; ++i) {  // all page ids first: their LDS reads overlap
-        const int p = i * NT + (int)threadIdx.x;
-        page[i] = pages[min((V ? p / D * VEC : p / KPIECES) >> page_shift, 15)];
+        unsigned ids = V ? v_ids[i / 8] : k_ids[i / 8];
+        __asm__ volatile("" : "+v"(ids));  // (the compiler would keep every load's id address, and its 64-bit source below, from tile to tile)
+        page[i] = pages[ids >> (4 * (i % 8)) & 15];
       }
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         if (PER * NT != TOTAL && i * NT + wave * 64 >= TOTAL) break;  // uniform for the wave
-        const T* src = (V ? v_pages : k_pages) + (long)max(page[i], 0) * page_stride + (V ? v_off[i % VV] : k_off[i % KV]);
+        int off = V ? v_off[i % VV] : k_off[i % KV];
+        __asm__ volatile("" : "+v"(off));
+        const T* src = (V ? v_pages : k_pages) + (long)max(page[i], 0) * page_stride + off;
         load_to_lds16(src, (lptr_t)((V ? v_lds : k_lds) + (i * NT + wave * 64) * 16));
       }
     }
   };
   constexpr std::false_type keys{};
   constexpr std::true_type values{};
+  // where a lane's operands lie but for a constant (the rotation is the same in every block of sixteen keys)
+  const unsigned char* k_at[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int row = key_of_row<T>(0, row16);
+    k_at[c] = k_lds + row * KROW + slot_of_piece<T>(row, min(c * 4 + g, KPIECES - 1)) * 16;
+  }
+  const unsigned char* v_at = v_lds + (key_of_row<T>(0, 4 * g) / VEC * D + row16) * 16;
 
   RowState run;
   run.reset();
@@ -973,10 +1003,8 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
       auto block_of = [](int idx) constexpr { return 2 * (idx / (2 * NC)) + idx % 2; };
       auto chunk_of = [](int idx) constexpr { return idx / 2 % NC; };
       auto k_read = [&](int idx) LS_INLINED -> vec_t {
-        const int row = key_of_row<T>(block_of(idx), row16);
         const int piece = chunk_of(idx) * 4 + g;
-        const int pc = (4 * NC == KPIECES) ? piece : min(piece, KPIECES - 1);
-        vec_t kv = *reinterpret_cast<const vec_t*>(k_lds + row * KROW + slot_of_piece<T>(row, pc) * 16);
+        vec_t kv = *reinterpret_cast<const vec_t*>(k_at[chunk_of(idx)] + key_of_row<T>(block_of(idx), 0) * KROW);
         if (4 * NC != KPIECES) kv = piece < KPIECES ? kv : A::zero();
         return kv;
       };
@@ -1073,8 +1101,8 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
       run.m = some ? m_new : run.m;
     }
     PROBE(4)
-    // V has landed; the next K, asked for after it, is still on its way
-    if (ONE_PAGE && ahead) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+    // V has landed; the next K, asked for after it (by every wave with as many loads as this at least), is still on its way
+    if (ahead) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * NT == TOTAL ? PER : PER - 1) : "memory");
     else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     ring_barrier();
     if (t0 + kTileKeys > sm.kv_len || t0 < lo_valid) {  // uniform: clean the values of keys that are not held
@@ -1098,9 +1126,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
         constexpr int STEPS = PAIR * NK, PARTS = PAIR * 4;   // products of such a set of blocks, and its sums a lane
         auto v_read = [&](int idx) LS_INLINED -> vec_t {
           const int kb = (idx / PAIR % NK) * KB16;
-          const int d = (PAIR * (idx / STEPS) + idx % PAIR) * 16 + row16;
-          const int key = key_of_row<T>(kb, 4 * g);  // the lane's first key inside the tile (its others follow)
-          return *reinterpret_cast<const vec_t*>(v_lds + ((key / VEC) * D + d) * 16);
+          return *reinterpret_cast<const vec_t*>(v_at + (key_of_row<T>(kb, 0) / VEC * D + (PAIR * (idx / STEPS) + idx % PAIR) * 16) * 16);
         };
         vec_t ring[RING];
 #pragma unroll
@@ -2374,7 +2400,7 @@ extern "C" int ls_attention_decode(int dtype, const void* qkv, long ld, void* k_
 // CU, 281 / 178), unless their loads need addresses of their own (float32, D = 80: 286 / 262, registers spill).
 constexpr int kLargeBlock = 128, kSmallBlock = 64;   // rows of variant 4's and variant 5's row blocks
 constexpr bool wide_has_eight_waves(int element_bytes) { return !wide_shares_cu(element_bytes) && D % 64 == 0; }
-static size_t wide_lds_bytes(int dtype) { return 2 * (size_t)kTileKeys * D * (dtype == kF32 ? 4 : 2) + kPageWindow * 16 * sizeof(int); }
+constexpr size_t wide_lds_bytes(int element_bytes) { return 2 * (size_t)kTileKeys * D * element_bytes + kPageWindow * 16 * sizeof(int); }
 template <typename T, int NW>
 static bool wide_kernel_ready(size_t bytes) {
   static int state = 0;  // 0 unknown, 1 granted, -1 refused
@@ -2387,17 +2413,14 @@ static bool wide_kernel_ready(size_t bytes) {
   return state == 1;
 }
 template <typename T>
-static bool wide_ready(size_t bytes) {
-  if constexpr (wide_has_eight_waves(sizeof(T)))
-    if (!wide_kernel_ready<T, 8>(bytes)) return false;
-  return wide_kernel_ready<T, 4>(bytes);
+static bool wide_ready() {
+  constexpr size_t bytes = wide_lds_bytes(sizeof(T));
+  if constexpr (bytes > kLdsLimit) return false;
+  else if constexpr (bytes <= 64 * 1024) return true;
+  else if constexpr (wide_has_eight_waves(sizeof(T))) return wide_kernel_ready<T, 8>(bytes) && wide_kernel_ready<T, 4>(bytes);
+  else return wide_kernel_ready<T, 4>(bytes);
 }
-static bool wide_supported(int dtype) {
-  const size_t bytes = wide_lds_bytes(dtype);
-  if (bytes > kLdsLimit) return false;
-  if (bytes <= 64 * 1024) return true;
-  return dtype == kF32 ? wide_ready<float>(bytes) : wide_ready<bf16_t>(bytes);
-}
+static bool wide_supported(int dtype) { return dtype == kF32 ? wide_ready<float>() : wide_ready<bf16_t>(); }
 // 1 if the wide kernel (variants 4 and 5) can run for this dtype.
 extern "C" int ls_attn_wide_supported(int dtype) { return wide_supported(dtype) ? 1 : 0; }
 // 1 if variant 4's row blocks have a workgroup of eight waves each (else two of variant 5's workgroups).
@@ -2410,24 +2433,26 @@ template <typename T>
 static void launch_wide(int variant, hipStream_t s, const void* q, long ldq, const void* k_pages, const void* v_pages, int nkv,
                         int page_size, int page_shift, const int* table, int table_stride, const void* seqs, const void* items,
                         int n_items, void* out, long ldo, float* part_acc, float* part_ml, int G, float scale, int window) {
-  const size_t bytes = wide_lds_bytes(sizeof(T) == 4 ? kF32 : kBF16);
-  // Workgroup ids go round the eight XCDs, and all row blocks of a kv head walk the same keys and values.  With the kv heads
-  // as the fast dimension a head's blocks meet on one XCD (8, 16, ... heads; fewer: on as many XCDs as share one), whose L2
-  // then answers most of their loads; with the row blocks as the fast dimension every XCD reads every head from beyond
-  // its L2, which bound the whole kernel.  (Numbered so inside the kernel instead, an item's record waits for the
-  // divisions: 97 tokens, 2 kv heads of 64, 7.3 us in place of 7.1.)
-  for (int first = 0; first < n_items; first += kMaxGridY) {
-    const int n = n_items - first < kMaxGridY ? n_items - first : kMaxGridY;
-    auto launch = [&](auto kernel, int waves, int halves) {
-      hipLaunchKernelGGL(kernel, dim3(nkv, n, halves), dim3(64 * waves), bytes, s, (const T*)q, ldq, (const T*)k_pages,
-                         (const T*)v_pages, nkv, page_size, page_shift, table, table_stride, (const SeqMeta*)seqs,
-                         (const AttnItem*)items + first, (T*)out, ldo, part_acc, part_ml, G, scale, window);
-    };
-    if (variant == 4) {
-      if constexpr (wide_has_eight_waves(sizeof(T))) launch(attention_wide_kernel<T, 8>, 8, 1);
-      else launch(attention_wide_kernel<T, 4>, 4, 2);
-    } else {
-      launch(attention_wide_kernel<T, 4>, 4, 1);
+  constexpr size_t bytes = wide_lds_bytes(sizeof(T));
+  if constexpr (bytes <= kLdsLimit) {
+    // Workgroup ids go round the eight XCDs, and all row blocks of a kv head walk the same keys and values.  With the kv heads
+    // as the fast dimension a head's blocks meet on one XCD (8, 16, ... heads; fewer: on as many XCDs as share one), whose L2
+    // then answers most of their loads; with the row blocks as the fast dimension every XCD reads every head from beyond
+    // its L2, which bound the whole kernel.  (Numbered so inside the kernel instead, an item's record waits for the
+    // divisions: 97 tokens, 2 kv heads of 64, 7.3 us in place of 7.1.)
+    for (int first = 0; first < n_items; first += kMaxGridY) {
+      const int n = n_items - first < kMaxGridY ? n_items - first : kMaxGridY;
+      auto launch = [&](auto kernel, int waves, int halves) {
+        hipLaunchKernelGGL(kernel, dim3(nkv, n, halves), dim3(64 * waves), bytes, s, (const T*)q, ldq, (const T*)k_pages,
+                           (const T*)v_pages, nkv, page_size, page_shift, table, table_stride, (const SeqMeta*)seqs,
+                           (const AttnItem*)items + first, (T*)out, ldo, part_acc, part_ml, G, scale, window);
+      };
+      if (variant == 4) {
+        if constexpr (wide_has_eight_waves(sizeof(T))) launch(attention_wide_kernel<T, 8>, 8, 1);
+        else launch(attention_wide_kernel<T, 4>, 4, 2);
+      } else {
+        launch(attention_wide_kernel<T, 4>, 4, 1);
+      }
     }
   }
 }

@@ -253,7 +253,7 @@ def build_attention_mutants(head_dim: int, force: bool = False) -> Path:
     return build(f"attention{head_dim}.mutants", ATTENTION_SOURCES, (f"-DLS_HEAD_DIM={head_dim}", MUTANT_DEFINE), force)
 
 
-DEFAULT_HEAD_DIMS = (16, 32, 48, 64, 80, 128, 256)
+DEFAULT_HEAD_DIMS = (16, 32, 48, 64, 80, 112, 128, 144, 160, 192, 256)
 MUTANT_HEAD_DIMS = (16, 32, 128)     # the head sizes of the tests that use the controls
 #: (query heads, kv heads, key size, value size) of the talking-heads attention the tests and measurements use
 DEFAULT_TALKING_SHAPES = ((4, 2, 32, 16), (6, 3, 48, 24), (3, 1, 24, 40), (2, 2, 16, 16), (16, 8, 128, 128),

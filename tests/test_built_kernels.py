@@ -21,15 +21,16 @@ import pytest
 LIB_DIR = pathlib.Path(__file__).resolve().parent.parent / "lockstep_amd" / "_lib"
 # kernels that are known to spill (256 registers a lane are not enough for them), by a part of their name
 SMALL = 64                                              # bytes a lane that need no entry here
-# paged attention of row blocks, bytes a lane by head size (float tiles of more than 64 elements do not fit LDS, and such
-# instances never run); head sizes that are not listed, and every other instance, keep to SMALL
-WIDE_MAY_SPILL = {"attention_wide_kernelIfLi8E": {80: 160, 96: 312, 112: 472, 128: 288, 144: 760},
-                  "attention_wide_kernelIfLi4E": {144: 216}, "attention_wide_kernelIDF16bLi8E": {144: 192}}
-# ... and registers a lane with which two workgroups of eight waves share a CU
-WIDE_REGISTERS = {"attention_wide_kernelIDF16bLi8E": {16: 128, 32: 128}}
+# paged attention of row blocks: in workgroups of four waves none may (the wait for a spilled register is a wait for every load
+# in flight), and a lane keeps to 256 registers where two of them share a CU; in workgroups of eight waves, which have 256
+# registers at most, bytes a lane by head size
+WIDE_MAY_SPILL = {"attention_wide_kernelIfLi8E": {128: 72}, "attention_wide_kernelIDF16bLi8E": {192: 104, 256: 220}}
+WIDE_SHARES_A_CU = {"attention_wide_kernelIfLi4E": 64, "attention_wide_kernelIDF16bLi4E": 144}     # largest such head size
 # recurrences of one wave a workgroup, whose registers let two waves share a SIMD
 TWO_WAVES = ("delta_rule_kernel",)
-MAY_SPILL_AT_HEAD_256 = ("attention_",)               # every float instance at a head size of 256, and some bfloat16
+# other kernels of paged attention, by head size: float instances of large heads, and some bfloat16
+MAY_SPILL_AT_HEAD = {160: ("attention_coop_kernelIf",), 192: ("attention_coop_kernelIf", "attention_staged_kernelIDF16b"),
+                     256: ("attention_coop_kernel", "attention_staged_kernel")}
 # sink attention with keys of more than 256 or values of more than 128 elements (a library of such a shape is built when a
 # model first asks for it): correct, not fast, or the instances of four row tiles, which only measurements use
 MAY_SPILL_AT_WIDE_HEADS = ("sink_attention_",)
@@ -121,7 +122,6 @@ LIBS = sorted(LIB_DIR.glob("liblockstep_*.so")) if LIB_DIR.is_dir() else []
 def test_no_kernel_calls_a_function_and_only_known_ones_spill():
     seen = 0
     for lib in LIBS:
-        head_256 = "attention256" in lib.name
         head = int(re.match(r"liblockstep_attention(\d+)", lib.name).group(1)) if "_attention" in lib.name else 0
         sizes = lib.name.split("sink")[1].split("-")[0].split("x") if "sink" in lib.name else None
         wide_heads = sizes is not None and (int(sizes[0]) > 256 or int(sizes[1]) > 128)
@@ -132,12 +132,13 @@ def test_no_kernel_calls_a_function_and_only_known_ones_spill():
             scratch = kernel.get(".private_segment_fixed_size", 0)
             if any(part in name for part in TWO_WAVES):
                 assert kernel[".vgpr_count"] <= 256, f"{lib.name}: {name}"
-            for part, limits in WIDE_REGISTERS.items():
-                if part in name:
-                    assert kernel[".vgpr_count"] <= limits.get(head, 512), f"{lib.name}: {name}"
-            if scratch <= max((limits.get(head, 0) for part, limits in WIDE_MAY_SPILL.items() if part in name), default=0):
+            if "attention_wide_kernel" in name:
+                most = max((limits.get(head, 0) for part, limits in WIDE_MAY_SPILL.items() if part in name), default=0)
+                assert scratch <= most, f"{lib.name}: {name} uses {scratch} bytes of scratch memory a lane"
+                shared = max((largest for part, largest in WIDE_SHARES_A_CU.items() if part in name), default=0)
+                assert head > shared or kernel[".vgpr_count"] <= 256, f"{lib.name}: {name}"
                 continue
-            allowed = (MAY_SPILL_AT_HEAD_256 if head_256 else ()) + (MAY_SPILL_AT_WIDE_HEADS if wide_heads else ())
+            allowed = MAY_SPILL_AT_HEAD.get(head, ()) + (MAY_SPILL_AT_WIDE_HEADS if wide_heads else ())
             if scratch > SMALL and not any(part in name for part in allowed):
                 pytest.fail(f"{lib.name}: {name} uses {scratch} bytes of scratch memory a lane")
     assert seen > 100, "the libraries' metadata was not found"

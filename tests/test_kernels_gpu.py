@@ -788,6 +788,26 @@ def test_wide_attention_at_the_edges_of_its_row_blocks_and_page_windows(dtype, n
                 assert torch.equal(got, want), (start, length, variant)
 
 
+@pytest.mark.parametrize("dtype,nq,nkv,d,ps", [(torch.bfloat16, 4, 2, 112, 16), (torch.bfloat16, 3, 1, 144, 8), (torch.float32, 4, 2, 144, 16),
+                                               (torch.float32, 3, 1, 112, 128), (torch.bfloat16, 4, 2, 160, 64), (torch.bfloat16, 2, 2, 192, 8)])
+@pytest.mark.parametrize("window", [0, 150])
+def test_wide_attention_where_a_load_spans_several_pages(dtype, nq, nkv, d, ps, window):
+    """Head sizes whose rows do not divide a wave's load: every lane looks its piece's page up, among the sixteen of a tile, and
+    the last round of loads is only some waves'.  The bits of the kernel that loads straight from global memory."""
+    n = 4000 + 130
+    qkv = rand_qkv(n, nq, nkv, d, dtype, seed=d + ps)
+    case = PagedCase(dtype, nq, nkv, d, ps, n, shuffle_seed=9)
+    dev = qkv.cuda()
+    case.write(dev, 0)
+    assert K().wide_supported(d, dtype, ps)
+    for start, length in ((0, 97), (127, 65), (4000, 130), (3967, 33)):
+        rows = dev[start:start + length]
+        want = case.attend(rows, start, d ** -0.5, window=window, variant=1, force_split=False)
+        for variant in (4, 5):
+            got = case.attend(rows, start, d ** -0.5, window=window, variant=variant, force_split=False)
+            assert torch.equal(got, want), (start, length, variant)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nq,nkv,d,ps", [(16, 8, 128, 16), (6, 3, 32, 8), (8, 1, 64, 16)])
 def test_attention_row_is_the_same_alone_in_a_portion_and_in_the_whole_prompt(dtype, nq, nkv, d, ps):
