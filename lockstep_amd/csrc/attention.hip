@@ -2393,13 +2393,17 @@ extern "C" int ls_attention_decode(int dtype, const void* qkv, long ld, void* k_
   return check_launch("attention (decode, fused)");
 }
 
-// The wide kernel: a K and a V tile, and the page ids.  Four waves (64 rows) where two workgroups share a CU:
-// never slower there than eight waves (128 rows; 2,048 tokens, D = 128, 16 over 8 heads 42 / 49 us, 32 over 8 58 / 58).  Where
-// one workgroup has the CU, eight waves fill it once there are more blocks of 128 rows than CUs (float32, D = 128: 2,048 tokens, 32
-// over 8 heads 309 us against 354 by four; bfloat16, D = 256, 2,048 tokens from 6,144 638 / 769; but float32, 16 over 8 heads, a block a
-// CU, 281 / 178), unless their loads need addresses of their own (float32, D = 80: 286 / 262, registers spill).
+// The wide kernel: a K and a V tile, and the page ids.  Four waves (64 rows) where two workgroups share a CU: eight (128 rows) were
+// measured at all such head sizes and are faster in twelve of 156 cases, by 7 % at most (2,048 tokens, D = 128, 16 over 8 heads
+// 46 / 54 us, 32 over 8 59 / 62).  Where one workgroup has the CU, eight waves once there are more blocks of 128 rows than CUs; us by
+// four / eight, 2,048 tokens of 32 over 8 heads from 0, from 6,144, and 512 of them from 1,000, which are half a block a CU:
+//   bfloat16 D = 160 130 / 84, 727 / 444, 48 / 54    D = 192 142 / 97, 801 / 508, 52 / 61    D = 208 152 / 148, 867 / 868, 56 / 97
+//            D = 224 174 / 129, 966 / 660, 63 / 81   D = 256 148 / 136, 782 / 679, 55 / 79
+//   float32  D = 80 261 / 218, 1645 / 1349, 95 / 147   D = 128 360 / 311, 2274 / 1963, 131 / 213   D = 144 434 / 372, 2720 / 2374, 158 / 258
+// At as many blocks as CUs either may be the faster (16 over 8 heads from 0 and from 6,144, D = 160 70 / 73, 364 / 249; float32 D = 128
+// 184 / 292, 1138 / 1112): four.
 constexpr int kLargeBlock = 128, kSmallBlock = 64;   // rows of variant 4's and variant 5's row blocks
-constexpr bool wide_has_eight_waves(int element_bytes) { return !wide_shares_cu(element_bytes) && D % 64 == 0; }
+constexpr bool wide_has_eight_waves(int element_bytes) { return !wide_shares_cu(element_bytes); }
 constexpr size_t wide_lds_bytes(int element_bytes) { return 2 * (size_t)kTileKeys * D * element_bytes + kPageWindow * 16 * sizeof(int); }
 template <typename T, int NW>
 static bool wide_kernel_ready(size_t bytes) {
@@ -2423,7 +2427,8 @@ static bool wide_ready() {
 static bool wide_supported(int dtype) { return dtype == kF32 ? wide_ready<float>() : wide_ready<bf16_t>(); }
 // 1 if the wide kernel (variants 4 and 5) can run for this dtype.
 extern "C" int ls_attn_wide_supported(int dtype) { return wide_supported(dtype) ? 1 : 0; }
-// 1 if variant 4's row blocks have a workgroup of eight waves each (else two of variant 5's workgroups).
+// 1 if variant 4's row blocks have a workgroup of eight waves each (else they are two of variant 5's workgroups, for callers that name
+// the variant; plans take variant 5).
 extern "C" int ls_attn_wide_eight_waves(int dtype) { return wide_has_eight_waves(dtype == kF32 ? 4 : 2) ? 1 : 0; }
 // Rows of one work item's row block: AttnItem.row_block counts blocks of this many rows.
 extern "C" int ls_attn_block_rows(int variant) {

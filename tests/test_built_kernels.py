@@ -24,7 +24,7 @@ SMALL = 64                                              # bytes a lane that need
 # paged attention of row blocks: in workgroups of four waves none may (the wait for a spilled register is a wait for every load
 # in flight), and a lane keeps to 256 registers where two of them share a CU; in workgroups of eight waves, which have 256
 # registers at most, bytes a lane by head size
-WIDE_MAY_SPILL = {"attention_wide_kernelIfLi8E": {128: 72}, "attention_wide_kernelIDF16bLi8E": {192: 104, 256: 220}}
+WIDE_MAY_SPILL = {"attention_wide_kernelIfLi8E": {112: 12, 128: 72, 144: 184}, "attention_wide_kernelIDF16bLi8E": {192: 104, 256: 220}}
 WIDE_SHARES_A_CU = {"attention_wide_kernelIfLi4E": 64, "attention_wide_kernelIDF16bLi4E": 144}     # largest such head size
 # recurrences of one wave a workgroup, whose registers let two waves share a SIMD
 TWO_WAVES = ("delta_rule_kernel",)

@@ -808,6 +808,14 @@ def test_wide_attention_where_a_load_spans_several_pages(dtype, nq, nkv, d, ps, 
             assert torch.equal(got, want), (start, length, variant)
 
 
+@pytest.mark.parametrize("dtype,largest_shared", [(torch.bfloat16, 144), (torch.float32, 64)])
+def test_wide_attention_has_eight_waves_where_a_workgroup_has_the_cu(dtype, largest_shared):
+    """Two workgroups' tiles and page ids fit a CU's 160 KB up to these head sizes."""
+    for d in (16, 32, 48, 64, 80, 112, 128, 144, 160, 192, 256):
+        if K().wide_supported(d, dtype, 16):
+            assert K().wide_eight_waves(d, dtype) == (d > largest_shared), d
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nq,nkv,d,ps", [(16, 8, 128, 16), (6, 3, 32, 8), (8, 1, 64, 16)])
 def test_attention_row_is_the_same_alone_in_a_portion_and_in_the_whole_prompt(dtype, nq, nkv, d, ps):
