@@ -420,6 +420,15 @@ template <typename T> struct Staged {
   static constexpr int kBytes = kKeyBytes + kValueBytes + kWindow * kTilePages * 4;
   static constexpr bool kFits = kBytes <= 64 * 1024 && D % Atom<T>::VEC == 0;
   static constexpr bool kOnePage = kKeyPieces % 8 == 0 && DV % 64 == 0;
+  // A lane's query and its sums are eight registers for each of these; with all else 256 hold them, and two workgroups share a CU, up
+  // to a limit, beyond which registers would spill, and the wait for one is a wait for every load in flight.  Loads that
+  // look pages up take a few more.  bfloat16, us, two / one a CU, 2,048 tokens from 6,000 on and 700 from 1,500 on in a window of 600:
+  // keys of 192 and values of 128 elements (14 of these) 169 / 262 and 34 / 36; 128 and 192 (16) 245 / 299 and 46 / 41; 192 and
+  // 192 (18) 289 / 325 and 53 / 42; 128 and 256 (20) 484 / 384 and 64 / 47; 112 and 112 (11, pages looked up) 158 / 255 and 32 / 34;
+  // 144 and 144 (14, looked up) 262 / 306 and 50 / 40.  float32 128 and 192 (20) 946 / 1120 and 92 / 91; 256 and 128 (24)
+  // 1336 / 1195 and 126 / 99; 144 and 144 (18, looked up) 884 / 1043 and 91 / 87; 160 and 160 (20, looked up) 1106 / 1132 and 111 / 94.
+  static constexpr int kRowRegisters = (D + Atom<T>::KCHUNK - 1) / Atom<T>::KCHUNK + (DV + 15) / 16;
+  static constexpr bool two_a_cu(bool one_page) { return kRowRegisters <= (sizeof(T) == 2 ? 14 : 20) - (one_page ? 0 : 2); }
 };
 
 // Which key of a tile row r (0..15) of the score block kb stands for.
@@ -443,7 +452,7 @@ __device__ __forceinline__ constexpr int slot_of_piece(int key, int piece) {
 }
 
 template <typename T, bool ONE_PAGE>
-__global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
+__global__ __launch_bounds__(256, Staged<T>::two_a_cu(ONE_PAGE) ? 2 : 1) void sink_attention_staged_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int page_size,
     const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs, const int* __restrict__ items,
     int H, int G, float scale, int window, int chunk, int keep_first, const float* __restrict__ sink,
@@ -606,6 +615,8 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
 #pragma unroll
   for (int c = 0; c < PERIOD; ++c) k_at[c] = k_lds + (key_of_row<T>(0, l16) * KP + slot_at<T>(l16, 4 * c + quad)) * 16;
 
+  const unsigned char* const v_at = v_lds + (quad * DV + l16) * 16;   // (a value operand: this and constants)
+
 #pragma unroll
   for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -672,10 +683,9 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
     const bool ahead = step + 1 < step_end && !opens(step + 1);
     if (ahead && !(ONE_PAGE && mine)) request(step + 1, keys);
     vec_t pb[2][NC];
+    float shrink[2] = {1.f, 1.f};            // of the sums so far; they are multiplied where the products add to them
     if (mine) {
       // -- 2. scale, bias, mask, online softmax; the next keys' loads among it --------------------------------
-      float shrink[2];
-      bool moved = false;
       unsigned long long from = 0;
       if (ONE_PAGE && ahead) from = loads_of(step + 1);
       auto softmax_tile = [&](auto whole, auto biased, auto with_loads) LS_INLINED {
@@ -720,7 +730,6 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
           sum = quad16_sum(sum);
           l_run[r] = l_run[r] * shrink[r] + sum;
           m_run[r] = m_new;
-          moved = moved || shrink[r] != 1.0f;
         }
       };
       const bool whole_tile = key0 + TK - 1 <= wave_first && (key0 >= wave_lo_last || key0 + TK <= keep_first) && wave_row0 + 31 < nrows;
@@ -734,14 +743,6 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
       } else {
         if (ONE_PAGE && ahead) softmax_of(std::false_type{}, std::bool_constant<ONE_PAGE>{});
         else softmax_of(std::false_type{}, std::false_type{});
-      }
-      if (__any(moved)) {
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
-#pragma unroll
-          for (int b = 0; b < VB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[r][b][i] = acc[r][b][i] * shrink[r];
       }
     }
     // the values have landed; the next keys, asked for after them, are still on their way
@@ -768,9 +769,8 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
       // -- 3. values ---------------------------------------------------------------------------
       constexpr int N = VB * NC, RING = N < 4 ? N : 4;
       auto v_read = [&](int idx) LS_INLINED -> vec_t {
-        const int col = 16 * (idx / NC) + l16;
-        const bool in = DV % 16 == 0 || col < DV;
-        vec_t a = *reinterpret_cast<const vec_t*>(v_lds + ((4 * (idx % NC) + quad) * DV + (in ? col : 0)) * 16);
+        const bool in = DV % 16 == 0 || 16 * (idx / NC) + l16 < DV;
+        vec_t a = *reinterpret_cast<const vec_t*>((in ? v_at : v_lds) + (4 * (idx % NC) * DV + (in ? 16 * (idx / NC) : 0)) * 16);
         return in ? a : A::zero();
       };
       __builtin_amdgcn_s_setprio(1);
@@ -781,7 +781,12 @@ __global__ __launch_bounds__(256, 2) void sink_attention_staged_kernel(
 #pragma unroll
       for (int idx = 0; idx < N; ++idx) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r) A::mma(acc[r][idx / NC], ring[idx % RING], pb[r][idx % NC]);
+        for (int r = 0; r < 2; ++r) {
+          if (idx % NC == 0)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[r][idx / NC][i] = acc[r][idx / NC][i] * shrink[r];
+          A::mma(acc[r][idx / NC], ring[idx % RING], pb[r][idx % NC]);
+        }
         if (idx + RING < N) ring[idx % RING] = v_read(idx + RING);
         __builtin_amdgcn_sched_barrier(0);
       }

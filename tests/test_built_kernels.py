@@ -33,7 +33,9 @@ MAY_SPILL_AT_HEAD = {160: ("attention_coop_kernelIf",), 192: ("attention_coop_ke
                      256: ("attention_coop_kernel", "attention_staged_kernel")}
 # sink attention with keys of more than 256 or values of more than 128 elements (a library of such a shape is built when a
 # model first asks for it): correct, not fast, or the instances of four row tiles, which only measurements use
-MAY_SPILL_AT_WIDE_HEADS = ("sink_attention_",)
+MAY_SPILL_AT_WIDE_HEADS = ("sink_attention_kernel",)
+# ... and its kernel for prompts, bytes a lane by key and value size (at 320 and 256 the tiles do not fit LDS, and it never runs)
+STAGED_MAY_SPILL = {("64", "320"): 112, ("320", "256"): 156}
 
 
 def code_object_notes(blob: bytes):
@@ -137,6 +139,8 @@ def test_no_kernel_calls_a_function_and_only_known_ones_spill():
                 assert scratch <= most, f"{lib.name}: {name} uses {scratch} bytes of scratch memory a lane"
                 shared = max((largest for part, largest in WIDE_SHARES_A_CU.items() if part in name), default=0)
                 assert head > shared or kernel[".vgpr_count"] <= 256, f"{lib.name}: {name}"
+                continue
+            if "sink_attention_staged_kernel" in name and scratch <= STAGED_MAY_SPILL.get(tuple(sizes), 0):
                 continue
             allowed = MAY_SPILL_AT_HEAD.get(head, ()) + (MAY_SPILL_AT_WIDE_HEADS if wide_heads else ())
             if scratch > SMALL and not any(part in name for part in allowed):
