@@ -42,6 +42,21 @@ ROW_TILES = int(__import__("os").environ.get("LOCKSTEP_SINK_ROW_TILES", "0"))   
 STAGED = 8             # the value of row_tiles that names the kernel with tiles staged in LDS
 
 
+def staged_runs(tiles, workgroups: int, cus: int, least: int):
+    """How many runs the kernel with tiles staged in LDS deals each row block of a prompt portion to; ``tiles`` are the blocks', an
+    item is ``workgroups`` workgroups.
+
+    A run is as long as a CU's share of the tiles, from ``least`` to four times as many.  With more work than that gives four
+    workgroups a CU it is longer, and the longest prompts are not cut: their blocks balance by themselves, and a run leaves its
+    partial results in memory (16,384 tokens, 16 heads over one, values of 128: 1.1 GB with runs of ``4 * least``, none now)."""
+    # bfloat16, keys of 192 and values of 128, 16 heads over one, us uncut / four times ``least`` at most / this rule: 2,048
+    # tokens 77 / 63 / 62, from 6,000 on in a window of 4,096 152 / 151 / 150, from 14,000 on 534 / 466 / 422; 8,192 513 / 530 / 439;
+    # 16,384 1,490 / 2,025 / 1,485; 700 from 1,500 on in a window of 600 40 / 34 / 34.  The longest runs first (see ``prepare``).
+    share = int(tiles.sum()) * workgroups // cus
+    a_run = max(least, min(share, 4 * least), share // 4)
+    return np.minimum(MAX_RUNS, -(-tiles // a_run))
+
+
 def distance_buckets(rows: int, farthest: float) -> list[int]:
     """``bucket(n)`` for n = 0 .. the first distance of the last bucket."""
     half = rows // 2
@@ -271,14 +286,8 @@ class SinkAttention(ProjectedMixer):
             lo_tile = self._first_seen(first) // tile_keys
             tiles = last // tile_keys - lo_tile + 1 + np.minimum(-(-self.keep_first // tile_keys), lo_tile)    # (as the kernel counts them)
             if row_tiles == STAGED:
-                # runs as long as a CU's share of the tiles, from TILES_A_RUN of 32 keys to four times as many, and the blocks of the
-                # longest runs first (2,048 tokens, 16 heads, keys of 192 and values of 128: 58 to 66 us with any rule near
-                # this one, 73 uncut; from 6,000 on 129, with runs half as long 164; 700 from 1,500 on 34, uncut 39)
-                least = TILES_A_RUN * TILE_KEYS // tile_keys
-                launched = int(tiles.sum()) * groups * -(-self.nq // groups // 4)
-                a_run = min(max(least, launched // cus), 4 * least)
-                runs = np.minimum(MAX_RUNS, -(-tiles // a_run))
-                order = np.argsort(-(-(-tiles // runs)), kind="stable")
+                runs = staged_runs(tiles, groups * -(-self.nq // groups // 4), cus, TILES_A_RUN * TILE_KEYS // tile_keys)
+                order = np.argsort(-(-(-tiles // runs)), kind="stable")     # (blocks of the longest runs first)
                 seq, block, rows, runs = seq[order], block[order], rows[order], runs[order]
             else:
                 # runs of at least TILES_A_RUN tiles, longer where the step has more work than a few items a CU

@@ -8,6 +8,7 @@ from __future__ import annotations
 import copy
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -267,3 +268,21 @@ def test_plain_model_runs_every_case_and_later_tokens_do_not_change_earlier_logi
     whole = plain.forward(raw, tensors, tokens)
     assert whole.shape == (50, raw["vocab"]) and bool(torch.isfinite(whole).all())
     assert torch.allclose(plain.forward(raw, tensors, tokens[:31]), whole[:31], atol=1e-9)
+
+
+@pytest.mark.parametrize("workgroups", [4, 8])
+@pytest.mark.parametrize("window", [0, 4096])
+def test_runs_of_prompt_portions_keep_their_partial_results_bounded(workgroups, window):
+    """The runs beyond one a row block are at most four workgroups a compute unit, however long the prompt is; blocks of fewer
+    tiles than the shortest run stay whole; every block has a run."""
+    from lockstep_amd.parts.sink_attention import MAX_RUNS, staged_runs
+
+    cus, least = 256, 4
+    for tokens in (40, 97, 700, 2048, 5000, 8192, 16384, 65536):
+        last = np.minimum(np.arange(32, tokens + 32, 32), tokens) - 1
+        first_seen = np.maximum(0, last // 32 * 32 - window + 1) if window else np.zeros_like(last)
+        tiles = last // 64 - first_seen // 64 + 1
+        runs = staged_runs(tiles, workgroups, cus, least)
+        assert runs.min() >= 1 and runs.max() <= MAX_RUNS
+        assert int(runs.sum()) - len(tiles) <= 4 * cus // workgroups, tokens
+        assert (runs[tiles <= least] == 1).all()
