@@ -444,10 +444,14 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(
   };
   if (is_v) {
     for (int i0 = 0; i0 < size; i0 += 128) {   // (two elements of a lane at a time, their loads together)
-      const float y0 = channel(c0 + min(i0 + lane, size - 1)), y1 = channel(c0 + min(i0 + 64 + lane, size - 1));
       float* dst = vv + (long)t * H * DV + (c0 - 2 * G * D) + i0 + lane;
-      if (i0 + lane < size) dst[0] = y0;
-      if (i0 + 64 + lane < size) dst[64] = y1;
+      if (i0 + 64 < size) {
+        const float y0 = channel(c0 + i0 + lane), y1 = channel(c0 + min(i0 + 64 + lane, size - 1));
+        dst[0] = y0;
+        if (i0 + 64 + lane < size) dst[64] = y1;
+      } else if (i0 + lane < size) {           // (the same for the wave but for this test: no second element to compute)
+        dst[0] = channel(c0 + i0 + lane);
+      }
     }
     return;
   }
