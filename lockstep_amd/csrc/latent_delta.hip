@@ -63,10 +63,16 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int e, int W
 // (N, the number of copies, is a template parameter: every copy's load stands in straight-line code, so all of a
 // thread's loads are on their way before the first is used.)  What bounds it at few rows is the chain of answers from memory, so a
 // thread's first run of four elements, the slices' sums, the mixing factors and the weights are asked for together, in front of the
-// first barrier, and what a run was read as stays in registers (rows of up to 1,024 elements are one run): requests of one
-// token through four copies of 1,024 (28 layers, all kernels) 2,633 -> 2,574 us a step
-template <typename T, int N>
-__global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X, long ldx, int W,
+// first barrier, and what a run was read as stays in registers: requests of one token through four copies of 1,024 (28 layers,
+// all kernels) 2,633 -> 2,574 us a step.  At many rows it is memory, and how many rows a CU has in flight: ONE, rows of up to
+// 1,024 elements, one run a thread, without the registers of further runs (2,048 rows, one slice, four copies of 1,024 elements 16.3 ->
+// 14.6 us, eight of 512 22.6 -> 18.6); and where seven or eight copies of longer rows are in registers, their first run is not
+// asked for in front of the barrier, and the registers are held to what three rows a CU need (seven of 2,048 43.4 -> 41.4, eight
+// 49.2 -> 48.3).
+constexpr bool streams_ahead(int copies, bool one) { return one || copies <= 6; }
+constexpr int streams_rows_a_cu(int copies, bool one) { return streams_ahead(copies, one) ? 1 : 3; }
+template <typename T, int N, bool ONE>
+__global__ __launch_bounds__(256, streams_rows_a_cu(N, ONE)) void streams_step_kernel(float* __restrict__ X, long ldx, int W,
                                                            const float* __restrict__ P, int slices, long p_stride,
                                                            const float* __restrict__ mix, const float* __restrict__ gain,
                                                            const float* __restrict__ take, const float* __restrict__ weight,
@@ -92,8 +98,9 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
     for (int u = 0; u < BATCH; ++u) got[u] = load4(p + (long)min(s0 + u, slices - 1) * p_stride, e, W, vec_ok);   // (clamped: no branch between the loads)
   };
   const int i_mix = min((int)threadIdx.x, N * N - 1), i_copy = min((int)threadIdx.x, N - 1);
+  constexpr bool AHEAD = streams_ahead(N, ONE);
   const float my_mix = P ? mix[i_mix] : 0.f, my_gain = P ? gain[i_copy] : 0.f, my_take = take ? take[i_copy] : 1.0f;
-  if (e_first < W) {
+  if (AHEAD && e_first < W) {
     load_run(e_first);
     if (P) load_sums(e_first, 0);
     if (out) {
@@ -110,12 +117,12 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
   float part = 0.f;
   f32x4 u_first = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-  for (int e = e_first; e < W; e += 1024) {
-    if (e != e_first) load_run(e);
+  for (int e = e_first; e < W; e += ONE ? W : 1024) {
+    if (!AHEAD || (!ONE && e != e_first)) load_run(e);
     if (P) {
       f32x4 y = {0.f, 0.f, 0.f, 0.f};
       for (int s0 = 0; s0 < slices; s0 += BATCH) {
-        if (s0 > 0 || e != e_first) load_sums(e, s0);
+        if (!AHEAD || s0 > 0 || (!ONE && e != e_first)) load_sums(e, s0);
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
           if (s0 + u < slices) y = y + got[u];
@@ -143,7 +150,7 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < N; ++t) sum = sum + take_s[t] * copy[t];
-    if (e == e_first) u_first = sum;
+    if (ONE || (AHEAD && e == e_first)) u_first = sum;
     else if (out) *reinterpret_cast<f32x4*>(u_s + e) = sum;
 #pragma unroll
     for (int i = 0; i < 4; ++i) part = part + (centred ? sum[i] : sum[i] * sum[i]);   // (elements beyond W are zeros)
@@ -161,8 +168,8 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
     mean = row_sum(part, sums_s) / (float)W;
     part = 0.f;
 #pragma unroll 1
-    for (int e = e_first; e < W; e += 1024) {
-      const f32x4 u = e == e_first ? u_first : *reinterpret_cast<const f32x4*>(u_s + e);
+    for (int e = e_first; e < W; e += ONE ? W : 1024) {
+      const f32x4 u = ONE || (AHEAD && e == e_first) ? u_first : *reinterpret_cast<const f32x4*>(u_s + e);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float d = e + i < W ? u[i] - mean : 0.f;
@@ -173,9 +180,9 @@ __global__ __launch_bounds__(256) void streams_step_kernel(float* __restrict__ X
   const float scale = 1.0f / sqrtf(row_sum(part, scratch) / (float)W + eps);
   const bool vec_out = vec_ok && ld_out % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(T)) == 0;
 #pragma unroll 1
-  for (int e0 = e_first; e0 < W; e0 += 1024) {
+  for (int e0 = e_first; e0 < W; e0 += ONE ? W : 1024) {
     f32x4 u = u_first, w = w_first, b = b_first;
-    if (e0 != e_first) {
+    if (!AHEAD || (!ONE && e0 != e_first)) {
       u = *reinterpret_cast<const f32x4*>(u_s + e0);
       w = load4(weight, e0, W, vec_ok);
       if (bias) b = load4(bias, e0, W, vec_ok);
@@ -683,19 +690,22 @@ extern "C" int ls_streams_step(int dtype, float* X, long ldx, int n, int width, 
   const long p_stride = (long)p_rows * width;
   LS_REQUIRE(dtype == kF32 || dtype == kBF16, "streams_step: unknown dtype %d", dtype);
   const size_t lds = out ? (size_t)((width + 3) / 4) * 16 : 0;
+#define LS_STREAMS_AS(T_, N_, ONE_)                                                                                  \
+  hipLaunchKernelGGL((streams_step_kernel<T_, N_, ONE_>), dim3(n_rows), dim3(256), lds, s, X, ldx, width, P, slices, \
+                     p_stride, mix, gain, take, weight, bias, centred, eps, (T_*)out, ld_out, rows)
 #define LS_STREAMS(N_)                                                                                               \
   case N_:                                                                                                           \
-    if (dtype == kF32)                                                                                               \
-      hipLaunchKernelGGL((streams_step_kernel<float, N_>), dim3(n_rows), dim3(256), lds, s, X, ldx, width, P, slices, \
-                         p_stride, mix, gain, take, weight, bias, centred, eps, (float*)out, ld_out, rows);                         \
-    else                                                                                                             \
-      hipLaunchKernelGGL((streams_step_kernel<bf16_t, N_>), dim3(n_rows), dim3(256), lds, s, X, ldx, width, P, slices, \
-                         p_stride, mix, gain, take, weight, bias, centred, eps, (bf16_t*)out, ld_out, rows);                        \
+    if (dtype == kF32) {                                                                                             \
+      if (width <= 1024) LS_STREAMS_AS(float, N_, true); else LS_STREAMS_AS(float, N_, false);                       \
+    } else {                                                                                                         \
+      if (width <= 1024) LS_STREAMS_AS(bf16_t, N_, true); else LS_STREAMS_AS(bf16_t, N_, false);                     \
+    }                                                                                                                \
     break;
   switch (n) {
     LS_STREAMS(1) LS_STREAMS(2) LS_STREAMS(3) LS_STREAMS(4) LS_STREAMS(5) LS_STREAMS(6) LS_STREAMS(7) LS_STREAMS(8)
   }
 #undef LS_STREAMS
+#undef LS_STREAMS_AS
   return check_launch("streams_step");
 }
 
