@@ -279,6 +279,54 @@ def test_staged_attention_with_value_rows_that_do_not_divide_a_load_of_the_workg
         assert rel_err(got, want) < bound, (runs, lengths)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, groups, d, dv, page", [(2, 1, 192, 128, 16), (2, 2, 64, 192, 8), (2, 1, 40, 40, 8), (4, 1, 128, 128, 128),
+                                                        (1, 1, 24, 20, 8)])
+@pytest.mark.parametrize("window, keep_first", [(70, 0), (2300, 5), (2300, 70), (130, 2100)])
+@pytest.mark.parametrize("runs", [1, 3])
+def test_staged_attention_over_pages_that_were_given_back(dtype, heads, groups, d, dv, page, window, keep_first, runs):
+    """Pages behind the window (but for the first tokens that stay) are no longer the request's: their table entries are -1,
+    and what the kernel loads in their place, page 0, must not reach a result, be it NaN.  The windows and the kept tokens are each
+    more tiles than a workgroup holds page ids for."""
+    start, n = 4700, 40
+    total = start + n
+    g = torch.Generator().manual_seed(d + dv + window + keep_first + runs)
+    k = (torch.randn(total, groups, d, generator=g) * 1.5).to(dtype)
+    v = torch.randn(total, groups, dv, generator=g).to(dtype)
+    q = (torch.randn(n, heads, d, generator=g) * 1.5).to(dtype)
+    first_seen = start - window + 1
+    order = (torch.randperm(-(-total // page), generator=g) + 1).tolist()
+    keys, values = paged(-(-total // page) + 1, groups, page, d, dv, dtype)
+    keys.fill_(float("nan")), values.fill_(float("nan"))       # page 0 among them, and what lies behind the last token
+    table = torch.full((1, -(-total // page) + 1), -1, dtype=torch.int32)
+    for logical, pg in enumerate(order):
+        lo, hi = logical * page, min(total, (logical + 1) * page)
+        if hi <= first_seen and lo >= keep_first:
+            continue                                            # given back
+        table[0, logical] = pg
+        keys[pg, :, :hi - lo] = k[lo:hi].transpose(0, 1).cuda()
+        values[pg, :, :, :hi - lo] = v[lo:hi].permute(1, 2, 0).cuda()
+    assert window + keep_first > total or (table[0, :-1] < 0).any()
+    _, _, seqs = step_meta([n], [start], [0])
+    rows = K().sink_staged_rows(heads, groups)
+    blocks = -(-n // rows)
+    items = torch.tensor([[0, b, r, runs] for b in range(blocks) for r in range(runs)], dtype=torch.int32, device="cuda").reshape(-1)
+    folds = torch.tensor([[b * runs, runs, b * rows, min(rows, n - b * rows)] for b in range(blocks)], dtype=torch.int32,
+                         device="cuda").reshape(-1) if runs > 1 else None
+    part = torch.full((blocks * runs * rows * heads * (dv + 2),), float("nan"), device="cuda") if runs > 1 else None
+    out = torch.empty(n, heads * dv, dtype=dtype, device="cuda")
+    K().sink_attention(q.reshape(n, heads * d).cuda(), heads, groups, d, dv, keys, values, page, table.cuda(), seqs, items,
+                       blocks * runs, 8, 0.1, window, 0, None, None, None, out, folds, blocks if runs > 1 else 0, part,
+                       keep_first=keep_first)
+    i_pos, j_pos = torch.arange(start, total)[:, None], torch.arange(total)[None, :]
+    visible = (j_pos <= i_pos) & ((i_pos - j_pos < window) | (j_pos < keep_first))
+    spread = torch.arange(heads) // (heads // groups)
+    scores = torch.einsum("nhd,mhd->hnm", q.double(), k.double()[:, spread]) * 0.1
+    weights = torch.softmax(scores.masked_fill(~visible, float("-inf")), -1)
+    want = torch.einsum("hnm,mhe->nhe", weights, v.double()[:, spread]).reshape(n, heads * dv)
+    assert rel_err(out.float().cpu(), want) < (6e-6 if dtype is torch.float32 else 2e-2)      # (as above)
+
+
 def test_a_sink_left_out_or_a_chunk_one_off_shows_in_the_kernel_test():
     """Controls of the test above: the same inputs against a plain result without the sink, or with the
     chunk one larger, differ by many times the bound."""
