@@ -128,8 +128,8 @@ __device__ __forceinline__ constexpr int key_of_row(int kb, int r) {
   return sizeof(T) == 2 ? 32 * (kb >> 1) + 8 * (r >> 2) + 4 * (kb & 1) + (r & 3) : 16 * kb + r;
 }
 // The rotation of a key row's 16-byte pieces in the LDS tile: the sixteen rows that a score block reads
-// together start in sixteen different slots.  (Lanes that LDS serves together come from more than one of them: counters of
-// the wide kernel at a head size of 128 show bank conflicts in 31 % of LDS's active cycles.)
+// together start in sixteen different slots.  (As a rotation alone it left bank conflicts in 31 % of LDS's active cycles at a head size
+// of 128, because lanes that LDS serves together come from more than one of those reads; as the exclusive-or below, none.)
 template <typename T>
 __device__ __forceinline__ constexpr int row_rotation(int row) {
   return sizeof(T) == 2 ? (row & 3) + 4 * ((row >> 3) & 3) : row & 15;
@@ -766,9 +766,9 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 // matrix products run under the other's exponentials and waits; with two buffers one workgroup of eight
 // waves had the CU, its waves in step, and LDS, vector unit and matrix cores took turns.  Raised priority during the
 // products lets a wave that has operands go first (2,048 tokens, 32 over 8 heads: 64.7 -> 57.7 us).
-// What bounds it: LDS (a tile's 64 KB are written once and read by each of the four waves: 2,600 of some 3,400 cycles a
-// workgroup's tile) and the vector unit (1,600 a wave).  Measured, bfloat16, us, two buffers / now, for 2,048 tokens from
-// position 0 of 16 over 8 heads, the same of 32 over 8, 2,048 tokens of 16 over 8 from 6,144, 808 from 8,192:
+// What bounds it: the vector unit (exponentials, scaling, the folds: instructions for 60 % of a SIMD's cycles while its CU is busy;
+// matrix pipes 28 %, LDS reads 28 %, no bank conflicts), and in prompts from position 0 the blocks that walk the most tiles
+// (a CU is busy four fifths of the launch).  Measured, bfloat16, us, two buffers / now, for 2,048 tokens from position 0 of 16 over 8 heads, the same of 32 over 8, 2,048 tokens of 16 over 8 from 6,144, 808 from 8,192:
 //   D = 128  62 / 46    71 / 59   211 / 171   196 / 158        D = 64   40 / 34   45 / 43   134 / 116   133 / 120
 //   D = 112  61 / 51    69 / 67   211 / 186   187 / 180        D = 80   51 / 43   58 / 57   181 / 157   155 / 155
 //   D = 144  89 / 60   101 / 79   311 / 225   235 / 216        D = 32   33 / 28   38 / 32   110 / 99    101 / 103

@@ -405,9 +405,9 @@ __global__ __launch_bounds__(64 * (DEC ? 1 : kMaxWaves)) void sink_attention_ker
 // wave's load lie in one page, whose address is a scalar; else every lane looks its piece's page up.
 //
 // What bounds it: the vector unit (scales, maxima, exponentials: 1,200 of a wave's cycles a tile of 64 keys) in turn with the
-// matrix cores (1,280 at keys of 192 and values of 128 elements), two workgroups a CU.  Measured with its fold, us, tiles through
-// registers with one workgroup a CU / now, 16 heads: 2,048 tokens, keys of 192 and values of 128, one key/value head 132 / 64, keys of
-// 128 and eight of them 121 / 55; 700 from 1,500 on in a window of 600 45 / 34; 2,048 from 6,000 on 434 / 129.
+// matrix cores (1,280 at keys of 192 and values of 128 elements), two workgroups a CU where the registers allow it.  Measured with its
+// fold, us, tiles through registers with one workgroup a CU / now, 16 heads: 2,048 tokens, keys of 192 and values of 128, one key/value
+// head 134 / 62, keys of 128 and eight of them 120 / 53; 700 from 1,500 on in a window of 600 45 / 34; 2,048 from 6,000 on 433 / 150.
 // ---------------------------------------------------------------------------
 template <typename T> struct Staged {
   static constexpr int kKeys = 128 / (int)sizeof(T);                 // keys of a tile
