@@ -117,6 +117,30 @@ def test_the_step_of_a_stream_of_several_copies(dtype, copies, width, rows):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("copies, width", [(1, 1024), (1, 1025), (4, 1023), (4, 1028), (6, 1024), (6, 2052), (7, 1024), (7, 1028), (8, 1020), (8, 1030)])
+@pytest.mark.parametrize("centred", [False, True])
+def test_the_step_of_the_copies_at_the_edges_of_a_row_of_one_run(dtype, copies, width, centred):
+    """Rows of up to 1,024 elements are one run of a thread and have an instance of their own; longer ones ask for their first run
+    ahead, up to six copies.  Nine slices are one more than a batch."""
+    g = torch.Generator().manual_seed(copies * width + centred)
+    rows = 3
+    x, partials = torch.randn((rows, copies, width), generator=g), torch.randn((9, rows, width), generator=g)
+    mix, gain, take = (torch.randn(s, generator=g) for s in ((copies, copies), (copies,), (copies,)))
+    weight, bias = torch.randn(width, generator=g), torch.randn(width, generator=g)
+    written = plain.write_streams(x.double(), partials.double().sum(0), mix.double(), gain.double())
+    read = plain.read_streams(written, take.double())
+    if centred:
+        read = read - read.mean(-1, keepdim=True)
+    want = plain.rms(read, 1e-5) * weight.double() + bias.double()
+    dev = x.view(rows, copies * width).cuda().clone()
+    out = torch.empty((rows, width), dtype=dtype, device="cuda")
+    K().streams_step(dev, copies, partials.cuda(), mix.view(-1).cuda(), gain.cuda(), take.cuda(), weight.cuda(), 1e-5, out,
+                     bias=bias.cuda(), centred=centred)
+    assert close(dev.view(rows, copies, width), written, torch.float32)
+    assert close(out, want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads, n, kk, rows", [(3, 20, 12, 5), (4, 64, 32, 130), (1, 7, 100, 17), (6, 36, 10, 66)])
 def test_a_product_a_head(dtype, heads, n, kk, rows):
     g = torch.Generator().manual_seed(heads * n + kk)
