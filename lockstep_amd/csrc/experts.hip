@@ -608,6 +608,148 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
 }
 
 // ---------------------------------------------------------------------------
+// The same two products for tiles of 16 rows where the sizes are whole chunks (`few_chunks`): decode steps, whose weights are
+// read once, by workgroups of 16 columns with a quarter of K a wave.  What bounds them is the weights (a CU keeps some 64 KB on
+// their way, so all of its workgroups' should be asked for at once) and, in front of those, the chain of what a workgroup has to
+// look up.  So: one load of the tile's entry, then every weight of the wave's quarter (U chunks at a time) in one batch,
+// without a branch, then the rows that the order names; registers for four workgroups a CU.  The kernels above, which take any
+// size, have a branch in front of every operand.  Both launches, 4 of 32 experts, width 1,024, 768 a piece, weights from HBM, us by the
+// kernels above / these (bytes at 5.96 TB/s): 1 token 10.9 / 8.6 (3.2), 8 tokens 31.7 / 26.9 (18.2), 40 tokens 42.3 / 34.5 (25.3);
+// 8 tokens of width 2,048, 1,024 a piece 69 / 61 (49); float32 8 tokens 96 / 54 (36), of width 2,048 238 / 130 (97).
+// The same sums in the same order as the kernels above give with a cut of K: the same bits.
+// ---------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+
+template <typename T, int U>
+__global__ __launch_bounds__(256, 4) void experts_few_gate_up_kernel(const i32x4_t* __restrict__ tiles, const T* __restrict__ w_gate,
+                                                                     const T* __restrict__ w_up, const int* __restrict__ order,
+                                                                     const T* __restrict__ x, long ldx, int F, int K, int top,
+                                                                     int real, float limit, float alpha, float shift,
+                                                                     const float* __restrict__ in_weight, T* __restrict__ act,
+                                                                     long ldy) {
+  typedef typename Atom<T>::vec_t vec_t;
+  constexpr int VEC = Atom<T>::VEC, KC = Atom<T>::KCHUNK, KS = 4;
+  const i32x4_t tile = tiles[blockIdx.x];
+  const int e = tile[0], first = tile[1], rows = tile[2];
+  if (e < 0 || e >= real) return;  // (an expert that returns its input has nothing to multiply)
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, quad = lane >> 4;
+  const int col0 = blockIdx.y * 16;
+  const int k_each = K / KS;
+  const long at = ((long)e * F + col0 + l16) * K + w * k_each + VEC * quad;
+  const T *g = w_gate + at, *u = w_up + at;
+  f32x4 acc_g = f32x4{0.f, 0.f, 0.f, 0.f}, acc_u = acc_g;
+  const int pair = order[first + min(l16, rows - 1)];  // (rows past the tile's repeat the last: their sums are not stored)
+  vec_t a_g[U], a_u[U];
+  auto request = [&](int k0) LS_INLINED {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      a_g[i] = *reinterpret_cast<const vec_t*>(g + k0 + i * KC);
+      a_u[i] = *reinterpret_cast<const vec_t*>(u + k0 + i * KC);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  request(0);  // before the order's entry is waited for
+  const T* xr = x + (long)(pair / top) * ldx + w * k_each + VEC * quad;
+  for (int k0 = 0;;) {
+    vec_t b[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) b[i] = *reinterpret_cast<const vec_t*>(xr + k0 + i * KC);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      Atom<T>::mma(acc_g, a_g[i], b[i]);
+      Atom<T>::mma(acc_u, a_u[i], b[i]);
+    }
+    k0 += U * KC;
+    if (k0 >= k_each) break;
+    request(k0);
+  }
+  const float wt = in_weight ? in_weight[pair] : 1.0f;
+  __shared__ f32x4 sums_s[KS - 1][2][64];
+  if (w > 0) {
+    sums_s[w - 1][0][lane] = acc_g;
+    sums_s[w - 1][1][lane] = acc_u;
+  }
+  __syncthreads();
+  if (w != 0 || l16 >= rows) return;
+#pragma unroll
+  for (int o = 0; o < KS - 1; ++o)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      acc_g[i] = acc_g[i] + sums_s[o][0][lane][i];
+      acc_u[i] = acc_u[i] + sums_s[o][1][lane][i];
+    }
+  T* dst = act + (long)(first + l16) * ldy + col0 + 4 * quad;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float gv = fminf(acc_g[i] * wt, limit);
+    const float uv = fminf(fmaxf(acc_u[i] * wt, -limit), limit);
+    dst[i] = from_f32<T>((gv * sigmoid_e(alpha * gv)) * (uv + shift));
+  }
+}
+
+template <typename T, int U>
+__global__ __launch_bounds__(256, 4) void experts_few_down_kernel(const i32x4_t* __restrict__ tiles, const T* __restrict__ w_down,
+                                                                  const T* __restrict__ act, long ldy,
+                                                                  const int* __restrict__ order, const float* __restrict__ weight,
+                                                                  float* __restrict__ P, int N, int F, int top, int n_tokens,
+                                                                  int real, const T* __restrict__ x, long ldx,
+                                                                  const float* __restrict__ share) {
+  typedef typename Atom<T>::vec_t vec_t;
+  constexpr int VEC = Atom<T>::VEC, KC = Atom<T>::KCHUNK, KS = 4;
+  const i32x4_t tile = tiles[blockIdx.x];
+  const int e = tile[0], first = tile[1], rows = tile[2];
+  if (e < 0) return;
+  const int col0 = blockIdx.y * 16;
+  if (e >= real) {  // (the whole workgroup)
+    pass_input<T, 256>(x, ldx, share, first, rows, col0, col0 + 16, top, n_tokens, N, order, P);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, quad = lane >> 4;
+  const int k_each = F / KS;
+  const T* d = w_down + ((long)e * N + col0 + l16) * F + w * k_each + VEC * quad;
+  const T* y = act + (long)(first + min(l16, rows - 1)) * ldy + w * k_each + VEC * quad;
+  const int pair = order[first + min(l16, rows - 1)];  // (rows past the tile's repeat the last: their sums are not stored)
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < k_each; k0 += U * KC) {
+    vec_t a[U], b[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) a[i] = *reinterpret_cast<const vec_t*>(d + k0 + i * KC);
+#pragma unroll
+    for (int i = 0; i < U; ++i) b[i] = *reinterpret_cast<const vec_t*>(y + k0 + i * KC);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < U; ++i) Atom<T>::mma(acc, a[i], b[i]);
+  }
+  const float factor = weight ? weight[pair] : 1.0f;
+  __shared__ f32x4 sums_s[KS - 1][64];
+  if (w > 0) sums_s[w - 1][lane] = acc;
+  __syncthreads();
+  if (w != 0 || l16 >= rows) return;
+#pragma unroll
+  for (int o = 0; o < KS - 1; ++o)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = acc[i] + sums_s[o][lane][i];
+  float* dst = P + ((long)(pair % top) * n_tokens + pair / top) * N + col0 + 4 * quad;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) dst[i] = factor * acc[i];
+}
+
+// Chunks that a wave of those kernels asks for at a time where K is a whole number of such rounds, else 0.
+static int few_chunks(int dtype, int K) {
+  const int quarter = 4 * (dtype == kF32 ? Atom<float>::KCHUNK : Atom<bf16_t>::KCHUNK);
+  if (K % quarter != 0) return 0;
+  for (int u : {8, 6, 4})
+    if (K / quarter % u == 0) return u;
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
 // The same two products for tiles of 64 rows (many tokens an expert), both operands through a ring of three stages in
 // LDS (128 bytes of K a row, written there by the loads themselves; layout, waits and barriers as gemm_ring.h describes
 // them).  A workgroup of eight waves takes 64 rows by 128 weight rows: 64 gate and the 64 up rows of the same columns, or
@@ -987,9 +1129,31 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
                        ring_lds(kDownCols<T_>), s, (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, \
                        out_weight, P, (const T_*)x, ldx, weight, real);                                                \
   } while (0)
+  // tiles of 16 rows of whole chunks and columns have kernels of their own
+  const int few_up = few_chunks(dtype, K), few_down = few_chunks(dtype, F);
+  const bool few = rows_a_tile == 16 && !with_shared && few_up && few_down && F % 16 == 0 && N % 16 == 0 && ldx % vec == 0 &&
+                   ldy % vec == 0 && reinterpret_cast<uintptr_t>(tiles) % 16 == 0 && (F + 15) / 16 < 65536 && (N + 15) / 16 < 65536;
+#define LS_FEW_UP(T_, U_)                                                                                             \
+  hipLaunchKernelGGL((experts_few_gate_up_kernel<T_, U_>), dim3(cap, F / 16), dim3(256), 0, s, (const i32x4_t*)tiles, \
+                     (const T_*)w_gate, (const T_*)w_up, order, (const T_*)x, ldx, F, K, top, real, limit, alpha, shift, \
+                     in_weight, (T_*)act, ldy)
+#define LS_FEW_DOWN(T_, U_)                                                                                           \
+  hipLaunchKernelGGL((experts_few_down_kernel<T_, U_>), dim3(cap, N / 16), dim3(256), 0, s, (const i32x4_t*)tiles,    \
+                     (const T_*)w_down, (const T_*)act, ldy, order, out_weight, P, N, F, top, n_tokens, real, (const T_*)x, \
+                     ldx, weight)
+#define LS_FEW(T_)                                                                                                    \
+  do {                                                                                                                \
+    if (few_up == 8) LS_FEW_UP(T_, 8); else if (few_up == 6) LS_FEW_UP(T_, 6); else LS_FEW_UP(T_, 4);                 \
+    if (few_down == 8) LS_FEW_DOWN(T_, 8); else if (few_down == 6) LS_FEW_DOWN(T_, 6); else LS_FEW_DOWN(T_, 4);       \
+  } while (0)
 #define LS_EXPERTS_BY_ROWS(T_)                 \
   switch (rows_a_tile) {                       \
-    case 16: LS_EXPERTS(T_, 1, 4); break;      \
+    case 16:                                   \
+      if (few)                                 \
+        LS_FEW(T_);                            \
+      else                                     \
+        LS_EXPERTS(T_, 1, 4);                  \
+      break;                                   \
     case 32: LS_EXPERTS(T_, 2, 1); break;      \
     default:                                   \
       if (staged)                              \
@@ -1004,6 +1168,9 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
     LS_EXPERTS_BY_ROWS(bf16_t)
   }
 #undef LS_EXPERTS_BY_ROWS
+#undef LS_FEW
+#undef LS_FEW_UP
+#undef LS_FEW_DOWN
 #undef LS_EXPERTS_STAGED
 #undef LS_EXPERTS
   return check_launch("experts_apply");
