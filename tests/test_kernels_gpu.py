@@ -951,6 +951,34 @@ def test_scores_of_great_size_leave_finite_results(dtype, nq, nkv, d, ps, scale)
             assert torch.isfinite(one).all() and rel_err(one, want[p:p + 1]) < ATT_TOL[dtype], (p, split)
 
 
+@pytest.mark.parametrize("nq,nkv,d,ps", [(4, 2, 64, 16), (16, 8, 128, 16), (6, 2, 48, 8), (2, 1, 256, 32)])
+def test_rows_of_great_scores_beside_others(nq, nkv, d, ps):
+    """Rows whose largest scores lie from 300 to 3,000, side by side: every kernel gives a row the same bits, alone or among the
+    others, walked or folded from splits, and they are right."""
+    n, dtype, scale = 300, torch.bfloat16, d ** -0.5
+    g = torch.Generator().manual_seed(d + nq)
+    along = torch.nn.functional.normalize(torch.randn(d, generator=g), dim=0)
+    qkv = torch.randn(n, (nq + 2 * nkv) * d, generator=g)
+    tops = 300.0 * 10.0 ** torch.rand(n, nq, 1, generator=g)
+    q, k = qkv[:, : nq * d].view(n, nq, d), qkv[:, nq * d:(nq + nkv) * d].view(n, nkv, d)
+    q += along * tops / (32.0 * scale)
+    k *= 0.1
+    k += along * 32.0
+    qkv = qkv.to(dtype)
+    case = PagedCase(dtype, nq, nkv, d, ps, n, shuffle_seed=4)
+    dev = qkv.cuda()
+    case.write(dev, 0)
+    q, k, v = split_qkv(qkv.double(), nq, nkv, d)
+    want = naive_attention(q, k, v, 0, scale)
+    out = case.attend(dev, 0, scale, variant=1, force_split=False)
+    assert rel_err(out, want) < ATT_TOL[dtype]
+    for variant in (0,) + ((4, 5) if K().wide_supported(d, dtype, ps) else ()):
+        assert torch.equal(case.attend(dev, 0, scale, variant=variant, force_split=False), out), variant
+    for p in (0, 127, 128, 200, n - 1):
+        for split in (False, True):
+            assert torch.equal(case.attend(dev[p:p + 1], p, scale, variant=3, force_split=split), out[p:p + 1]), (p, split)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_norm_rotation_and_cache_write(dtype):
     nq, nkv, d, ps, t, start = 6, 3, 32, 8, 21, 5
