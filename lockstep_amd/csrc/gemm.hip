@@ -355,11 +355,12 @@ template <typename T, int MT, int EPI, int XC>
 __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                            void* __restrict__ C, int M, int N, int K, long ldx,
                                                            long ldc, int kslice, int aligned, int vec_ok,
-                                                           int out_cols, int blocks, int row_groups,
+                                                           int out_cols, int blocks, int row_groups, int block_cols,
                                                            const float* __restrict__ act) {
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   constexpr int NT = (EPI == kSwiGLU) ? 2 : 1;  // weight tiles per column block
+  const int cols = NT == 2 ? 16 : block_cols;   // of a block: 16, 12 or 8
   const Factors factors = load_factors<EPI>(act);
   constexpr int UC = 4;                          // chunks per unit
   constexpr int UQ = XC / UC;                    // units per tile
@@ -387,11 +388,11 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
   const int m_base = row_group * MT * 16;
 
   auto fetch = [&](int b, int t, int q, vec_t (&dst)[UC]) LS_INLINED {
-    const int n = (b * NT + t) * 16 + row16;
+    const int n = (b * NT + t) * cols + row16;
 #pragma unroll
     for (int c = 0; c < UC; ++c) {
       const int kc = k_begin + (q * UC + c) * A::KCHUNK;
-      dst[c] = load_vec<T>(W, n, kc + g * A::VEC, K, K, n < N && kc < k_end, aligned);
+      dst[c] = load_vec<T>(W, n, kc + g * A::VEC, K, K, row16 < cols && n < N && kc < k_end, aligned);
     }
   };
 
@@ -467,10 +468,12 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
       const int m = m_base + j * 16 + row16;
       if (EPI == kSwiGLU)
         epilogue_swiglu4<T>(C, ldc, m, b * 16 + g * 4, M, out_cols, total[0], total[NT - 1], vec_ok);
+      else if (g * 4 >= cols)
+        continue;  // (the next block's columns)
       else if constexpr (EPI == kXielu)
-        epilogue_xielu4<T>(C, ldc, m, b * 16 + g * 4, M, N, total[0], vec_ok, factors);
+        epilogue_xielu4<T>(C, ldc, m, b * cols + g * 4, M, N, total[0], vec_ok, factors);
       else
-        epilogue4<T, EPI>(C, ldc, m, b * 16 + g * 4, M, N, total[0], vec_ok);
+        epilogue4<T, EPI>(C, ldc, m, b * cols + g * 4, M, N, total[0], vec_ok);
     }
   };
 
@@ -1214,8 +1217,21 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   if (!norm_w && mt_rows <= 4 && !tiles && xc % 4 == 0 && xc * group_tiles <= 16 && nslices >= 8 && nslices <= 16 &&
       col_blocks * row_groups > stream_wgs && stream_lds <= 128 * 1024 && LS_GEMM_STREAM) {
     int walkers = stream_wgs / row_groups;
-    const int rounds = (col_blocks + walkers - 1) / walkers;
-    walkers = (col_blocks + rounds - 1) / rounds;
+    // Blocks of 16 columns, or of 12 or 8 where a walker has fewer columns with those: the one with the most decides
+    // (8 rows, weights from HBM, blocks of 16 / of these, us: 4,608 x 4,096 15.9 / 14.2, 5,120 x 4,096 16.1 / 14.4, 6,144 x 4,096 16.4 / 15.0,
+    // 7,168 x 4,096 17.9 / 16.9, 9,216 x 4,096 22.2 / 20.4, 4,608 x 3,584 14.2 / 12.8; 1 row 6,144 x 4,096 15.0 / 13.8, 16 rows 18.1 / 16.8).
+    int cols = 16, blocks = col_blocks;
+    if (EPI != kSwiGLU) {
+      for (int c : {12, 8}) {
+        const int n = (N + c - 1) / c;
+        if ((n + walkers - 1) / walkers * c < (blocks + walkers - 1) / walkers * cols) {
+          cols = c;
+          blocks = n;
+        }
+      }
+    }
+    const int rounds = (blocks + walkers - 1) / walkers;
+    walkers = (blocks + rounds - 1) / rounds;
     if (row_groups > 1) walkers = (walkers + 7) / 8 * 8;  // whole rounds of the XCDs, see the kernel
     dim3 grid(walkers * row_groups);
     bool launched = true;
@@ -1223,7 +1239,7 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   if (stream_lds_ready<T, MT_, EPI, XC_>(stream_lds))                                                             \
     hipLaunchKernelGGL((gemm_stream_kernel<T, MT_, EPI, XC_>), grid, dim3(nslices * 64), stream_lds, stream,      \
                        reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice, aligned, vec_ok, out_cols, \
-                       col_blocks, row_groups, act);                                                              \
+                       blocks, row_groups, cols, act);                                                            \
   else                                                                                                            \
     launched = false
     if (group_tiles == 1 && xc == 8) LS_STREAM(1, 8);
