@@ -617,30 +617,75 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
 // kernels above / these (bytes at 5.96 TB/s): 1 token 10.9 / 8.6 (3.2), 8 tokens 31.7 / 26.9 (18.2), 40 tokens 42.3 / 34.5 (25.3);
 // 8 tokens of width 2,048, 1,024 a piece 69 / 61 (49); float32 8 tokens 96 / 54 (36), of width 2,048 238 / 130 (97).
 // The same sums in the same order as the kernels above give with a cut of K: the same bits.
+//
+// A table that names the experts, and at most 64 pairs in the step: a workgroup then stands for an expert (and sixteen of its
+// rows), and each of its waves finds the rows by itself: lane l has pair l's expert, ballots give the expert's pairs and how many
+// lie in front of them.  The launch that would put the pairs in order is saved.  The first product looks the experts up (a table's
+// rows come from HBM, which takes as long as that launch did) and leaves them for the second one.  Whole requests of the design that is
+// measured (28 layers, eight decode): 74.3 ms with the launch, 75.0 with an expert's blocks all on one XCD, 72.8 spread over the eight,
+// 71.9 with two column tiles in the second product.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+constexpr int kTablePairs = 64;
+enum RowsFrom : int {
+  kListed,  // tiles and order
+  kTable,   // token ids and the table
+  kPicked,  // the pairs' experts
+};
 
-template <typename T, int U>
-__global__ __launch_bounds__(256, 4) void experts_few_gate_up_kernel(const i32x4_t* __restrict__ tiles, const T* __restrict__ w_gate,
-                                                                     const T* __restrict__ w_up, const int* __restrict__ order,
+// Sixteen rows of an expert: its first place among the pairs in the order of their experts, how many, and the pair of this lane's row
+// (l % 16; lanes past the last row repeat it).
+struct FewRows {
+  int expert, first, rows, pair;
+};
+// at, more: tiles and order; token ids and table; the picks.  picks: where workgroup (0, 0) leaves what the table named.
+template <int FROM>
+__device__ __forceinline__ FewRows few_rows(const int* __restrict__ at, const int* __restrict__ more, int top, int n_tokens, int E,
+                                            int (*places_s)[kTablePairs], int* __restrict__ picks) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15;
+  if constexpr (FROM == kListed) {
+    const i32x4_t tile = reinterpret_cast<const i32x4_t*>(at)[blockIdx.x];
+    const int rows = tile[2];
+    return {tile[0], tile[1], rows, tile[0] < 0 ? 0 : more[tile[1] + min(l16, rows - 1)]};
+  } else {
+    // (workgroups go round the eight XCDs: an expert's column blocks shift from one to the next, or one XCD would have all of them)
+    const int at_x = ((int)blockIdx.x + (int)blockIdx.y) % (int)gridDim.x;
+    const int e = at_x % E, skip = 16 * (at_x / E), P = n_tokens * top;
+    int mine = 0x7fffffff;
+    if (lane < P) mine = FROM == kTable ? more[(long)at[lane / top] * top + lane % top] : at[lane];
+    if (FROM == kTable && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < P) picks[threadIdx.x] = mine;  // (its first wave)
+    const unsigned long long held = __ballot(mine == e);
+    const int n = __popcll(held) - skip, first = __popcll(__ballot(mine < e)) + skip;
+    if (n <= 0) return {-1, 0, 0, 0};  // uniform
+    int* places = places_s[threadIdx.x >> 6];  // (the wave's own)
+    if (mine == e) places[__popcll(held & ((1ull << lane) - 1ull))] = lane;
+    __builtin_amdgcn_wave_barrier();
+    const int rows = min(16, n);
+    return {e, first, rows, places[skip + min(l16, rows - 1)]};
+  }
+}
+
+template <typename T, int U, int FROM>
+__global__ __launch_bounds__(256, 4) void experts_few_gate_up_kernel(const int* __restrict__ at, const T* __restrict__ w_gate,
+                                                                     const T* __restrict__ w_up, const int* __restrict__ more,
                                                                      const T* __restrict__ x, long ldx, int F, int K, int top,
                                                                      int real, float limit, float alpha, float shift,
                                                                      const float* __restrict__ in_weight, T* __restrict__ act,
-                                                                     long ldy) {
+                                                                     long ldy, int n_tokens, int E, int* __restrict__ picks) {
   typedef typename Atom<T>::vec_t vec_t;
   constexpr int VEC = Atom<T>::VEC, KC = Atom<T>::KCHUNK, KS = 4;
-  const i32x4_t tile = tiles[blockIdx.x];
-  const int e = tile[0], first = tile[1], rows = tile[2];
+  __shared__ int places_s[FROM == kListed ? 1 : KS][kTablePairs];
+  const FewRows mine = few_rows<FROM>(at, more, top, n_tokens, E, places_s, picks);
+  const int e = mine.expert, first = mine.first, rows = mine.rows, pair = mine.pair;
   if (e < 0 || e >= real) return;  // (an expert that returns its input has nothing to multiply)
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, quad = lane >> 4;
   const int col0 = blockIdx.y * 16;
   const int k_each = K / KS;
-  const long at = ((long)e * F + col0 + l16) * K + w * k_each + VEC * quad;
-  const T *g = w_gate + at, *u = w_up + at;
+  const long from = ((long)e * F + col0 + l16) * K + w * k_each + VEC * quad;
+  const T *g = w_gate + from, *u = w_up + from;
   f32x4 acc_g = f32x4{0.f, 0.f, 0.f, 0.f}, acc_u = acc_g;
-  const int pair = order[first + min(l16, rows - 1)];  // (rows past the tile's repeat the last: their sums are not stored)
   vec_t a_g[U], a_u[U];
   auto request = [&](int k0) LS_INLINED {
     __builtin_amdgcn_sched_barrier(0);
@@ -691,21 +736,24 @@ __global__ __launch_bounds__(256, 4) void experts_few_gate_up_kernel(const i32x4
   }
 }
 
-template <typename T, int U>
-__global__ __launch_bounds__(256, 4) void experts_few_down_kernel(const i32x4_t* __restrict__ tiles, const T* __restrict__ w_down,
+// COLS: tiles of 16 columns a workgroup.  Two where its waves have to find their rows and a weight has two bytes (8 tokens, 23 of 32
+// experts, 1,024 x 768 10.9 -> 10.4 us in the decode step); with a list one is the faster (both launches 26.9 / 28.1, float32 54 / 60).
+template <typename T, int U, int FROM, int COLS>
+__global__ __launch_bounds__(256, 4) void experts_few_down_kernel(const int* __restrict__ at, const T* __restrict__ w_down,
                                                                   const T* __restrict__ act, long ldy,
-                                                                  const int* __restrict__ order, const float* __restrict__ weight,
-                                                                  float* __restrict__ P, int N, int F, int top, int n_tokens,
-                                                                  int real, const T* __restrict__ x, long ldx,
-                                                                  const float* __restrict__ share) {
+                                                                  const int* __restrict__ more,
+                                                                  const float* __restrict__ weight, float* __restrict__ P, int N,
+                                                                  int F, int top, int n_tokens, int real, const T* __restrict__ x,
+                                                                  long ldx, const float* __restrict__ share, int E) {
   typedef typename Atom<T>::vec_t vec_t;
   constexpr int VEC = Atom<T>::VEC, KC = Atom<T>::KCHUNK, KS = 4;
-  const i32x4_t tile = tiles[blockIdx.x];
-  const int e = tile[0], first = tile[1], rows = tile[2];
+  __shared__ int places_s[FROM == kListed ? 1 : KS][kTablePairs];
+  const FewRows mine = few_rows<FROM>(at, more, top, n_tokens, E, places_s, nullptr);
+  const int e = mine.expert, first = mine.first, rows = mine.rows, pair = mine.pair;
   if (e < 0) return;
-  const int col0 = blockIdx.y * 16;
-  if (e >= real) {  // (the whole workgroup)
-    pass_input<T, 256>(x, ldx, share, first, rows, col0, col0 + 16, top, n_tokens, N, order, P);
+  const int col0 = blockIdx.y * 16 * COLS;
+  if (FROM == kListed && e >= real) {  // (the whole workgroup)
+    pass_input<T, 256>(x, ldx, share, first, rows, col0, col0 + 16 * COLS, top, n_tokens, N, more, P);
     return;
   }
   const int lane = threadIdx.x & 63;
@@ -714,30 +762,41 @@ __global__ __launch_bounds__(256, 4) void experts_few_down_kernel(const i32x4_t*
   const int k_each = F / KS;
   const T* d = w_down + ((long)e * N + col0 + l16) * F + w * k_each + VEC * quad;
   const T* y = act + (long)(first + min(l16, rows - 1)) * ldy + w * k_each + VEC * quad;
-  const int pair = order[first + min(l16, rows - 1)];  // (rows past the tile's repeat the last: their sums are not stored)
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < k_each; k0 += U * KC) {
-    vec_t a[U], b[U];
+  f32x4 acc[COLS];
 #pragma unroll
-    for (int i = 0; i < U; ++i) a[i] = *reinterpret_cast<const vec_t*>(d + k0 + i * KC);
+  for (int c = 0; c < COLS; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < k_each; k0 += U * KC) {
+    vec_t a[COLS][U], b[U];
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+#pragma unroll
+      for (int i = 0; i < U; ++i) a[c][i] = *reinterpret_cast<const vec_t*>(d + (long)(16 * c) * F + k0 + i * KC);
 #pragma unroll
     for (int i = 0; i < U; ++i) b[i] = *reinterpret_cast<const vec_t*>(y + k0 + i * KC);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < U; ++i) Atom<T>::mma(acc, a[i], b[i]);
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) Atom<T>::mma(acc[c], a[c][i], b[i]);
   }
-  const float factor = weight ? weight[pair] : 1.0f;
-  __shared__ f32x4 sums_s[KS - 1][64];
-  if (w > 0) sums_s[w - 1][lane] = acc;
+  const float factor = FROM != kListed ? 1.0f / (float)top : weight ? weight[pair] : 1.0f;
+  __shared__ f32x4 sums_s[KS - 1][COLS][64];
+  if (w > 0) {
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) sums_s[w - 1][c][lane] = acc[c];
+  }
   __syncthreads();
   if (w != 0 || l16 >= rows) return;
-#pragma unroll
-  for (int o = 0; o < KS - 1; ++o)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = acc[i] + sums_s[o][lane][i];
   float* dst = P + ((long)(pair % top) * n_tokens + pair / top) * N + col0 + 4 * quad;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) dst[i] = factor * acc[i];
+  for (int c = 0; c < COLS; ++c) {
+#pragma unroll
+    for (int o = 0; o < KS - 1; ++o)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[c][i] = acc[c][i] + sums_s[o][c][lane][i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[16 * c + i] = factor * acc[c][i];
+  }
 }
 
 // Chunks that a wave of those kernels asks for at a time where K is a whole number of such rounds, else 0.
@@ -1134,13 +1193,13 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
   const bool few = rows_a_tile == 16 && !with_shared && few_up && few_down && F % 16 == 0 && N % 16 == 0 && ldx % vec == 0 &&
                    ldy % vec == 0 && reinterpret_cast<uintptr_t>(tiles) % 16 == 0 && (F + 15) / 16 < 65536 && (N + 15) / 16 < 65536;
 #define LS_FEW_UP(T_, U_)                                                                                             \
-  hipLaunchKernelGGL((experts_few_gate_up_kernel<T_, U_>), dim3(cap, F / 16), dim3(256), 0, s, (const i32x4_t*)tiles, \
+  hipLaunchKernelGGL((experts_few_gate_up_kernel<T_, U_, kListed>), dim3(cap, F / 16), dim3(256), 0, s, tiles,          \
                      (const T_*)w_gate, (const T_*)w_up, order, (const T_*)x, ldx, F, K, top, real, limit, alpha, shift, \
-                     in_weight, (T_*)act, ldy)
+                     in_weight, (T_*)act, ldy, n_tokens, E, (int*)nullptr)
 #define LS_FEW_DOWN(T_, U_)                                                                                           \
-  hipLaunchKernelGGL((experts_few_down_kernel<T_, U_>), dim3(cap, N / 16), dim3(256), 0, s, (const i32x4_t*)tiles,    \
+  hipLaunchKernelGGL((experts_few_down_kernel<T_, U_, kListed, 1>), dim3(cap, N / 16), dim3(256), 0, s, tiles,        \
                      (const T_*)w_down, (const T_*)act, ldy, order, out_weight, P, N, F, top, n_tokens, real, (const T_*)x, \
-                     ldx, weight)
+                     ldx, weight, E)
 #define LS_FEW(T_)                                                                                                    \
   do {                                                                                                                \
     if (few_up == 8) LS_FEW_UP(T_, 8); else if (few_up == 6) LS_FEW_UP(T_, 6); else LS_FEW_UP(T_, 4);                 \
@@ -1174,4 +1233,55 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
 #undef LS_EXPERTS_STAGED
 #undef LS_EXPERTS
   return check_launch("experts_apply");
+}
+
+// Whether ls_experts_apply_table takes a step of these sizes.
+extern "C" int ls_experts_apply_table_ok(int dtype, int n_tokens, int E, int top, int K, int F, int N) {
+  return n_tokens > 0 && (long)n_tokens * top <= kTablePairs && few_chunks(dtype, K) && few_chunks(dtype, F) && F % 16 == 0 && N % 16 == 0 &&
+         F / 16 < 65536 && N / 16 < 65536 && (long)E * ((n_tokens + 15) / 16) <= 0x7fffffffL;
+}
+
+// ls_experts_route_table and ls_experts_apply in two launches, for few pairs: token t uses the experts that row token_ids[t] of
+// table [vocab][top] names (entries in [0, E), those of a row differ), each with the weight 1 / top.  picks: scratch of n_tokens * top
+// ints, the pairs' experts afterwards.
+extern "C" int ls_experts_apply_table(int dtype, const void* x, long ldx, const void* w_gate, const void* w_up, const void* w_down,
+                                      const int* token_ids, const int* table, int n_tokens, int E, int top, int K, int F, int N,
+                                      float limit, float alpha, float shift, void* act, long ldy, int* picks, float* P,
+                                      void* stream) {
+  LS_REQUIRE(dtype == kF32 || dtype == kBF16, "experts_apply_table: unknown dtype %d", dtype);
+  LS_REQUIRE(n_tokens > 0 && E > 0 && top > 0 && top <= E && K > 0 && F > 0 && N > 0 && ldx >= K && ldy >= F &&
+                 ls_experts_apply_table_ok(dtype, n_tokens, E, top, K, F, N),
+             "experts_apply_table: %d tokens, %d of %d experts, sizes %d, %d, %d", n_tokens, top, E, K, F, N);
+  LS_REQUIRE(x && w_gate && w_up && w_down && token_ids && table && act && picks && P, "experts_apply_table: null operand");
+  LS_REQUIRE(limit > 0.f, "experts_apply_table: the limit must be positive");
+  const int vec = dtype == kF32 ? 4 : 8;
+  LS_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(act) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(w_gate) % 16 == 0 && reinterpret_cast<uintptr_t>(w_up) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(w_down) % 16 == 0 && ldx % vec == 0 && ldy % vec == 0,
+             "experts_apply_table: operands must be 16-byte aligned");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int groups = E * ((n_tokens + 15) / 16);
+#define LS_TABLE_UP(T_, U_)                                                                                           \
+  hipLaunchKernelGGL((experts_few_gate_up_kernel<T_, U_, kTable>), dim3(groups, F / 16), dim3(256), 0, s, token_ids,    \
+                     (const T_*)w_gate, (const T_*)w_up, table, (const T_*)x, ldx, F, K, top, E, limit, alpha, shift, \
+                     (const float*)nullptr, (T_*)act, ldy, n_tokens, E, picks)
+#define LS_TABLE_DOWN_COLS(T_, U_, COLS_)                                                                             \
+  hipLaunchKernelGGL((experts_few_down_kernel<T_, U_, kPicked, COLS_>), dim3(groups, N / (16 * COLS_)), dim3(256), 0, s, picks, \
+                     (const T_*)w_down, (const T_*)act, ldy, (const int*)nullptr, (const float*)nullptr, P, N, F, top, n_tokens, E, \
+                     (const T_*)nullptr, 0L, (const float*)nullptr, E)
+#define LS_TABLE_DOWN(T_, U_) \
+  if (sizeof(T_) == 2 && N % 32 == 0) LS_TABLE_DOWN_COLS(T_, U_, 2); else LS_TABLE_DOWN_COLS(T_, U_, 1)
+#define LS_TABLE(T_)                                                                                                  \
+  do {                                                                                                                \
+    const int up = few_chunks(dtype, K), down = few_chunks(dtype, F);                                                 \
+    if (up == 8) LS_TABLE_UP(T_, 8); else if (up == 6) LS_TABLE_UP(T_, 6); else LS_TABLE_UP(T_, 4);                   \
+    if (down == 8) { LS_TABLE_DOWN(T_, 8); } else if (down == 6) { LS_TABLE_DOWN(T_, 6); } else { LS_TABLE_DOWN(T_, 4); } \
+  } while (0)
+  if (dtype == kF32) LS_TABLE(float);
+  else LS_TABLE(bf16_t);
+#undef LS_TABLE
+#undef LS_TABLE_UP
+#undef LS_TABLE_DOWN
+#undef LS_TABLE_DOWN_COLS
+  return check_launch("experts_apply_table");
 }

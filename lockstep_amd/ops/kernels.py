@@ -1302,6 +1302,42 @@ class Kernels:
             _ptr(token_ids), _ptr(table), c_int(t), c_int(experts), c_int(top), c_int(rows_a_tile), _ptr(expert),
             _ptr(weight), _ptr(order), _ptr(tiles), c_int(cap), _ptr(counts), _stream()))
 
+    def experts_apply_table_ok(self, dtype: torch.dtype, tokens: int, experts: int, top: int, k: int, f: int, n: int) -> bool:
+        """Whether ``experts_apply_table`` takes a step of these sizes."""
+        return self._memo(("experts_apply_table_ok", dtype, tokens, experts, top, k, f, n), lambda: bool(
+            self.experts_lib().ls_experts_apply_table_ok(c_int(DTYPE_CODE[dtype]), c_int(tokens), c_int(experts), c_int(top), c_int(k),
+                                                         c_int(f), c_int(n))))
+
+    def experts_apply_table(self, x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
+                            token_ids: torch.Tensor, table: torch.Tensor, limit: float, alpha: float, act: torch.Tensor,
+                            expert: torch.Tensor, partials: torch.Tensor, shift: float = 1.0) -> None:
+        """``experts_route_table`` and ``experts_apply`` at once, for the few pairs of a decode step
+        (``experts_apply_table_ok``): the workgroups of the products find their rows themselves.  ``expert [T * top]``
+        gets what the table names, as by ``experts_route_table``."""
+        _rows_ok(x, "experts_apply_table x"); _rows_ok(act, "experts_apply_table act")
+        t, k = x.shape
+        if not (table.is_cuda and table.dtype == torch.int32 and table.dim() == 2 and table.is_contiguous()):
+            raise KernelError("experts_apply_table table must be int32 [vocab, top] on the GPU")
+        if not (w_gate.dim() == 3 and w_gate.shape == w_up.shape and w_gate.shape[2] == k and w_down.dim() == 3
+                and w_down.shape[0] == w_gate.shape[0] and w_down.shape[2] == w_gate.shape[1]
+                and w_gate.is_contiguous() and w_up.is_contiguous() and w_down.is_contiguous()
+                and w_gate.dtype == x.dtype == w_up.dtype == w_down.dtype == act.dtype and x.dtype in DTYPE_CODE):
+            raise KernelError("experts_apply_table weights must be [E, F, K], [E, F, K], [E, N, F] of the compute dtype")
+        e, f, n, top = w_gate.shape[0], w_gate.shape[1], w_down.shape[1], table.shape[1]
+        if not (act.shape[0] >= t * top and act.shape[1] == f):
+            raise KernelError(f"experts_apply_table act must be [>= {t * top}, {f}]")
+        if not (partials.is_cuda and partials.dtype == torch.float32 and partials.is_contiguous()
+                and tuple(partials.shape) == (top, t, n)):
+            raise KernelError(f"experts_apply_table partials must be float32 [{top}, {t}, {n}]")
+        self._i32(token_ids, t, "experts_apply_table token_ids"); self._i32(expert, t * top, "experts_apply_table expert")
+        if t == 0:
+            return
+        lib = self.experts_lib()
+        self._launch(lib, lib.ls_experts_apply_table, (
+            c_int(DTYPE_CODE[x.dtype]), _ptr(x), c_long(x.stride(0)), _ptr(w_gate), _ptr(w_up), _ptr(w_down), _ptr(token_ids),
+            _ptr(table), c_int(t), c_int(e), c_int(top), c_int(k), c_int(f), c_int(n), c_float(limit), c_float(alpha),
+            c_float(shift), _ptr(act), c_long(act.stride(0)), _ptr(expert), _ptr(partials), _stream()))
+
     # -- a residual stream of several copies ------------------------------------------------------
     def streams_max(self) -> tuple[int, int]:
         """(the most copies, the widest row) that ``streams_step`` takes."""

@@ -153,6 +153,13 @@ class RoutedExperts(FeedForward):
         rt = ctx.rt
         k = rt.kernels
         t, e, top = ctx.n_tokens, self.routed, self.top
+        if self.tabled and self.shared is None and self.weigh == "output" and \
+                k.experts_apply_table_ok(rt.dtype, t, e, top, self.hidden, self.inter, self.hidden):   # a few tokens: no launch to put them in order
+            partials = ctx.buf("experts.slices", (top * t, self.hidden), torch.float32).view(top, t, self.hidden)
+            k.experts_apply_table(x, self.w_gate, self.w_up, self.w_down, ctx.token_ids, self.table, self.limit, self.alpha,
+                                  ctx.buf("experts.act", (t * top, self.inter), rt.dtype),
+                                  ctx.buf("experts.chosen", (t * top,), torch.int32), partials, shift=self.shift)
+            return self._leave(ctx, out, partials, accumulate, defer)
         rows = self.rows_a_tile(t, top, e)
         cap = k.experts_tile_capacity(t, e, top, rows)
         chosen = ctx.buf("experts.chosen", (t * top,), torch.int32)
@@ -182,8 +189,11 @@ class RoutedExperts(FeedForward):
                         act, partials[:top], shift=self.shift, weigh_input=self.weigh == "input", identity=self.identity, shared=beside)
         if self.shared is not None and beside is None:
             self.shared.forward(ctx, x, partials[top], accumulate=False)
+        return self._leave(ctx, out, partials, accumulate, defer)
+
+    def _leave(self, ctx, out, partials, accumulate: bool, defer):
         pending = PendingAdd(partials)
-        if defer == "any" or (defer and t <= DEFER_ROWS and self.hidden % 4 == 0):
+        if defer == "any" or (defer and ctx.n_tokens <= DEFER_ROWS and self.hidden % 4 == 0):
             return pending                 # (the slices are the result: ``out`` is not touched)
         if not accumulate:
             out.zero_()

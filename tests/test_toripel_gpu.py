@@ -445,6 +445,65 @@ def test_experts_that_a_table_names(dtype, tokens, experts, top, width, ff):
     assert close(partials.sum(0), want, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("weigh_input,identity", [(False, 0), (True, 0), (False, 2)])
+@pytest.mark.parametrize("tokens,experts,top,width,ff", [(1, 4, 1, 512, 512), (9, 8, 2, 1024, 768), (40, 6, 3, 1536, 2048), (17, 1, 1, 768, 16 * 48),
+                                                         (150, 32, 1, 1024, 512)])
+def test_experts_of_few_rows_have_the_bits_of_the_kernels_for_any_size(dtype, tokens, experts, top, width, ff, weigh_input, identity):
+    """Tiles of 16 rows of whole chunks (one round and several of 4, 6 and 8; a last tile of one row; experts that return their
+    input) against the kernels for any size, which a tile list off 16 bytes goes to."""
+    g = torch.Generator().manual_seed(tokens + width)
+    k, all_of = K(), experts + identity
+    ids = torch.arange(tokens, dtype=torch.int32).cuda()
+    table = torch.stack([torch.randperm(all_of, generator=g)[:top] for _ in range(tokens)]).to(torch.int32).cuda()
+    x = torch.randn((tokens, width), generator=g).to(dtype).cuda()
+    w_gate, w_up, w_down = ((torch.randn((experts, *s), generator=g) * s[1] ** -0.5).to(dtype).cuda() for s in ((ff, width), (ff, width), (width, ff)))
+    cap = k.experts_tile_capacity(tokens, all_of, top, 16)
+    outs = []
+    for shift in (0, 1):
+        i32 = lambda n: torch.empty(n, dtype=torch.int32, device="cuda")  # noqa: E731
+        chosen, order, tiles, counts = i32(tokens * top), i32(tokens * top), i32(4 * cap + shift)[shift:], i32(all_of)
+        share = torch.empty(tokens * top, dtype=torch.float32, device="cuda")
+        k.experts_route_table(ids, table, all_of, 16, chosen, share, order, tiles, counts)
+        share.copy_(torch.rand(tokens * top, generator=torch.Generator().manual_seed(5)))
+        act = torch.zeros((tokens * top, ff), dtype=dtype, device="cuda")
+        partials = torch.full((top, tokens, width), float("nan"), device="cuda")
+        k.experts_apply(x, w_gate, w_up, w_down, top, 16, order, tiles, share, 3.0, 1.5, act, partials, shift=0.5, weigh_input=weigh_input,
+                        identity=identity)
+        assert not torch.isnan(partials).any()
+        outs.append(partials)
+    assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,experts,top,width,ff", [(1, 4, 1, 512, 512), (8, 32, 4, 1024, 768), (21, 6, 3, 1536, 2048), (64, 3, 1, 512, 1536),
+                                                         (33, 1, 1, 768, 768), (1, 64, 64, 512, 512), (16, 300, 4, 512, 512)])
+def test_few_pairs_that_a_table_names_without_a_launch_to_order_them(dtype, tokens, experts, top, width, ff):
+    """Steps of up to 64 pairs (one expert's rows in one, two and four workgroups; a table that names every expert) against the
+    routing and the products in launches of their own: the same bits, tokens that repeat among them."""
+    g = torch.Generator().manual_seed(tokens * top + width)
+    k, vocab = K(), 40
+    assert k.experts_apply_table_ok(dtype, tokens, experts, top, width, ff, width)
+    assert not k.experts_apply_table_ok(dtype, 64 // top + 1, experts, top, width, ff, width)
+    assert not k.experts_apply_table_ok(dtype, tokens, experts, top, width + 16, ff, width)
+    ids = torch.randint(0, vocab, (tokens,), generator=g).to(torch.int32).cuda()
+    table = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(vocab)]).to(torch.int32).cuda()
+    x = torch.randn((tokens, width), generator=g).to(dtype).cuda()
+    w_gate, w_up, w_down = ((torch.randn((experts, *s), generator=g) * s[1] ** -0.5).to(dtype).cuda() for s in ((ff, width), (ff, width), (width, ff)))
+    cap = k.experts_tile_capacity(tokens, experts, top, 16)
+    i32 = lambda n: torch.empty(n, dtype=torch.int32, device="cuda")  # noqa: E731
+    chosen, order, tiles, counts = i32(tokens * top), i32(tokens * top), i32(4 * cap), i32(experts)
+    share = torch.empty(tokens * top, dtype=torch.float32, device="cuda")
+    k.experts_route_table(ids, table, experts, 16, chosen, share, order, tiles, counts)
+    act = torch.full((tokens * top, ff), float("nan"), dtype=dtype, device="cuda")
+    want, got = (torch.full((top, tokens, width), float("nan"), device="cuda") for _ in range(2))
+    k.experts_apply(x, w_gate, w_up, w_down, top, 16, order, tiles, share, 3.0, 1.5, act, want, shift=0.5)
+    act.fill_(float("nan"))
+    picked = torch.full_like(chosen, -1)
+    k.experts_apply_table(x, w_gate, w_up, w_down, ids, table, 3.0, 1.5, act, picked, got, shift=0.5)
+    assert not torch.isnan(want).any() and torch.equal(got, want) and torch.equal(picked, chosen)
+
+
 # ---------------------------------------------------------------------------
 # whole models
 # ---------------------------------------------------------------------------
