@@ -389,7 +389,8 @@ __global__ __launch_bounds__(256) void heads_product_kernel(const T* __restrict_
 //     (the sums: a lane's rows in four interleaved chains of fused multiply-adds, then the lanes of a column by moves inside their row of sixteen; the
 //     decay multiplies the sum of the old state with the key, which is the decayed state's sum up to rounding).
 //     A token's operands are requested eight (four) tokens before it is worked on.
-// (3) delta_conv_state: the last M - 1 inputs of every channel become the state of the next step.
+//     The request's waves also make the last M - 1 inputs of every channel, which (1) has read, the state of the next step
+//     (a launch of its own for that took 5 us of a decode step's 29 a layer).
 // ---------------------------------------------------------------------------
 // MM: the taps of the convolution where they are one aligned vector (4; all of an element's loads are then on their way
 // together: 2,048 tokens, 4,096 channels 51.7 -> 31.3 us, eight tokens 8.4 -> 5.6), or 0: any number, in a loop.
@@ -499,6 +500,27 @@ __device__ __forceinline__ float lanes_sum(float v) {
   return v;
 }
 
+// The last M - 1 inputs of the channels c, c + step, ...: place a holds the input at position kv_len - (M - 1) + a, one of this
+// step's, or one the state already holds further on.
+__device__ __forceinline__ void keep_inputs(const float* __restrict__ raw, long ld, int C, int M, const SeqMeta& m, float* __restrict__ kept,
+                                            int c, int step) {
+  for (; c < C; c += step) {
+    auto input = [&](int a) LS_INLINED -> const float* {
+      const int p = m.kv_len - (M - 1) + a;
+      return p >= m.q_start ? raw + (long)(m.q_off + p - m.q_start) * ld + c : kept + (long)(p - m.q_start + M - 1) * C + c;
+    };
+    constexpr int kAtOnce = 3;
+    for (int a0 = 0; a0 < M - 1; a0 += kAtOnce) {  // (read before the ascending walk overwrites it)
+      float v[kAtOnce];
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) v[u] = *input(min(a0 + u, M - 2));
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u)
+        if (a0 + u < M - 1) kept[(long)(a0 + u) * C + c] = v[u];
+    }
+  }
+}
+
 // R rows a lane, L lanes a column (R * L rows, the head size rounded up), 64 / L columns a wave.  CH: the decay is a
 // number a row of the state (decays [T][H][dp]) instead of one a head: S[r] <- g[r] S[r] first, then the rule as stated.
 //
@@ -521,7 +543,8 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
                                                         const float* __restrict__ gates, const float* __restrict__ decays,
                                                         int G, int H, int D, int DV,
                                                         const SeqMeta* __restrict__ seqs, float* __restrict__ state,
-                                                        long state_stride, float* __restrict__ out, long ldo) {
+                                                        long state_stride, float* __restrict__ out, long ldo,
+                                                        const float* __restrict__ raw, long ld, int C, int M, long conv_at) {
   typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
   typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
   constexpr int dp = L * R, COLS = 64 / L;
@@ -615,6 +638,9 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) fetch(ring[j], qkb, vb, gb, db, min(j, n - 1));
   }
+  if (M > 1)
+    keep_inputs(raw, ld, C, M, m, state + (long)m.table_row * state_stride + conv_at, (head * (int)gridDim.y + (int)blockIdx.y) * 64 + lane,
+                64 * H * (int)gridDim.y);
   auto next_block = [&]() LS_INLINED {
     qk_at += (long)DEPTH * 2 * G * dp;
     v_at += (long)DEPTH * H * DV;
@@ -653,22 +679,6 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[r]), mine, s_off[r], 0, 0);
-}
-
-__global__ __launch_bounds__(256) void delta_conv_state_kernel(const float* __restrict__ raw, long ld, int C, int M,
-                                                               const SeqMeta* __restrict__ seqs, float* __restrict__ state,
-                                                               long state_stride, long conv_at) {
-  const SeqMeta m = seqs[blockIdx.x];
-  const int c = blockIdx.y * 256 + threadIdx.x;
-  if (m.q_len <= 0 || c >= C) return;
-  float* kept = state + (long)m.table_row * state_stride + conv_at;
-  // place a holds the input at position kv_len - (M - 1) + a: one of this step's, or one the state already holds
-  // further on (read before the ascending walk overwrites it)
-  for (int a = 0; a < M - 1; ++a) {
-    const int p = m.kv_len - (M - 1) + a;
-    kept[(long)a * C + c] = p >= m.q_start ? raw[(long)(m.q_off + p - m.q_start) * ld + c]
-                                           : kept[(long)(p - m.q_start + M - 1) * C + c];
-  }
 }
 
 }  // namespace ls
@@ -849,7 +859,7 @@ extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, in
   const bool far = ldo >= (1L << 26);  // output rows that a block's 32-bit offsets do not reach: a block of one token
 #define LS_DELTA_RULE(R_, L_, CH_, DEPTH_)                                                                               \
   hipLaunchKernelGGL((delta_rule_kernel<R_, L_, CH_, DEPTH_>), dim3(n_seqs * H, (DV * L_ + 63) / 64), dim3(64), 0, s, qk, vv, \
-                     gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo)
+                     gates, decays, G, H, D, DV, (const SeqMeta*)seqs, state, state_stride, out, ldo, raw, ld, (int)C, M, conv_at)
 #define LS_DELTA(R_, L_)                                                          \
   do {                                                                            \
     if (far) {                                                                    \
@@ -871,9 +881,6 @@ extern "C" int ls_delta_rule_longest(const float* raw, long ld, int n_tokens, in
   }
 #undef LS_DELTA
 #undef LS_DELTA_RULE
-  if (M > 1)
-    hipLaunchKernelGGL(delta_conv_state_kernel, dim3(n_seqs, (unsigned)((C + 255) / 256)), dim3(256), 0, s, raw, ld, (int)C,
-                       M, (const SeqMeta*)seqs, state, state_stride, conv_at);
   return check_launch("delta_rule");
 }
 

@@ -285,6 +285,33 @@ def test_the_delta_rule_with_its_convolutions_over_unequal_requests_in_steps(hea
         assert close(torch.cat(got[s]), want[s], torch.float32, scale=1e-2), s
 
 
+@pytest.mark.parametrize("heads, groups, d, dv, taps", [(1, 1, 250, 4, 9), (2, 1, 16, 5, 2), (1, 1, 64, 3, 4), (3, 3, 128, 16, 6)])
+def test_the_delta_rule_keeps_the_last_inputs_of_every_channel(heads, groups, d, dv, taps):
+    """The inputs that a step leaves for the next one's convolutions, exactly: more channels than a request has lanes, more
+    taps than are moved at once, steps shorter than the taps, a request that sits a step out."""
+    g = torch.Generator().manual_seed(d + taps)
+    k, channels = K(), 2 * groups * d + heads * dv
+    conv, a_log, dt_bias = torch.randn((channels, taps), generator=g).cuda(), torch.zeros(heads).cuda(), torch.zeros(heads).cuda()
+    conv_at = heads * d * dv
+    state = torch.zeros((3, conv_at + (taps - 1) * channels), dtype=torch.float32, device="cuda")
+    seen = {s: torch.zeros(taps - 1, channels) for s in (0, 2)}
+    done = {0: 0, 2: 0}
+    for portion in ({0: 1, 2: 7}, {2: 2}, {0: 3, 2: 1}, {0: 20, 2: 1}, {0: 1, 2: 1}):
+        order = list(portion)
+        tok_seq, tok_pos, seqs = step_meta([portion[s] for s in order], [done[s] for s in order], order)
+        raws = [torch.randn((portion[s], channels + 2 * heads), generator=g) for s in order]
+        out = torch.empty((sum(portion.values()), heads * dv), dtype=torch.float32, device="cuda")
+        scratch = torch.empty(k.delta_scratch_floats(len(out), groups, heads, d, dv), dtype=torch.float32, device="cuda")
+        k.delta_rule(torch.cat(raws).cuda(), groups, heads, d, dv, conv, a_log, dt_bias, 1e-6, tok_seq, tok_pos, seqs, len(order), state,
+                     scratch, out)
+        for s, raw in zip(order, raws):
+            seen[s] = torch.cat([seen[s], raw[:, :channels]])
+            done[s] += portion[s]
+        for s in seen:
+            assert torch.equal(state[s, conv_at:].cpu().view(taps - 1, channels), seen[s][-(taps - 1):]), (portion, s)
+    assert not state[1].any()
+
+
 @pytest.mark.parametrize("heads, groups, d, dv", [(2, 1, 16, 17), (2, 2, 30, 5), (1, 1, 64, 64), (4, 2, 128, 20), (1, 1, 200, 9)])
 @pytest.mark.parametrize("channel_decays", [False, True])
 def test_the_delta_rule_has_the_same_bits_however_many_tokens_a_step_brings(heads, groups, d, dv, channel_decays):
