@@ -194,7 +194,8 @@ __device__ __forceinline__ f32x4 and_vec(f32x4 a, f32x4 b) {
 // Prompts, D = 128, us: 2,048 tokens of 16 over 8 heads from 0 48.1 -> 47.2, from 6,144 177 -> 168, of 32 over 8 heads from 0 65.0 -> 61.9,
 // 9,000 from 0 481 -> 457.  (One fused multiply-add in place of the product and the subtraction gives another 3 %, but needs the other form
 // beside it for scores whose rounding it does not cancel, and decode steps took 0.3 to 2 % longer for that.)
-template <typename T> __device__ __forceinline__ float score_factor(float scale) { return sizeof(T) == 2 ? scale * 1.44269504088896340736f : scale; }
+// (`factor` is c, or the scale in float32; formed on the host: a kernel would keep it in a register, where it reads an argument again)
+static float score_factor(int dtype, float scale) { return dtype == kBF16 ? scale * 1.44269504088896340736f : scale; }
 template <typename T> __device__ __forceinline__ float score_exp(float x);
 template <> __device__ __forceinline__ float score_exp<float>(float x) { return softmax_exp<float>(x); }
 template <> __device__ __forceinline__ float score_exp<bf16_t>(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -254,9 +255,8 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs,
     const AttnItem* __restrict__ items, T* __restrict__ out, long ldo, float* __restrict__ part_acc,
-    float* __restrict__ part_ml, int G, float scale, int window) {
+    float* __restrict__ part_ml, int G, float factor, int window) {
   typedef Atom<T> A;
-  const float factor = score_factor<T>(scale);
   typedef typename A::vec_t vec_t;
   constexpr int NC = (D + A::KCHUNK - 1) / A::KCHUNK;  // chunks over the head
 
@@ -440,9 +440,8 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, int page_shift, const int* __restrict__ table, int table_stride,
     const SeqMeta* __restrict__ seqs, const AttnItem* __restrict__ items, T* __restrict__ out, long ldo,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float scale, int window) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float factor, int window) {
   typedef Atom<T> A;
-  const float factor = score_factor<T>(scale);
   typedef typename A::vec_t vec_t;
   constexpr int SZ = sizeof(T);
   constexpr int NC = (D + A::KCHUNK - 1) / A::KCHUNK;
@@ -804,9 +803,8 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, int page_shift, const int* __restrict__ table, int table_stride,
     const SeqMeta* __restrict__ seqs, const AttnItem* __restrict__ items, T* __restrict__ out, long ldo,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float scale, int window) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float factor, int window) {
   typedef Atom<T> A;
-  const float factor = score_factor<T>(scale);
   typedef typename A::vec_t vec_t;
   constexpr int SZ = sizeof(T);
   constexpr int NT = 64 * NW;
@@ -1245,14 +1243,13 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     const float* __restrict__ head_k_weight, const float* __restrict__ cos_table, const float* __restrict__ sin_table,
     int G, int nkv, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int page_size, int page_shift,
     const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs, T* __restrict__ out, long ldo,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, float scale, int window, DecodeFuse<T> fz_rest) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, float factor, int window, DecodeFuse<T> fz_rest) {
   DecodeFuse<T> fz = fz_rest;
   fz.q_weight = head_q_weight;
   fz.k_weight = head_k_weight;
   fz.cos_table = cos_table;
   fz.sin_table = sin_table;
   typedef Atom<T> A;
-  const float factor = score_factor<T>(scale);
   typedef typename A::vec_t vec_t;
   constexpr int SZ = sizeof(T);
   constexpr int NT = 256;
@@ -1301,7 +1298,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     // every other argument is requested now, while the item is on its way: left to themselves their loads
     // stand where each is first used, each with a wait of its own for memory that no cache holds yet
     __asm__ volatile("" ::"s"(k_pages), "s"(v_pages), "s"(page_size), "s"(page_shift), "s"(part_acc), "s"(part_ml),
-                     "s"(scale), "s"(window), "s"(fz.eps), "s"(fz.rot), "s"(fz.nq), "s"(fz.write_kv), "s"(fz.k_out),
+                     "s"(factor), "s"(window), "s"(fz.eps), "s"(fz.rot), "s"(fz.nq), "s"(fz.write_kv), "s"(fz.k_out),
                      "s"(fz.v_out), "s"(out), "s"(ldo), "s"(table), "s"(table_stride));
   }
   const SeqMeta sm = item.sm;
@@ -2390,6 +2387,7 @@ extern "C" int ls_attention_decode(int dtype, const void* qkv, long ld, void* k_
   LS_REQUIRE(!cos_table || (sin_table && table_positions > max_pos),
              "decode attention: rotation tables hold %d positions, the step reaches %d", table_positions, max_pos);
   LS_REQUIRE(decode_fused_supported(dtype), "decode attention: the fused kernel does not fit into LDS for this head size");
+  scale = score_factor(dtype, scale);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   dim3 grid(n_items, nkv);
   int page_shift = 0;
@@ -2499,6 +2497,7 @@ extern "C" int ls_attention(int dtype, const void* q, long ldq, const void* k_pa
   LS_REQUIRE(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
                  reinterpret_cast<uintptr_t>(k_pages) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pages) % 16 == 0,
              "attention: operands must be 16-byte aligned");
+  scale = score_factor(dtype, scale);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   dim3 grid(n_items, nkv);
   int page_shift = 0;
