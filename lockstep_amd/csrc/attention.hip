@@ -186,21 +186,6 @@ __device__ __forceinline__ f32x4 and_vec(f32x4 a, f32x4 b) {
   return __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, a) & __builtin_bit_cast(u32x4, b));
 }
 
-// From a tile's products q.k to its probabilities e^(s scale - m), m being the largest s scale of the row's in the tile.
-// float32: as written, the library's exponential.  bfloat16: in powers of two, 2^(s c - m2) with c = scale log2 e and m2 the largest
-// s c: the product with log2 e that the hardware's exponential needs is in the scale, an instruction a score less (the attention of
-// prompts is bound by what its vector unit and matrix cores take to issue).  s c is rounded as s scale was, the largest
-// probability of a row is exactly 1 however great the scores are, and what a split leaves for its fold, m = m2 ln 2, is in natural units.
-// Prompts, D = 128, us: 2,048 tokens of 16 over 8 heads from 0 48.1 -> 47.2, from 6,144 177 -> 168, of 32 over 8 heads from 0 65.0 -> 61.9,
-// 9,000 from 0 481 -> 457.  (One fused multiply-add in place of the product and the subtraction gives another 3 %, but needs the other form
-// beside it for scores whose rounding it does not cancel, and decode steps took 0.3 to 2 % longer for that.)
-// (`factor` is c, or the scale in float32; formed on the host: a kernel would keep it in a register, where it reads an argument again)
-static float score_factor(int dtype, float scale) { return dtype == kBF16 ? scale * 1.44269504088896340736f : scale; }
-template <typename T> __device__ __forceinline__ float score_exp(float x);
-template <> __device__ __forceinline__ float score_exp<float>(float x) { return softmax_exp<float>(x); }
-template <> __device__ __forceinline__ float score_exp<bf16_t>(float x) { return __builtin_amdgcn_exp2f(x); }
-template <typename T> __device__ __forceinline__ float natural(float m) { return sizeof(T) == 2 ? m * 0.69314718055994530942f : m; }
-
 struct RowState {
   f32x4 acc[DB];
   float m, l;
@@ -255,7 +240,7 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs,
     const AttnItem* __restrict__ items, T* __restrict__ out, long ldo, float* __restrict__ part_acc,
-    float* __restrict__ part_ml, int G, float factor, int window) {
+    float* __restrict__ part_ml, int G, float scale, int window) {
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   constexpr int NC = (D + A::KCHUNK - 1) / A::KCHUNK;  // chunks over the head
@@ -330,7 +315,7 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            s[kb][e] = s[kb][e] * factor;
+            s[kb][e] = s[kb][e] * scale;
             tile_max = fmaxf(tile_max, s[kb][e]);
           }
       } else {
@@ -339,24 +324,24 @@ __global__ __launch_bounds__(256) void attention_direct_kernel(
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * factor : kMasked;
+            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * scale : kMasked;
             s[kb][e] = v;
             tile_max = fmaxf(tile_max, v);
           }
       }
       tile_max = quad16_max(tile_max);
-      const float m_new = fmaxf(cur.m, tile_max);  // (a split is one tile: tile_max, or kNegSentinel)
-      const float alpha = score_exp<T>(cur.m - m_new);
+      const float m_new = fmaxf(cur.m, tile_max);
+      const float alpha = softmax_exp<T>(cur.m - m_new);
       float p_sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[kb][e] = score_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
+        for (int e = 0; e < 4; ++e) s[kb][e] = softmax_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
         p_sum = p_sum + ((s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]));
       }
       p_sum = quad16_sum(p_sum);
       cur.l = cur.l * alpha + p_sum;
-      cur.m = natural<T>(m_new);
+      cur.m = m_new;
 #pragma unroll
       for (int blk = 0; blk < DB; ++blk)
 #pragma unroll
@@ -440,7 +425,7 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, int page_shift, const int* __restrict__ table, int table_stride,
     const SeqMeta* __restrict__ seqs, const AttnItem* __restrict__ items, T* __restrict__ out, long ldo,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float factor, int window) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float scale, int window) {
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   constexpr int SZ = sizeof(T);
@@ -657,7 +642,7 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            s[kb][e] = s[kb][e] * factor;
+            s[kb][e] = s[kb][e] * scale;
             tile_max = fmaxf(tile_max, s[kb][e]);
           }
       } else {
@@ -666,24 +651,24 @@ __global__ __launch_bounds__(256, LS_STAGED_MIN_BLOCKS) void attention_staged_ke
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * factor : kMasked;
+            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * scale : kMasked;
             s[kb][e] = v;
             tile_max = fmaxf(tile_max, v);
           }
       }
       tile_max = quad16_max(tile_max);
-      const float m_new = fmaxf(cur.m, tile_max);  // (a split is one tile: tile_max, or kNegSentinel)
-      const float alpha = score_exp<T>(cur.m - m_new);
+      const float m_new = fmaxf(cur.m, tile_max);
+      const float alpha = softmax_exp<T>(cur.m - m_new);
       float p_sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[kb][e] = score_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
+        for (int e = 0; e < 4; ++e) s[kb][e] = softmax_exp<T>(s[kb][e] - m_new);  // masked: exp(-inf) = 0
         p_sum = p_sum + ((s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]));
       }
       p_sum = quad16_sum(p_sum);
       cur.l = cur.l * alpha + p_sum;
-      cur.m = natural<T>(m_new);
+      cur.m = m_new;
 #pragma unroll
       for (int blk = 0; blk < DB; ++blk)
 #pragma unroll
@@ -803,7 +788,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int nkv,
     int page_size, int page_shift, const int* __restrict__ table, int table_stride,
     const SeqMeta* __restrict__ seqs, const AttnItem* __restrict__ items, T* __restrict__ out, long ldo,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float factor, int window) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, int G, float scale, int window) {
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   constexpr int SZ = sizeof(T);
@@ -1072,7 +1057,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            s[kb][e] = s[kb][e] * factor;
+            s[kb][e] = s[kb][e] * scale;
             tile_max = fmaxf(tile_max, s[kb][e]);
           }
       } else {
@@ -1081,12 +1066,12 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * factor : kMasked;
+            const float v = ((key <= key_hi) & (key >= key_lo)) ? s[kb][e] * scale : kMasked;
             s[kb][e] = v;
             tile_max = fmaxf(tile_max, v);
           }
       }
-      const float top = quad16_max(tile_max), m = natural<T>(top);
+      const float m = quad16_max(tile_max);
       float p_sum = 0.f;
       auto probabilities = [&](auto with_loads) LS_INLINED {
 #pragma unroll
@@ -1094,7 +1079,7 @@ __global__ __launch_bounds__(64 * NW, wide_shares_cu(sizeof(T)) ? 2 : 1) void at
           float pr[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            pr[e] = score_exp<T>(s[kb][e] - top);  // masked: exp(-inf) = 0
+            pr[e] = softmax_exp<T>(s[kb][e] - m);  // masked: exp(-inf) = 0
             pv[kb / KB16][kb % KB16 * 4 + e] = from_f32<T>(pr[e]);
           }
           p_sum = p_sum + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
@@ -1243,7 +1228,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     const float* __restrict__ head_k_weight, const float* __restrict__ cos_table, const float* __restrict__ sin_table,
     int G, int nkv, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int page_size, int page_shift,
     const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs, T* __restrict__ out, long ldo,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, float factor, int window, DecodeFuse<T> fz_rest) {
+    float* __restrict__ part_acc, float* __restrict__ part_ml, float scale, int window, DecodeFuse<T> fz_rest) {
   DecodeFuse<T> fz = fz_rest;
   fz.q_weight = head_q_weight;
   fz.k_weight = head_k_weight;
@@ -1298,7 +1283,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     // every other argument is requested now, while the item is on its way: left to themselves their loads
     // stand where each is first used, each with a wait of its own for memory that no cache holds yet
     __asm__ volatile("" ::"s"(k_pages), "s"(v_pages), "s"(page_size), "s"(page_shift), "s"(part_acc), "s"(part_ml),
-                     "s"(factor), "s"(window), "s"(fz.eps), "s"(fz.rot), "s"(fz.nq), "s"(fz.write_kv), "s"(fz.k_out),
+                     "s"(scale), "s"(window), "s"(fz.eps), "s"(fz.rot), "s"(fz.nq), "s"(fz.write_kv), "s"(fz.k_out),
                      "s"(fz.v_out), "s"(out), "s"(ldo), "s"(table), "s"(table_stride));
   }
   const SeqMeta sm = item.sm;
@@ -1707,7 +1692,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = t0 + key_of_row<T>(kb, 4 * g + e);
-          const float v = ((key <= key_hi) & (key >= key_lo)) ? s[j][e] * factor : kMasked;
+          const float v = ((key <= key_hi) & (key >= key_lo)) ? s[j][e] * scale : kMasked;
           s[j][e] = v;
           my_max = fmaxf(my_max, v);
         }
@@ -1720,13 +1705,13 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     PROBE(8)
     if (NBUF == 1 && ahead) issue_k(ti + 1);  // every wave has its scores: the K half of the buffer is free
     const float tile_max = fmaxf(fmaxf(wmax[row16], wmax[16 + row16]), fmaxf(wmax[32 + row16], wmax[48 + row16]));
-    const float m_new = fmaxf(cur_m, tile_max);  // (a split is one tile: tile_max, or kNegSentinel)
-    const float alpha = score_exp<T>(cur_m - m_new);
+    const float m_new = fmaxf(cur_m, tile_max);
+    const float alpha = softmax_exp<T>(cur_m - m_new);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int kb = 2 * wave + j;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[j][e] = score_exp<T>(s[j][e] - m_new);  // masked: exp(-inf) = 0
+      for (int e = 0; e < 4; ++e) s[j][e] = softmax_exp<T>(s[j][e] - m_new);  // masked: exp(-inf) = 0
       psum[kb * 64 + lane] = (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
       prob[kb * 64 + lane] = s[j];
     }
@@ -1815,7 +1800,7 @@ __global__ __launch_bounds__(256) void attention_coop_kernel(
     for (int kb = 0; kb < NB; ++kb) p_sum = p_sum + psum[kb * 64 + lane];
     p_sum = quad16_sum(p_sum);
     cur_l = cur_l * alpha + p_sum;
-    cur_m = natural<T>(m_new);
+    cur_m = m_new;
 #pragma unroll
     for (int j = 0; j < MYDB; ++j)
 #pragma unroll
@@ -2387,7 +2372,6 @@ extern "C" int ls_attention_decode(int dtype, const void* qkv, long ld, void* k_
   LS_REQUIRE(!cos_table || (sin_table && table_positions > max_pos),
              "decode attention: rotation tables hold %d positions, the step reaches %d", table_positions, max_pos);
   LS_REQUIRE(decode_fused_supported(dtype), "decode attention: the fused kernel does not fit into LDS for this head size");
-  scale = score_factor(dtype, scale);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   dim3 grid(n_items, nkv);
   int page_shift = 0;
@@ -2497,7 +2481,6 @@ extern "C" int ls_attention(int dtype, const void* q, long ldq, const void* k_pa
   LS_REQUIRE(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
                  reinterpret_cast<uintptr_t>(k_pages) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pages) % 16 == 0,
              "attention: operands must be 16-byte aligned");
-  scale = score_factor(dtype, scale);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   dim3 grid(n_items, nkv);
   int page_shift = 0;

@@ -951,6 +951,39 @@ def test_scores_of_great_size_leave_finite_results(dtype, nq, nkv, d, ps, scale)
             assert torch.isfinite(one).all() and rel_err(one, want[p:p + 1]) < ATT_TOL[dtype], (p, split)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq,nkv,d,ps", [(4, 2, 64, 16), (16, 8, 128, 16), (6, 2, 48, 8)])
+@pytest.mark.parametrize("largest", [0.95 * 2.0 ** 128, -0.95e30])
+def test_scores_at_the_ends_of_their_range(dtype, nq, nkv, d, ps, largest):
+    """Scores close to the largest float32, and scores close above the -1e30 that running maxima start at: they are finite as
+    they are, so they are not to be multiplied by a constant beyond 1 before the row's largest is taken off.  Queries are 2^60 in
+    every element and keys +-2^60, so every partial sum is a whole multiple of 2^120 that float32 holds exactly in any order."""
+    n = 300
+    g = torch.Generator().manual_seed(d)
+    qkv = torch.randn(n, (nq + 2 * nkv) * d, generator=g)
+    keys = torch.full((n, nkv, d), 2.0 ** 60)
+    for i in range(n):
+        for h in range(nkv):         # (up to an eighth of the elements turned: scores from 3/4 of the largest size on)
+            turned = int(torch.randint(0, d // 8 + 1, (1,), generator=g))
+            keys[i, h, torch.randperm(d, generator=g)[:turned]] *= -1.0
+    qkv[:, : nq * d] = 2.0 ** 60
+    qkv[:, nq * d:(nq + nkv) * d] = keys.flatten(1)
+    qkv = qkv.to(dtype)
+    scale = largest / (d * 2.0 ** 120)
+    case = PagedCase(dtype, nq, nkv, d, ps, n, shuffle_seed=2)
+    dev = qkv.cuda()
+    case.write(dev, 0)
+    q, k, v = split_qkv(qkv.double(), nq, nkv, d)
+    want = naive_attention(q, k, v, 0, scale)
+    for variant in (0, 1) + ((4, 5) if K().wide_supported(d, dtype, ps) else ()):
+        got = case.attend(dev, 0, scale, variant=variant, force_split=False)
+        assert torch.isfinite(got).all() and rel_err(got, want) < ATT_TOL[dtype], variant
+    for p in (0, 5, 127, 128, n - 1):
+        for split in (False, True):
+            one = case.attend(dev[p:p + 1], p, scale, variant=3, force_split=split)
+            assert torch.isfinite(one).all() and rel_err(one, want[p:p + 1]) < ATT_TOL[dtype], (p, split)
+
+
 @pytest.mark.parametrize("nq,nkv,d,ps", [(4, 2, 64, 16), (16, 8, 128, 16), (6, 2, 48, 8), (2, 1, 256, 32)])
 def test_rows_of_great_scores_beside_others(nq, nkv, d, ps):
     """Rows whose largest scores lie from 300 to 3,000, side by side: every kernel gives a row the same bits, alone or among the
