@@ -659,7 +659,10 @@ __device__ __forceinline__ FewRows few_rows(const int* __restrict__ at, const in
     if (n <= 0) return {-1, 0, 0, 0};  // uniform
     int* places = places_s[threadIdx.x >> 6];  // (the wave's own)
     if (mine == e) places[__popcll(held & ((1ull << lane) - 1ull))] = lane;
+    // (other lanes read what this one wrote: the barrier orders instructions, the fences the memory between them)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int rows = min(16, n);
     return {e, first, rows, places[skip + min(l16, rows - 1)]};
   }

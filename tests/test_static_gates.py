@@ -34,6 +34,18 @@ def test_kernels_are_built_without_contraction_and_for_gfx950_only():
     assert not any("fast-math" in f for f in build.FLAGS)
 
 
+def test_a_barrier_inside_a_wave_has_its_fences():
+    """__builtin_amdgcn_wave_barrier orders instructions and is declared to touch no memory: where lanes of a wave hand each other
+    values through LDS, it takes a release fence in front of it and an acquire fence behind it."""
+    barrier = "__builtin_amdgcn_wave_barrier();"
+    for path in sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.h")):
+        lines = [line.strip() for line in strip_comments(path.read_text()).splitlines() if line.strip()]
+        for i, line in enumerate(lines):
+            if barrier in line:
+                assert lines[i - 1] == '__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");', (path.name, lines[i - 1])
+                assert lines[i + 1] == '__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");', (path.name, lines[i + 1])
+
+
 def test_product_path_calls_no_library_model_code():
     """No torch matrix products, attention, softmax or norms in the package:
     those are the hand-written kernels' job (the sampler's float64 top-p on the
