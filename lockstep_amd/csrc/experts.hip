@@ -619,7 +619,8 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const T* __restrict__
 // The same sums in the same order as the kernels above give with a cut of K: the same bits.
 //
 // A table that names the experts, and at most 64 pairs in the step: a workgroup then stands for an expert (and sixteen of its
-// rows), and each of its waves finds the rows by itself: lane l has pair l's expert, ballots give the expert's pairs and how many
+// rows), or for a pair where there are fewer of those, and works if that is the first of sixteen of its expert's
+// (`table_groups`).  Each of its waves finds the rows by itself: lane l has pair l's expert, ballots give the expert's pairs and how many
 // lie in front of them.  The launch that would put the pairs in order is saved.  The first product looks the experts up (a table's
 // rows come from HBM, which takes as long as that launch did) and leaves them for the second one.  Whole requests of the design that is
 // measured (28 layers, eight decode): 74.3 ms with the launch, 75.0 with an expert's blocks all on one XCD, 72.8 spread over the eight,
@@ -649,14 +650,16 @@ __device__ __forceinline__ FewRows few_rows(const int* __restrict__ at, const in
     return {tile[0], tile[1], rows, tile[0] < 0 ? 0 : more[tile[1] + min(l16, rows - 1)]};
   } else {
     // (workgroups go round the eight XCDs: an expert's column blocks shift from one to the next, or one XCD would have all of them)
-    const int at_x = ((int)blockIdx.x + (int)blockIdx.y) % (int)gridDim.x;
-    const int e = at_x % E, skip = 16 * (at_x / E), P = n_tokens * top;
+    const int at_x = ((int)blockIdx.x + (int)blockIdx.y) % (int)gridDim.x, P = n_tokens * top;
     int mine = 0x7fffffff;
     if (lane < P) mine = FROM == kTable ? more[(long)at[lane / top] * top + lane % top] : at[lane];
     if (FROM == kTable && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < P) picks[threadIdx.x] = mine;  // (its first wave)
+    const bool by_pair = (long)gridDim.x < (long)E * ((n_tokens + 15) / 16);  // table_groups
+    const int e = by_pair ? __builtin_amdgcn_readlane(mine, at_x) : at_x % E;
     const unsigned long long held = __ballot(mine == e);
+    const int skip = by_pair ? __popcll(held & ((1ull << at_x) - 1ull)) : 16 * (at_x / E);
     const int n = __popcll(held) - skip, first = __popcll(__ballot(mine < e)) + skip;
-    if (n <= 0) return {-1, 0, 0, 0};  // uniform
+    if (n <= 0 || skip % 16 != 0) return {-1, 0, 0, 0};  // uniform
     int* places = places_s[threadIdx.x >> 6];  // (the wave's own)
     if (mine == e) places[__popcll(held & ((1ull << lane) - 1ull))] = lane;
     // (other lanes read what this one wrote: the barrier orders instructions, the fences the memory between them)
@@ -739,7 +742,7 @@ __global__ __launch_bounds__(256, 4) void experts_few_gate_up_kernel(const int* 
   }
 }
 
-// COLS: tiles of 16 columns a workgroup.  Two where its waves have to find their rows and a weight has two bytes (8 tokens, 23 of 32
+// COLS: tiles of 16 columns a workgroup.  Two where its waves have to find their rows and a weight has two bytes (8 tokens, some 21 of 32
 // experts, 1,024 x 768 10.9 -> 10.4 us in the decode step); with a list one is the faster (both launches 26.9 / 28.1, float32 54 / 60).
 template <typename T, int U, int FROM, int COLS>
 __global__ __launch_bounds__(256, 4) void experts_few_down_kernel(const int* __restrict__ at, const T* __restrict__ w_down,
@@ -1238,10 +1241,25 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
   return check_launch("experts_apply");
 }
 
+// Workgroups along x that find their rows in a table: for every expert and sixteen tokens, or for every pair.  (For every expert
+// alone, one token of 4 of 32, 64, 256 and 512 experts, 1,024 x 768, both launches us: 16.1, 18.5, 27.6 and 42.9; now 11.2, 11.4, 11.4 and 11.3;
+// with a list, the launch that makes it included, 14.4, 17.0, 39.4 and 86.5.  Eight tokens of 32 experts are 32 either way: 27.7 for 29.5.)
+static int table_groups(int n_tokens, int E, int top) {
+  return (int)std::min<long>((long)n_tokens * top, (long)E * ((n_tokens + 15) / 16));
+}
+
 // Whether ls_experts_apply_table takes a step of these sizes.
 extern "C" int ls_experts_apply_table_ok(int dtype, int n_tokens, int E, int top, int K, int F, int N) {
   return n_tokens > 0 && (long)n_tokens * top <= kTablePairs && few_chunks(dtype, K) && few_chunks(dtype, F) && F % 16 == 0 && N % 16 == 0 &&
          F / 16 < 65536 && N / 16 < 65536 && (long)E * ((n_tokens + 15) / 16) <= 0x7fffffffL;
+}
+
+// ... and whether it is the faster route: where it has no more workgroups than a list has room for tiles.  Each of them looks its rows up before
+// it knows whether it has any (table / list, 1,024 x 768, us: 17 tokens 3 of 4, 8 workgroups for 7, 13.4 / 16.0; 3 of 64 51 for 54, 40.7 / 44.2;
+// 1 of 12 17 for 13, 20.2 / 19.6; 64 tokens 1 of 16 64 for 20, 31.2 / 24.6; 2,048 x 2,048 32 tokens 1 of 4 8 for 6, 38.2 / 30.5;
+// up to a ratio of 1 the table was ahead or level at every size tried, beyond it now one, now the other).
+extern "C" int ls_experts_apply_table_pays(int n_tokens, int E, int top) {
+  return n_tokens > 0 && table_groups(n_tokens, E, top) <= ls_experts_tile_capacity(n_tokens, E, top, 16);
 }
 
 // ls_experts_route_table and ls_experts_apply in two launches, for few pairs: token t uses the experts that row token_ids[t] of
@@ -1263,7 +1281,7 @@ extern "C" int ls_experts_apply_table(int dtype, const void* x, long ldx, const 
                  reinterpret_cast<uintptr_t>(w_down) % 16 == 0 && ldx % vec == 0 && ldy % vec == 0,
              "experts_apply_table: operands must be 16-byte aligned");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int groups = E * ((n_tokens + 15) / 16);
+  const int groups = table_groups(n_tokens, E, top);
 #define LS_TABLE_UP(T_, U_)                                                                                           \
   hipLaunchKernelGGL((experts_few_gate_up_kernel<T_, U_, kTable>), dim3(groups, F / 16), dim3(256), 0, s, token_ids,    \
                      (const T_*)w_gate, (const T_*)w_up, table, (const T_*)x, ldx, F, K, top, E, limit, alpha, shift, \

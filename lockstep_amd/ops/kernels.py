@@ -1308,6 +1308,11 @@ class Kernels:
             self.experts_lib().ls_experts_apply_table_ok(c_int(DTYPE_CODE[dtype]), c_int(tokens), c_int(experts), c_int(top), c_int(k),
                                                          c_int(f), c_int(n))))
 
+    def experts_apply_table_pays(self, tokens: int, experts: int, top: int) -> bool:
+        """Whether ``experts_apply_table`` is the faster route for that many tokens."""
+        return self._memo(("experts_apply_table_pays", tokens, experts, top), lambda: bool(
+            self.experts_lib().ls_experts_apply_table_pays(c_int(tokens), c_int(experts), c_int(top))))
+
     def experts_apply_table(self, x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                             token_ids: torch.Tensor, table: torch.Tensor, limit: float, alpha: float, act: torch.Tensor,
                             expert: torch.Tensor, partials: torch.Tensor, shift: float = 1.0) -> None:

@@ -153,7 +153,7 @@ class RoutedExperts(FeedForward):
         rt = ctx.rt
         k = rt.kernels
         t, e, top = ctx.n_tokens, self.routed, self.top
-        if self.tabled and self.shared is None and self.weigh == "output" and \
+        if self.tabled and self.shared is None and self.weigh == "output" and k.experts_apply_table_pays(t, e, top) and \
                 k.experts_apply_table_ok(rt.dtype, t, e, top, self.hidden, self.inter, self.hidden):   # a few tokens: no launch to put them in order
             partials = ctx.buf("experts.slices", (top * t, self.hidden), torch.float32).view(top, t, self.hidden)
             k.experts_apply_table(x, self.w_gate, self.w_up, self.w_down, ctx.token_ids, self.table, self.limit, self.alpha,

@@ -262,3 +262,17 @@ def test_plain_model_prefix_property_and_generation():
     assert torch.allclose(model.forward(tokens[:7]), whole[:7], atol=1e-10)
     new = model.generate_greedy(tokens[:5], 3)
     assert new[0] == int(torch.argmax(model.forward(tokens[:5])[-1])) and len(new) == 3
+
+
+def test_the_route_of_few_pairs_is_taken_where_it_has_no_more_workgroups_than_a_list():
+    """One workgroup an expert would be hundreds that look up and leave where a design has hundreds of experts: never more than pairs, and
+    the list is taken where even so there are more than it has tiles."""
+    import ctypes
+
+    from lockstep_amd.ops import build
+
+    lib = ctypes.CDLL(str(build.build_experts()))
+    for tokens, experts, top in ((1, 4, 4), (1, 32, 4), (8, 32, 4), (1, 512, 8), (16, 300, 4), (63, 64, 1), (33, 1, 1), (17, 3, 3)):
+        assert lib.ls_experts_apply_table_pays(tokens, experts, top), (tokens, experts, top)
+    for tokens, experts, top in ((17, 12, 1), (32, 4, 1), (64, 4, 1), (64, 16, 1), (21, 32, 3), (0, 4, 1)):
+        assert not lib.ls_experts_apply_table_pays(tokens, experts, top), (tokens, experts, top)

@@ -531,6 +531,32 @@ def test_few_pairs_that_a_table_names_without_a_launch_to_order_them(dtype, toke
     assert not torch.isnan(want).any() and torch.equal(got, want) and torch.equal(picked, chosen)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,experts,top,rows", [(1, 512, 4, 9), (7, 32, 4, 40), (33, 40, 1, 1), (63, 64, 1, 2), (16, 64, 4, 3), (21, 33, 3, 1),
+                                                     (16, 4, 4, 5)])
+def test_pairs_of_many_experts_that_a_table_names(dtype, tokens, experts, top, rows):
+    """Fewer pairs than experts and sixteens of tokens, so that a workgroup stands for a pair: one expert's rows in one, two, three and four
+    of them (a table of one row and of few), pairs in no order, one pair, as many workgroups by pairs as by experts."""
+    g = torch.Generator().manual_seed(tokens * top + experts)
+    k, width, ff = K(), 512, 512
+    ids = torch.randint(0, rows, (tokens,), generator=g).to(torch.int32).cuda()
+    table = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(rows)]).to(torch.int32).cuda()
+    x = torch.randn((tokens, width), generator=g).to(dtype).cuda()
+    w_gate, w_up, w_down = ((torch.randn((experts, *s), generator=g) * s[1] ** -0.5).to(dtype).cuda() for s in ((ff, width), (ff, width), (width, ff)))
+    cap = k.experts_tile_capacity(tokens, experts, top, 16)
+    i32 = lambda n: torch.empty(n, dtype=torch.int32, device="cuda")  # noqa: E731
+    chosen, order, tiles, counts = i32(tokens * top), i32(tokens * top), i32(4 * cap), i32(experts)
+    share = torch.empty(tokens * top, dtype=torch.float32, device="cuda")
+    k.experts_route_table(ids, table, experts, 16, chosen, share, order, tiles, counts)
+    act = torch.full((tokens * top, ff), float("nan"), dtype=dtype, device="cuda")
+    want, got = (torch.full((top, tokens, width), float("nan"), device="cuda") for _ in range(2))
+    k.experts_apply(x, w_gate, w_up, w_down, top, 16, order, tiles, share, 3.0, 1.5, act, want, shift=0.5)
+    act.fill_(float("nan"))
+    picked = torch.full_like(chosen, -1)
+    k.experts_apply_table(x, w_gate, w_up, w_down, ids, table, 3.0, 1.5, act, picked, got, shift=0.5)
+    assert not torch.isnan(want).any() and torch.equal(got, want) and torch.equal(picked, chosen)
+
+
 # ---------------------------------------------------------------------------
 # whole models
 # ---------------------------------------------------------------------------
