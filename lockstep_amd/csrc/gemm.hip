@@ -360,7 +360,7 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   constexpr int NT = (EPI == kSwiGLU) ? 2 : 1;  // weight tiles per column block
-  const int cols = NT == 2 ? 16 : block_cols;   // of a block: 16, 12 or 8
+  const int cols = NT == 2 ? 16 : block_cols;   // of a block: 16 or 12
   const Factors factors = load_factors<EPI>(act);
   constexpr int UC = 4;                          // chunks per unit
   constexpr int UQ = XC / UC;                    // units per tile
@@ -1178,6 +1178,17 @@ static int launch_ring(int tile, const T* X, const T* W, void* C, int M, int N, 
 #undef LS_RING
 }
 
+// Columns of the streaming kernel's blocks: 12 where the walks have no more rounds with those than with 16, else 16 (a round costs its
+// barrier, its fold and a fragment's instructions whatever its columns).  Weights from HBM, blocks of 16 / 12, us.  The same rounds, two or three:
+// 8 rows 4,608 x 4,096 16.0 / 14.4, 5,120 x 4,096 16.2 / 14.6, 6,144 x 4,096 16.7 / 15.2, 9,216 x 4,096 22.8 / 21.0, 1 row 6,144 x 4,096 15.3 / 13.9,
+// 6,144 x 5,120 23.5 / 22.7, 9,216 x 2,048 14.3 / 12.6, 16 rows 6,144 x 4,096 18.3 / 16.9, 40 rows 3,072 x 4,096 19.8 / 18.2, float32 1 row
+// 5,120 x 4,096 31.9 / 30.9.  A round more: 1 row 7,168 x 4,096 15.8 / 18.5, 10,240 21.8 / 24.0, 18,432 34.5 / 36.3, 151,936 232 / 272, 40 rows 5,056
+// 24.5 / 27.8.  Blocks of 8 never won (1 row 6,144 16.8, 14,336 36.0 for 28.0).  SwiGLU keeps its pairs of 16.
+static int stream_columns(int N, int walkers) {
+  auto rounds = [&](int cols) { return ((N + cols - 1) / cols + walkers - 1) / walkers; };
+  return rounds(12) <= rounds(16) ? 12 : 16;
+}
+
 template <typename T, int EPI>
 int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long ldx, long ldc, const float* norm_w,
                 float eps, int out_cols, hipStream_t stream, const float* act = nullptr) {
@@ -1217,19 +1228,8 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   if (!norm_w && mt_rows <= 4 && !tiles && xc % 4 == 0 && xc * group_tiles <= 16 && nslices >= 8 && nslices <= 16 &&
       col_blocks * row_groups > stream_wgs && stream_lds <= 128 * 1024 && LS_GEMM_STREAM) {
     int walkers = stream_wgs / row_groups;
-    // Blocks of 16 columns, or of 12 or 8 where a walker has fewer columns with those: the one with the most decides
-    // (8 rows, weights from HBM, blocks of 16 / of these, us: 4,608 x 4,096 15.9 / 14.2, 5,120 x 4,096 16.1 / 14.4, 6,144 x 4,096 16.4 / 15.0,
-    // 7,168 x 4,096 17.9 / 16.9, 9,216 x 4,096 22.2 / 20.4, 4,608 x 3,584 14.2 / 12.8; 1 row 6,144 x 4,096 15.0 / 13.8, 16 rows 18.1 / 16.8).
-    int cols = 16, blocks = col_blocks;
-    if (EPI != kSwiGLU) {
-      for (int c : {12, 8}) {
-        const int n = (N + c - 1) / c;
-        if ((n + walkers - 1) / walkers * c < (blocks + walkers - 1) / walkers * cols) {
-          cols = c;
-          blocks = n;
-        }
-      }
-    }
+    const int cols = NT == 2 ? 16 : stream_columns(N, walkers);
+    const int blocks = NT == 2 ? col_blocks : (N + cols - 1) / cols;
     const int rounds = (blocks + walkers - 1) / walkers;
     walkers = (blocks + rounds - 1) / rounds;
     if (row_groups > 1) walkers = (walkers + 7) / 8 * 8;  // whole rounds of the XCDs, see the kernel
@@ -1337,6 +1337,9 @@ extern "C" int ls_gemm_ring_tile(int dtype, int epilogue, int M, int N, int K) {
   return epilogue == kSwiGLU ? LS_TILE(bf16_t, kSwiGLU) : LS_TILE(bf16_t, kStore);
 #undef LS_TILE
 }
+
+// Columns of a block of the streaming kernel for N columns and that many walkers (workgroups of a group of rows).
+extern "C" int ls_gemm_stream_columns(int N, int walkers) { return ls::stream_columns(N, walkers); }
 
 // Number of K slices of a product over K (the first dimension of the partial sums of ls_gemm_slices).
 extern "C" int ls_gemm_slices_count(int K) {

@@ -58,6 +58,27 @@ def test_gemm_matches_linear(dtype, m, n, k):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k,n", [(4096, 4608), (4096, 4613), (4096, 6144), (4096, 6148), (2560, 9210), (2048, 8200), (3584, 2571)])
+def test_products_of_few_rows_by_blocks_of_twelve_columns(dtype, k, n):
+    """Walks over blocks of 12 columns and, one column block more, of 16 (columns that end inside a block and off a vector, a last round of few
+    walkers, one and two groups of rows), against the same rows among 300, which other kernels take: the same bits."""
+    from lockstep_amd.ops import ADD_F32, STORE, STORE_F32
+
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(300, k, generator=g).to(dtype).cuda()
+    w = torch.randn(n, k, generator=g).to(dtype).cuda()
+    start = torch.randn(300, n, generator=g).cuda()
+    for epilogue, kind in ((STORE, dtype), (STORE_F32, torch.float32), (ADD_F32, torch.float32)):
+        full = start.to(kind, copy=True)
+        K().gemm(x, w, full, epilogue)
+        for rows in (1, 7, 16, 24, 31, 40, 55):
+            part = torch.full((rows + 1, n), 3.0, dtype=kind, device="cuda")
+            part[:rows] = start[:rows]
+            K().gemm(x[:rows], w, part[:rows], epilogue)
+            assert torch.equal(part[:rows], full[:rows]) and (part[rows] == 3.0).all(), (epilogue, rows)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_row_does_not_depend_on_the_batch(dtype):
     """Row i alone, in a 16-row batch, in a 64-row batch and in a 300-row batch:
     same bits (the kernels of few and of many rows share one summation order)."""

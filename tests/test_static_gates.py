@@ -66,6 +66,21 @@ def test_engine_does_not_import_tests_or_working_files():
         assert not re.search(r"^\s*(from|import)\s+(tests|plain)\b", code, flags=re.M), path
 
 
+def test_narrow_column_blocks_cost_the_streaming_products_no_round():
+    """A round of a walk costs its barrier and its fold however narrow its block is: blocks of 12 columns only where the walks
+    have no more rounds with them (the heads of 151,936 columns and the widths of three rounds and more do)."""
+    import ctypes
+
+    from lockstep_amd.ops import build
+
+    columns = ctypes.CDLL(str(build.build_core())).ls_gemm_stream_columns
+    for walkers in (128, 256, 512):
+        for n in [*range(1, 20 * walkers, 7), 10240, 14336, 22016, 32000, 151936]:
+            rounds = {c: -(-(-(-n // c)) // walkers) for c in (12, 16)}
+            assert columns(n, walkers) == (12 if rounds[12] == rounds[16] else 16), (n, walkers)
+    assert [columns(n, 256) for n in (4608, 6144, 7168, 9216, 10240, 14336, 22016, 151936)] == [12, 12, 16, 12, 16, 16, 16, 16]
+
+
 def test_the_products_tile_numbering_refuses_a_band_of_no_rows():
     """A tuning macro of 0 would be a division by zero in device code."""
     import shutil
