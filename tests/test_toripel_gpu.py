@@ -23,7 +23,7 @@ import torch
 
 from helpers import feed, make_mixed_trace, max_live_tokens, random_tokens, rel_err, replay_in_process
 from plain import toripel_plain as plain
-from toripel_cases import CASES, SINGLE, bare, config, delta, latent, make_tensors, windowed, write_model
+from toripel_cases import CASES, SINGLE, bare, config, delta, latent, make_tensors, tabled, windowed, write_model
 
 pytestmark = pytest.mark.gpu
 ROOT = Path(__file__).resolve().parent.parent
@@ -634,6 +634,52 @@ def test_mixed_batches_of_unequal_requests_with_pages_and_slots_used_again(model
     assert cache.free_slots == 4 and all(g.pool.taken_total > g.pool.num_pages for g in cache.groups)
     for rid, toks in requests.items():
         assert rel_err(got[rid], oracle.forward(toks)) < TOL[dtype], rid
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_model_whose_few_pairs_find_their_experts_themselves(tmp_path, monkeypatch, dtype):
+    """A model wide enough for ``experts_apply_table``: a prompt in portions on both sides of the rule, a mixed batch, and two requests
+    through replayed graphs, against the plain model, and with the same bits as the engine that puts the pairs in order first."""
+    from lockstep_amd import load_model
+    from lockstep_amd.engine.batch import StepEntry
+
+    raw = config(512, 96, [tabled(windowed(4, 2, 32, 16, window=21, scale=0.5), 512, experts=6, top=2),
+                           tabled(delta(2, 1, 32, 24, taps=3), 768, experts=40, top=3)], streams=2)
+    tensors = make_tensors(raw, seed=31)
+    folder, oracle = write_model(tmp_path / "m", raw, tensors), plain.PlainToripel(raw, tensors)
+    kernels, calls = type(K()), []
+    apply_table = kernels.experts_apply_table
+    monkeypatch.setattr(kernels, "experts_apply_table", lambda self, x, *rest, **named: (calls.append(x.shape[0]), apply_table(self, x, *rest, **named))[1])
+    prompt = random_tokens(140, raw["vocab"], seed=6)
+    requests = {f"r{i}": random_tokens(n, raw["vocab"], seed=50 + i) for i, n in enumerate([1, 23, 61, 2, 40])}
+    steps = make_mixed_trace(requests, seed=4, max_live=4, decode_tail=8, max_portion=19)
+    pair = random_tokens(90, raw["vocab"], seed=8), random_tokens(80, raw["vocab"], seed=9)
+    runs = {}
+    for listed in (False, True):
+        if listed:
+            monkeypatch.setattr(kernels, "experts_apply_table_pays", lambda self, tokens, experts, top: False)
+        model = load_model(folder, dtype=dtype)
+        cache = new_cache(model, 8, tokens=512)
+        got = [feed(model, cache, "r", prompt, [1, 3, 16, 17, 21, 22, 5, 32, 1, 8])]
+        cache.close("r")
+        out = replay_in_process(model, cache, steps)
+        got += [out[rid] for rid in requests]
+        cache.open("a"), cache.open("b")
+        model.step(cache, [StepEntry("a", pair[0][:30], []), StepEntry("b", pair[1][:20], [])])
+        replays, rows = model.graph_replays, []
+        for t in range(60):
+            rows.append(model.step(cache, [StepEntry("a", [pair[0][30 + t]], [0]), StepEntry("b", [pair[1][20 + t]], [0])]).cpu())
+        assert model.graph_replays - replays >= 40
+        got += [torch.stack([r[i] for r in rows]) for i in range(2)]
+        runs[listed] = [torch.as_tensor(g).cpu() for g in got]
+        if not listed:
+            assert {1, 2, 3, 8, 16} <= set(calls) and max(calls) <= 32, sorted(set(calls))
+            taken = len(calls)
+        assert len(calls) == taken
+    want = [oracle.forward(prompt), *(oracle.forward(toks) for toks in requests.values()), oracle.forward(pair[0])[30:], oracle.forward(pair[1])[20:]]
+    for i, (mine, other, plain_rows) in enumerate(zip(runs[False], runs[True], want)):
+        assert torch.equal(mine, other), i
+        assert rel_err(mine, plain_rows) < TOL[dtype], i
 
 
 # ---------------------------------------------------------------------------
