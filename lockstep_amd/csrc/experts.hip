@@ -805,7 +805,9 @@ __global__ __launch_bounds__(256, 4) void experts_few_down_kernel(const int* __r
   }
 }
 
-// Chunks that a wave of those kernels asks for at a time where K is a whole number of such rounds, else 0.
+// Chunks that a wave of those kernels asks for at a time where K is a whole number of such rounds, else 0.  (Rounds of eight, six and four, for
+// both products of an expert: what was built and measured, ahead at widths of 512 to 8,192.  Widths that only other rounds divide, 640, 896, 1,280 or
+// 1,408 say, keep the kernels for any size in both, and the launch that orders the pairs: other rounds were not tried, nor one product by each.)
 static int few_chunks(int dtype, int K) {
   const int quarter = 4 * (dtype == kF32 ? Atom<float>::KCHUNK : Atom<bf16_t>::KCHUNK);
   if (K % quarter != 0) return 0;
