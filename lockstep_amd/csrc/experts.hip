@@ -859,9 +859,9 @@ struct RingProduct {
     const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) void*)ring + wave * 1024;
     const int stages = (K + BK - 1) / BK;
     auto request = [&](int st, int buf) LS_INLINED {
-      buffer_to_lds16(x_off, st * 128, x, lds0 + S * W_BYTES + buf * X_BYTES);
-      buffer_to_lds16(w_off, st * 128, w0, lds0 + buf * W_BYTES);
-      if constexpr (TI == 2) buffer_to_lds16(w_off, st * 128, w1, lds0 + buf * W_BYTES + 64 * 128);
+      buffer_to_lds16(x_off + st * 128, x, lds0 + S * W_BYTES + buf * X_BYTES);
+      buffer_to_lds16(w_off + st * 128, w0, lds0 + buf * W_BYTES);
+      if constexpr (TI == 2) buffer_to_lds16(w_off + st * 128, w1, lds0 + buf * W_BYTES + 64 * 128);
     };
     auto clear_past_k = [&](int buf) LS_INLINED {
       const int first = (K % BK) / Atom<T>::VEC;  // the first piece of a row that lies past K

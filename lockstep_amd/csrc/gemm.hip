@@ -1046,7 +1046,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ X
 // workgroup on every CU and with as many as it holds (bfloat16, K = 4,096, weights from HBM).  The larger the tile, the
 // fewer operand bytes a product loads; the smaller, the more CUs have one, and the fuller the last round.
 enum RingTile { kRing256x192, kRing256x128, kRing192x192, kRing128x192, kRing192x128, kRing128x128, kRing128x64, kRing64x128,
-                kRing64x64, kRingTiles, kRing64x32 = kRingTiles };
+                kRing64x64, kRingTiles, kRing64x32 = kRingTiles, kRing32x64, kRing32x32 };
 struct RingShape {
   int rows, cols, a_cu;
   float one, full;
@@ -1117,16 +1117,53 @@ static bool ring_takes(int M, int N, int K) {
   return blocks >= 32 && M >= (GATED ? 48 : 56);
 }
 
+// The narrow tiles: 32 rows by 32 or by 64 columns where those are so few that a wider tile would leave CUs idle, or few
+// rows over many columns; -1 where the table's tiles or the other kernels serve as well.  Every workgroup loads 32 rows of both
+// operands or 96 a stage in place of 128, and the 32 x 32 tile's stages are of 256 bytes, so that a barrier and an LDS latency
+// stand every 128 elements of K.  Against what ran before them (64 x 64 tiles, the streaming kernel, a wave a slice), weights
+// from HBM, us:
+//   one round of 32 x 32    8 x 6,144 x 4,096 15.6 / 11.9, SwiGLU 8 x 6,144 x 1,024 6.6 / 5.6, 1 x 6,144 x 1,024 6.3 / 5.4, 64 x 4,096 x 1,024
+//                           7.5 / 5.1, 64 x 4,096 x 4,096 22 / 13, 97 x 1,024 x 2,048 11.9 / 6.8, 200 x 1,024 x 4,096 20 / 11
+//   one round of 32 x 64    8 x 10,240 x 5,120 26.4 / 23.8, SwiGLU 1 x 14,336 x 1,024 9.6 / 7.8, 64 x 6,144 x 4,096 23 / 18.5, 97 x 4,096
+//                           x 1,024 7.6 / 5.9; 32 x 32 tiles, two a CU, 6.5 for the last
+//   up to three rounds and 32 rows  SwiGLU 8 x 24,576 x 4,096 41.8 / 36.2 in 32 x 32 (64 x 64 as they are now 39); below 2,048 of K 32 x 64
+//                           are ahead up to 512 (8 x 24,576 x 512 9.8 / 7.8); 18,432 columns, a round and an eighth, gain nothing
+// Up to 16 rows of a plain product a wave a slice and 16 columns keeps the lead while those blocks fit one round (8 x 4,096 x 1,024
+// 4.7 / 4.8, 1 x 1,024 x 4,096 7.3 / 10.3), beyond 320 of K (1 x 4,096 x 256 3.4 / 3.3).  And four rounds of 32,768 columns ask
+// for 128 rows of weights a multiple of 4 KB apart together (8 x 32,768 x 4,096 54.8 / 69.9): they keep the table's tiles.
+// float32 multiplies longer than it loads, so every CU that has a tile counts, up to six rounds (64 x 4,096 x 1,024 17.6 / 10.2, 8 x
+// 24,576 x 1,024 29.3 / 24.0, 33 x 24,576 x 1,024 40 / 35, 128 x 10,240 x 4,096 145 / 105; 2,000 x 1,024 x 1,024, eight rounds, 40.4 / 42.3); up to 64
+// rows over columns that 64 x 32 tiles cover in one round keep those.  A wave a slice stays ahead where a tile's one chain of
+// products is the longer way: up to 24 rows of few columns (17 x 2,048 x 2,048 14.9 / 16.4, 17 x 4,096 x 512 7.0 / 6.0), one to four of long K (1 x
+// 6,144 x 4,096 29.7 / 31.7, 8 rows 35.5 / 32.5), SwiGLU of few rows and columns (1 x 2,048 x 1,024 9.2 / 10.0, 1 x 6,144 x 1,024 11.2 / 10.4).
+template <typename T, int EPI>
+static int narrow_tile(int M, int N, int K) {
+  const long cus = compute_units();
+  const long rows = (M + 31) / 32, small = rows * ((N + 31) / 32), wide = rows * ((N + 63) / 64);
+  if (sizeof(T) == 4) {
+    if (EPI != kSwiGLU && (N + 15) / 16 <= cus && M <= (K <= 512 ? 16 : K <= 1024 || N > 512 ? 24 : 32)) return -1;
+    if (EPI != kSwiGLU && M <= 4 && K > 2048 && (N + 31) / 32 <= cus) return -1;
+    if (M <= 16 && (K < 256 || (EPI == kSwiGLU && (N + 31) / 32 <= (K > 1024 ? cus : cus / 2)))) return -1;
+    return small <= cus || (small <= 6 * cus && (EPI == kSwiGLU || M > 64 || (N + 31) / 32 > cus)) ? kRing32x32 : -1;
+  }
+  if (M <= 16 && EPI != kSwiGLU && (N + 15) / 16 <= cus && K > 320) return -1;
+  if (small <= cus) return kRing32x32;
+  if (wide <= cus) return kRing32x64;
+  if (M > 32) return -1;
+  if (K >= 2048) return small <= 3 * cus ? kRing32x32 : -1;
+  return K <= 512 && 2 * wide >= 3 * cus && wide <= 2 * cus ? kRing32x64 : -1;
+}
+
 // Whether the ring kernel's 32-bit byte offsets inside a tile reach every operand: the rows of the largest tile, and what
 // the last stage reads behind the last row.  (Rows further apart go to the other kernels, which form 64-bit addresses.)
 static bool ring_reaches(long ldx, long K, long size) { return (256 * std::max(ldx, K) + 128) * size <= 0xffffffffL; }
 
 // Dynamic LDS beyond 64 KB has to be granted per kernel (once).
-template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS>
+template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS, int SUB>
 static bool ring_lds_ready(int bytes) {
   static const bool granted = [bytes] {
     if (bytes <= 64 * 1024) return true;
-    const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS>),
+    const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS, SUB>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
     if (!ok) (void)hipGetLastError();
     return ok;
@@ -1138,14 +1175,13 @@ constexpr int kNotLaunched = 1;  // the LDS was refused: the caller has another 
 constexpr int kMutantNoRing = 16;  // bit of the controls' mask (common.h): that refusal, as a test wants it
 
 // groups: workgroups along K (kSliceSums: out_cols slices each); otherwise 1.
-template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS>
+template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS, int SUB = 1>
 static int launch_ring_tile(const T* X, const T* W, void* C, int M, int N, int K, long ldx, long ldc, int kslice, int vec_ok,
                             int out_cols, int groups, const float* act, hipStream_t stream) {
-  constexpr int kBytes = (WS * BN + XS * BM) * 128;
-  static_assert(kBytes <= 160 * 1024, "the rings fit the LDS of a CU");
-  if (LS_MUTANT_HOST(kMutantNoRing) || !ring_lds_ready<T, EPI, BM, BN, NWM, NWN, WS, XS>(kBytes)) return kNotLaunched;
+  constexpr int kBytes = (WS * BN + XS * BM) * SUB * 128;
+  if (LS_MUTANT_HOST(kMutantNoRing) || !ring_lds_ready<T, EPI, BM, BN, NWM, NWN, WS, XS, SUB>(kBytes)) return kNotLaunched;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  hipLaunchKernelGGL((gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS>), dim3(tiles_m * tiles_n, groups),
+  hipLaunchKernelGGL((gemm_ring_kernel<T, EPI, BM, BN, NWM, NWN, WS, XS, SUB>), dim3(tiles_m * tiles_n, groups),
                      dim3(64 * NWM * NWN), kBytes, stream, X, W, C, M, N, K, ldx, ldc, kslice, vec_ok, tiles_m, tiles_n,
                      out_cols, act);
   return check_launch("gemm");
@@ -1159,8 +1195,11 @@ static int launch_ring(int tile, const T* X, const T* W, void* C, int M, int N, 
   if constexpr (sizeof(T) == 4) {
     if constexpr (EPI != kSwiGLU && EPI != kSliceSums)
       if (tile == kRing64x32) LS_RING(64, 32, 2, 2, 5, 5);
+    if constexpr (EPI != kSliceSums)
+      if (tile == kRing32x32) LS_RING(32, 32, 2, 2, 5, 5);
     LS_RING(64, 64, 2, 2, 3, 3);
   } else if constexpr (EPI == kSliceSums) {
+    if (tile == kRing32x64) LS_RING(32, 64, 2, 2, 5, 5);
     LS_RING(64, 64, 4, 2, 5, 5);
   } else {
     switch (tile) {
@@ -1172,6 +1211,8 @@ static int launch_ring(int tile, const T* X, const T* W, void* C, int M, int N, 
       case kRing128x128: LS_RING(128, 128, 4, 2, 4, 4);
       case kRing128x64: LS_RING(128, 64, 4, 2, 5, 5);
       case kRing64x128: LS_RING(64, 128, 2, 4, 3, 3);
+      case kRing32x64: LS_RING(32, 64, 2, 2, 5, 5);
+      case kRing32x32: LS_RING(32, 32, 2, 2, 5, 5, 2);
       default: LS_RING(64, 64, 4, 2, 5, 5);
     }
   }
@@ -1206,9 +1247,10 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   const int mt_rows = (M + 15) / 16;
   const int col_blocks = (N + 16 * NT - 1) / (16 * NT);
   bool ring = aligned && ring_reaches(ldx, K, sizeof(T));
-  if (!norm_w && ring && ring_takes<T, EPI>(M, N, K)) {
-    const int rc = launch_ring<T, EPI>(ring_tile<T, EPI>(M, N, K), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice,
-                                       vec_ok, out_cols, 1, act, stream);
+  const int narrow = !norm_w && ring ? narrow_tile<T, EPI>(M, N, K) : -1;
+  if (!norm_w && ring && (narrow >= 0 || ring_takes<T, EPI>(M, N, K))) {
+    const int rc = launch_ring<T, EPI>(narrow >= 0 ? narrow : ring_tile<T, EPI>(M, N, K), reinterpret_cast<const T*>(X), w, C, M,
+                                       N, K, ldx, ldc, kslice, vec_ok, out_cols, 1, act, stream);
     if (rc != kNotLaunched) return rc;
     ring = false;
   }
@@ -1329,13 +1371,23 @@ extern "C" int ls_gemm_xielu(int dtype, const void* X, const void* W, void* C, i
 
 extern "C" int ls_gemm_kslice(int K) { return ls::kslice_for(K); }
 
-// The tile (enum RingTile) that ls_gemm gives the ring kernel for a product of aligned operands; -1: another kernel's.
+// The tile (enum RingTile) that the table gives the ring kernel for a product of aligned operands; -1: another kernel's.  A narrow
+// tile (ls_gemm_narrow_tile) goes before it.
 extern "C" int ls_gemm_ring_tile(int dtype, int epilogue, int M, int N, int K) {
   using namespace ls;
 #define LS_TILE(T_, EPI_) (ring_takes<T_, EPI_>(M, N, K) ? ring_tile<T_, EPI_>(M, N, K) : -1)
   if (dtype == kF32) return epilogue == kSwiGLU ? LS_TILE(float, kSwiGLU) : LS_TILE(float, kStore);
   return epilogue == kSwiGLU ? LS_TILE(bf16_t, kSwiGLU) : LS_TILE(bf16_t, kStore);
 #undef LS_TILE
+}
+
+// The rows times columns of the narrow tile that ls_gemm gives a product of aligned operands; 0: none.
+extern "C" int ls_gemm_narrow_tile(int dtype, int epilogue, int M, int N, int K) {
+  using namespace ls;
+#define LS_TILE(T_) (epilogue == kSwiGLU ? narrow_tile<T_, kSwiGLU>(M, N, K) : narrow_tile<T_, kStore>(M, N, K))
+  const int tile = dtype == kF32 ? LS_TILE(float) : LS_TILE(bf16_t);
+#undef LS_TILE
+  return tile == kRing32x32 ? 32 * 32 : tile == kRing32x64 ? 32 * 64 : 0;
 }
 
 // Columns of a block of the streaming kernel for N columns and that many walkers (workgroups of a group of rows).
@@ -1354,6 +1406,54 @@ extern "C" int ls_gemm_slices_max_rows(int dtype, int K) {
   const int xc = ls::kslice_for(K) / (dtype == ls::kF32 ? 16 : 32);
   return (LS_GEMM_STREAM && (xc == 8 || xc == 16)) ? 256 : 64;
 }
+
+namespace ls {
+
+// Rows from which the slice sums of a product come from the ring kernel.
+static int slices_ring_from(int dtype, int N, int K) {
+  if (dtype == kF32) return 33;
+  return (long)N * K * 2 >= (32L << 20) ? 4 : 17;
+}
+
+// The ring kernel's tile for slice sums and the slices a workgroup takes; per 0: another kernel.
+struct SlicesPlan {
+  int tile, per;
+};
+// bfloat16: the cheaper of 32 x 64 and 64 x 64 tiles with one, two or four slices a workgroup, a stage 0.18 and 0.25 us where a CU has one
+// workgroup, twice that where it has two, and a round about four stages besides.  Before (64 x 64, every CU a workgroup or another
+// kernel) / now, us: 8 x 4,096 x 4,096 10.9 / 8.4, 8 x 4,096 x 12,288 24.0 / 21.8, 17 x 1,024 x 3,072 4.3 / 4.0, 64 x 1,024 x 2,048 5.4 / 4.2, 64 x 1,024 x
+// 3,072 6.7 / 5.0, 64 x 4,096 x 4,096 13.3 / 12.8, 97 x 1,024 x 2,048 5.2 / 5.0.  One row 5,120 x 8,192 19.4 / 20.8, hence four rows at least; 17 to
+// 32 rows of less than five slices over few columns 3.8 / 4.0.  From 65 rows on longer runs of stages lose what fewer rounds gain (128 x 5,120 x
+// 5,120 with one, two and four slices a workgroup 28, 30, 31).
+static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
+  const int kslice = kslice_for(K), nslices = (K + kslice - 1) / kslice;
+  const long cus = compute_units();
+  if (dtype == kF32) {  // sixteen stages a workgroup where every CU gets two (33 x 4,096 x 4,096 in eight 28, in sixteen 23), eight where it gets one
+    const int a_slice = kslice / 32;
+    int per = std::min(nslices, std::max(1, (16 + a_slice - 1) / a_slice));
+    auto workgroups = [&](int p) LS_INLINED { return (long)((M + 63) / 64) * ((N + 63) / 64) * ((nslices + p - 1) / p); };
+    while (per > 1 && workgroups(per) < (per * a_slice > 8 ? 2 * cus : cus)) per = (per + 1) / 2;
+    return workgroups(per) >= cus ? SlicesPlan{kRing64x64, per} : SlicesPlan{kRing64x64, 0};
+  }
+  if (M <= 32 && nslices < 5) return {kRing32x64, 0};
+  SlicesPlan best{kRing64x64, 0};
+  float least = 0.f;
+  for (int rows = 32; rows <= 64; rows += 32)
+    for (int per = M > 64 ? std::max(1, 512 / kslice) : 4; per >= 1; per /= 2) {
+      const long groups = (nslices + per - 1) / per, all = (long)((M + rows - 1) / rows) * ((N + 63) / 64) * groups;
+      if (M > 64 && per > 1 && all < cus) continue;
+      const float stages = (float)std::min(per, nslices) * (kslice / 64), one = rows == 32 ? 0.18f : 0.25f;
+      const long rest = all % (2 * cus), twos = all / (2 * cus) + (rest > cus);
+      const float time = (float)twos * (1.6f + 2.f * one * stages) + (rest > 0 && rest <= cus ? 1.f + one * stages : 0.f);
+      if (best.per == 0 || time < least) {
+        least = time;
+        best = {rows == 32 ? kRing32x64 : kRing64x64, per};
+      }
+    }
+  return best;
+}
+
+}  // namespace ls
 
 // Slice sums of X [M,K] @ W [N,K]^T for M <= ls_gemm_slices_max_rows: P [slices][M][N] float, P[s] = the
 // sum over K slice s.  The product is P[0] + P[1] + ... added in this order, starting from +0.
@@ -1390,32 +1490,19 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
   int rounds =
       (int)std::min<long>(4, (long)col_blocks * groups * std::max(row_groups, 1) / (2L * compute_units()));
   if (mt > 4 && rounds < 1) rounds = 1;  // more than 64 rows: this kernel only, if with one column block a workgroup
-  // Enough rows over weights large enough that 64 x 64 tiles times groups of slices give every CU a
-  // workgroup: the ring kernel, which has four stages of both operands in flight (measured against tiles staged
-  // through registers: 17 x 4,096 x 4,096 11.1 -> 9.0 us, 64 x 4,096 x 12,288 29.9 -> 26.4, 256 x 1,024 x 2,048 8.3 ->
-  // 6.5; those were ahead of the wide kernel by a third).  A workgroup takes as many slices as give it eight stages, fewer
-  // where that leaves CUs without one.
-  // From 17 rows on in bfloat16 (from 8 over weights of 64 MB and more, where the kernels of a wave a slice
-  // fall to 3.7 TB/s; below that and over smaller weights those are ahead), from 33 rows on in float32.
-  const long weight_bytes = (long)N * K * (dtype == kF32 ? 4 : 2);
-  const int tiled_from = dtype == kF32 ? 33 : (weight_bytes >= (64L << 20) ? 8 : 17);
-  if (LS_GEMM_SLICES_TILED && aligned && ring_reaches(ldx, K, dtype == kF32 ? 4 : 2) && M >= tiled_from && N % 4 == 0) {
-    const int stages_a_slice = kslice / (128 / (dtype == kF32 ? 4 : 2));
-    int per = std::min(nslices, std::max(1, (8 + stages_a_slice - 1) / stages_a_slice));
-    const int tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64;
-    auto workgroups = [&](int p) LS_INLINED { return (long)tiles_m * tiles_n * ((nslices + p - 1) / p); };
-    while (per > 1 && workgroups(per) < compute_units()) per = (per + 1) / 2;
-    if (workgroups(per) >= compute_units()) {
-      const int groups_y = (nslices + per - 1) / per;
-      int rc;
-      if (dtype == kF32)
-        rc = launch_ring<float, kSliceSums>(kRing64x64, (const float*)X, (const float*)W, P, M, N, K, ldx, N, kslice, 1, per,
-                                            groups_y, nullptr, s);
-      else if (dtype == kBF16)
-        rc = launch_ring<bf16_t, kSliceSums>(kRing64x64, (const bf16_t*)X, (const bf16_t*)W, P, M, N, K, ldx, N, kslice, 1,
-                                             per, groups_y, nullptr, s);
-      else
-        return fail("gemm_slices: unknown dtype %d", dtype);
+  // The ring kernel (float32: where its 64 x 64 tiles times groups of slices give every CU a workgroup), with four stages of
+  // both operands in flight: from 17 rows on (from 4 over weights of 32 MB and more, where the kernels of a wave a slice fall
+  // to 3.7 TB/s), from 33 rows on in float32.  bfloat16 takes the tile and the slices a workgroup that slices_plan finds cheapest.
+  const int ring_from = slices_ring_from(dtype, N, K);
+  if (LS_GEMM_SLICES_TILED && aligned && ring_reaches(ldx, K, dtype == kF32 ? 4 : 2) && M >= ring_from && N % 4 == 0 &&
+      (dtype == kF32 || dtype == kBF16)) {
+    const SlicesPlan plan = slices_plan(dtype, M, N, K);
+    if (plan.per > 0) {
+      const int groups_y = (nslices + plan.per - 1) / plan.per;
+      const int rc = dtype == kF32 ? launch_ring<float, kSliceSums>(plan.tile, (const float*)X, (const float*)W, P, M, N, K, ldx, N,
+                                                                    kslice, 1, plan.per, groups_y, nullptr, s)
+                                   : launch_ring<bf16_t, kSliceSums>(plan.tile, (const bf16_t*)X, (const bf16_t*)W, P, M, N, K, ldx,
+                                                                     N, kslice, 1, plan.per, groups_y, nullptr, s);
       if (rc != kNotLaunched) return rc;
     }
   }
@@ -1479,16 +1566,16 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
 
 // Whether ls_gemm_slices_folded takes this product: at most 16 rows, whole heads of a size that is a
 // multiple of four, K a multiple of the load width, at most 32 splits, the folded rows of a slice within
-// 64 KB of LDS -- and the plain slice kernel is what ls_gemm_slices itself would run for these sizes (over
-// large weights it prefers the ring kernel from eight rows on, which reads its operand from memory).
+// 64 KB of LDS -- and not so many rows over large weights (eight over 64 MB) that a fold of its own and the ring kernel's
+// slice sums are ahead.
 extern "C" int ls_gemm_slices_folded_ok(int dtype, int M, int N, int K, int head_dim, int splits) {
   using namespace ls;
   if (dtype != kF32 && dtype != kBF16) return 0;
   if (M < 1 || M > 16 || N < 1 || K < 1 || head_dim < 4 || head_dim % 4 || K % head_dim) return 0;
   if (splits < 1 || splits > 32 || K % (dtype == kF32 ? 4 : 8)) return 0;
   const long weight_bytes = (long)N * K * (dtype == kF32 ? 4 : 2);
-  const int tiled_from = dtype == kF32 ? 33 : (weight_bytes >= (64L << 20) ? 8 : 17);
-  if (LS_GEMM_SLICES_TILED && M >= tiled_from && N % 4 == 0) return 0;
+  const int ring_better_from = dtype == kF32 ? 33 : (weight_bytes >= (64L << 20) ? 8 : 17);
+  if (LS_GEMM_SLICES_TILED && M >= ring_better_from && N % 4 == 0) return 0;
   const size_t element = dtype == kF32 ? 4 : 2;
   return (size_t)M * (kslice_for(K) + 16 / element) * element <= 64 * 1024;
 }

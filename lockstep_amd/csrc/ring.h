@@ -23,14 +23,15 @@ __device__ __forceinline__ u32x4_t buffer_of(const void* p, long bytes) {
 // (Naming m0 keeps the compiler from relying on a value of its own there; that it warns of the name is all the diagnostic says.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-// Sixteen bytes a lane from buffer + lane_off + off straight into LDS: the wave's 64 pieces land at lds_base + 16 *
+// Sixteen bytes a lane from buffer + at straight into LDS: the wave's 64 pieces land at lds_base + 16 *
 // lane.  The instruction itself, because the compiler would wait for the compiler's own form of it in front of every
 // later LDS read.  The whole offset goes through the vector register: the buffer's bound counts that one for certain.
-__device__ __forceinline__ void buffer_to_lds16(unsigned lane_off, unsigned off, u32x4_t buffer, unsigned lds_base) {
-  unsigned at;
-  __asm__ volatile("v_add_u32 %0, %2, %1\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %3, 0 offen lds"
-                   : "=&v"(at)
-                   : "v"(lane_off), "s"(off), "s"(buffer), "s"(lds_base)
+// The descriptor may come from vector instructions (v_readfirstlane): the s_mov and the s_nop are the five wait states that
+// a memory instruction needs behind those (see load_to_lds16_from).
+__device__ __forceinline__ void buffer_to_lds16(unsigned at, u32x4_t buffer, unsigned lds_base) {
+  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                   :
+                   : "v"(at), "s"(buffer), "s"(lds_base)
                    : "memory", "m0");
 }
 // One 16-byte piece per lane from global memory straight into LDS: the wave's 64 pieces land at

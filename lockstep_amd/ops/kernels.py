@@ -265,9 +265,14 @@ class Kernels:
             c_long(out.stride(0)), _ptr(act), _stream()))
 
     def gemm_ring_tile(self, dtype: torch.dtype, epilogue: int, m: int, n: int, k: int) -> int:
-        """Which tile of the ring kernel a product of these sizes (and of 16-byte aligned operands) takes: its place in
-        ``RingTile`` of gemm.hip, -1 where another kernel computes it."""
+        """Which tile of the ring kernel's table a product of these sizes (and of 16-byte aligned operands) takes, unless a
+        narrow tile is better: its place in ``RingTile`` of gemm.hip, -1 where another kernel computes it."""
         return int(self.core.ls_gemm_ring_tile(c_int(DTYPE_CODE[dtype]), c_int(epilogue), c_int(m), c_int(n), c_int(k)))
+
+    def gemm_narrow_tile(self, dtype: torch.dtype, epilogue: int, m: int, n: int, k: int) -> int:
+        """Rows times columns of the narrow tile of the ring kernel that a product of these sizes (and of 16-byte aligned
+        operands) takes before any other kernel; 0: none."""
+        return int(self.core.ls_gemm_narrow_tile(c_int(DTYPE_CODE[dtype]), c_int(epilogue), c_int(m), c_int(n), c_int(k)))
 
     def gemm_slices_count(self, k: int) -> int:
         """K slices of a product over ``k`` (first dimension of ``gemm_slices``'s output)."""

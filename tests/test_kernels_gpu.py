@@ -315,6 +315,69 @@ def test_products_on_both_sides_of_the_lines_between_the_kernels_have_the_same_b
             assert torch.equal(part, out[first:first + 5]), (m, n, k, gated, first)
 
 
+# (rows, columns, K, whether SwiGLU) on both sides of the lines of the narrow tiles, and rows times columns of the tile (0: none)
+NARROW_LINES = {
+    torch.float32: [(16, 4096, 264, False, 0), (17, 4096, 512, False, 1024), (24, 4096, 516, False, 0), (25, 4093, 516, False, 1024),
+                    (32, 512, 1028, False, 0), (32, 513, 1028, False, 1024), (4, 8192, 2056, False, 0), (5, 8192, 2056, False, 1024),
+                    (16, 8224, 248, False, 0), (16, 8211, 264, False, 1024), (64, 4112, 264, False, 0), (65, 4112, 264, False, 1024),
+                    (97, 12289, 72, False, 0), (33, 24544, 72, True, 1024), (16, 4096, 264, True, 0), (16, 4128, 264, True, 1024)],
+    torch.bfloat16: [(16, 4096, 328, False, 0), (16, 4109, 328, False, 1024), (1, 1000, 320, False, 1024), (17, 24, 8, False, 1024),
+                     (5, 4096, 1032, True, 1024), (33, 4096, 72, False, 1024), (33, 4097, 72, False, 2048), (64, 8192, 264, False, 2048),
+                     (64, 8193, 264, False, 0), (97, 4091, 72, False, 2048), (97, 4097, 72, False, 0), (257, 909, 4424, False, 2048),
+                     (32, 16384, 520, True, 2048), (32, 16416, 520, True, 0), (32, 24544, 512, False, 2048), (32, 24544, 520, False, 0),
+                     (31, 24544, 2056, True, 1024), (31, 24608, 2056, True, 0), (33, 24544, 2056, True, 0)],
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_products_on_both_sides_of_the_lines_of_the_narrow_tiles_have_the_same_bits(dtype):
+    """Weights one element behind a 16-byte boundary go to kernels of another kind (a wave a slice, tiles through registers): the
+    same bits.  The sum of every element is at most sum(|x||w|) 2^-24 (K + K / 256) off (each addition rounds once)."""
+    from lockstep_amd.ops import ADD_F32, STORE_F32, SWIGLU
+
+    for m, n, k, gated, tile in NARROW_LINES[dtype]:
+        epilogue = SWIGLU if gated else STORE_F32
+        assert K().gemm_narrow_tile(dtype, epilogue, m, n, k) == tile, (m, n, k, gated)
+        g = torch.Generator(device="cuda").manual_seed(m + n + k)
+        x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+        w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+        x[-1] = float("inf")                                     # a row must not reach another one
+        off = torch.empty(n * k + 8, dtype=dtype, device="cuda")[1:1 + n * k].view(n, k)
+        off.copy_(w)
+        a, b = (torch.full((m, n // 2 if gated else n), 7.0, dtype=dtype if gated else torch.float32, device="cuda") for _ in range(2))
+        K().gemm(x, w, a, epilogue)
+        K().gemm(x, off, b, epilogue)
+        assert torch.equal(a[:-1], b[:-1]), (m, n, k, gated)
+        if not gated and m > 1:
+            want, most = x[:-1].double() @ w.double().T, x[:-1].double().abs() @ w.double().abs().T
+            assert ((a[:-1] - want).abs() <= most * 2.0 ** -24 * (k + k / 256 + 1)).all(), (m, n, k)
+            K().gemm(x, w, a, ADD_F32)
+            assert torch.equal(a[:-1], b[:-1] + b[:-1]), (m, n, k)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(4, 4096, 4096), (3, 4096, 4096), (17, 1028, 1288), (32, 1020, 4424), (33, 1024, 8), (40, 260, 328), (64, 1024, 2048),
+                                   (64, 4092, 1032), (65, 508, 2048), (200, 1024, 3072), (256, 4096, 520)])
+def test_slice_sums_in_either_tile_add_up_to_the_product(dtype, m, n, k):
+    """Slice sums on both sides of the choice between tiles of 32 and 64 rows and of one, two and four slices a workgroup, with rows and
+    columns that end inside a tile: every sum is there, and added in ascending order they are the product, bit for bit."""
+    from lockstep_amd.ops import STORE_F32
+
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+    if m > K().gemm_slices_max_rows(k, dtype):
+        pytest.skip("more rows than the slice sums take")
+    sums = torch.full((K().gemm_slices_count(k), m, n), float("nan"), device="cuda")
+    K().gemm_slices(x, w, sums)
+    want = torch.empty(m, n, device="cuda")
+    K().gemm(x, w, want, STORE_F32)
+    total = torch.zeros(m, n, device="cuda")
+    for part in sums:
+        total = total + part
+    assert torch.equal(total, want)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,k,gated", [(16352, 200, False), (16352, 200, True), (32768 + 40, 96, False), (32768, 72, True)])
 def test_products_off_a_16_byte_boundary_with_few_rows_have_the_bits_of_aligned_ones(dtype, n, k, gated):
