@@ -24,7 +24,7 @@
 // tiles of a wave.
 
 #include "common.h"
-#include "ring.h"
+#include "ring_product.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -817,195 +817,193 @@ static int few_chunks(int dtype, int K) {
 }
 
 // ---------------------------------------------------------------------------
-// The same two products for tiles of 64 rows (many tokens an expert), both operands through a ring of three stages in
-// LDS (128 bytes of K a row, written there by the loads themselves; layout, waits and barriers as gemm_ring.h describes
-// them).  A workgroup of eight waves takes 64 rows by 128 weight rows: 64 gate and the 64 up rows of the same columns, or
-// 128 columns of the down product (float32: 64); two workgroups share a CU.  A row's contraction is still one chain over ascending
-// chunks from zero: the same bits as the kernels above give without a cut of K.  Measured against tiles staged through
-// registers (64 x 64 by four waves; 2,048 tokens with 4 of 32 experts, width 1,024, 768 a piece): gate and up 94 -> 65
-// us (395 TFLOP/s), down 65 -> 52.  What bounds it now is the L2: 855 MB of requests in gate and up, 13 TB/s, three
-// quarters of them hits.  Four neighbouring tiles kept on one XCD, so that an expert's weights reach an L2 once, moved
-// this by no more than the runs differ (67 and 50 us): a row tile of 64 asks for too many bytes an operation.
+// The same two products for tiles of 64 rows (many tokens an expert), both operands through rings of three stages in LDS
+// (ring_product.h).  Eight waves, NWM along the rows by NWN along the weights, take 64 rows by WEIGHTS weight rows: half of them gate rows
+// and half the up rows of the same columns, which lie in LDS in tiles of 16 in turn, or columns of the down product; two workgroups share a
+// CU.  A row's contraction is one chain over ascending chunks from zero: the same bits as the kernels above give without a cut of K.
+// What bounds it: the loads, most of them answered by L2 once neighbouring tiles of an expert share one (below).  Measured (2,048
+// tokens with 4 of 32 experts, width 1,024, 768 a piece, weights from HBM, us, before / now): gate and up 64 / 51 (510 TFLOP/s), down
+// 52 / 31; 520, 1,024 and 4,096 tokens, both, 65 / 45, 77 / 54, 188 / 139; 2,048 tokens of 4,096 and 1,536 a piece 614 / 579.  Of that the loop's
+// order is a third (70 and 45 with the columns of a tile on one XCD), the units of tiles two.  Other shapes, gate and up / down: 64 x 256
+// 68 / 36, five stages 70 / 38 (one workgroup a CU), 128 rows x 256 47 to 59 / 34, x 192 50; 128 rows are ahead for wide experts (441 for the 579).
 // ---------------------------------------------------------------------------
-constexpr int kRingRows = 64, kRingStages = 3;
-constexpr int ring_lds(int weights) { return kRingStages * (kRingRows + weights) * 128; }
-// WEIGHTS: weight rows, 128 or 64 (two tiles a wave or one).  PAIRED: a wave's two weight tiles lie 64 rows apart (gate,
-// up), else side by side.
-template <typename T, int WEIGHTS, bool PAIRED>
-struct RingProduct {
-  typedef typename Atom<T>::vec_t vec_t;
-  static constexpr int BK = 128 / (int)sizeof(T), S = kRingStages;
-  static constexpr int W_BYTES = WEIGHTS * 128, X_BYTES = kRingRows * 128;
-  static constexpr int TI = WEIGHTS / 64;  // weight tiles a wave
-  static constexpr int LOADS = 1 + TI;     // a wave's loads a stage: eight rows of X, TI times eight of W
-  f32x4 acc[TI][2];                        // [weight tile][row tile]
+template <typename T, int WEIGHTS, int NWM, int NWN>
+struct ExpertTile {
+  static constexpr int ROWS = 64, S = 3;
+  static constexpr int NW = NWM * NWN, TI = WEIGHTS / (16 * NWN), TJ = ROWS / (16 * NWM);
+  static constexpr int LW = WEIGHTS / (8 * NW), LX = ROWS / (8 * NW);  // a wave's loads a stage: eight rows each
+  static_assert(LW * 8 * NW == WEIGHTS && LX * 8 * NW == ROWS && TI * 16 * NWN == WEIGHTS && TJ * 16 * NWM == ROWS, "tile shape");
+  typedef RingProduct<T, TI, TJ, 2048, WEIGHTS, ROWS, LW, LX, S, S, 1, false> Product;
+  static constexpr int kLds = Product::LDS_BYTES, kThreads = 64 * NW;
+  Product product;
 
-  // row and column of this lane's outputs acc[i][j][0..3] inside the workgroup's tile
-  static __device__ __forceinline__ int row_of(int j) { return ((threadIdx.x >> 8) & 1) * 32 + j * 16 + (threadIdx.x & 15); }
+  static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+  // the row of this lane's outputs of row tile j, and the first of its four weight rows of weight tile i, inside the tile
+  static __device__ __forceinline__ int row_of(int j) { return (wave() / NWN) * (ROWS / NWM) + j * 16 + (threadIdx.x & 15); }
   static __device__ __forceinline__ int weight_of(int i) {
-    const int w4 = (threadIdx.x >> 6) & 3;
-    return PAIRED ? i * 64 + w4 * 16 : w4 * 16 * TI + i * 16;
+    return (wave() % NWN) * (WEIGHTS / NWN) + i * 16 + ((threadIdx.x & 63) >> 4) * 4;
   }
+  // the row of the tile that this lane loads in the wave's load i, of either operand
+  static __device__ __forceinline__ int loaded_row(int i) { return (i * NW + wave()) * 8 + ((threadIdx.x & 63) >> 3); }
 
-  // x_off: this lane's row of X (row wave * 8 + lane / 8 of the tile) from the start of its buffer, in bytes; w0, w1: the
-  // buffers of the first and the second 64 weight rows, rows of K elements
-  __device__ __forceinline__ void run(u32x4_t x, unsigned x_off, u32x4_t w0, u32x4_t w1, int K, unsigned char* ring) {
+  // x_at[i]: the bytes from the start of x to row loaded_row(i) of the tile (~0: no such row); w: the buffer that this wave's
+  // weights come from, w_row(i): the row in it that load i begins with
+  template <typename WeightRow>
+  __device__ __forceinline__ void run(u32x4_t x, const unsigned (&x_at)[LX], u32x4_t w, WeightRow w_row, int K, unsigned char* ring) {
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int row16 = lane & 15, g = lane >> 4;
     const unsigned piece = ((lane & 7) ^ (lane >> 3)) * 16;
-    x_off += piece;
-    const unsigned w_off = (unsigned)((wave * 8 + (lane >> 3)) * (long)K * sizeof(T)) + piece;
-    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) void*)ring + wave * 1024;
-    const int stages = (K + BK - 1) / BK;
-    auto request = [&](int st, int buf) LS_INLINED {
-      buffer_to_lds16(x_off + st * 128, x, lds0 + S * W_BYTES + buf * X_BYTES);
-      buffer_to_lds16(w_off + st * 128, w0, lds0 + buf * W_BYTES);
-      if constexpr (TI == 2) buffer_to_lds16(w_off + st * 128, w1, lds0 + buf * W_BYTES + 64 * 128);
+    const unsigned w_off = (unsigned)((lane >> 3) * (long)K * sizeof(T)) + piece;
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) void*)ring + wave() * 1024;
+    const int limit = K * (int)sizeof(T) - (int)piece;  // bytes of a row from this lane's piece on
+    const int stages = (K + 128 / (int)sizeof(T) - 1) / (128 / (int)sizeof(T));
+    auto request_w = [&](int st, int buf, int n) LS_INLINED {
+      const int k = st * 128;
+      buffer_to_lds16(k < limit ? w_off + k + (unsigned)((long)w_row(n) * K * sizeof(T)) : ~0u, w,
+                      lds0 + buf * Product::W_BYTES + n * NW * 1024);
     };
-    auto clear_past_k = [&](int buf) LS_INLINED {
-      const int first = (K % BK) / Atom<T>::VEC;  // the first piece of a row that lies past K
-      for (int idx = threadIdx.x; idx < (WEIGHTS + kRingRows) * 8; idx += 512) {
-        const int row = idx >> 3;
-        if (((idx & 7) ^ (row & 7)) < first) continue;
-        unsigned char* at = row < WEIGHTS ? ring + buf * W_BYTES + idx * 16
-                                               : ring + S * W_BYTES + buf * X_BYTES + (idx - WEIGHTS * 8) * 16;
-        *reinterpret_cast<vec_t*>(at) = Atom<T>::zero();
-      }
-      ring_barrier();
+    auto request_x = [&](int st, int buf, int n) LS_INLINED {
+      const int k = st * 128;
+      buffer_to_lds16(k < limit && x_at[n] != ~0u ? x_at[n] + k + piece : ~0u, x,
+                      lds0 + S * Product::W_BYTES + buf * Product::X_BYTES + n * NW * 1024);
     };
-    const unsigned at = row16 * 128 + ((g ^ (row16 & 7)) << 4);
-    const int wm = ((wave >> 2) & 1) * 32;
-    vec_t a[TI], b[2][2];
-    auto read_a = [&](int i, int buf, int c) LS_INLINED {
-      a[i] = *reinterpret_cast<const vec_t*>(ring + buf * W_BYTES + weight_of(i) * 128 + (at ^ (c * 64)));
-    };
-    auto read_b = [&](vec_t (&dst)[2], int buf, int c) LS_INLINED {
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        dst[j] = *reinterpret_cast<const vec_t*>(ring + S * W_BYTES + buf * X_BYTES + (wm + j * 16) * 128 + (at ^ (c * 64)));
-    };
-    auto multiply = [&](const vec_t (&mine)[2], vec_t (&next)[2], int buf, int c) LS_INLINED {
-      read_b(next, buf, c);
-#pragma unroll
-      for (int i = 0; i < TI; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) Atom<T>::mma(acc[i][j], a[i], mine[j]);
-        read_a(i, buf, c);
-      }
-    };
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-      if (s < stages) request(s, s);
-    if (stages >= S) wait_loads<(S - 1) * LOADS>(); else wait_loads<0>();
-    ring_barrier();
-    if (K % BK && stages == 1) clear_past_k(0);
-    read_b(b[0], 0, 0);
-#pragma unroll
-    for (int i = 0; i < TI; ++i) read_a(i, 0, 0);
-    int buf = 0;
-    for (int st = 0; st < stages; ++st) {
-      multiply(b[0], b[1], buf, 1);
-      if (st + S > stages) wait_loads<0>(); else wait_loads<(S - 2) * LOADS>();  // stage st + 1 is there
-      ring_barrier();                                                            // ... for everyone, and stage st is read
-      if (st + S < stages) request(st + S, buf);
-      buf = buf + 1 == S ? 0 : buf + 1;
-      if (K % BK && st + 2 == stages) clear_past_k(buf);
-      multiply(b[1], b[0], buf, 0);
-    }
+    product.run(ring + (wave() % NWN) * (WEIGHTS / NWN) * 128, ring + S * Product::W_BYTES + (wave() / NWN) * (ROWS / NWM) * 128, stages,
+                stages, request_w, request_x, [](int) LS_INLINED {});
   }
 };
 
-template <typename T>
-__global__ __launch_bounds__(512) void experts_gate_up_ring_kernel(const T* __restrict__ x, long ldx,
-                                                                   const T* __restrict__ w_gate,
-                                                                   const T* __restrict__ w_up, int F, int K, int top,
-                                                                   const int* __restrict__ order,
-                                                                   const int* __restrict__ tiles, float limit, float alpha,
-                                                                   float shift, const float* __restrict__ in_weight,
-                                                                   T* __restrict__ act, long ldy, int real, int n_tokens) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
-  const int tile = blockIdx.y;
-  const int e = tiles[4 * tile];
-  if (e < 0 || e >= real) return;
-  const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
-  const int col0 = blockIdx.x * 64;
-  const int mine = min((int)(threadIdx.x >> 3), rows - 1);  // (rows past the tile's: the last one again, not stored)
-  const long left = (long)(F - col0) * K * sizeof(T), from = ((long)e * F + col0) * K;
-  RingProduct<T, 128, true> product;
-  product.run(buffer_of(x, ((long)(n_tokens - 1) * ldx + K) * sizeof(T)), (unsigned)((long)(order[first + mine] / top) * ldx * sizeof(T)),
-              buffer_of(w_gate + from, left), buffer_of(w_up + from, left), K, ring);
-  const int quad = (threadIdx.x & 63) >> 4;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = product.row_of(j);
-    if (r >= rows) continue;
-    T* dst = act + (long)(first + r) * ldy;
-    const float wt = in_weight ? in_weight[order[first + r]] : 1.0f;
-    const int c0 = col0 + product.weight_of(0) + 4 * quad;
-    float y[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float g = fminf(product.acc[0][j][i] * wt, limit);
-      const float u = fminf(fmaxf(product.acc[1][j][i] * wt, -limit), limit);
-      y[i] = (g * sigmoid_e(alpha * g)) * (u + shift);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (c0 + i < F) dst[c0 + i] = from_f32<T>(y[i]);
-  }
-}
-
-// Columns of the down product a workgroup.  float32 is bound by the matrix cores of the CUs that have a workgroup, so narrow
-// tiles, of which there are more, are never slower (gate and up included, us, 64 / 128 columns: 700 tokens of one expert, width
-// 1,024, 2,048 a piece 112 / 144; 2,048 tokens with 4 of 32 experts, 1,024 and 768 367 / 379; staged through registers 140 and
-// 487).  bfloat16 is bound by the operands that a tile asks for (2,048 tokens of 4,096 and 1,536 a piece 646 / 610).
+// Columns of the down product a workgroup.  float32 is bound by the matrix cores of the CUs that have a workgroup, so
+// narrow tiles, of which there are more, are never slower.
 template <typename T>
 constexpr int kDownCols = sizeof(T) == 4 ? 64 : 128;
 
-template <typename T>
-__global__ __launch_bounds__(512) void experts_down_ring_kernel(const T* __restrict__ act, long ldy,
+// Workgroups go round the eight XCDs: units of four tiles (mostly one expert's) by four columns stay on one, so that a unit's rows
+// and weights are read from beyond an L2 once.  How many of the cap tiles are used nobody knows here: the units go round the XCDs in
+// turn, which leaves an XCD at most one unit behind another (whole runs of tiles an XCD, 20 tiles by 11 columns: 47 us for 32; gate and up
+// above with units of one, two and four tiles by all columns 70, 56, 56, of four by two, four and eight columns 55, 51, 63).
+// False: no such tile.
+constexpr int kUnitTiles = 4, kUnitColumns = 4;
+__device__ __forceinline__ bool tile_and_column(int columns, int cap, int& tile, int& column) {
+  constexpr int UNIT = kUnitTiles * kUnitColumns;
+  const int at = blockIdx.x >> 3, unit = at / UNIT * 8 + (blockIdx.x & 7), in_unit = at % UNIT;
+  const int across = (columns + kUnitColumns - 1) / kUnitColumns;
+  tile = unit / across * kUnitTiles + in_unit % kUnitTiles;
+  column = unit % across * kUnitColumns + in_unit / kUnitTiles;
+  return tile < cap && column < columns;
+}
+static long tile_grid(int columns, int cap) {
+  const long units = (long)((cap + kUnitTiles - 1) / kUnitTiles) * ((columns + kUnitColumns - 1) / kUnitColumns);
+  return (units + 7) / 8 * 8 * kUnitTiles * kUnitColumns;
+}
+
+template <typename T, int WEIGHTS, int NWM, int NWN>
+__global__ __launch_bounds__(64 * NWM * NWN) void experts_gate_up_ring_kernel(const T* __restrict__ x, long ldx,
+                                                                   const T* __restrict__ w_gate,
+                                                                   const T* __restrict__ w_up, int F, int K, int top,
+                                                                   const int* __restrict__ order,
+                                                                   const int* __restrict__ tiles, int cap, float limit, float alpha,
+                                                                   float shift, const float* __restrict__ in_weight,
+                                                                   T* __restrict__ act, long ldy, int real, int n_tokens) {
+  typedef ExpertTile<T, WEIGHTS, NWM, NWN> Tile;
+  static_assert(Tile::TI % 2 == 0, "a wave holds the gate and the up tile of its columns");
+  static_assert(Tile::NW % 4 == 0, "all loads of a wave are of gate rows, or all of up rows");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
+  constexpr int COLS = WEIGHTS / 2;
+  int tile, column;
+  if (!tile_and_column((F + COLS - 1) / COLS, cap, tile, column)) return;
+  const int e = tiles[4 * tile];
+  if (e < 0 || e >= real) return;
+  const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
+  const int col0 = column * COLS;
+  const int wave = Tile::wave();
+  unsigned x_at[Tile::LX];
+#pragma unroll
+  for (int i = 0; i < Tile::LX; ++i) {
+    const int r = Tile::loaded_row(i);
+    x_at[i] = r < rows ? (unsigned)((long)(order[first + r] / top) * ldx * sizeof(T)) : ~0u;
+  }
+  const long left = (long)(F - col0) * K * sizeof(T), from = ((long)e * F + col0) * K;
+  Tile t;
+  // (rows 32 p to 32 p + 15 of the weights in LDS are gate rows 16 p .., the next sixteen the same up rows)
+  t.run(buffer_of(x, ((long)(n_tokens - 1) * ldx + K) * sizeof(T)), x_at, buffer_of(((wave >> 1) & 1 ? w_up : w_gate) + from, left),
+        [&](int i) LS_INLINED { return ((i * Tile::NW + wave) >> 2) * 16 + (wave & 1) * 8; }, K, ring);
+#pragma unroll
+  for (int j = 0; j < Tile::TJ; ++j) {
+    const int r = Tile::row_of(j);
+    if (r >= rows) continue;
+    T* dst = act + (long)(first + r) * ldy;
+    const float wt = in_weight ? in_weight[order[first + r]] : 1.0f;
+#pragma unroll
+    for (int p = 0; p < Tile::TI; p += 2) {
+      const int w0 = Tile::weight_of(p), c0 = col0 + (w0 >> 5) * 16 + (w0 & 15);
+      typedef __attribute__((ext_vector_type(4))) T four_t;
+      four_t y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float g = fminf(t.product.acc[p][j][i] * wt, limit);
+        const float u = fminf(fmaxf(t.product.acc[p + 1][j][i] * wt, -limit), limit);
+        y[i] = from_f32<T>((g * sigmoid_e(alpha * g)) * (u + shift));
+      }
+      if (c0 + 3 < F) {  // (act and its rows start on 16 bytes)
+        *reinterpret_cast<four_t*>(dst + c0) = y;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (c0 + i < F) dst[c0 + i] = y[i];
+      }
+    }
+  }
+}
+
+template <typename T, int COLS, int NWM, int NWN>
+__global__ __launch_bounds__(64 * NWM * NWN) void experts_down_ring_kernel(const T* __restrict__ act, long ldy,
                                                                 const T* __restrict__ w_down, int N, int F, int top,
                                                                 int n_tokens, const int* __restrict__ order,
-                                                                const int* __restrict__ tiles,
+                                                                const int* __restrict__ tiles, int cap,
                                                                 const float* __restrict__ weight, float* __restrict__ P,
                                                                 const T* __restrict__ x, long ldx,
-                                                                const float* __restrict__ share, int real) {
+                                                                const float* __restrict__ share, int real, int vec_out) {
+  typedef ExpertTile<T, COLS, NWM, NWN> Tile;
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
-  constexpr int COLS = kDownCols<T>;
-  const int tile = blockIdx.y;
+  int tile, column;
+  if (!tile_and_column((N + COLS - 1) / COLS, cap, tile, column)) return;
   const int e = tiles[4 * tile];
   if (e < 0) return;
   const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
-  const int col0 = blockIdx.x * COLS;
+  const int col0 = column * COLS;
   if (e >= real) {
-    pass_input<T, 512>(x, ldx, share, first, rows, col0, min(N, col0 + COLS), top, n_tokens, N, order, P);
+    pass_input<T, Tile::kThreads>(x, ldx, share, first, rows, col0, min(N, col0 + COLS), top, n_tokens, N, order, P);
     return;
   }
-  const int mine = min((int)(threadIdx.x >> 3), rows - 1);
-  const T* from = w_down + ((long)e * N + col0) * F;
-  const long left = (long)(N - col0) * F * sizeof(T), half = 64L * F * sizeof(T);
-  RingProduct<T, COLS, false> product;
-  product.run(buffer_of(act + (long)first * ldy, ((long)(rows - 1) * ldy + F) * sizeof(T)), (unsigned)(mine * ldy * sizeof(T)),
-              buffer_of(from, left), buffer_of(from + 64L * F, left > half ? left - half : 0), F, ring);
-  const int quad = (threadIdx.x & 63) >> 4;
+  const int wave = Tile::wave();
+  unsigned x_at[Tile::LX];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = product.row_of(j);
+  for (int i = 0; i < Tile::LX; ++i) {
+    const int r = Tile::loaded_row(i);
+    x_at[i] = r < rows ? (unsigned)(r * ldy * sizeof(T)) : ~0u;
+  }
+  Tile t;
+  t.run(buffer_of(act + (long)first * ldy, ((long)(rows - 1) * ldy + F) * sizeof(T)), x_at,
+        buffer_of(w_down + ((long)e * N + col0) * F, (long)(N - col0) * F * sizeof(T)),
+        [&](int i) LS_INLINED { return (i * Tile::NW + wave) * 8; }, F, ring);
+#pragma unroll
+  for (int j = 0; j < Tile::TJ; ++j) {
+    const int r = Tile::row_of(j);
     if (r >= rows) continue;
     const int pair = order[first + r];
     const float wt = weight ? weight[pair] : 1.0f;
     float* dst = P + ((long)(pair % top) * n_tokens + pair / top) * N;
 #pragma unroll
-    for (int i = 0; i < product.TI; ++i) {
-      const int c0 = col0 + product.weight_of(i) + 4 * quad;
+    for (int i = 0; i < Tile::TI; ++i) {
+      const int c0 = col0 + Tile::weight_of(i);
+      const f32x4& acc = t.product.acc[i][j];
+      const f32x4 y = f32x4{wt * acc[0], wt * acc[1], wt * acc[2], wt * acc[3]};
+      if (vec_out && c0 + 3 < N) {
+        *reinterpret_cast<f32x4*>(dst + c0) = y;
+      } else {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (c0 + q < N) dst[c0 + q] = wt * product.acc[i][j][q];
+        for (int q = 0; q < 4; ++q)
+          if (c0 + q < N) dst[c0 + q] = y[q];
+      }
     }
   }
 }
@@ -1018,17 +1016,22 @@ using namespace ls;
 
 extern "C" int ls_experts_max_top() { return kMaxTop; }
 
+// The two kernels of 64-row tiles.
+#define LS_EXPERTS_UP(T_) experts_gate_up_ring_kernel<T_, 128, 2, 4>
+#define LS_EXPERTS_DOWN(T_) experts_down_ring_kernel<T_, kDownCols<T_>, 4, 2>
+template <typename T> constexpr int kUpLds = ExpertTile<T, 128, 2, 4>::kLds;
+template <typename T> constexpr int kDownLds = ExpertTile<T, kDownCols<T>, 4, 2>::kLds;
+
 // Dynamic LDS beyond 64 KB has to be granted per kernel (once).
-static bool ring_lds_ready(int dtype) {
-  auto grant = [](const void* kernel) {
-    const bool ok = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, ring_lds(128)) == hipSuccess;
+template <typename T>
+static bool ring_lds_ready() {
+  auto grant = [](const void* kernel, int bytes) {
+    const bool ok = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
     if (!ok) (void)hipGetLastError();
     return ok;
   };
-  static const bool granted[2] = {
-      grant((const void*)&experts_gate_up_ring_kernel<float>) && grant((const void*)&experts_down_ring_kernel<float>),
-      grant((const void*)&experts_gate_up_ring_kernel<bf16_t>) && grant((const void*)&experts_down_ring_kernel<bf16_t>)};
-  return granted[dtype == kF32 ? 0 : 1];
+  static const bool granted = grant((const void*)&LS_EXPERTS_UP(T), kUpLds<T>) && grant((const void*)&LS_EXPERTS_DOWN(T), kDownLds<T>);
+  return granted;
 }
 
 // Tiles that the pairs of n_tokens tokens can need at most, with rows_a_tile rows each.
@@ -1182,19 +1185,20 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
                        shared_of((T_*)nullptr));                                                                      \
   } while (0)
   // tiles of 64 rows go through LDS where every row of every operand starts on a 16-byte boundary, 32-bit offsets reach the
-  // rows (all of x, whose rows are picked; 64 of the weights and of act) and what the last stage reads behind them, and the
-  // tiles fit a grid's second dimension.  Rows further apart go to the kernel that forms 64-bit addresses.
-  const long across = 64 * std::max({(long)K, (long)F, ldy}), all_of_x = (n_tokens - 1) * ldx + K;
+  // rows (all of x, whose rows are picked; 128 of the weights, 64 of act), and a grid has room for the tiles.  Rows further apart go to the kernel that forms 64-bit addresses.
+  const long across = 128 * std::max({(long)K, (long)F, ldy}), all_of_x = (n_tokens - 1) * ldx + K;
+  const long wgs_up = tile_grid((F + 63) / 64, cap), wgs_down = tile_grid((N + 63) / 64, cap);
   const bool staged = rows_a_tile == 64 && K % vec == 0 && F % vec == 0 && ldx % vec == 0 && ldy % vec == 0 &&
-                      std::max(across, all_of_x) * (16 / vec) + 128 <= 0xffffffffL && cap < 65536 && ring_lds_ready(dtype);
+                      std::max(across, all_of_x) * (16 / vec) + 128 <= 0xffffffffL && std::max(wgs_up, wgs_down) < (1L << 22) &&
+                      (dtype == kF32 ? ring_lds_ready<float>() : ring_lds_ready<bf16_t>());
+  const int vec_out = N % 4 == 0 && reinterpret_cast<uintptr_t>(P) % 16 == 0;
 #define LS_EXPERTS_STAGED(T_)                                                                                         \
   do {                                                                                                                \
-    hipLaunchKernelGGL(experts_gate_up_ring_kernel<T_>, dim3((F + 63) / 64, cap), dim3(512), ring_lds(128), s, (const T_*)x, \
-                       ldx, (const T_*)w_gate, (const T_*)w_up, F, K, top, order, tiles, limit, alpha, shift, in_weight, \
-                       (T_*)act, ldy, real, n_tokens);                                                                  \
-    hipLaunchKernelGGL(experts_down_ring_kernel<T_>, dim3((N + kDownCols<T_> - 1) / kDownCols<T_>, cap), dim3(512),  \
-                       ring_lds(kDownCols<T_>), s, (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, \
-                       out_weight, P, (const T_*)x, ldx, weight, real);                                                \
+    hipLaunchKernelGGL((LS_EXPERTS_UP(T_)), dim3(wgs_up), dim3(512), kUpLds<T_>, s, (const T_*)x, ldx, (const T_*)w_gate,  \
+                       (const T_*)w_up, F, K, top, order, tiles, cap, limit, alpha, shift, in_weight, (T_*)act, ldy, real, n_tokens); \
+    hipLaunchKernelGGL((LS_EXPERTS_DOWN(T_)), dim3(tile_grid((N + kDownCols<T_> - 1) / kDownCols<T_>, cap)), dim3(512),    \
+                       kDownLds<T_>, s, (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, cap, out_weight, P, \
+                       (const T_*)x, ldx, weight, real, vec_out);                                                     \
   } while (0)
   // tiles of 16 rows of whole chunks and columns have kernels of their own
   const int few_up = few_chunks(dtype, K), few_down = few_chunks(dtype, F);

@@ -528,6 +528,37 @@ def test_tiles_of_64_rows_have_the_bits_of_tiles_of_32(dtype, width, ff):
     assert not torch.isnan(results[1][1]).any()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width, ff, sizes", [(520, 584, [700, 64, 1, 0, 300, 129]), (264, 64, [65] * 33), (1160, 1032, [1] * 3 + [900])])
+def test_units_of_tiles_and_columns_cover_every_output_once(dtype, width, ff, sizes):
+    """Tiles of 64 rows in units of four tiles by four columns dealt to the XCDs: more units than XCDs, units that end inside the columns
+    and inside the tiles, outputs that start on 16 bytes and off them, against tiles of 32 rows (another kernel), bit for bit."""
+    g = torch.Generator().manual_seed(width + ff)
+    k = K()
+    tokens, experts = sum(sizes), len(sizes)
+    owner = torch.repeat_interleave(torch.arange(experts), torch.tensor(sizes))[torch.randperm(tokens, generator=g)]
+    logits = torch.zeros(tokens, experts)
+    logits[torch.arange(tokens), owner] = 9.0
+    x = torch.randn(tokens, width, generator=g).to(dtype).cuda()
+    gate, up, down = ((torch.randn(experts, *shape, generator=g) * 0.3).to(dtype).cuda() for shape in ((ff, width), (ff, width), (width, ff)))
+    results = []
+    for rows, off in ((32, 0), (64, 0), (64, 1)):
+        cap = k.experts_tile_capacity(tokens, experts, 1, rows)
+        i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+        chosen, order, tiles, counts = i32(tokens), i32(tokens), i32(4 * cap), i32(experts)
+        share = torch.empty(tokens, device="cuda")
+        k.experts_route(logits.cuda(), torch.zeros(experts).cuda(), 1, rows, chosen, share, order, tiles, counts)
+        act = torch.full((tokens, ff), float("nan"), dtype=dtype, device="cuda")
+        room = torch.full((tokens * width + 8,), float("nan"), device="cuda")
+        partials = room[off:off + tokens * width].view(1, tokens, width)
+        k.experts_apply(x, gate, up, down, 1, rows, order, tiles, share, 1.3, 1.702, act, partials)
+        assert torch.isnan(room[:off]).all() and torch.isnan(room[off + tokens * width:]).all()
+        results.append((act, partials))
+    for act, partials in results[1:]:
+        assert torch.equal(results[0][0], act) and torch.equal(results[0][1], partials)
+    assert not torch.isnan(results[0][1]).any()
+
+
 # ---------------------------------------------------------------------------
 # one-layer models of each mechanism, then whole models
 # ---------------------------------------------------------------------------
