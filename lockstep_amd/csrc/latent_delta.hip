@@ -517,6 +517,10 @@ __device__ __forceinline__ void keep_inputs(const float* __restrict__ raw, long 
 #pragma unroll
       for (int u = 0; u < kAtOnce; ++u)
         if (a0 + u < M - 1) kept[(long)(a0 + u) * C + c] = v[u];
+      // (every load is used on every path: one that might still be on its way to its register when the recurrence reuses that
+      // was waited for in each of the recurrence's blocks, with all but seven of the loads that are ahead there)
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) __asm__ volatile("" ::"v"(v[u]));
     }
   }
 }
@@ -531,7 +535,8 @@ __device__ __forceinline__ void keep_inputs(const float* __restrict__ raw, long 
 // branches; only the blocks whose requests would leave the request hold them at its last token.  beta and the decay come
 // by one vector load at the same address in every lane (as scalar loads, which return in any order, a wait for one would
 // be a wait for all, also for those of the tokens ahead).
-// DEPTH: the tokens whose operands are on their way.  2,048 tokens (16 heads over 8, 128 x 128): 258 us, 281 with a decay
+// DEPTH: the tokens whose operands are on their way.  2,048 tokens (16 heads over 8, 128 x 128): 258 us under the profiler (271 with a wait
+// for all of them in every block, see keep_inputs and the order of the first requests), 281 with a decay
 // a channel; with lane pointers, a conditional step of each, and a branch a token it took 490.  Where the longest request brings a token or two,
 // two are enough and leave room for twice the waves: eight requests decoding 28 -> 13 us.  Where most requests decode beside
 // a longer one, the longest's chain counts as much as the room: four (63 requests of one token and one of 64, two / four / eight
@@ -636,7 +641,10 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
   {
     const auto qkb = buffer(qk_at, kNowhere), vb = buffer(v_at, kNowhere), gb = buffer(g_at, kNowhere), db = buffer(d_at, kNowhere);
 #pragma unroll
-    for (int j = 0; j < DEPTH; ++j) fetch(ring[j], qkb, vb, gb, db, min(j, n - 1));
+    for (int j = 0; j < DEPTH; ++j) {
+      fetch(ring[j], qkb, vb, gb, db, min(j, n - 1));
+      __builtin_amdgcn_sched_barrier(0);  // (in the order in which the loop waits for them)
+    }
   }
   if (M > 1)
     keep_inputs(raw, ld, C, M, m, state + (long)m.table_row * state_stride + conv_at, (head * (int)gridDim.y + (int)blockIdx.y) * 64 + lane,
