@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "row_piece.h"
 #include "core_api.h"
 
 namespace ls {
@@ -191,7 +192,7 @@ __device__ __forceinline__ void row_scales(const float* __restrict__ H, long ldh
 // slices w, w + NW, ...; slice sums meet in LDS and are folded in ascending
 // order by the thread that owns the output element.
 // ---------------------------------------------------------------------------
-template <typename T, int MT, int NW, int EPI, bool NORM>
+template <typename T, int MT, int NW, int EPI, bool NORM, bool WHOLE>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const void* __restrict__ Xv, const T* __restrict__ W,
                                                                void* __restrict__ C, int M, int N, int K, long ldx,
                                                                long ldc, int kslice, int aligned, int vec_ok,
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const void* __rest
   extern __shared__ float part[];                // [nslices][NT][MT][256] (+ 80 floats with NORM)
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16 * NT;
   const int row16 = lane & 15;
   const int g = lane >> 4;
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const void* __rest
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int n = n0 + t * 16 + row16;
-        w[t][u] = load_vec<T>(W, n, k, K, K, n < N && in, aligned);
+        w[t][u] = row_piece<T, WHOLE>(W + (long)n0 * K, t * 16 + row16, k, K, K, (n < N) & in, aligned);
       }
     }
   };
@@ -294,12 +295,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const void* __rest
         } else {
 #pragma unroll
           for (int j = 0; j < MT; ++j)
-            x[j][u] = load_vec<T>(X, j * 16 + row16, k, K, ldx, j * 16 + row16 < M && in, aligned);
+            x[j][u] = row_piece<T, WHOLE>(X, j * 16 + row16, k, K, ldx, (j * 16 + row16 < M) & in, aligned);
         }
       }
+      if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);  // (the scheduler would move the loads down to their products, two in flight at a time)
 #pragma unroll
       for (int u = 0; u < UNR; ++u) {
-        if (k0 + u * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
+        if (!WHOLE && k0 + u * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -351,7 +353,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const void* __rest
 // fold.  Slice sums meet in LDS and are folded in ascending order, as in the
 // skinny kernel.
 // ---------------------------------------------------------------------------
-template <typename T, int MT, int EPI, int XC>
+template <typename T, int MT, int EPI, int XC, bool WHOLE>
 __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                            void* __restrict__ C, int M, int N, int K, long ldx,
                                                            long ldc, int kslice, int aligned, int vec_ok,
@@ -371,7 +373,7 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
   extern __shared__ float part[];  // [2][waves][NT][MT][256]
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;  // = number of K slices
   const int row16 = lane & 15;
   const int g = lane >> 4;
@@ -392,29 +394,38 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
 #pragma unroll
     for (int c = 0; c < UC; ++c) {
       const int kc = k_begin + (q * UC + c) * A::KCHUNK;
-      dst[c] = load_vec<T>(W, n, kc + g * A::VEC, K, K, row16 < cols && n < N && kc < k_end, aligned);
+      dst[c] = row_piece<T, WHOLE>(W + (long)(b * NT + t) * cols * K, row16, kc + g * A::VEC, K, K, (row16 < cols) & (n < N) & (kc < k_end),
+                                   aligned, b < blocks);
     }
   };
 
   // Units are numbered through the walk: unit u of the workgroup is unit u % UNITS of its block u / UNITS
   // and lives in buffer u % RING.
-  vec_t wbuf[RING][UC];
-  int b = walker;
-#pragma unroll
-  for (int u = 0; u < AHEAD; ++u) {
-    const int bu = b + (u / UNITS) * walkers;
-    if (bu < blocks) fetch(bu, (u % UNITS) / UQ, (u % UNITS) % UQ, wbuf[u % RING]);
-  }
-
   vec_t xs[MT][XC];
 #pragma unroll
   for (int j = 0; j < MT; ++j)
 #pragma unroll
     for (int c = 0; c < XC; ++c) {
       const int kc = k_begin + c * A::KCHUNK;
-      xs[j][c] = load_vec<T>(X, m_base + j * 16 + row16, kc + g * A::VEC, K, ldx,
-                             m_base + j * 16 + row16 < M && kc < k_end, aligned);
+      xs[j][c] = row_piece<T, WHOLE>(X, m_base + j * 16 + row16, kc + g * A::VEC, K, ldx,
+                                     m_base + j * 16 + row16 < M && kc < k_end, aligned);
     }
+  if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);
+  vec_t wbuf[RING][UC];
+  int b = walker;
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) {
+    const int bu = b + (u / UNITS) * walkers;
+    fetch(bu, (u % UNITS) / UQ, (u % UNITS) % UQ, wbuf[u % RING]);
+    if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);  // (in the order in which they are waited for)
+  }
+  // (X has come before the walk begins: inside it the first product's wait for X would be one for every unit in flight)
+  if constexpr (WHOLE) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int c = 0; c < XC; ++c) __asm__ volatile("" ::"v"(__builtin_bit_cast(f32x4, xs[j][c])));
+  }
 
   // One column block; `par` is the buffer that holds the block's first unit (static, so that the
   // register buffers are addressed statically).
@@ -432,11 +443,11 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
         for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
       const int far_block = b + ((idx + AHEAD) / UNITS) * walkers;  // the block of the unit AHEAD units on
-      if (far_block < blocks)
-        fetch(far_block, ((idx + AHEAD) % UNITS) / UQ, ((idx + AHEAD) % UNITS) % UQ, wbuf[(P + idx + AHEAD) % RING]);
+      fetch(far_block, ((idx + AHEAD) % UNITS) / UQ, ((idx + AHEAD) % UNITS) % UQ, wbuf[(P + idx + AHEAD) % RING]);
+      if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);  // (the scheduler would move the loads down to their products, two in flight at a time)
 #pragma unroll
       for (int c = 0; c < UC; ++c) {
-        if (k_begin + (q * UC + c) * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
+        if (!WHOLE && k_begin + (q * UC + c) * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
 #pragma unroll
         for (int j = 0; j < MT; ++j) A::mma(acc[j], wbuf[(P + idx) % RING][c], xs[j][q * UC + c]);
       }
@@ -478,27 +489,31 @@ __global__ __launch_bounds__(1024) void gemm_stream_kernel(const T* __restrict__
   };
 
   // the first buffer of a block advances by UNITS % RING from block to block
-  for (int it = 0; b < blocks;) {
-    block_step(std::integral_constant<int, 0>{}, it);
-    b += walkers;
-    ++it;
-    if (UNITS % RING != 0) {  // UNITS = 2, RING = 4: every other block starts in buffer 2
-      if (b >= blocks) break;
-      block_step(std::integral_constant<int, UNITS % RING>{}, it);
+  int it = 0;
+  if constexpr (UNITS % RING != 0) {  // UNITS = 2, RING = 4: every other block starts in buffer 2
+    for (; b + walkers < blocks;) {   // (no way out between the two, which the loop's waits would be counted by)
+      block_step(std::integral_constant<int, 0>{}, it++);
       b += walkers;
-      ++it;
+      block_step(std::integral_constant<int, UNITS % RING>{}, it++);
+      b += walkers;
     }
+    if (b < blocks) block_step(std::integral_constant<int, 0>{}, it);
+  } else {
+    for (; b < blocks; b += walkers) block_step(std::integral_constant<int, 0>{}, it++);
   }
 }
 
+// Whether row_piece's 31-bit offsets reach up to 64 aligned rows of both operands.
+static bool pieces_reach(long ldx, long K, long size) { return 65 * std::max(ldx, K) * size <= kNoPiece; }
+
 // Dynamic LDS beyond 64 KB has to be granted per kernel (once).
-template <typename T, int MT, int EPI, int XC>
+template <typename T, int MT, int EPI, int XC, bool WHOLE>
 static bool stream_lds_ready(size_t bytes) {
   if (bytes <= 64 * 1024) return true;
   if (bytes > 128 * 1024) return false;
   static int state = 0;  // 0 unknown, 1 granted, -1 refused
   if (state == 0) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_stream_kernel<T, MT, EPI, XC>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_stream_kernel<T, MT, EPI, XC, WHOLE>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
     if (e != hipSuccess) (void)hipGetLastError();
     state = e == hipSuccess ? 1 : -1;
@@ -516,14 +531,14 @@ static bool stream_lds_ready(size_t bytes) {
 // slowly), at the price of the fold, which the consumer (add_rmsnorm_kernel)
 // does on the way.
 // ---------------------------------------------------------------------------
-template <typename T, int MT>
+template <typename T, int MT, bool WHOLE>
 __global__ __launch_bounds__(256) void gemm_slices_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                           float* __restrict__ P, int M, int N, int K, long ldx,
                                                           int kslice, int aligned, int slices_per_group) {
   typedef Atom<T> A;
   typedef typename A::vec_t vec_t;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16;
   const int row16 = lane & 15;
   const int g = lane >> 4;
@@ -543,14 +558,15 @@ __global__ __launch_bounds__(256) void gemm_slices_kernel(const T* __restrict__ 
     for (int u = 0; u < UNR; ++u) {
       const int k = k0 + u * A::KCHUNK + g * A::VEC;
       const bool in = k0 + u * A::KCHUNK < k_end;
-      w[u] = load_vec<T>(W, n0 + row16, k, K, K, n0 + row16 < N && in, aligned);
+      w[u] = row_piece<T, WHOLE>(W + (long)n0 * K, row16, k, K, K, (n0 + row16 < N) & in, aligned);
 #pragma unroll
       for (int j = 0; j < MT; ++j)
-        x[j][u] = load_vec<T>(X, j * 16 + row16, k, K, ldx, j * 16 + row16 < M && in, aligned);
+        x[j][u] = row_piece<T, WHOLE>(X, j * 16 + row16, k, K, ldx, (j * 16 + row16 < M) & in, aligned);
     }
+    if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);  // (the scheduler would move the loads down to their products, two in flight at a time)
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
-      if (k0 + u * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
+      if (!WHOLE && k0 + u * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
 #pragma unroll
       for (int j = 0; j < MT; ++j) A::mma(acc[j], w[u], x[j][u]);
     }
@@ -594,7 +610,7 @@ __global__ __launch_bounds__(256) void gemm_slices_folded_kernel(const float* __
   typedef typename A::vec_t vec_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char folded_lds[];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 64 + wave * 16;
   const int row16 = lane & 15;
   const int g = lane >> 4;
@@ -612,7 +628,7 @@ __global__ __launch_bounds__(256) void gemm_slices_folded_kernel(const float* __
 #pragma unroll
   for (int u = 0; u < UNR; ++u) {
     const int k = k_begin + u * A::KCHUNK + g * A::VEC;
-    w_first[u] = load_vec<T>(W, n0 + row16, k, K, K, n0 + row16 < N && k_begin + u * A::KCHUNK < k_end, true);
+    w_first[u] = row_piece<T, true>(W + (long)n0 * K, row16, k, K, K, n0 + row16 < N && k_begin + u * A::KCHUNK < k_end, true);
   }
   __builtin_amdgcn_sched_barrier(0);  // (the scheduler would move these loads down to their use, behind the fold)
 
@@ -676,15 +692,12 @@ __global__ __launch_bounds__(256) void gemm_slices_folded_kernel(const float* __
     for (int u = 0; u < UNR; ++u) {
       const int k = k0 + u * A::KCHUNK + g * A::VEC;
       const bool in = k0 + u * A::KCHUNK < k_end;
-      w[u] = k0 == k_begin ? w_first[u] : load_vec<T>(W, n0 + row16, k, K, K, n0 + row16 < N && in, true);
+      w[u] = k0 == k_begin ? w_first[u] : row_piece<T, true>(W + (long)n0 * K, row16, k, K, K, n0 + row16 < N && in, true);
       x[u] = (row16 < M && in && k < k_end) ? *reinterpret_cast<const vec_t*>(xs + (long)row16 * row_stride + (k - k_begin))
                                             : A::zero();
     }
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      if (k0 + u * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
-      A::mma(acc, w[u], x[u]);
-    }
+    for (int u = 0; u < UNR; ++u) A::mma(acc, w[u], x[u]);  // (beyond the slice zeros, as row_piece has it)
   }
   const int n = n0 + g * 4;
   if (row16 < M && n < N) {
@@ -774,7 +787,7 @@ __global__ __launch_bounds__(256) void gemm_slices_wide_kernel(const T* __restri
 // in registers, the weights of the next units are in flight across column
 // blocks as in the streaming kernel.  The waves share nothing, so there is no
 // barrier.
-template <typename T, int MT, int XC>
+template <typename T, int MT, int XC, bool WHOLE>
 __global__ __launch_bounds__(256) void gemm_slices_stream_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                                  float* __restrict__ P, int M, int N, int K, long ldx,
                                                                  int kslice, int aligned, int slices_per_group,
@@ -787,7 +800,7 @@ __global__ __launch_bounds__(256) void gemm_slices_stream_kernel(const T* __rest
   constexpr int AHEAD = RING - 1;
   static_assert(XC % UC == 0 && (UNITS % RING == 0 || (2 * UNITS) % RING == 0), "units and ring");
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row16 = lane & 15;
   const int g = lane >> 4;
   const int nslices = (K + kslice - 1) / kslice;
@@ -803,25 +816,34 @@ __global__ __launch_bounds__(256) void gemm_slices_stream_kernel(const T* __rest
 #pragma unroll
     for (int c = 0; c < UC; ++c) {
       const int kc = k_begin + (q * UC + c) * A::KCHUNK;
-      dst[c] = load_vec<T>(W, n, kc + g * A::VEC, K, K, n < N && kc < k_end, aligned);
+      dst[c] = row_piece<T, WHOLE>(W + (long)b * 16 * K, row16, kc + g * A::VEC, K, K, (n < N) & (kc < k_end), aligned, b < blocks);
     }
   };
-  vec_t wbuf[RING][UC];
-  int b = blockIdx.x;
-#pragma unroll
-  for (int u = 0; u < AHEAD; ++u) {
-    const int bu = b + (u / UNITS) * walkers;
-    if (bu < blocks) fetch(bu, u % UNITS, wbuf[u % RING]);
-  }
   vec_t xs[MT][XC];
 #pragma unroll
   for (int j = 0; j < MT; ++j)
 #pragma unroll
     for (int c = 0; c < XC; ++c) {
       const int kc = k_begin + c * A::KCHUNK;
-      xs[j][c] = load_vec<T>(X, m_base + j * 16 + row16, kc + g * A::VEC, K, ldx,
-                             m_base + j * 16 + row16 < M && kc < k_end, aligned);
+      xs[j][c] = row_piece<T, WHOLE>(X + (long)m_base * ldx, j * 16 + row16, kc + g * A::VEC, K, ldx,
+                                     m_base + j * 16 + row16 < M && kc < k_end, aligned);
     }
+  if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);
+  vec_t wbuf[RING][UC];
+  int b = blockIdx.x;
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) {
+    const int bu = b + (u / UNITS) * walkers;
+    fetch(bu, u % UNITS, wbuf[u % RING]);
+    if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);  // (in the order in which they are waited for)
+  }
+  // (X has come before the walk begins: inside it the first product's wait for X would be one for every unit in flight)
+  if constexpr (WHOLE) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int c = 0; c < XC; ++c) __asm__ volatile("" ::"v"(__builtin_bit_cast(f32x4, xs[j][c])));
+  }
 
   auto block_step = [&](auto par) LS_INLINED {
     constexpr int P0 = decltype(par)::value;
@@ -831,10 +853,11 @@ __global__ __launch_bounds__(256) void gemm_slices_stream_kernel(const T* __rest
 #pragma unroll
     for (int idx = 0; idx < UNITS; ++idx) {
       const int far_block = b + ((idx + AHEAD) / UNITS) * walkers;
-      if (far_block < blocks) fetch(far_block, (idx + AHEAD) % UNITS, wbuf[(P0 + idx + AHEAD) % RING]);
+      fetch(far_block, (idx + AHEAD) % UNITS, wbuf[(P0 + idx + AHEAD) % RING]);
+      if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);  // (the scheduler would move the loads down to their products, two in flight at a time)
 #pragma unroll
       for (int c = 0; c < UC; ++c) {
-        if (k_begin + (idx * UC + c) * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
+        if (!WHOLE && k_begin + (idx * UC + c) * A::KCHUNK >= k_end) break;  // uniform: a chunk is visited iff it starts inside the slice
 #pragma unroll
         for (int j = 0; j < MT; ++j) A::mma(acc[j], wbuf[(P0 + idx) % RING][c], xs[j][idx * UC + c]);
       }
@@ -854,14 +877,16 @@ __global__ __launch_bounds__(256) void gemm_slices_stream_kernel(const T* __rest
       }
     }
   };
-  while (b < blocks) {
-    block_step(std::integral_constant<int, 0>{});
-    b += walkers;
-    if (UNITS % RING != 0) {
-      if (b >= blocks) break;
+  if constexpr (UNITS % RING != 0) {
+    while (b + walkers < blocks) {
+      block_step(std::integral_constant<int, 0>{});
+      b += walkers;
       block_step(std::integral_constant<int, UNITS % RING>{});
       b += walkers;
     }
+    if (b < blocks) block_step(std::integral_constant<int, 0>{});
+  } else {
+    for (; b < blocks; b += walkers) block_step(std::integral_constant<int, 0>{});
   }
 }
 
@@ -1242,6 +1267,7 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
                       (reinterpret_cast<uintptr_t>(W) % 16 == 0);
   const size_t out_size = (EPI == kStore || EPI == kSwiGLU || EPI == kXielu) ? sizeof(T) : sizeof(float);
   const int vec_ok = (ldc % 4 == 0) && (reinterpret_cast<uintptr_t>(C) % (4 * out_size) == 0);
+  const bool whole = aligned && pieces_reach(ldx, K, sizeof(T));
   const T* w = reinterpret_cast<const T*>(W);
   if (norm_w && M > 16) return fail("gemm: the fused norm prologue takes at most 16 rows, got %d", M);
   const int mt_rows = (M + 15) / 16;
@@ -1277,18 +1303,26 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
     if (row_groups > 1) walkers = (walkers + 7) / 8 * 8;  // whole rounds of the XCDs, see the kernel
     dim3 grid(walkers * row_groups);
     bool launched = true;
-#define LS_STREAM(MT_, XC_)                                                                                       \
-  if (stream_lds_ready<T, MT_, EPI, XC_>(stream_lds))                                                             \
-    hipLaunchKernelGGL((gemm_stream_kernel<T, MT_, EPI, XC_>), grid, dim3(nslices * 64), stream_lds, stream,      \
-                       reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice, aligned, vec_ok, out_cols, \
-                       blocks, row_groups, cols, act);                                                            \
-  else                                                                                                            \
+#define LS_STREAM_AS(MT_, XC_, WHOLE_)                                                                             \
+  if (stream_lds_ready<T, MT_, EPI, XC_, WHOLE_>(stream_lds))                                                      \
+    hipLaunchKernelGGL((gemm_stream_kernel<T, MT_, EPI, XC_, WHOLE_>), grid, dim3(nslices * 64), stream_lds, stream, \
+                       reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice, aligned, vec_ok, out_cols,  \
+                       blocks, row_groups, cols, act);                                                             \
+  else                                                                                                             \
     launched = false
-    if (group_tiles == 1 && xc == 8) LS_STREAM(1, 8);
-    else if (group_tiles == 1 && xc == 16) LS_STREAM(1, 16);
-    else if (group_tiles == 2 && xc == 8) LS_STREAM(2, 8);
-    else launched = false;
+#define LS_STREAM(MT_, XC_) \
+  if (whole) { LS_STREAM_AS(MT_, XC_, true); } else { LS_STREAM_AS(MT_, XC_, false); }
+    if (group_tiles == 1 && xc == 8) {
+      LS_STREAM(1, 8)
+    } else if (group_tiles == 1 && xc == 16) {
+      LS_STREAM(1, 16)
+    } else if (group_tiles == 2 && xc == 8) {
+      LS_STREAM(2, 8)
+    } else {
+      launched = false;
+    }
 #undef LS_STREAM
+#undef LS_STREAM_AS
     if (launched) return check_launch("gemm");
   }
   if (M <= 64 && !tiles && (ring || M <= 16 || N < 32768)) {
@@ -1297,23 +1331,26 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
     const int nw = (nslices > 8 && mt * NT <= 2) ? 16 : (nslices > 4 ? 8 : 4);
     dim3 grid((N + 16 * NT - 1) / (16 * NT));
     const size_t lds = ((size_t)nslices * NT * mt * 256 + (norm_w ? 80 : 0)) * sizeof(float);
-#define LS_SKINNY(MT_, NW_, NORM_)                                                                              \
-  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT_, NW_, EPI, NORM_>), grid, dim3(NW_ * 64), lds, stream, X, w, C, M, N, \
-                     K, ldx, ldc, kslice, aligned, vec_ok, norm_w, eps, out_cols, act)
+#define LS_SKINNY_AS(MT_, NW_, NORM_, WHOLE_)                                                                    \
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT_, NW_, EPI, NORM_, WHOLE_>), grid, dim3(NW_ * 64), lds, stream, X, w, C, \
+                     M, N, K, ldx, ldc, kslice, aligned, vec_ok, norm_w, eps, out_cols, act)
+#define LS_SKINNY(MT_, NW_) \
+  if (whole) LS_SKINNY_AS(MT_, NW_, false, true); else LS_SKINNY_AS(MT_, NW_, false, false)
     if (norm_w) {
       if constexpr (EPI == kXielu) return fail("gemm: the xIELU epilogue has no norm prologue");
-      else if (nw >= 8) LS_SKINNY(1, 8, true);
-      else LS_SKINNY(1, 4, true);
+      else if (nw >= 8) LS_SKINNY_AS(1, 8, true, false);
+      else LS_SKINNY_AS(1, 4, true, false);
     } else if (nw == 16) {
-      if (mt == 1) LS_SKINNY(1, 16, false); else LS_SKINNY(2, 16, false);
+      if (mt == 1) { LS_SKINNY(1, 16); } else { LS_SKINNY(2, 16); }
     } else if (nw == 8) {
-      if (mt == 1) LS_SKINNY(1, 8, false); else if (mt == 2) LS_SKINNY(2, 8, false);
-      else if (mt == 3) LS_SKINNY(3, 8, false); else LS_SKINNY(4, 8, false);
+      if (mt == 1) { LS_SKINNY(1, 8); } else if (mt == 2) { LS_SKINNY(2, 8); }
+      else if (mt == 3) { LS_SKINNY(3, 8); } else { LS_SKINNY(4, 8); }
     } else {
-      if (mt == 1) LS_SKINNY(1, 4, false); else if (mt == 2) LS_SKINNY(2, 4, false);
-      else if (mt == 3) LS_SKINNY(3, 4, false); else LS_SKINNY(4, 4, false);
+      if (mt == 1) { LS_SKINNY(1, 4); } else if (mt == 2) { LS_SKINNY(2, 4); }
+      else if (mt == 3) { LS_SKINNY(3, 4); } else { LS_SKINNY(4, 4); }
     }
 #undef LS_SKINNY
+#undef LS_SKINNY_AS
   } else {
     const int tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64;
     hipLaunchKernelGGL((gemm_tiled_kernel<T, EPI>), dim3(tiles_m * tiles_n), dim3(256), 0, stream,
@@ -1478,6 +1515,7 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
   const int vec = dtype == kF32 ? 4 : 8;
   const int aligned = (K % vec == 0) && (ldx % vec == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0) &&
                       (reinterpret_cast<uintptr_t>(W) % 16 == 0);
+  const bool whole = aligned && pieces_reach(ldx, K, dtype == kF32 ? 4 : 2);
   const int mt = (M + 15) / 16;
   // With more than 16 rows, where the rows of X outweigh the weights of a column block, and at least four
   // workgroups a CU, workgroups walk two or more column blocks each with X in registers (the walk keeps
@@ -1531,27 +1569,32 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
     if (row_groups > 1) walkers = (walkers + 7) / 8 * 8;  // the groups' workgroups of a walk sit on the same XCD
     dim3 walk_grid(walkers, groups, row_groups);
     bool launched = true;
-#define LS_WALK(T_, MT_, XC_)                                                                                     \
-  hipLaunchKernelGGL((gemm_slices_stream_kernel<T_, MT_, XC_>), walk_grid, dim3(64 * per_group), 0, s, (const T_*)X, \
+#define LS_WALK_AS(T_, MT_, XC_, WHOLE_)                                                                           \
+  hipLaunchKernelGGL((gemm_slices_stream_kernel<T_, MT_, XC_, WHOLE_>), walk_grid, dim3(64 * per_group), 0, s, (const T_*)X, \
                      (const T_*)W, P, M, N, K, ldx, kslice, aligned, per_group, col_blocks)
+#define LS_WALK(T_, MT_, XC_) \
+  { if (whole) LS_WALK_AS(T_, MT_, XC_, true); else LS_WALK_AS(T_, MT_, XC_, false); }
 #define LS_WALK_T(T_)                                                          \
-  if (group_tiles == 2 && xc == 8) LS_WALK(T_, 2, 8);                          \
-  else if (group_tiles == 3 && xc == 8) LS_WALK(T_, 3, 8);                     \
-  else if (group_tiles == 4 && xc == 8) LS_WALK(T_, 4, 8);                     \
-  else if (group_tiles == 2 && xc == 16) LS_WALK(T_, 2, 16);                   \
+  if (group_tiles == 2 && xc == 8) LS_WALK(T_, 2, 8)                           \
+  else if (group_tiles == 3 && xc == 8) LS_WALK(T_, 3, 8)                      \
+  else if (group_tiles == 4 && xc == 8) LS_WALK(T_, 4, 8)                      \
+  else if (group_tiles == 2 && xc == 16) LS_WALK(T_, 2, 16)                    \
   else launched = false
     if (dtype == kF32) { LS_WALK_T(float); } else if (dtype == kBF16) { LS_WALK_T(bf16_t); } else launched = false;
 #undef LS_WALK_T
 #undef LS_WALK
+#undef LS_WALK_AS
     if (launched) return check_launch("gemm_slices");
   }
   LS_REQUIRE(mt <= 4, "gemm_slices: no kernel for %d rows with K=%d", M, K);
-#define LS_SLICES(T_, MT_)                                                                                       \
-  hipLaunchKernelGGL((gemm_slices_kernel<T_, MT_>), grid, dim3(64 * per_group), 0, s, (const T_*)X, (const T_*)W, P, M, \
-                     N, K, ldx, kslice, aligned, per_group)
+#define LS_SLICES_AS(T_, MT_, WHOLE_)                                                                            \
+  hipLaunchKernelGGL((gemm_slices_kernel<T_, MT_, WHOLE_>), grid, dim3(64 * per_group), 0, s, (const T_*)X,       \
+                     (const T_*)W, P, M, N, K, ldx, kslice, aligned, per_group)
+#define LS_SLICES(T_, MT_) \
+  { if (whole) LS_SLICES_AS(T_, MT_, true); else LS_SLICES_AS(T_, MT_, false); }
 #define LS_SLICES_MT(T_)                                              \
-  if (mt == 1) LS_SLICES(T_, 1); else if (mt == 2) LS_SLICES(T_, 2); \
-  else if (mt == 3) LS_SLICES(T_, 3); else LS_SLICES(T_, 4)
+  if (mt == 1) LS_SLICES(T_, 1) else if (mt == 2) LS_SLICES(T_, 2)   \
+  else if (mt == 3) LS_SLICES(T_, 3) else LS_SLICES(T_, 4)
   if (dtype == kF32) {
     LS_SLICES_MT(float);
   } else if (dtype == kBF16) {
@@ -1561,6 +1604,7 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
   }
 #undef LS_SLICES_MT
 #undef LS_SLICES
+#undef LS_SLICES_AS
   return check_launch("gemm_slices");
 }
 

@@ -243,6 +243,29 @@ def test_rows_of_x_further_apart_than_offsets_of_32_bits_reach(dtype):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,k", [(40, 8), (100, 264), (1000, 1032), (4099, 2056), (6148, 4096), (9000, 4424)])
+def test_few_rows_read_by_whole_pieces_have_the_bits_of_element_by_element_reads(dtype, n, k):
+    """Rows of X one element behind a 16-byte boundary take the general loads, aligned ones buffer loads: columns that end inside a
+    block, slices that end inside a round of loads, walks of an even and an odd number of blocks; the slice sums likewise."""
+    from lockstep_amd.ops import STORE_F32
+
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    x = torch.randn(64, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+    off = torch.empty(64 * k + 8, dtype=dtype, device="cuda")[1:1 + 64 * k].view(64, k)
+    off.copy_(x)
+    for m in (1, 3, 16, 17, 40, 64):
+        a, b = (torch.full((m, n), float("nan"), device="cuda") for _ in range(2))
+        K().gemm(x[:m], w, a, STORE_F32)
+        K().gemm(off[:m], w, b, STORE_F32)
+        assert torch.equal(a, b), m
+        a, b = (torch.full((K().gemm_slices_count(k), m, n), float("nan"), device="cuda") for _ in range(2))
+        K().gemm_slices(x[:m], w, a)
+        K().gemm_slices(off[:m], w, b)
+        assert torch.equal(a, b), f"slice sums, {m}"
+
+
 # (rows, columns) that take each tile of the ring kernel, in the order of RingTile, with both ending inside a tile
 RING_TILE_SIZES = [(2041, 4448), (1003, 6176), (1501, 5408), (1003, 5408), (700, 5408), (500, 4128), (130, 5472), (300, 5472), (97, 96)]
 
