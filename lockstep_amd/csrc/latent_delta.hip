@@ -11,6 +11,7 @@
 
 #include "common.h"
 #include "ring.h"
+#include "row_piece.h"
 #include "mixers_api.h"
 
 namespace ls {
@@ -68,10 +69,11 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int e, int W
 // 1,024 elements, one run a thread, without the registers of further runs (2,048 rows, one slice, four copies of 1,024 elements 16.3 ->
 // 14.6 us, eight of 512 22.6 -> 18.6); and where seven or eight copies of longer rows are in registers, their first run is not
 // asked for in front of the barrier, and the registers are held to what three rows a CU need (seven of 2,048 43.4 -> 41.4, eight
-// 49.2 -> 48.3).
+// 49.2 -> 48.3).  WHOLE, rows of whole vectors of four, is an instance of its own: with the test at every load the compiler put each
+// into a block with the element-by-element loads behind it (eight rows of four copies of 1,024, 5.6 -> 5.1 us in a decode step).
 constexpr bool streams_ahead(int copies, bool one) { return one || copies <= 6; }
 constexpr int streams_rows_a_cu(int copies, bool one) { return streams_ahead(copies, one) ? 1 : 3; }
-template <typename T, int N, bool ONE>
+template <typename T, int N, bool ONE, bool WHOLE>
 __global__ __launch_bounds__(256, streams_rows_a_cu(N, ONE)) void streams_step_kernel(float* __restrict__ X, long ldx, int W,
                                                            const float* __restrict__ P, int slices, long p_stride,
                                                            const float* __restrict__ mix, const float* __restrict__ gain,
@@ -82,8 +84,7 @@ __global__ __launch_bounds__(256, streams_rows_a_cu(N, ONE)) void streams_step_k
   const int r_out = blockIdx.x;
   const long row = rows ? rows[r_out] : r_out;
   float* x = X + row * ldx;
-  // rows of whole vectors of four: a copy's elements and a slice's move as 16 bytes
-  const bool vec_ok = W % 4 == 0 && ldx % 4 == 0;
+  constexpr bool vec_ok = WHOLE;   // rows of whole vectors of four: a copy's elements and a slice's move as 16 bytes
   extern __shared__ float u_s[];   // what the row's read gave, until the row's sum of squares is known (a thread's own elements)
   const int e_first = 4 * (int)threadIdx.x;
   constexpr int BATCH = 8;         // slice sums requested together
@@ -309,29 +310,27 @@ __global__ __launch_bounds__(256) void latent_query_kernel(const float* __restri
 // ---------------------------------------------------------------------------
 // A product a head: out[t][head * o_stride + n] = sum_k w[head][n][k] x[t][head * x_stride + k], w [H][N][K].
 // A workgroup: 16 * RT rows of one head, four waves with 16 columns each.  The 16x16 MFMA atom with the weight rows
-// as first operand; a row's contraction is one chain over ascending K from zero.
+// as first operand; a row's contraction is one chain over ascending K from zero.  WHOLE (row_piece.h): rows that buffer loads
+// read (eight rows, sixteen heads of 128 x 128 3.5 -> 3.2 us in a decode step).
 // ---------------------------------------------------------------------------
-template <typename T, int RT>
+template <typename T, int RT, bool WHOLE>
 __global__ __launch_bounds__(256) void heads_product_kernel(const T* __restrict__ x, long ldx, int x_stride,
                                                             const T* __restrict__ w, int N, int K, int n_rows,
                                                             T* __restrict__ out, long ldo, int o_stride, int x_aligned,
                                                             int out_vec) {
   constexpr int VEC = Atom<T>::VEC, KC = Atom<T>::KCHUNK;
   const int head = blockIdx.y;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, quad = lane >> 4;
   const int col0 = (blockIdx.z * 4 + wv) * 16;
   if (col0 >= N) return;
   const bool w_ok = col0 + l16 < N;
-  const T* w_row = w + ((long)head * N + (w_ok ? col0 + l16 : 0)) * K;
+  const T* w_base = w + ((long)head * N + col0) * K;
   const int row0 = blockIdx.x * 16 * RT;
-  const T* x_row[RT];
+  const T* x_base = x + (long)row0 * ldx + (long)head * x_stride;
   bool x_ok[RT];
 #pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    x_ok[r] = row0 + 16 * r + l16 < n_rows;
-    x_row[r] = x + (long)(x_ok[r] ? row0 + 16 * r + l16 : 0) * ldx + (long)head * x_stride;
-  }
+  for (int r = 0; r < RT; ++r) x_ok[r] = row0 + 16 * r + l16 < n_rows;
   f32x4 acc[RT];
 #pragma unroll
   for (int r = 0; r < RT; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -342,10 +341,11 @@ __global__ __launch_bounds__(256) void heads_product_kernel(const T* __restrict_
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = k0 + u * KC + VEC * quad;
-      a[u] = load_vec<T>(w_row, 0, k, K, 0, w_ok, w_aligned);
+      a[u] = row_piece<T, WHOLE>(w_base, l16, k, K, K, w_ok, w_aligned);
 #pragma unroll
-      for (int r = 0; r < RT; ++r) b[u][r] = load_vec<T>(x_row[r], 0, k, K, 0, x_ok[r], x_aligned != 0);
+      for (int r = 0; r < RT; ++r) b[u][r] = row_piece<T, WHOLE>(x_base, 16 * r + l16, k, K, ldx, x_ok[r], x_aligned != 0);
     }
+    if constexpr (WHOLE) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -708,15 +708,18 @@ extern "C" int ls_streams_step(int dtype, float* X, long ldx, int n, int width, 
   const long p_stride = (long)p_rows * width;
   LS_REQUIRE(dtype == kF32 || dtype == kBF16, "streams_step: unknown dtype %d", dtype);
   const size_t lds = out ? (size_t)((width + 3) / 4) * 16 : 0;
-#define LS_STREAMS_AS(T_, N_, ONE_)                                                                                  \
-  hipLaunchKernelGGL((streams_step_kernel<T_, N_, ONE_>), dim3(n_rows), dim3(256), lds, s, X, ldx, width, P, slices, \
+  const bool whole = width % 4 == 0 && ldx % 4 == 0;
+#define LS_STREAMS_AS(T_, N_, ONE_) \
+  if (whole) LS_STREAMS_ROWS(T_, N_, ONE_, true); else LS_STREAMS_ROWS(T_, N_, ONE_, false)
+#define LS_STREAMS_ROWS(T_, N_, ONE_, WHOLE_)                                                                        \
+  hipLaunchKernelGGL((streams_step_kernel<T_, N_, ONE_, WHOLE_>), dim3(n_rows), dim3(256), lds, s, X, ldx, width, P, slices, \
                      p_stride, mix, gain, take, weight, bias, centred, eps, (T_*)out, ld_out, rows)
 #define LS_STREAMS(N_)                                                                                               \
   case N_:                                                                                                           \
     if (dtype == kF32) {                                                                                             \
-      if (width <= 1024) LS_STREAMS_AS(float, N_, true); else LS_STREAMS_AS(float, N_, false);                       \
+      if (width <= 1024) { LS_STREAMS_AS(float, N_, true); } else { LS_STREAMS_AS(float, N_, false); }               \
     } else {                                                                                                         \
-      if (width <= 1024) LS_STREAMS_AS(bf16_t, N_, true); else LS_STREAMS_AS(bf16_t, N_, false);                     \
+      if (width <= 1024) { LS_STREAMS_AS(bf16_t, N_, true); } else { LS_STREAMS_AS(bf16_t, N_, false); }             \
     }                                                                                                                \
     break;
   switch (n) {
@@ -724,6 +727,7 @@ extern "C" int ls_streams_step(int dtype, float* X, long ldx, int n, int width, 
   }
 #undef LS_STREAMS
 #undef LS_STREAMS_AS
+#undef LS_STREAMS_ROWS
   return check_launch("streams_step");
 }
 
@@ -802,8 +806,11 @@ extern "C" int ls_heads_product(int dtype, const void* x, long ldx, int x_stride
   const bool many = n_rows > 64;
   const int rows_a_block = many ? 64 : 16;
   const dim3 grid((n_rows + rows_a_block - 1) / rows_a_block, H, (N + 63) / 64);
-#define LS_HEADS(T_, RT_)                                                                                            \
-  hipLaunchKernelGGL((heads_product_kernel<T_, RT_>), grid, dim3(256), 0, s, (const T_*)x, ldx, x_stride, (const T_*)w, N, \
+  const bool whole = x_aligned && K % vec == 0 && 65 * std::max(ldx, (long)K) * (long)(16 / vec) <= kNoPiece;
+#define LS_HEADS(T_, RT_) \
+  if (whole) LS_HEADS_AS(T_, RT_, true); else LS_HEADS_AS(T_, RT_, false)
+#define LS_HEADS_AS(T_, RT_, WHOLE_)                                                                                 \
+  hipLaunchKernelGGL((heads_product_kernel<T_, RT_, WHOLE_>), grid, dim3(256), 0, s, (const T_*)x, ldx, x_stride, (const T_*)w, N, \
                      K, n_rows, (T_*)out, ldo, o_stride, x_aligned, out_vec)
   if (dtype == kF32) {
     if (many) LS_HEADS(float, 4); else LS_HEADS(float, 1);
@@ -811,6 +818,7 @@ extern "C" int ls_heads_product(int dtype, const void* x, long ldx, int x_stride
     if (many) LS_HEADS(bf16_t, 4); else LS_HEADS(bf16_t, 1);
   }
 #undef LS_HEADS
+#undef LS_HEADS_AS
   return check_launch("heads_product");
 }
 

@@ -155,6 +155,22 @@ def test_a_product_a_head(dtype, heads, n, kk, rows):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, n, kk, rows", [(2, 20, 8, 5), (3, 64, 136, 16), (2, 72, 40, 64), (2, 33, 264, 130)])
+def test_a_product_a_head_of_aligned_rows_has_the_bits_of_others(dtype, heads, n, kk, rows):
+    """Aligned rows are read by buffer loads, rows an odd number of elements apart one element at a time: columns, rows and
+    contractions that end inside a block."""
+    g = torch.Generator().manual_seed(heads * n + kk)
+    x = torch.randn((rows, heads * kk), generator=g).to(dtype).cuda()
+    apart = torch.zeros((rows, heads * kk + 3), dtype=dtype, device="cuda")
+    apart[:, :heads * kk] = x
+    w = torch.randn((heads, n, kk), generator=g).to(dtype).cuda()
+    out, want = (torch.zeros((rows, heads * n), dtype=dtype, device="cuda") for _ in range(2))
+    K().heads_product(x, kk, w, out, n)
+    K().heads_product(apart, kk, w, want, n)
+    assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_the_passes_around_attention_over_a_latent(dtype):
     """Norms of both latents, the shared key part rotated into the pages at the tokens' positions, the queries'
     rotated part behind the latent's dimensions; two requests at different positions on scattered pages."""
