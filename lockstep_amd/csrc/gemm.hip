@@ -1159,16 +1159,17 @@ static bool ring_takes(int M, int N, int K) {
 // float32 multiplies longer than it loads, so every CU that has a tile counts, up to six rounds (64 x 4,096 x 1,024 17.6 / 10.2, 8 x
 // 24,576 x 1,024 29.3 / 24.0, 33 x 24,576 x 1,024 40 / 35, 128 x 10,240 x 4,096 145 / 105; 2,000 x 1,024 x 1,024, eight rounds, 40.4 / 42.3); up to 64
 // rows over columns that 64 x 32 tiles cover in one round keep those.  A wave a slice stays ahead where a tile's one chain of
-// products is the longer way: up to 24 rows of few columns (17 x 2,048 x 2,048 14.9 / 16.4, 17 x 4,096 x 512 7.0 / 6.0), one to four of long K (1 x
-// 6,144 x 4,096 29.7 / 31.7, 8 rows 35.5 / 32.5), SwiGLU of few rows and columns (1 x 2,048 x 1,024 9.2 / 10.0, 1 x 6,144 x 1,024 11.2 / 10.4).
+// products is the longer way (its times / 32 x 32): up to 32 rows of few columns (32 x 2,048 x 1,024 8.3 / 9.5, 32 x 4,096 x 4,096 27.3 / 30.0; 32 x
+// 6,144 x 1,024 14.0 / 10.0), eight of up to a round and a half (8 x 6,144 x 4,096 23.0 / 30.1, 1 x 12,288 x 1,024 11.2 / 14.0; 16 x 8,192 x 2,048
+// 19.1 / 17.5), SwiGLU of 16 in a round (8 x 6,144 x 1,024 9.4 / 10.7; 8 x 12,288 x 1,024 15.9 / 14.6, 16 x 8,192 x 512 7.6 / 7.0).
 template <typename T, int EPI>
 static int narrow_tile(int M, int N, int K) {
   const long cus = compute_units();
   const long rows = (M + 31) / 32, small = rows * ((N + 31) / 32), wide = rows * ((N + 63) / 64);
   if (sizeof(T) == 4) {
-    if (EPI != kSwiGLU && (N + 15) / 16 <= cus && M <= (K <= 512 ? 16 : K <= 1024 || N > 512 ? 24 : 32)) return -1;
-    if (EPI != kSwiGLU && M <= 4 && K > 2048 && (N + 31) / 32 <= cus) return -1;
-    if (M <= 16 && (K < 256 || (EPI == kSwiGLU && (N + 31) / 32 <= (K > 1024 ? cus : cus / 2)))) return -1;
+    if (EPI != kSwiGLU && (N + 15) / 16 <= cus && M <= (K <= 512 ? 16 : K <= 1024 && N <= 1024 ? 24 : 32)) return -1;
+    if (EPI != kSwiGLU && M <= 8 && K >= 512 && 2 * small <= 3 * cus) return -1;
+    if (M <= 16 && (K < 256 || (EPI == kSwiGLU && (N + 31) / 32 <= (K > 512 ? cus : cus / 2)))) return -1;
     return small <= cus || (small <= 6 * cus && (EPI == kSwiGLU || M > 64 || (N + 31) / 32 > cus)) ? kRing32x32 : -1;
   }
   if (M <= 16 && EPI != kSwiGLU && (N + 15) / 16 <= cus && K > 320) return -1;
@@ -1458,9 +1459,10 @@ struct SlicesPlan {
 };
 // bfloat16: the cheaper of 32 x 64 and 64 x 64 tiles with one, two or four slices a workgroup, a stage 0.18 and 0.25 us where a CU has one
 // workgroup, twice that where it has two, and a round about four stages besides.  Before (64 x 64, every CU a workgroup or another
-// kernel) / now, us: 8 x 4,096 x 4,096 10.9 / 8.4, 8 x 4,096 x 12,288 24.0 / 21.8, 17 x 1,024 x 3,072 4.3 / 4.0, 64 x 1,024 x 2,048 5.4 / 4.2, 64 x 1,024 x
+// kernel) / now, us: 8 x 4,096 x 4,096 10.9 / 8.4, 8 x 4,096 x 12,288 24.0 / 21.8, 64 x 1,024 x 2,048 5.4 / 4.2, 64 x 1,024 x
 // 3,072 6.7 / 5.0, 64 x 4,096 x 4,096 13.3 / 12.8, 97 x 1,024 x 2,048 5.2 / 5.0.  One row 5,120 x 8,192 19.4 / 20.8, hence four rows at least; 17 to
-// 32 rows of less than five slices over few columns 3.8 / 4.0.  From 65 rows on longer runs of stages lose what fewer rounds gain (128 x 5,120 x
+// 32 rows of less than five slices over few columns 3.8 / 4.0, and of up to twelve over the fewest, by a wave a slice / tiles (17 x 1,024 x 2,048
+// 3.1 / 3.8, 32 rows 3.5 / 3.9, 24 x 1,024 x 3,072 4.4 / 4.6; 32 rows 4.9 / 4.7, 24 x 2,048 x 2,048 5.0 / 4.8).  From 65 rows on longer runs of stages lose what fewer rounds gain (128 x 5,120 x
 // 5,120 with one, two and four slices a workgroup 28, 30, 31).
 static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
   const int kslice = kslice_for(K), nslices = (K + kslice - 1) / kslice;
@@ -1472,7 +1474,7 @@ static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
     while (per > 1 && workgroups(per) < (per * a_slice > 8 ? 2 * cus : cus)) per = (per + 1) / 2;
     return workgroups(per) >= cus ? SlicesPlan{kRing64x64, per} : SlicesPlan{kRing64x64, 0};
   }
-  if (M <= 32 && nslices < 5) return {kRing32x64, 0};
+  if (M <= 32 && (nslices < 5 || (N <= 1024 && nslices <= (M <= 24 ? 12 : 8)))) return {kRing32x64, 0};
   SlicesPlan best{kRing64x64, 0};
   float least = 0.f;
   for (int rows = 32; rows <= 64; rows += 32)

@@ -340,10 +340,12 @@ def test_products_on_both_sides_of_the_lines_between_the_kernels_have_the_same_b
 
 # (rows, columns, K, whether SwiGLU) on both sides of the lines of the narrow tiles, and rows times columns of the tile (0: none)
 NARROW_LINES = {
-    torch.float32: [(16, 4096, 264, False, 0), (17, 4096, 512, False, 1024), (24, 4096, 516, False, 0), (25, 4093, 516, False, 1024),
-                    (32, 512, 1028, False, 0), (32, 513, 1028, False, 1024), (4, 8192, 2056, False, 0), (5, 8192, 2056, False, 1024),
+    torch.float32: [(16, 4096, 264, False, 0), (17, 4096, 512, False, 1024), (32, 4096, 516, False, 0), (33, 4093, 516, False, 1024),
+                    (24, 1024, 1024, False, 0), (25, 1024, 1024, False, 1024), (32, 1025, 1024, False, 0), (32, 513, 1028, False, 0),
+                    (8, 12288, 512, False, 0), (8, 12320, 512, False, 1024), (8, 8192, 508, False, 1024), (9, 8192, 512, False, 1024),
                     (16, 8224, 248, False, 0), (16, 8211, 264, False, 1024), (64, 4112, 264, False, 0), (65, 4112, 264, False, 1024),
-                    (97, 12289, 72, False, 0), (33, 24544, 72, True, 1024), (16, 4096, 264, True, 0), (16, 4128, 264, True, 1024)],
+                    (97, 12289, 72, False, 0), (33, 24544, 72, True, 1024), (16, 4096, 264, True, 0), (16, 4128, 264, True, 1024),
+                    (16, 8192, 520, True, 0), (16, 8224, 520, True, 1024), (17, 8192, 520, True, 1024)],
     torch.bfloat16: [(16, 4096, 328, False, 0), (16, 4109, 328, False, 1024), (1, 1000, 320, False, 1024), (17, 24, 8, False, 1024),
                      (5, 4096, 1032, True, 1024), (33, 4096, 72, False, 1024), (33, 4097, 72, False, 2048), (64, 8192, 264, False, 2048),
                      (64, 8193, 264, False, 0), (97, 4091, 72, False, 2048), (97, 4097, 72, False, 0), (257, 909, 4424, False, 2048),
