@@ -240,9 +240,10 @@ __global__ __launch_bounds__(64 * (DEC ? 1 : kMaxWaves)) void sink_attention_ker
           if constexpr (kKeepQ) {
             Atom<T>::mma(s[r][half], now.kv[half][c], qv[r][c]);
           } else {
+            // (with a choice, or the compiler would keep all of these in registers it does not have)
             const bool in = c * KC + VEC * quad + VEC <= D;
             Atom<T>::mma(s[r][half], now.kv[half][c],
-                         load_piece<T>(q_row[r] + (in ? c * KC + VEC * quad : 0), in));
+                         load_or_zero<T>(q_row[r] + (in ? c * KC + VEC * quad : 0), row_ok[r] && in));
           }
         }
       }
