@@ -23,7 +23,8 @@ __device__ __forceinline__ typename Atom<T>::vec_t row_piece(const T* __restrict
     __asm__("" : "+v"(offset));  // (a choice of offsets, not a branch to one of two loads)
     return __builtin_bit_cast(typename Atom<T>::vec_t, __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, 0));
   } else {
-    return load_vec<T>(base, row, k, limit, ld, ok && any, aligned);
+    if (!any) return Atom<T>::zero();  // (load_vec may read at `base` for a lane without a piece)
+    return load_vec<T>(base, row, k, limit, ld, ok, aligned);
   }
 }
 

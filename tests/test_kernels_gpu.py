@@ -266,6 +266,26 @@ def test_few_rows_read_by_whole_pieces_have_the_bits_of_element_by_element_reads
         assert torch.equal(a, b), f"slice sums, {m}"
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k,n", [(2048, 9000), (4096, 8209)])
+def test_walks_over_aligned_rows_too_far_apart_for_whole_pieces(dtype, k, n):
+    """Three rows of X whose distance puts 65 of them past 2 GiB: the streaming kernel's general instance, whose walks end at
+    different blocks, with the bits of the rows side by side."""
+    from lockstep_amd.ops import STORE_F32
+
+    size = torch.finfo(dtype).bits // 8
+    ldx = (1 << 25) // size + 16
+    g = torch.Generator(device="cuda").manual_seed(size + k)
+    near = torch.randn(3, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
+    far = torch.empty(2 * ldx + k, dtype=dtype, device="cuda").as_strided((3, k), (ldx, 1))
+    far.copy_(near)
+    out, want = (torch.empty(3, n, device="cuda") for _ in range(2))
+    K().gemm(far, w, out, STORE_F32)
+    K().gemm(near, w, want, STORE_F32)
+    assert torch.equal(out, want)
+
+
 # (rows, columns) that take each tile of the ring kernel, in the order of RingTile, with both ending inside a tile
 RING_TILE_SIZES = [(2041, 4448), (1003, 6176), (1501, 5408), (1003, 5408), (700, 5408), (500, 4128), (130, 5472), (300, 5472), (97, 96)]
 
