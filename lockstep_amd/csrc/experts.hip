@@ -858,12 +858,12 @@ struct ExpertTile {
     const int stages = (K + 128 / (int)sizeof(T) - 1) / (128 / (int)sizeof(T));
     auto request_w = [&](int st, int buf, int n) LS_INLINED {
       const int k = st * 128;
-      buffer_to_lds16(k < limit ? w_off + k + (unsigned)((long)w_row(n) * K * sizeof(T)) : ~0u, w,
+      buffer_to_lds16(k < limit ? w_off + k + (unsigned)((long)w_row(n) * K * sizeof(T)) : kNothing, w,
                       lds0 + buf * Product::W_BYTES + n * NW * 1024);
     };
     auto request_x = [&](int st, int buf, int n) LS_INLINED {
       const int k = st * 128;
-      buffer_to_lds16(k < limit && x_at[n] != ~0u ? x_at[n] + k + piece : ~0u, x,
+      buffer_to_lds16(k < limit && x_at[n] != kNothing ? x_at[n] + k + piece : kNothing, x,
                       lds0 + S * Product::W_BYTES + buf * Product::X_BYTES + n * NW * 1024);
     };
     product.run(ring + (wave() % NWN) * (WEIGHTS / NWN) * 128, ring + S * Product::W_BYTES + (wave() / NWN) * (ROWS / NWM) * 128, stages,
@@ -919,7 +919,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void experts_gate_up_ring_kernel(co
 #pragma unroll
   for (int i = 0; i < Tile::LX; ++i) {
     const int r = Tile::loaded_row(i);
-    x_at[i] = r < rows ? (unsigned)((long)(order[first + r] / top) * ldx * sizeof(T)) : ~0u;
+    x_at[i] = r < rows ? (unsigned)((long)(order[first + r] / top) * ldx * sizeof(T)) : kNothing;
   }
   const long left = (long)(F - col0) * K * sizeof(T), from = ((long)e * F + col0) * K;
   Tile t;
@@ -979,7 +979,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void experts_down_ring_kernel(const
 #pragma unroll
   for (int i = 0; i < Tile::LX; ++i) {
     const int r = Tile::loaded_row(i);
-    x_at[i] = r < rows ? (unsigned)(r * ldy * sizeof(T)) : ~0u;
+    x_at[i] = r < rows ? (unsigned)(r * ldy * sizeof(T)) : kNothing;
   }
   Tile t;
   t.run(buffer_of(act + (long)first * ldy, ((long)(rows - 1) * ldy + F) * sizeof(T)), x_at,
@@ -1189,7 +1189,7 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
   const long across = 128 * std::max({(long)K, (long)F, ldy}), all_of_x = (n_tokens - 1) * ldx + K;
   const long wgs_up = tile_grid((F + 63) / 64, cap), wgs_down = tile_grid((N + 63) / 64, cap);
   const bool staged = rows_a_tile == 64 && K % vec == 0 && F % vec == 0 && ldx % vec == 0 && ldy % vec == 0 &&
-                      std::max(across, all_of_x) * (16 / vec) + 128 <= 0xffffffffL && std::max(wgs_up, wgs_down) < (1L << 22) &&
+                      std::max(across, all_of_x) * (16 / vec) + 128 <= (long)kNothing && std::max(wgs_up, wgs_down) < (1L << 22) &&
                       (dtype == kF32 ? ring_lds_ready<float>() : ring_lds_ready<bf16_t>());
   const int vec_out = N % 4 == 0 && reinterpret_cast<uintptr_t>(P) % 16 == 0;
 #define LS_EXPERTS_STAGED(T_)                                                                                         \

@@ -1182,7 +1182,7 @@ static int narrow_tile(int M, int N, int K) {
 
 // Whether the ring kernel's 32-bit byte offsets inside a tile reach every operand: the rows of the largest tile, and what
 // the last stage reads behind the last row.  (Rows further apart go to the other kernels, which form 64-bit addresses.)
-static bool ring_reaches(long ldx, long K, long size) { return (256 * std::max(ldx, K) + 128) * size <= 0xffffffffL; }
+static bool ring_reaches(long ldx, long K, long size) { return (256 * std::max(ldx, K) + 128) * size <= (long)kNothing; }
 
 // Dynamic LDS beyond 64 KB has to be granted per kernel (once).
 template <typename T, int EPI, int BM, int BN, int NWM, int NWN, int WS, int XS, int SUB>

@@ -73,12 +73,12 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_ring_kernel(const T* __re
 
   auto request_w = [&](int st, int buf, int n) LS_INLINED {
     const int i = n / SUB, part = n % SUB, k = ((first_stage + st) * SUB + part) * 128;
-    buffer_to_lds16(k < limit ? w_off + k + i * w_step : ~0u, w_buffer,
+    buffer_to_lds16(k < limit ? w_off + k + i * w_step : kNothing, w_buffer,
                     lds0 + buf * Product::W_BYTES + part * BN * 128 + i * NW * 1024);
   };
   auto request_x = [&](int st, int buf, int n) LS_INLINED {
     const int i = n / SUB, part = n % SUB, k = ((first_stage + st) * SUB + part) * 128;
-    buffer_to_lds16(k < limit ? x_off + k + i * x_step : ~0u, x_buffer,
+    buffer_to_lds16(k < limit ? x_off + k + i * x_step : kNothing, x_buffer,
                     lds0 + WS * Product::W_BYTES + buf * Product::X_BYTES + part * BM * 128 + i * NW * 1024);
   };
   Product product;

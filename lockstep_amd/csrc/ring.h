@@ -9,13 +9,17 @@ namespace ls {
 
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
 
-// A buffer descriptor over `bytes` bytes from `p`: loads at offsets from there on return zeros.
+// The offset of a load that is to read nothing, and the most bytes a descriptor is given: an operand that goes on for 4 GiB and
+// more ends there for the hardware too, and neither this offset nor its sixteen bytes come round to the operand's start.
+constexpr unsigned kNothing = 0xfffffff0u;
+
+// A buffer descriptor over `bytes` bytes from `p` (kNothing of them at most): loads at offsets from there on return zeros.
 __device__ __forceinline__ u32x4_t buffer_of(const void* p, long bytes) {
   const unsigned long a = reinterpret_cast<unsigned long>(p);
   u32x4_t r;
   r[0] = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a));
   r[1] = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a >> 32) & 0xffffu);
-  r[2] = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(bytes > 0xffffffffL ? 0xffffffffL : bytes));
+  r[2] = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(bytes > (long)kNothing ? (long)kNothing : bytes));
   r[3] = 0x00020000u;
   return r;
 }

@@ -243,6 +243,30 @@ def test_rows_of_x_further_apart_than_offsets_of_32_bits_reach(dtype):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("big", ["weights", "rows"])
+def test_what_a_stage_reads_behind_the_last_column_of_an_operand_of_4_gib(big):
+    """An operand that goes on for more than 4 GiB behind the first tile, K that ends inside a stage: the last stage's loads behind K
+    read zeros and not the operand, whatever its bytes are a byte off.  The first and the last tile have the bits of the same rows alone."""
+    from lockstep_amd.ops import STORE_F32
+
+    k, many, few = 4104, 530_000, 97                             # 4.05 GiB
+    g = torch.Generator(device="cuda").manual_seed(k)
+    large = torch.empty(many, k, dtype=torch.bfloat16, device="cuda").normal_(0, 0.1, generator=g)
+    small = torch.randn(few, k, generator=g, device="cuda").to(torch.bfloat16)
+    x, w = (small, large) if big == "weights" else (large, small)
+    out = torch.empty(x.shape[0], w.shape[0], device="cuda")
+    K().gemm(x, w, out, STORE_F32)
+    for part in (slice(0, 300), slice(many - 300, many)):
+        a, b = (x, w[part]) if big == "weights" else (x[part], w)
+        want = torch.empty(a.shape[0], b.shape[0], device="cuda")
+        K().gemm(a, b, want, STORE_F32)
+        assert torch.equal(out[:, part] if big == "weights" else out[part], want)
+        exact = a[:4].double() @ b.double().T
+        assert rel_err(want[:4], exact) < 2e-5
+    del large, x, w, out
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,k", [(40, 8), (100, 264), (1000, 1032), (4099, 2056), (6148, 4096), (9000, 4424)])
 def test_few_rows_read_by_whole_pieces_have_the_bits_of_element_by_element_reads(dtype, n, k):
