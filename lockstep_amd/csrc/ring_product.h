@@ -33,8 +33,13 @@
 // as its last product is issued, at least TJ * TI / 2 products before its next use.  With the barrier between the second half's two
 // groups nothing is read from a stage that is not whole, and the reads that the barrier waits for are a group old.
 //
-// Parts of 256 and 512 bytes (SUB 2, 4) have a barrier and an LDS latency every 128 (256) elements of K: worth it where few products stand between
+// Stages of two parts (SUB 2) have a barrier and an LDS latency every 128 elements of K: worth it where few products stand between
 // two barriers and one workgroup has the CU (97 x 1,024 x 2,048 in tiles of 64 x 64: 10.2 / 9.4 us), not where a second one fills the gaps.
+//
+// float32 multiplies four times as long a byte: with four tiles a wave the compiler's own order has products enough between a read and
+// its use, and the order above only holds products back (us, above / compiler's: 128 x 6,144 x 5,120 102.0 / 99.0, 256 x 3,072 x 12,288
+// 238 / 229, SwiGLU 256 x 4,096 x 4,096 85.6 / 79.5, slice sums 40 x 10,240 x 8,192 102.1 / 94.0; 2,000 x 6,144 x 1,024 level).  With one
+// or two tiles it stays ahead (32 x 32, 128 x 4,096 x 12,288 136 / 153).
 #pragma once
 
 #include <type_traits>
@@ -54,10 +59,16 @@ struct RingProduct {
   static constexpr int LDS_BYTES = WS * W_BYTES + XS * X_BYTES;
   static constexpr bool IN_PLACE = SUB == 1 && TI % 2 == 0 && TI * TJ >= 8;
   static constexpr bool TAIL = TI * TJ < 24;
+  static constexpr bool ORDERED = sizeof(T) == 2 || TI * TJ < 4;
   static_assert(WS >= XS && XS >= 2 && WS >= 3, "rings");
+  static_assert(!TAIL || WS <= XS + 1, "X's last stage is requested before the tail begins");
   static_assert(LDS_BYTES <= 160 * 1024, "the rings fit the LDS of a CU");
 
   f32x4 total[TI][TJ], acc[TI][TJ];  // [weight tile][row tile]
+
+  static __device__ __forceinline__ void in_order() {
+    if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
+  }
 
   template <bool FIRST>  // FIRST: the tile's first product of a slice
   __device__ __forceinline__ void product(int i, int j, const vec_t& a, const vec_t& b) {
@@ -142,7 +153,7 @@ struct RingProduct {
 #pragma unroll
           for (int i = 0; i < TI; ++i) a[set][u][i] = w_frag(wbuf, i, half * SUB + u);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        in_order();
       };
       auto multiply = [&](auto first, int set, auto load, auto loads) LS_INLINED {
         constexpr int ROWS = SUB * TI, L = decltype(loads)::value;
@@ -158,7 +169,7 @@ struct RingProduct {
               if (u == 0) product<decltype(first)::value>(i, j, a[set][u][i], b[set][u][j]);
               else product<false>(i, j, a[set][u][i], b[set][u][j]);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            in_order();
           }
       };
       read(0, 0, 0, 0);
@@ -190,7 +201,7 @@ struct RingProduct {
 #pragma unroll
           for (int i = I0; i < I0 + G; ++i) product<decltype(first)::value>(i, j, a[i], b[j]);
           then(j);
-          __builtin_amdgcn_sched_barrier(0);
+          in_order();
         }
       };
       auto read_a = [&](int group, int c) LS_INLINED {
@@ -222,7 +233,7 @@ struct RingProduct {
         wb = after(wb, WS);
         xb = after(xb, XS);
         read_a(0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        in_order();
         columns(no, high, [&](int j) LS_INLINED {
 #pragma unroll
           for (int n = 0; n < LX; ++n)
