@@ -501,7 +501,11 @@ __device__ __forceinline__ float lanes_sum(float v) {
 }
 
 // The last M - 1 inputs of the channels c, c + step, ...: place a holds the input at position kv_len - (M - 1) + a, one of this
-// step's, or one the state already holds further on.
+// step's, or one the state already holds further on.  SETTLE: every load is used on every path.  One that might still be on its way to
+// its register when the recurrence reuses that was waited for in each of the recurrence's blocks, with all but seven of the loads that are
+// ahead there (2,048 tokens 301 / 290 us).  With a decay a channel the compiler finds other registers, and the wait itself costs (16 heads
+// over 8 of 128 x 128 352 / 338 without it, 4 over 2 of 96 x 80 313 / 302).
+template <bool SETTLE>
 __device__ __forceinline__ void keep_inputs(const float* __restrict__ raw, long ld, int C, int M, const SeqMeta& m, float* __restrict__ kept,
                                             int c, int step) {
   for (; c < C; c += step) {
@@ -517,10 +521,9 @@ __device__ __forceinline__ void keep_inputs(const float* __restrict__ raw, long 
 #pragma unroll
       for (int u = 0; u < kAtOnce; ++u)
         if (a0 + u < M - 1) kept[(long)(a0 + u) * C + c] = v[u];
-      // (every load is used on every path: one that might still be on its way to its register when the recurrence reuses that
-      // was waited for in each of the recurrence's blocks, with all but seven of the loads that are ahead there)
+      if constexpr (SETTLE)
 #pragma unroll
-      for (int u = 0; u < kAtOnce; ++u) __asm__ volatile("" ::"v"(v[u]));
+        for (int u = 0; u < kAtOnce; ++u) __asm__ volatile("" ::"v"(v[u]));
     }
   }
 }
@@ -647,7 +650,7 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(const float* __restrict_
     }
   }
   if (M > 1)
-    keep_inputs(raw, ld, C, M, m, state + (long)m.table_row * state_stride + conv_at, (head * (int)gridDim.y + (int)blockIdx.y) * 64 + lane,
+    keep_inputs<!CH>(raw, ld, C, M, m, state + (long)m.table_row * state_stride + conv_at, (head * (int)gridDim.y + (int)blockIdx.y) * 64 + lane,
                 64 * H * (int)gridDim.y);
   auto next_block = [&]() LS_INLINED {
     qk_at += (long)DEPTH * 2 * G * dp;
