@@ -809,7 +809,10 @@ extern "C" int ls_heads_product(int dtype, const void* x, long ldx, int x_stride
   const bool many = n_rows > 64;
   const int rows_a_block = many ? 64 : 16;
   const dim3 grid((n_rows + rows_a_block - 1) / rows_a_block, H, (N + 63) / 64);
-  const bool whole = x_aligned && K % vec == 0 && 65 * std::max(ldx, (long)K) * (long)(16 / vec) <= kNoPiece;
+  // (many rows of bfloat16 are bound by their products, and a last round of loads that is not whole is multiplied to its end: 2,048 rows, 32
+  // heads of 64 x 192 18.6 / 17.7 us by the general loads, of 64 x 128 12.1 / 12.3, eight of 40 x 24 3.0 / 3.4)
+  const bool padded = dtype == kBF16 && many && K > 64 && K % 128 != 0;
+  const bool whole = x_aligned && !padded && 65 * std::max(ldx, (long)K) * (long)(16 / vec) <= kNoPiece;
 #define LS_HEADS(T_, RT_) \
   if (whole) LS_HEADS_AS(T_, RT_, true); else LS_HEADS_AS(T_, RT_, false)
 #define LS_HEADS_AS(T_, RT_, WHOLE_)                                                                                 \
