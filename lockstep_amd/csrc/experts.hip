@@ -879,20 +879,24 @@ constexpr int kDownCols = sizeof(T) == 4 ? 64 : 128;
 // Workgroups go round the eight XCDs: units of four tiles (mostly one expert's) by four columns stay on one, so that a unit's rows
 // and weights are read from beyond an L2 once.  How many of the cap tiles are used nobody knows here: the units go round the XCDs in
 // turn, which leaves an XCD at most one unit behind another (whole runs of tiles an XCD, 20 tiles by 11 columns: 47 us for 32; gate and up
-// above with units of one, two and four tiles by all columns 70, 56, 56, of four by two, four and eight columns 55, 51, 63).
+// above with units of one, two and four tiles by all columns 70, 56, 56, of four by two, four and eight columns 55, 51, 63).  float32, bound by
+// the CUs that have a workgroup, evens them out with units of two by two (2,048 tokens with 2 of 16 experts, width 256, 128 a piece, both products
+// 29.7 / 22.1; 260 with 2 of 2, 7,168 and 2,048 631 / 602; others within 2 %).
 // False: no such tile.
-constexpr int kUnitTiles = 4, kUnitColumns = 4;
+template <typename T>
+constexpr int kUnit = sizeof(T) == 4 ? 2 : 4;  // tiles, and columns
+template <int U>
 __device__ __forceinline__ bool tile_and_column(int columns, int cap, int& tile, int& column) {
-  constexpr int UNIT = kUnitTiles * kUnitColumns;
-  const int at = blockIdx.x >> 3, unit = at / UNIT * 8 + (blockIdx.x & 7), in_unit = at % UNIT;
-  const int across = (columns + kUnitColumns - 1) / kUnitColumns;
-  tile = unit / across * kUnitTiles + in_unit % kUnitTiles;
-  column = unit % across * kUnitColumns + in_unit / kUnitTiles;
+  const int at = blockIdx.x >> 3, unit = at / (U * U) * 8 + (blockIdx.x & 7), in_unit = at % (U * U);
+  const int across = (columns + U - 1) / U;
+  tile = unit / across * U + in_unit % U;
+  column = unit % across * U + in_unit / U;
   return tile < cap && column < columns;
 }
+template <int U>
 static long tile_grid(int columns, int cap) {
-  const long units = (long)((cap + kUnitTiles - 1) / kUnitTiles) * ((columns + kUnitColumns - 1) / kUnitColumns);
-  return (units + 7) / 8 * 8 * kUnitTiles * kUnitColumns;
+  const long units = (long)((cap + U - 1) / U) * ((columns + U - 1) / U);
+  return (units + 7) / 8 * 8 * U * U;
 }
 
 template <typename T, int WEIGHTS, int NWM, int NWN>
@@ -909,7 +913,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void experts_gate_up_ring_kernel(co
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
   constexpr int COLS = WEIGHTS / 2;
   int tile, column;
-  if (!tile_and_column((F + COLS - 1) / COLS, cap, tile, column)) return;
+  if (!tile_and_column<kUnit<T>>((F + COLS - 1) / COLS, cap, tile, column)) return;
   const int e = tiles[4 * tile];
   if (e < 0 || e >= real) return;
   const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
@@ -965,7 +969,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void experts_down_ring_kernel(const
   typedef ExpertTile<T, COLS, NWM, NWN> Tile;
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
   int tile, column;
-  if (!tile_and_column((N + COLS - 1) / COLS, cap, tile, column)) return;
+  if (!tile_and_column<kUnit<T>>((N + COLS - 1) / COLS, cap, tile, column)) return;
   const int e = tiles[4 * tile];
   if (e < 0) return;
   const int first = tiles[4 * tile + 1], rows = tiles[4 * tile + 2];
@@ -1185,18 +1189,22 @@ extern "C" int ls_experts_apply(int dtype, const void* x, long ldx, const void* 
                        shared_of((T_*)nullptr));                                                                      \
   } while (0)
   // tiles of 64 rows go through LDS where every row of every operand starts on a 16-byte boundary, 32-bit offsets reach the
-  // rows (all of x, whose rows are picked; 128 of the weights, 64 of act), and a grid has room for the tiles.  Rows further apart go to the kernel that forms 64-bit addresses.
+  // rows (all of x, whose rows are picked; 128 of the weights, 64 of act), and a grid of 512 threads a workgroup has room
+  // for the tiles (2^32 threads).  Rows further apart go to the kernel that forms 64-bit addresses.
   const long across = 128 * std::max({(long)K, (long)F, ldy}), all_of_x = (n_tokens - 1) * ldx + K;
-  const long wgs_up = tile_grid((F + 63) / 64, cap), wgs_down = tile_grid((N + 63) / 64, cap);
+  auto grid_of = [&](int width, int columns) {
+    return dtype == kF32 ? tile_grid<kUnit<float>>((width + columns - 1) / columns, cap) : tile_grid<kUnit<bf16_t>>((width + columns - 1) / columns, cap);
+  };
+  const long wgs_up = grid_of(F, 64), wgs_down = grid_of(N, dtype == kF32 ? kDownCols<float> : kDownCols<bf16_t>);
   const bool staged = rows_a_tile == 64 && K % vec == 0 && F % vec == 0 && ldx % vec == 0 && ldy % vec == 0 &&
-                      std::max(across, all_of_x) * (16 / vec) + 128 <= (long)kNothing && std::max(wgs_up, wgs_down) < (1L << 22) &&
+                      std::max(across, all_of_x) * (16 / vec) + 128 <= (long)kNothing && std::max(wgs_up, wgs_down) < (1L << 23) &&
                       (dtype == kF32 ? ring_lds_ready<float>() : ring_lds_ready<bf16_t>());
   const int vec_out = N % 4 == 0 && reinterpret_cast<uintptr_t>(P) % 16 == 0;
 #define LS_EXPERTS_STAGED(T_)                                                                                         \
   do {                                                                                                                \
     hipLaunchKernelGGL((LS_EXPERTS_UP(T_)), dim3(wgs_up), dim3(512), kUpLds<T_>, s, (const T_*)x, ldx, (const T_*)w_gate,  \
                        (const T_*)w_up, F, K, top, order, tiles, cap, limit, alpha, shift, in_weight, (T_*)act, ldy, real, n_tokens); \
-    hipLaunchKernelGGL((LS_EXPERTS_DOWN(T_)), dim3(tile_grid((N + kDownCols<T_> - 1) / kDownCols<T_>, cap)), dim3(512),    \
+    hipLaunchKernelGGL((LS_EXPERTS_DOWN(T_)), dim3(wgs_down), dim3(512), \
                        kDownLds<T_>, s, (const T_*)act, ldy, (const T_*)w_down, N, F, top, n_tokens, order, tiles, cap, out_weight, P, \
                        (const T_*)x, ldx, weight, real, vec_out);                                                     \
   } while (0)
