@@ -1081,6 +1081,16 @@ constexpr RingShape kRingShapes[kRingTiles] = {
     {192, 128, 1, 0.73f, 0.73f}, {128, 128, 1, 0.58f, 0.58f}, {128, 64, 1, 0.43f, 0.43f},  {64, 128, 2, 0.52f, 0.74f},
     {64, 64, 2, 0.33f, 0.52f}};
 
+// What `tiles` workgroups cost that a CU holds a_cu of: each round `start` and, for each of a workgroup's stages, stage[n - 1] where the fullest CU
+// has n of them.  (Microseconds; a cost, to compare tiles by, and not a time.)
+static float rounds_cost(long tiles, int a_cu, int stages, float start, const float* stage) {
+  const long cus = compute_units(), rest = tiles % (cus * a_cu);
+  float cost = (float)(tiles / (cus * a_cu)) * (start + stage[a_cu - 1] * stages);
+  if (rest) cost += start + stage[(rest + cus - 1) / cus - 1] * stages;
+  return cost;
+}
+constexpr float kStages64x64[3] = {0.59f, 1.15f, 1.7f};  // float32
+
 // The tile whose rounds of workgroups take least by that table.  (Every tile forced in turn over 65 to 2,048 rows and nine
 // shapes of weights: within 2 % of the best one everywhere.)  Two rules stand in front of it: up to 64 rows whose rows of
 // weights lie a multiple of 4 KB apart take 64 x 64 tiles (128 such rows asked for together meet in few memory channels: 16 x
@@ -1447,45 +1457,37 @@ extern "C" int ls_gemm_slices_max_rows(int dtype, int K) {
 
 namespace ls {
 
-// Rows from which the slice sums of a product come from the ring kernel.
-static int slices_ring_from(int dtype, int N, int K) {
-  if (dtype == kF32) return 33;
-  return (long)N * K * 2 >= (32L << 20) ? 4 : 17;
-}
-
 // The ring kernel's tile for slice sums and the slices a workgroup takes; per 0: another kernel.
 struct SlicesPlan {
   int tile, per;
 };
-// bfloat16: the cheaper of 32 x 64 and 64 x 64 tiles with one, two or four slices a workgroup, a stage 0.18 and 0.25 us where a CU has one
-// workgroup, twice that where it has two, and a round about four stages besides.  Before (64 x 64, every CU a workgroup or another
-// kernel) / now, us: 8 x 4,096 x 4,096 10.9 / 8.4, 8 x 4,096 x 12,288 24.0 / 21.8, 64 x 1,024 x 2,048 5.4 / 4.2, 64 x 1,024 x
-// 3,072 6.7 / 5.0, 64 x 4,096 x 4,096 13.3 / 12.8, 97 x 1,024 x 2,048 5.2 / 5.0.  One row 5,120 x 8,192 19.4 / 20.8, hence four rows at least; 17 to
-// 32 rows of less than five slices over few columns 3.8 / 4.0, and of up to twelve over the fewest, by a wave a slice / tiles (17 x 1,024 x 2,048
-// 3.1 / 3.8, 32 rows 3.5 / 3.9, 24 x 1,024 x 3,072 4.4 / 4.6; 32 rows 4.9 / 4.7, 24 x 2,048 x 2,048 5.0 / 4.8).  From 65 rows on longer runs of stages lose what fewer rounds gain (128 x 5,120 x
-// 5,120 with one, two and four slices a workgroup 28, 30, 31).
+// The cheapest of the tiles and of one, two or four slices a workgroup by rounds_cost.  (us)
+// float32, from 33 rows on: 64 x 64 tiles, from nine workgroups for sixteen CUs on (48 x 1,024 x 2,048, eight, 7.1 by a wave a slice / 8.6), eight or
+// sixteen stages a workgroup (33 x 4,096 x 4,096 24.9 / 22.1, 160 x 10,240 x 768 31.7 / 36.4, 200 x 5,120 x 1,024 27.4 / 30.4); slices of sixteen
+// stages by themselves (56 x 8,192 x 8,192 83, two of them 98).
+// bfloat16, from 4 rows on: 32 x 64 or 64 x 64 tiles, two a CU.  What a wave a slice does instead grows with the rows that every block of 16 columns
+// reads again, and a tile's time hardly: the line is a number of products a CU, the same from 4 rows to 256 (a wave a slice / tiles: 17 x 1,024 x
+// 3,072 4.0 / 4.7, 17 x 2,048 x 3,072 7.1 / 5.5, 32 x 4,096 x 552 3.4 / 4.2, 32 x 16,384 x 768 11.7 / 8.4, 48 x 5,120 x 1,576 15.2 / 8.3, 16 x 1,024
+// x 4,096 4.2 / 4.8, 8 x 4,096 x 12,288 23.9 / 20.2, 8 x 4,096 x 4,096 9.6 / 8.0, 64 x 1,024 x 2,048 4.5 / 4.1, 256 x 512 x 512 3.3 / 3.8; one row
+// 5,120 x 8,192 17.9 / 18.7).  Sixteen stages a workgroup at most, eight with more than 64 rows, and beyond 32 rows slices of eight and more by
+// themselves (128 x 5,120 x 5,120 with one, two and four 27.6, 29.5, 30.7; 64 x 10,240 x 5,120 31.3, 33.6, 34.9).
 static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
   const int kslice = kslice_for(K), nslices = (K + kslice - 1) / kslice;
   const long cus = compute_units();
-  if (dtype == kF32) {  // sixteen stages a workgroup where every CU gets two (33 x 4,096 x 4,096 in eight 28, in sixteen 23), eight where it gets one
-    const int a_slice = kslice / 32;
-    int per = std::min(nslices, std::max(1, (16 + a_slice - 1) / a_slice));
-    auto workgroups = [&](int p) LS_INLINED { return (long)((M + 63) / 64) * ((N + 63) / 64) * ((nslices + p - 1) / p); };
-    while (per > 1 && workgroups(per) < (per * a_slice > 8 ? 2 * cus : cus)) per = (per + 1) / 2;
-    return workgroups(per) >= cus ? SlicesPlan{kRing64x64, per} : SlicesPlan{kRing64x64, 0};
-  }
-  if (M <= 32 && (nslices < 5 || (N <= 1024 && nslices <= (M <= 24 ? 12 : 8)))) return {kRing32x64, 0};
+  const bool f32 = dtype == kF32;
   SlicesPlan best{kRing64x64, 0};
+  if (f32 ? M < 33 : M < 4 || (long)((N + 15) / 16) * std::max(K, 256) * M <= 72 * 256 * cus) return best;
+  constexpr float k32x64[2] = {0.18f, 0.39f}, k64x64[2] = {0.33f, 0.52f};
+  const int most = f32 || M > 64 || (M > 32 && kslice > 256) ? 512 : 1024;  // elements of K a workgroup
   float least = 0.f;
-  for (int rows = 32; rows <= 64; rows += 32)
-    for (int per = M > 64 ? std::max(1, 512 / kslice) : 4; per >= 1; per /= 2) {
-      const long groups = (nslices + per - 1) / per, all = (long)((M + rows - 1) / rows) * ((N + 63) / 64) * groups;
-      if (M > 64 && per > 1 && all < cus) continue;
-      const float stages = (float)std::min(per, nslices) * (kslice / 64), one = rows == 32 ? 0.18f : 0.25f;
-      const long rest = all % (2 * cus), twos = all / (2 * cus) + (rest > cus);
-      const float time = (float)twos * (1.6f + 2.f * one * stages) + (rest > 0 && rest <= cus ? 1.f + one * stages : 0.f);
-      if (best.per == 0 || time < least) {
-        least = time;
+  for (int rows = f32 ? 64 : 32; rows <= 64; rows += 32)
+    for (int per = 1; per == 1 || (per <= nslices && per * kslice <= most); per *= 2) {
+      const long all = (long)((M + rows - 1) / rows) * ((N + 63) / 64) * ((nslices + per - 1) / per);
+      const int stages = std::min(per, nslices) * (kslice / (f32 ? 32 : 64));
+      if (f32 && 16 * all < 9 * cus) continue;
+      const float cost = f32 ? rounds_cost(all, 3, stages, 1.2f, kStages64x64) : rounds_cost(all, 2, stages, 1.5f, rows == 32 ? k32x64 : k64x64);
+      if (best.per == 0 || cost < least) {
+        least = cost;
         best = {rows == 32 ? kRing32x64 : kRing64x64, per};
       }
     }
@@ -1493,6 +1495,13 @@ static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
 }
 
 }  // namespace ls
+
+// How ls_gemm_slices computes the sums of aligned operands: rows of the ring kernel's tile times 16 plus slices a workgroup; 0: another kernel.
+extern "C" int ls_gemm_slices_plan(int dtype, int M, int N, int K) {
+  using namespace ls;
+  const SlicesPlan plan = N % 4 == 0 ? slices_plan(dtype, M, N, K) : SlicesPlan{kRing64x64, 0};
+  return plan.per == 0 ? 0 : (plan.tile == kRing32x64 ? 32 : 64) * 16 + plan.per;
+}
 
 // Slice sums of X [M,K] @ W [N,K]^T for M <= ls_gemm_slices_max_rows: P [slices][M][N] float, P[s] = the
 // sum over K slice s.  The product is P[0] + P[1] + ... added in this order, starting from +0.
@@ -1530,12 +1539,8 @@ extern "C" int ls_gemm_slices(int dtype, const void* X, const void* W, float* P,
   int rounds =
       (int)std::min<long>(4, (long)col_blocks * groups * std::max(row_groups, 1) / (2L * compute_units()));
   if (mt > 4 && rounds < 1) rounds = 1;  // more than 64 rows: this kernel only, if with one column block a workgroup
-  // The ring kernel (float32: where its 64 x 64 tiles times groups of slices give every CU a workgroup), with four stages of
-  // both operands in flight: from 17 rows on (from 4 over weights of 32 MB and more, where the kernels of a wave a slice fall
-  // to 3.7 TB/s), from 33 rows on in float32.  bfloat16 takes the tile and the slices a workgroup that slices_plan finds cheapest.
-  const int ring_from = slices_ring_from(dtype, N, K);
-  if (LS_GEMM_SLICES_TILED && aligned && ring_reaches(ldx, K, dtype == kF32 ? 4 : 2) && M >= ring_from && N % 4 == 0 &&
-      (dtype == kF32 || dtype == kBF16)) {
+  // The ring kernel, with four stages of both operands in flight, where slices_plan finds its tiles the better ones.
+  if (LS_GEMM_SLICES_TILED && aligned && ring_reaches(ldx, K, dtype == kF32 ? 4 : 2) && N % 4 == 0 && (dtype == kF32 || dtype == kBF16)) {
     const SlicesPlan plan = slices_plan(dtype, M, N, K);
     if (plan.per > 0) {
       const int groups_y = (nslices + plan.per - 1) / plan.per;

@@ -274,6 +274,11 @@ class Kernels:
         operands) takes before any other kernel; 0: none."""
         return int(self.core.ls_gemm_narrow_tile(c_int(DTYPE_CODE[dtype]), c_int(epilogue), c_int(m), c_int(n), c_int(k)))
 
+    def gemm_slices_plan(self, dtype: torch.dtype, m: int, n: int, k: int) -> tuple[int, int]:
+        """(rows of the ring kernel's tile, slices a workgroup) of the slice sums of a product of these sizes (and of 16-byte
+        aligned operands); (0, 0) where another kernel computes them."""
+        return divmod(int(self.core.ls_gemm_slices_plan(c_int(DTYPE_CODE[dtype]), c_int(m), c_int(n), c_int(k))), 16)
+
     def gemm_slices_count(self, k: int) -> int:
         """K slices of a product over ``k`` (first dimension of ``gemm_slices``'s output)."""
         return self._memo(("slices", k), lambda: int(self.core.ls_gemm_slices_count(c_int(k))))

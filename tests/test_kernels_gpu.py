@@ -424,21 +424,34 @@ def test_products_on_both_sides_of_the_lines_of_the_narrow_tiles_have_the_same_b
             assert torch.equal(a[:-1], b[:-1] + b[:-1]), (m, n, k)
 
 
+# (rows, columns, K) of slice sums, and (rows of the tile, slices a workgroup) of the ring kernel that computes them in bfloat16 and in float32
+SLICES_PLANS = [(3, 4096, 4096, (0, 0), (0, 0)), (4, 4096, 4096, (0, 0), (0, 0)), (17, 1028, 1288, (0, 0), (0, 0)), (33, 1024, 8, (0, 0), (0, 0)),
+                (40, 260, 328, (0, 0), (0, 0)), (65, 508, 2048, (0, 0), (0, 0)), (32, 1020, 4424, (32, 1), (0, 0)), (64, 1024, 2048, (32, 1), (0, 0)),
+                (8, 5116, 8192, (32, 2), (0, 0)), (24, 8188, 1032, (32, 4), (0, 0)), (64, 4092, 1032, (64, 1), (64, 1)),
+                (64, 1020, 3072, (64, 1), (64, 1)), (128, 5116, 5120, (64, 1), (64, 1)), (56, 8188, 4424, (64, 1), (64, 1)),
+                (33, 4092, 4096, (64, 2), (64, 2)), (64, 4092, 4096, (64, 2), (64, 2)), (200, 1024, 3072, (64, 2), (64, 1)),
+                (256, 4096, 520, (64, 2), (64, 1)), (33, 12284, 3080, (64, 4), (64, 1))]
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("m,n,k", [(4, 4096, 4096), (3, 4096, 4096), (17, 1028, 1288), (32, 1020, 4424), (33, 1024, 8), (40, 260, 328), (64, 1024, 2048),
-                                   (64, 4092, 1032), (65, 508, 2048), (200, 1024, 3072), (256, 4096, 520)])
-def test_slice_sums_in_either_tile_add_up_to_the_product(dtype, m, n, k):
-    """Slice sums on both sides of the choice between tiles of 32 and 64 rows and of one, two and four slices a workgroup, with rows and
-    columns that end inside a tile: every sum is there, and added in ascending order they are the product, bit for bit."""
+@pytest.mark.parametrize("m,n,k,plan,plan_f32", SLICES_PLANS)
+def test_slice_sums_by_either_tile_add_up_to_the_product(dtype, m, n, k, plan, plan_f32):
+    """Slice sums of every plan, with rows and columns that end inside a tile and a last workgroup with fewer slices: every sum is there, they
+    have the bits that another kernel gives for weights off a 16-byte boundary, and added in ascending order they are the product, bit for bit."""
     from lockstep_amd.ops import STORE_F32
 
+    if m > K().gemm_slices_max_rows(k, dtype):
+        pytest.skip("more rows than the slice sums take")
+    assert K().gemm_slices_plan(dtype, m, n, k) == (plan if dtype is torch.bfloat16 else plan_f32)
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
     w = (torch.randn(n, k, generator=g, device="cuda") * 0.1).to(dtype)
-    if m > K().gemm_slices_max_rows(k, dtype):
-        pytest.skip("more rows than the slice sums take")
-    sums = torch.full((K().gemm_slices_count(k), m, n), float("nan"), device="cuda")
+    off = torch.empty(n * k + 8, dtype=dtype, device="cuda")[1:1 + n * k].view(n, k)
+    off.copy_(w)
+    sums, others = (torch.full((K().gemm_slices_count(k), m, n), float("nan"), device="cuda") for _ in range(2))
     K().gemm_slices(x, w, sums)
+    K().gemm_slices(x, off, others)
+    assert torch.equal(sums, others)
     want = torch.empty(m, n, device="cuda")
     K().gemm(x, w, want, STORE_F32)
     total = torch.zeros(m, n, device="cuda")
