@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ X
 // workgroup on every CU and with as many as it holds (bfloat16, K = 4,096, weights from HBM).  The larger the tile, the
 // fewer operand bytes a product loads; the smaller, the more CUs have one, and the fuller the last round.
 enum RingTile { kRing256x192, kRing256x128, kRing192x192, kRing128x192, kRing192x128, kRing128x128, kRing128x64, kRing64x128,
-                kRing64x64, kRingTiles, kRing64x32 = kRingTiles, kRing32x64, kRing32x32 };
+                kRing64x64, kRingTiles, kRing32x64 = kRingTiles, kRing32x32 };
 struct RingShape {
   int rows, cols, a_cu;
   float one, full;
@@ -1089,26 +1089,45 @@ static float rounds_cost(long tiles, int a_cu, int stages, float start, const fl
   if (rest) cost += start + stage[(rest + cus - 1) / cus - 1] * stages;
   return cost;
 }
-constexpr float kStages64x64[3] = {0.59f, 1.15f, 1.7f};  // float32
+constexpr float kStages32x32[4] = {0.218f, 0.365f, 0.515f, 0.68f}, kStages64x64[3] = {0.59f, 1.15f, 1.7f};  // float32
 
-// The tile whose rounds of workgroups take least by that table.  (Every tile forced in turn over 65 to 2,048 rows and nine
-// shapes of weights: within 2 % of the best one everywhere.)  Two rules stand in front of it: up to 64 rows whose rows of
-// weights lie a multiple of 4 KB apart take 64 x 64 tiles (128 such rows asked for together meet in few memory channels: 16 x
-// 32,768 x 4,096 62.6 -> 55.1 us, 16 x 24,576 x 4,096 49.2 -> 45.5; other K 0.9 to 1.05 times as long).  float32 has four times
-// the matrix work a byte and takes 64 x 64 tiles, three a CU (2,000 x 6,144 x 1,024 192 us, 128 x 128 tiles 204), and for up
-// to 64 rows 64 x 32 tiles where every CU gets at most one (64 x 6,144 x 1,024 15.5, 64 x 64 tiles 23.8).
-template <typename T, int EPI>
+// The ring kernel's tile of a product that it runs.
+// float32 has four times the matrix work a byte: 32 x 32 tiles, four a CU, or 64 x 64, three a CU, whichever the costs above (fitted to 1,900
+// products each) give less (us, 32 x 32 / 64 x 64: 64 x 4,096 x 1,024 10.0 / 22.3, 24 x 51,200 x 2,048 90 / 137, 128 x 10,240 x 4,096 107 / 143, 200
+// x 4,096 x 8,344 181 / 164, SwiGLU 64 x 16,384 x 2,048 49.6 / 45.7, 256 x 4,096 x 408 13.9 / 11.7, 2,000 x 1,024 x 1,024 41.4 / 38.1).  64 x 32
+// tiles beside these two gained 0.4 %.
+// bfloat16: 32 x 32 (stages of 256 bytes, so that a barrier and an LDS latency stand every 128 elements of K) and then 32 x 64 where those tiles are
+// one round: a wider one would leave CUs idle, and every workgroup loads 32 rows of both operands or 96 a stage in place of 128.  Up to 32 rows 32 x
+// 32 also for three rounds of at least 2,048 of K, 32 x 64 for one and a half to two of at most 512.  Weights from HBM, us, 64 x 64 / these:
+//   one round of 32 x 32    SwiGLU 8 x 6,144 x 1,024 7.1 / 5.7, 64 x 4,096 x 1,024 7.9 / 5.4, 64 x 4,096 x 4,096 21.3 / 12.4, 97 x 1,024 x 2,048 9.6 /
+//                           6.5, 200 x 1,024 x 4,096 17.0 / 11.4
+//   one round of 32 x 64    8 x 10,240 x 5,120 23.1 / 22.3, SwiGLU 1 x 14,336 x 1,024 8.0 / 7.5, 64 x 6,144 x 4,096 22.3 / 18.0, 97 x 4,096
+//                           x 1,024 7.6 / 6.5; 32 x 32 tiles, two a CU, 6.9 for the last
+//   up to 32 rows           SwiGLU 8 x 24,576 x 4,096 40.2 / 35.6 in 32 x 32, 32 x 24,544 x 512 in 32 x 64; four rounds ask for 128 rows of weights a
+//                           multiple of 4 KB apart together (8 x 32,768 x 4,096 51.9 / 64.9)
+// Others the tile whose rounds of workgroups take least by the table above.  (Every tile forced in turn over 65 to 2,048 rows and nine shapes of
+// weights: within 2 % of the best one everywhere.)  One rule stands in front of it: up to 64 rows whose rows of weights lie a multiple of 4 KB apart
+// take 64 x 64 tiles (128 such rows asked for together meet in few memory channels: 16 x 32,768 x 4,096 62.6 -> 55.1 us; other K 0.9 to 1.05 times as long).
+template <typename T>
 static int ring_tile(int M, int N, int K) {
-  if (sizeof(T) == 4) return EPI != kSwiGLU && M <= 64 && (N + 31) / 32 <= compute_units() ? kRing64x32 : kRing64x64;
-  if (M <= 64 && K % 2048 == 0) return kRing64x64;
   const long cus = compute_units();
+  auto tiles = [&](int rows, int cols) { return (long)((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
+  if (sizeof(T) == 4) {
+    const int stages = (K + 31) / 32;
+    return rounds_cost(tiles(32, 32), 4, stages, 0.9f, kStages32x32) <= rounds_cost(tiles(64, 64), 3, stages, 1.2f, kStages64x64) ? kRing32x32
+                                                                                                                                : kRing64x64;
+  }
+  if (tiles(32, 32) <= cus) return kRing32x32;
+  if (tiles(32, 64) <= cus) return kRing32x64;
+  if (M <= 32 && K >= 2048 && tiles(32, 32) <= 3 * cus) return kRing32x32;
+  if (M <= 32 && K <= 512 && 2 * tiles(32, 64) >= 3 * cus && tiles(32, 64) <= 2 * cus) return kRing32x64;
+  if (M <= 64 && K % 2048 == 0) return kRing64x64;
   int best = 0;
   float least = 0.f;
   for (int t = 0; t < kRingTiles; ++t) {
     const RingShape& s = kRingShapes[t];
-    const long tiles = (long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols);
-    const long rest = tiles % (cus * s.a_cu);
-    const float time = (float)(tiles / (cus * s.a_cu)) * s.full + (rest == 0 ? 0.f : rest <= cus ? s.one : s.full);
+    const long all = tiles(s.rows, s.cols), rest = all % (cus * s.a_cu);
+    const float time = (float)(all / (cus * s.a_cu)) * s.full + (rest == 0 ? 0.f : rest <= cus ? s.one : s.full);
     if (t == 0 || time < least) {
       least = time;
       best = t;
@@ -1117,77 +1136,37 @@ static int ring_tile(int M, int N, int K) {
   return best;
 }
 
-// Whether the ring kernel runs a product of aligned operands: more than 64 rows, or so many columns that its 64-column
-// tiles beat the kernels of a wave a slice, which read the rows of X once for 16 columns.  A stage costs the ring kernel the
-// same at any number of rows, so the line is a number of rows, lower the more columns there are (and for SwiGLU, where a wave
-// of the other kernels holds two weight tiles).  Measured on both sides, us, those kernels / this one:
-//   10,240 columns and more  8 x 10,240 x 5,120 36 / 28, SwiGLU 8 x 24,576 x 4,096 48 / 43, 8 x 151,936 x 1,024 66 / 58
-//   5,057 and more           17 x 6,144 x 5,120 29 / 25, 20 x 6,144 x 1,024 7.9 / 7.6 (17 rows 7.5 / 7.5), 40 x 5,696 x 5,120
-//                            42 / 26; SwiGLU 24 x 8,192 x 4,096 24 / 22, 32 x 6,144 x 1,024 7.6 / 8.0, 40 rows 8.8 / 8.0
-//   1,985 and more           48 x 2,048 x 5,120 25 / 27, 56 rows 27.7 / 27.8, 64 rows 29.5 / 28.3; SwiGLU 48 x 2,048 x 4,096 25 / 21
-// Below 768 of K there are few stages behind the first, which everybody waits for; up to 320 they are all asked for at once:
-//   K = 520                  16 x 10,240 4.9 / 6.0, 32 rows 8.1 / 6.2, 17 x 16,384 8.8 / 7.1, 64 x 5,696 6.0 / 6.4; SwiGLU 17 x
-//                            10,240 6.4 / 6.2, 48 x 6,144 6.2 / 6.3, 56 rows 6.9 / 6.3, 8 x 32,768 12.8 / 11.0
-//   K = 264                  17 x 16,384 6.9 / 5.3, 16 rows 4.3 / 5.2, 48 x 2,048 4.8 / 4.5, 8 x 65,536 12.5 / 11.0; SwiGLU 17 x
-//                            2,048 5.1 / 4.5, 16 rows 4.2 / 4.5
-// float32 multiplies too slowly for 64 rows in place of 32 to pay while the other kernels have a block of 16 columns for every
-// CU and no more (33 x 4,096 x 1,024 12.9 / 15.2); beyond that they take a second round (32 x 5,120 x 1,024 18.1 / 15.3, 64 x
-// 10,240 x 5,120 203 / 103; K = 264: 32 x 10,240 7.8 / 9.3, 33 rows 16.5 / 9.4), for SwiGLU and for 17 to 31 rows later (SwiGLU
-// 33 x 16,384 x 1,024 31 / 26, 17 x 32,768 x 1,024 53 / 39).
+// Whether the ring kernel runs a product of aligned operands: more than 32 rows, or where its tiles beat the kernels of a wave a slice, which read
+// the rows of X once for 16 columns.  Its stages cost the same at any number of rows, so the line is lower the more columns there are, and for
+// SwiGLU, where a wave of the other kernels holds two weight tiles.  Measured on both sides, us, those kernels / the ring kernel in its best tile:
+//   plain, 16 rows and less  8 x 4,096 x 256 2.7 / 3.0, 1 x 12,288 x 256 3.6 / 4.1, 7 x 20,000 x 1,024 10.0 / 10.8, 8 x 6,144 x 4,096 13.8 / 11.5, 16 x 6,144 x 4,096 14.7 /
+//                            11.8, 16 x 12,288 x 2,048 15.0 / 12.6, 8 x 151,936 x 1,024 58.9 / 55.3, 7 x 65,536 x 64 6.3 / 4.4, 12 x 12,288 x 392 4.3 / 5.2
+//   plain, 17 to 32 rows     17 x 1,536 x 1,024 4.5 / 4.4; rows of weights that are no whole lines of 128 bytes: 31 x 1,536 x 1,272 4.6 / 5.1, 20 x 204 x 1,624 4.7 /
+//                            5.6, 24 x 371 x 472 2.9 / 3.7, 20 x 6,144 x 144 2.8 / 3.2, 20 x 768 x 4,384 11.0 / 11.9, 32 x 12,288 x 520 6.7 / 6.4
+//   SwiGLU                   6 x 6,144 x 512 4.3 / 4.8, 8 x 2,048 x 1,024 5.3 / 4.9, 16 x 12,288 x 512 6.0 / 5.3, 8 x 1,280 x 912 4.2 / 4.8, 16 x 512 x 408 3.2 / 3.8,
+//                            8 x 512 x 2,032 5.9 / 6.8
+// float32 multiplies longer than it loads, and a tile's one chain of products is the longer way where few columns leave it alone on its CU: 8 x 2,048
+// x 1,024 6.2 / 9.7, 8 x 6,144 x 4,096 25.9 / 30.7, 24 x 2,048 x 1,024 8.1 / 9.7, 24 x 2,048 x 256 4.9 / 4.2, 32 x 4,096 x 4,096 27.6 / 29.8, 16 x
+// 8,192 x 2,048 19.2 / 17.4, 32 x 6,144 x 1,024 14.5 / 10.2, SwiGLU 8 x 6,144 x 1,024 10.0 / 11.0, 3 x 1,024 x 256 5.6 / 4.5, 16 x 12,288 x 1,024
+// 17.5 / 15.2, 3 x 32,768 x 1,024 29.7 / 33.9.
 template <typename T, int EPI>
 static bool ring_takes(int M, int N, int K) {
-  if (M > 64) return true;
-  const int blocks = (N + 63) / 64;
   constexpr bool GATED = EPI == kSwiGLU;
+  if (M > 32 || (GATED && M > 16)) return true;
+  const bool one_round = (N + 15) / 16 <= compute_units();  // of the other kernels' blocks
   if (sizeof(T) == 4) {
-    if (GATED) return blocks >= 256 && M > 32;
-    return M >= (K >= 512 ? 32 : 33) ? (N + 15) / 16 > compute_units() : M > 16 && blocks >= 512;
+    if (GATED) return N <= 8192 ? K <= 512 : M > 8 || N < 30000;
+    if (M <= 16) return M > 8 && !one_round && K >= 256;
+    return !one_round || K <= 384;
   }
-  if (K < 768) {
-    if (GATED) return blocks >= 32 && M >= (blocks >= 512 ? 8 : K <= 320 || blocks >= 160 ? 17 : 56);
-    return blocks >= 256 ? M >= (blocks >= 1024 ? 8 : 17) : blocks >= 90 ? M >= 32 : blocks >= 32 && K <= 320 && M >= 48;
-  }
-  if (blocks >= 160) return M >= 8;
-  if (blocks >= 80) return M >= (GATED ? (K >= 2048 ? 24 : 40) : K >= 2048 ? 17 : 20);
-  return blocks >= 32 && M >= (GATED ? 48 : 56);
-}
-
-// The narrow tiles: 32 rows by 32 or by 64 columns where those are so few that a wider tile would leave CUs idle, or few
-// rows over many columns; -1 where the table's tiles or the other kernels serve as well.  Every workgroup loads 32 rows of both
-// operands or 96 a stage in place of 128, and the 32 x 32 tile's stages are of 256 bytes, so that a barrier and an LDS latency
-// stand every 128 elements of K.  Against what ran before them (64 x 64 tiles, the streaming kernel, a wave a slice), weights
-// from HBM, us:
-//   one round of 32 x 32    8 x 6,144 x 4,096 15.6 / 11.9, SwiGLU 8 x 6,144 x 1,024 6.6 / 5.6, 1 x 6,144 x 1,024 6.3 / 5.4, 64 x 4,096 x 1,024
-//                           7.5 / 5.1, 64 x 4,096 x 4,096 22 / 13, 97 x 1,024 x 2,048 11.9 / 6.8, 200 x 1,024 x 4,096 20 / 11
-//   one round of 32 x 64    8 x 10,240 x 5,120 26.4 / 23.8, SwiGLU 1 x 14,336 x 1,024 9.6 / 7.8, 64 x 6,144 x 4,096 23 / 18.5, 97 x 4,096
-//                           x 1,024 7.6 / 5.9; 32 x 32 tiles, two a CU, 6.5 for the last
-//   up to three rounds and 32 rows  SwiGLU 8 x 24,576 x 4,096 41.8 / 36.2 in 32 x 32 (64 x 64 as they are now 39); below 2,048 of K 32 x 64
-//                           are ahead up to 512 (8 x 24,576 x 512 9.8 / 7.8); 18,432 columns, a round and an eighth, gain nothing
-// Up to 16 rows of a plain product a wave a slice and 16 columns keeps the lead while those blocks fit one round (8 x 4,096 x 1,024
-// 4.7 / 4.8, 1 x 1,024 x 4,096 7.3 / 10.3), beyond 320 of K (1 x 4,096 x 256 3.4 / 3.3).  And four rounds of 32,768 columns ask
-// for 128 rows of weights a multiple of 4 KB apart together (8 x 32,768 x 4,096 54.8 / 69.9): they keep the table's tiles.
-// float32 multiplies longer than it loads, so every CU that has a tile counts, up to six rounds (64 x 4,096 x 1,024 17.6 / 10.2, 8 x
-// 24,576 x 1,024 29.3 / 24.0, 33 x 24,576 x 1,024 40 / 35, 128 x 10,240 x 4,096 145 / 105; 2,000 x 1,024 x 1,024, eight rounds, 40.4 / 42.3); up to 64
-// rows over columns that 64 x 32 tiles cover in one round keep those.  A wave a slice stays ahead where a tile's one chain of
-// products is the longer way (its times / 32 x 32): up to 32 rows of few columns (32 x 2,048 x 1,024 8.3 / 9.5, 32 x 4,096 x 4,096 27.3 / 30.0; 32 x
-// 6,144 x 1,024 14.0 / 10.0), eight of up to a round and a half (8 x 6,144 x 4,096 23.0 / 30.1, 1 x 12,288 x 1,024 11.2 / 14.0; 16 x 8,192 x 2,048
-// 19.1 / 17.5), SwiGLU of 16 in a round (8 x 6,144 x 1,024 9.4 / 10.7; 8 x 12,288 x 1,024 15.9 / 14.6, 16 x 8,192 x 512 7.6 / 7.0).
-template <typename T, int EPI>
-static int narrow_tile(int M, int N, int K) {
-  const long cus = compute_units();
-  const long rows = (M + 31) / 32, small = rows * ((N + 31) / 32), wide = rows * ((N + 63) / 64);
-  if (sizeof(T) == 4) {
-    if (EPI != kSwiGLU && (N + 15) / 16 <= cus && M <= (K <= 512 ? 16 : K <= 1024 && N <= 1024 ? 24 : 32)) return -1;
-    if (EPI != kSwiGLU && M <= 8 && K >= 512 && 2 * small <= 3 * cus) return -1;
-    if (M <= 16 && (K < 256 || (EPI == kSwiGLU && (N + 31) / 32 <= (K > 512 ? cus : cus / 2)))) return -1;
-    return small <= cus || (small <= 6 * cus && (EPI == kSwiGLU || M > 64 || (N + 31) / 32 > cus)) ? kRing32x32 : -1;
-  }
-  if (M <= 16 && EPI != kSwiGLU && (N + 15) / 16 <= cus && K > 320) return -1;
-  if (small <= cus) return kRing32x32;
-  if (wide <= cus) return kRing32x64;
-  if (M > 32) return -1;
-  if (K >= 2048) return small <= 3 * cus ? kRing32x32 : -1;
-  return K <= 512 && 2 * wide >= 3 * cus && wide <= 2 * cus ? kRing32x64 : -1;
+  const bool lines = K % 64 == 0;  // rows of weights are whole lines
+  if (N >= 32768 && M <= 16 && (K <= 128 || M > 8 || (M == 8 && K >= 320))) return true;
+  if (GATED) return K >= (!lines && N <= 8192 ? 2600 : M <= 8 ? 640 : 320);
+  if (M > 16) return lines || (one_round ? M > 24 && K >= 4096 : K > 256 || N >= 20000);
+  if (one_round) return false;
+  if (M > 8) return K >= (lines ? 384 : 640);
+  const int tile = ring_tile<T>(M, N, K);
+  return K >= 640 && (tile == kRing32x32 || tile == kRing32x64);
 }
 
 // Whether the ring kernel's 32-bit byte offsets inside a tile reach every operand: the rows of the largest tile, and what
@@ -1229,8 +1208,6 @@ static int launch_ring(int tile, const T* X, const T* W, void* C, int M, int N, 
 #define LS_RING(...) \
   return launch_ring_tile<T, EPI, __VA_ARGS__>(X, W, C, M, N, K, ldx, ldc, kslice, vec_ok, out_cols, groups, act, stream)
   if constexpr (sizeof(T) == 4) {
-    if constexpr (EPI != kSwiGLU && EPI != kSliceSums)
-      if (tile == kRing64x32) LS_RING(64, 32, 2, 2, 5, 5);
     if constexpr (EPI != kSliceSums)
       if (tile == kRing32x32) LS_RING(32, 32, 2, 2, 5, 5);
     LS_RING(64, 64, 2, 2, 3, 3);
@@ -1284,10 +1261,9 @@ int launch_gemm(const void* X, const void* W, void* C, int M, int N, int K, long
   const int mt_rows = (M + 15) / 16;
   const int col_blocks = (N + 16 * NT - 1) / (16 * NT);
   bool ring = aligned && ring_reaches(ldx, K, sizeof(T));
-  const int narrow = !norm_w && ring ? narrow_tile<T, EPI>(M, N, K) : -1;
-  if (!norm_w && ring && (narrow >= 0 || ring_takes<T, EPI>(M, N, K))) {
-    const int rc = launch_ring<T, EPI>(narrow >= 0 ? narrow : ring_tile<T, EPI>(M, N, K), reinterpret_cast<const T*>(X), w, C, M,
-                                       N, K, ldx, ldc, kslice, vec_ok, out_cols, 1, act, stream);
+  if (!norm_w && ring && ring_takes<T, EPI>(M, N, K)) {
+    const int rc = launch_ring<T, EPI>(ring_tile<T>(M, N, K), reinterpret_cast<const T*>(X), w, C, M, N, K, ldx, ldc, kslice, vec_ok,
+                                       out_cols, 1, act, stream);
     if (rc != kNotLaunched) return rc;
     ring = false;
   }
@@ -1419,23 +1395,13 @@ extern "C" int ls_gemm_xielu(int dtype, const void* X, const void* W, void* C, i
 
 extern "C" int ls_gemm_kslice(int K) { return ls::kslice_for(K); }
 
-// The tile (enum RingTile) that the table gives the ring kernel for a product of aligned operands; -1: another kernel's.  A narrow
-// tile (ls_gemm_narrow_tile) goes before it.
+// The tile (enum RingTile) in which ls_gemm has the ring kernel compute a product of aligned operands; -1: another kernel does.
 extern "C" int ls_gemm_ring_tile(int dtype, int epilogue, int M, int N, int K) {
   using namespace ls;
-#define LS_TILE(T_, EPI_) (ring_takes<T_, EPI_>(M, N, K) ? ring_tile<T_, EPI_>(M, N, K) : -1)
-  if (dtype == kF32) return epilogue == kSwiGLU ? LS_TILE(float, kSwiGLU) : LS_TILE(float, kStore);
-  return epilogue == kSwiGLU ? LS_TILE(bf16_t, kSwiGLU) : LS_TILE(bf16_t, kStore);
-#undef LS_TILE
-}
-
-// The rows times columns of the narrow tile that ls_gemm gives a product of aligned operands; 0: none.
-extern "C" int ls_gemm_narrow_tile(int dtype, int epilogue, int M, int N, int K) {
-  using namespace ls;
-#define LS_TILE(T_) (epilogue == kSwiGLU ? narrow_tile<T_, kSwiGLU>(M, N, K) : narrow_tile<T_, kStore>(M, N, K))
-  const int tile = dtype == kF32 ? LS_TILE(float) : LS_TILE(bf16_t);
-#undef LS_TILE
-  return tile == kRing32x32 ? 32 * 32 : tile == kRing32x64 ? 32 * 64 : 0;
+#define LS_TAKES(T_) (epilogue == kSwiGLU ? ring_takes<T_, kSwiGLU>(M, N, K) : ring_takes<T_, kStore>(M, N, K))
+  if (dtype == kF32) return LS_TAKES(float) ? ring_tile<float>(M, N, K) : -1;
+  return LS_TAKES(bf16_t) ? ring_tile<bf16_t>(M, N, K) : -1;
+#undef LS_TAKES
 }
 
 // Columns of a block of the streaming kernel for N columns and that many walkers (workgroups of a group of rows).

@@ -265,14 +265,9 @@ class Kernels:
             c_long(out.stride(0)), _ptr(act), _stream()))
 
     def gemm_ring_tile(self, dtype: torch.dtype, epilogue: int, m: int, n: int, k: int) -> int:
-        """Which tile of the ring kernel's table a product of these sizes (and of 16-byte aligned operands) takes, unless a
-        narrow tile is better: its place in ``RingTile`` of gemm.hip, -1 where another kernel computes it."""
+        """In which tile the ring kernel computes a product of these sizes (and of 16-byte aligned operands): its place in
+        ``RingTile`` of gemm.hip, -1 where another kernel computes it."""
         return int(self.core.ls_gemm_ring_tile(c_int(DTYPE_CODE[dtype]), c_int(epilogue), c_int(m), c_int(n), c_int(k)))
-
-    def gemm_narrow_tile(self, dtype: torch.dtype, epilogue: int, m: int, n: int, k: int) -> int:
-        """Rows times columns of the narrow tile of the ring kernel that a product of these sizes (and of 16-byte aligned
-        operands) takes before any other kernel; 0: none."""
-        return int(self.core.ls_gemm_narrow_tile(c_int(DTYPE_CODE[dtype]), c_int(epilogue), c_int(m), c_int(n), c_int(k)))
 
     def gemm_slices_plan(self, dtype: torch.dtype, m: int, n: int, k: int) -> tuple[int, int]:
         """(rows of the ring kernel's tile, slices a workgroup) of the slice sums of a product of these sizes (and of 16-byte
