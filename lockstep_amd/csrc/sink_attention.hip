@@ -78,9 +78,16 @@ __device__ __forceinline__ int first_seen(int p, int window, int chunk) {
   return lo;
 }
 
+// Waves a SIMD that the registers of a decoded token's wave are held to.  Two, where 256 registers hold its queries, keys, values and sums
+// without a spill; left to itself the compiler takes accumulation registers besides and leaves room for one.  More than 1,024 waves want
+// the second (bfloat16, keys of 192 and values of 128, eight key/value heads over 1,024 keys, us, one / two a SIMD: 160 requests 171 / 151,
+// 128 requests 115 / 115; values of 192 and keys of 64, 16 requests in four runs 21.5 / 19.7).
+template <typename T>
+constexpr int decode_waves() { return sizeof(T) == 2 && (D + 31) / 32 + (DV + 15) / 16 <= 15 ? 2 : 1; }
+
 // DEC: a step of single decoded tokens (the rows of a tile are the heads of a key/value group).
 template <typename T, int RT, bool DEC>
-__global__ __launch_bounds__(64 * (DEC ? 1 : kMaxWaves)) void sink_attention_kernel(
+__global__ __launch_bounds__(64 * (DEC ? 1 : kMaxWaves), DEC ? decode_waves<T>() : 1) void sink_attention_kernel(
     const T* __restrict__ q, long ldq, const T* __restrict__ k_pages, const T* __restrict__ v_pages, int page_size,
     const int* __restrict__ table, int table_stride, const SeqMeta* __restrict__ seqs, const int* __restrict__ items,
     int H, int G, float scale, int window, int chunk, int keep_first, const float* __restrict__ sink,

@@ -148,6 +148,22 @@ def test_no_kernel_calls_a_function_and_only_known_ones_spill():
     assert seen > 100, "the libraries' metadata was not found"
 
 
+@pytest.mark.skipif(not LIBS, reason="no library has been built in the tree")
+def test_decoded_tokens_of_the_sink_attention_leave_room_for_two_waves_a_simd():
+    """bfloat16, keys of d and values of dv elements: up to fifteen of their chunks (32 of a key, 16 of a value) 256 registers hold them."""
+    seen = 0
+    for lib in LIBS:
+        sizes = re.match(r"liblockstep_sink(\d+)x(\d+)-", lib.name)
+        if not sizes or -(-int(sizes.group(1)) // 32) + -(-int(sizes.group(2)) // 16) > 15:
+            continue
+        for kernel in kernels_of(lib):
+            if "sink_attention_kernelIDF16bLi1ELb1E" in kernel[".name"]:
+                seen += 1
+                assert kernel[".vgpr_count"] <= 256, lib.name
+                assert kernel.get(".private_segment_fixed_size", 0) == 0, lib.name
+    assert seen, "no such kernel was found"
+
+
 def test_early_reads_of_scalar_registers_are_seen():
     listing = "0000 <f>:\n\tv_readlane_b32 s8, v1, 3\n\ts_mov_b32 m0, s5\n\t{}\n\tglobal_load_lds_dwordx4 v2, s[8:9]  // 00"
     assert len(list(early_scalar_reads(listing.format("s_nop 0")))) == 1
