@@ -26,9 +26,9 @@
 // The tiles of a row block are dealt to several work items in contiguous runs where that fills the GPU;
 // each leaves (unnormalised output, max, sum) of its run for every row and a second kernel folds the
 // runs in ascending order, adds the sink and applies the gate.
-// Scores, weights, statistics and accumulators are float; products read the compute dtype T.  Keys a
-// request does not hold (beyond its length, pages that a window or a chunk's end has released) enter as
-// zeros and are masked; their values are replaced by zeros before the product.
+// Scores, weights, statistics and accumulators are float; products read the compute dtype T.  For keys
+// that a request does not hold (beyond its length, pages that a window or a chunk's end has released) the first
+// row of page 0 is multiplied, whatever it holds, and their scores are masked; their values are replaced by zeros before the product.
 
 #include "common.h"
 #include "ring.h"

@@ -327,6 +327,53 @@ def test_staged_attention_over_pages_that_were_given_back(dtype, heads, groups, 
     assert rel_err(out.float().cpu(), want) < (6e-6 if dtype is torch.float32 else 2e-2)      # (as above)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, groups, d, dv, page", [(16, 1, 192, 128, 16), (20, 1, 24, 20, 8), (4, 2, 40, 40, 8), (6, 3, 128, 128, 16), (2, 1, 320, 256, 8)])
+@pytest.mark.parametrize("window, keep_first", [(70, 0), (70, 5), (1, 40)])
+@pytest.mark.parametrize("row_tiles, n", [(0, 1), (1, 16), (1, 5), (2, 40), (4, 70)])
+def test_keys_of_pages_that_were_given_back_reach_no_row(dtype, heads, groups, d, dv, page, window, keep_first, row_tiles, n):
+    """The kernel that takes fragments from global memory walks tiles some of whose keys lie on pages that are no longer the request's: what
+    it loads for those, the first row of page 0, is multiplied and must not reach a result, be it NaN."""
+    start = 150
+    total, step = start + n, 16 * row_tiles if row_tiles else 1
+    g = torch.Generator().manual_seed(d + dv + window + keep_first + n)
+    k = (torch.randn(total, groups, d, generator=g) * 1.5).to(dtype)
+    v = torch.randn(total, groups, dv, generator=g).to(dtype)
+    q = (torch.randn(n, heads, d, generator=g) * 1.5).to(dtype)
+    first_seen = start - window + 1
+    order = (torch.randperm(-(-total // page), generator=g) + 1).tolist()
+    keys, values = paged(-(-total // page) + 1, groups, page, d, dv, dtype)
+    keys.fill_(float("nan")), values.fill_(float("nan"))       # page 0 among them, and what lies behind the last token
+    table = torch.full((1, -(-total // page) + 1), -1, dtype=torch.int32)
+    for logical, pg in enumerate(order):
+        lo, hi = logical * page, min(total, (logical + 1) * page)
+        if hi <= first_seen and lo >= keep_first:
+            continue                                            # given back
+        table[0, logical] = pg
+        keys[pg, :, :hi - lo] = k[lo:hi].transpose(0, 1).cuda()
+        values[pg, :, :, :hi - lo] = v[lo:hi].permute(1, 2, 0).cuda()
+    walked = {key // page for tile in {*range(0, keep_first, 32), *range(first_seen // 32 * 32, total, 32)} for key in range(tile, min(total, tile + 32))}
+    assert (table[0, sorted(walked)] < 0).any()
+    _, _, seqs = step_meta([n], [start], [0])
+    blocks = -(-n // step)
+    spread = torch.arange(heads) // (heads // groups)
+    i_pos, j_pos = torch.arange(start, total)[:, None], torch.arange(total)[None, :]
+    visible = (j_pos <= i_pos) & ((i_pos - j_pos < window) | (j_pos < keep_first))
+    scores = torch.einsum("nhd,mhd->hnm", q.double(), k.double()[:, spread]) * 0.1
+    weights = torch.softmax(scores.masked_fill(~visible, float("-inf")), -1)
+    want = torch.einsum("hnm,mhe->nhe", weights, v.double()[:, spread]).reshape(n, heads * dv)
+    as_dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda").reshape(-1)
+    for runs in (1, 2):
+        items = as_dev([[0, b, r, runs] for b in range(blocks) for r in range(runs)])
+        folds = as_dev([[b * runs, runs, b * step, min(step, n - b * step)] for b in range(blocks)]) if runs > 1 else None
+        part = torch.full((blocks * runs * step * heads * (dv + 2),), float("nan"), device="cuda") if runs > 1 else None
+        out = torch.empty(n, heads * dv, dtype=dtype, device="cuda")
+        K().sink_attention(q.reshape(n, heads * d).cuda(), heads, groups, d, dv, keys, values, page, table.cuda(), seqs, items,
+                           blocks * runs, row_tiles, 0.1, window, 0, None, None, None, out, folds, blocks if runs > 1 else 0, part,
+                           keep_first=keep_first)
+        assert rel_err(out.float().cpu(), want) < (6e-6 if dtype is torch.float32 else 2e-2), runs      # (as above)
+
+
 def test_a_sink_left_out_or_a_chunk_one_off_shows_in_the_kernel_test():
     """Controls of the test above: the same inputs against a plain result without the sink, or with the
     chunk one larger, differ by many times the bound."""
