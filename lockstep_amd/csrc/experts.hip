@@ -822,10 +822,11 @@ static int few_chunks(int dtype, int K) {
 // and half the up rows of the same columns, which lie in LDS in tiles of 16 in turn, or columns of the down product; two workgroups share a
 // CU.  A row's contraction is one chain over ascending chunks from zero: the same bits as the kernels above give without a cut of K.
 // What bounds it: the loads, most of them answered by L2 once neighbouring tiles of an expert share one (below).  Measured (2,048
-// tokens with 4 of 32 experts, width 1,024, 768 a piece, weights from HBM, us, before / now): gate and up 64 / 51 (510 TFLOP/s), down
-// 52 / 31; 520, 1,024 and 4,096 tokens, both, 65 / 45, 77 / 54, 188 / 139; 2,048 tokens of 4,096 and 1,536 a piece 614 / 579.  Of that the loop's
-// order is a third (70 and 45 with the columns of a tile on one XCD), the units of tiles two.  Other shapes, gate and up / down: 64 x 256
-// 68 / 36, five stages 70 / 38 (one workgroup a CU), 128 rows x 256 47 to 59 / 34, x 192 50; 128 rows are ahead for wide experts (441 for the 579).
+// tokens with 4 of 32 experts, width 1,024, 768 a piece, us, before / now): in a prompt gate and up 62 / 55 (470 TFLOP/s), down 51 / 38; both products
+// alone, one call behind the other, weights from HBM, 122 / 100, of 520, 1,024 and 4,096 tokens 62 / 52, 82 / 67, 198 / 167, of 2,048 tokens of
+// 4,096 and 1,536 a piece 613 / 581.  Two thirds of that are the units of tiles, a third is the loop's order.  Other shapes, gate and up / down of the
+// first, alone (51 / 31 so): 64 x 256 68 / 36, five stages 70 / 38 (one workgroup a CU), 128 rows x 256 47 to 59 / 34, x 192 50; 128 rows are ahead
+// for wide experts (441 for the 581).
 // ---------------------------------------------------------------------------
 template <typename T, int WEIGHTS, int NWM, int NWN>
 struct ExpertTile {

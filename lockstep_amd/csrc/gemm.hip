@@ -1105,8 +1105,8 @@ constexpr float kStages32x32[4] = {0.218f, 0.365f, 0.515f, 0.68f}, kStages64x64[
 //                           x 1,024 7.6 / 6.5; 32 x 32 tiles, two a CU, 6.9 for the last
 //   up to 32 rows           SwiGLU 8 x 24,576 x 4,096 40.2 / 35.6 in 32 x 32, 32 x 24,544 x 512 in 32 x 64; four rounds ask for 128 rows of weights a
 //                           multiple of 4 KB apart together (8 x 32,768 x 4,096 51.9 / 64.9)
-// Others the tile whose rounds of workgroups take least by the table above.  (Every tile forced in turn over 65 to 2,048 rows and nine shapes of
-// weights: within 2 % of the best one everywhere.)  One rule stands in front of it: up to 64 rows whose rows of weights lie a multiple of 4 KB apart
+// Others the tile whose rounds of workgroups take least by the table above.  (Every tile forced in turn over 65 to 2,048 rows and nine
+// shapes of weights: within 2 % of the best one at 130 of 135 sizes, 5 % at the rest.)  One rule stands in front of it: up to 64 rows whose rows of weights lie a multiple of 4 KB apart
 // take 64 x 64 tiles (128 such rows asked for together meet in few memory channels: 16 x 32,768 x 4,096 62.6 -> 55.1 us; other K 0.9 to 1.05 times as long).
 template <typename T>
 static int ring_tile(int M, int N, int K) {

@@ -7,9 +7,10 @@
 // multiply it, and takes 1 to 2 us from the memory side; a CU's 160 KB of LDS hold two to five stages, so the
 // larger the tile, the more multiplications stand behind a byte in flight.  Loads without any product between them bring
 // 55 GB/s a CU (256 x 192 outputs) to 75 (128 x 64), 95 where L2 holds everything.  Measured (bfloat16, weights from
-// HBM, us): 2,048 x 24,576 x 4,096 326 (1,265 TFLOP/s), 2,048 x 6,144 x 4,096 83, 2,048 x 4,096 x 12,288 177 (1,165), 999 x
-// 4,096 x 4,096 39, 97 x 4,096 x 1,024 7.0; the clock falls to 1.9 GHz under the large ones, and products alone, without a load
-// or a fragment read, take 235 us where the first takes 326.
+// HBM, us): 2,048 x 24,576 x 4,096 326 (1,265 TFLOP/s; 356 in a long run of them), 2,048 x 6,144 x 4,096 83 to 89, 2,048 x 4,096 x 12,288 172 to 177
+// (1,195), 1,000 x 4,096 x 4,096 42, 97 x 4,096 x 1,024 6.4; the clock falls to 1.9 GHz under the large ones, and products alone, without a load
+// or a fragment read, take 235 us where the first takes 326.  Counters of the first: matrix pipes busy 67 % of the cycles that its CU is, LDS 28 %, no
+// bank conflicts.
 #pragma once
 
 #include "ring_product.h"
