@@ -1437,6 +1437,9 @@ struct SlicesPlan {
 // x 4,096 4.2 / 4.8, 8 x 4,096 x 12,288 23.9 / 20.2, 8 x 4,096 x 4,096 9.6 / 8.0, 64 x 1,024 x 2,048 4.5 / 4.1, 256 x 512 x 512 3.3 / 3.8; one row
 // 5,120 x 8,192 17.9 / 18.7).  Sixteen stages a workgroup at most, eight with more than 64 rows, and beyond 32 rows slices of eight and more by
 // themselves (128 x 5,120 x 5,120 with one, two and four 27.6, 29.5, 30.7; 64 x 10,240 x 5,120 31.3, 33.6, 34.9).
+// Up to 32 rows also two longer slices, where that is one nearly full round of one or of two a CU (one slice a workgroup / two: 8 x 1,280 x 14,472
+// 13.8 / 12.5, 6 x 1,472 x 9,576 10.9 / 9.9, 8 x 4,096 x 12,288 23.1 / 22.1), unless both the rows of weights and the workgroups' first columns lie a
+// multiple of 4 KB apart, so that all ask the same memory channels at once (18 x 2,240 x 14,336 14.2 / 17.0).
 static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
   const int kslice = kslice_for(K), nslices = (K + kslice - 1) / kslice;
   const long cus = compute_units();
@@ -1447,9 +1450,11 @@ static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
   const int most = f32 || M > 64 || (M > 32 && kslice > 256) ? 512 : 1024;  // elements of K a workgroup
   float least = 0.f;
   for (int rows = f32 ? 64 : 32; rows <= 64; rows += 32)
-    for (int per = 1; per == 1 || (per <= nslices && per * kslice <= most); per *= 2) {
+    for (int per = 1; per == 1 || (per <= 4 && per <= nslices); per *= 2) {
       const long all = (long)((M + rows - 1) / rows) * ((N + 63) / 64) * ((nslices + per - 1) / per);
       const int stages = std::min(per, nslices) * (kslice / (f32 ? 32 : 64));
+      const bool one_round = per == 2 && M <= 32 && ((16 * all > 9 * cus && all <= cus) || (16 * all > 30 * cus && all <= 2 * cus));
+      if (per > 1 && per * kslice > most && !(one_round && (K % 2048 || per * kslice % 2048))) continue;
       if (f32 && 16 * all < 9 * cus) continue;
       const float cost = f32 ? rounds_cost(all, 3, stages, 1.2f, kStages64x64) : rounds_cost(all, 2, stages, 1.5f, rows == 32 ? k32x64 : k64x64);
       if (best.per == 0 || cost < least) {

@@ -404,7 +404,9 @@ SLICES_PLANS = [(3, 4096, 4096, (0, 0), (0, 0)), (4, 4096, 4096, (0, 0), (0, 0))
                 (8, 5116, 8192, (32, 2), (0, 0)), (24, 8188, 1032, (32, 4), (0, 0)), (64, 4092, 1032, (64, 1), (64, 1)),
                 (64, 1020, 3072, (64, 1), (64, 1)), (128, 5116, 5120, (64, 1), (64, 1)), (56, 8188, 4424, (64, 1), (64, 1)),
                 (33, 4092, 4096, (64, 2), (64, 2)), (64, 4092, 4096, (64, 2), (64, 2)), (200, 1024, 3072, (64, 2), (64, 1)),
-                (256, 4096, 520, (64, 2), (64, 1)), (33, 12284, 3080, (64, 4), (64, 1))]
+                (256, 4096, 520, (64, 2), (64, 1)), (33, 12284, 3080, (64, 4), (64, 1)),
+                (8, 4092, 12288, (32, 2), (0, 0)), (6, 1468, 9576, (32, 2), (0, 0)), (18, 2236, 14336, (32, 1), (0, 0)), (32, 1020, 9576, (32, 1), (0, 0)),
+                (24, 3004, 9576, (32, 1), (0, 0))]
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
