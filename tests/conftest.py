@@ -15,7 +15,7 @@ sys.path.insert(0, str(ROOT / "tests"))
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs an AMD GPU (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs an AMD GPU")
 
 
 def pytest_collection_modifyitems(config, items):
