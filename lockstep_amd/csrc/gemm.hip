@@ -1427,16 +1427,23 @@ namespace ls {
 struct SlicesPlan {
   int tile, per;
 };
+// The products a CU (in 256) from which slice sums of bfloat16 come from tiles: what a wave a slice does instead grows with the rows that every
+// block of 16 columns reads again, a tile's time hardly.  Measured over 10,655 sizes (us, a wave a slice / tiles): fewer products for rows of weights
+// that are whole lines of 128 bytes (17 x 1,408 x 3,072 6.9 / 5.1, 16 x 1,792 x 3,328 6.2 / 5.5, 8 x 4,096 x 2,560 6.5 / 7.6, 32 x 1,280 x 1,280 3.6 / 4.0, 256 x 512 x 512
+// 3.3 / 3.9; no whole lines 10 x 6,784 x 1,128 6.0 / 7.9, 48 x 5,120 x 1,576 16.3 / 8.6); under eight rows, which cost little to read again, many more (6 x
+// 6,656 x 2,304 8.2 / 10.2), but for long slices (4 x 4,096 x 12,288 24.0 / 21.8) and rows of weights a multiple of 4 KB apart, sixteen of which
+// meet in few memory channels (4 x 4,096 x 4,096 9.7 / 8.3).  One row never (5,120 x 8,192 19.8 / 20.4).
+static long slices_line(int M, int K) {
+  if (K > 4096) return M < 8 ? 50 : 72;  // slices of more than 256
+  if (M < 8) return K % 2048 == 0 ? 56 : 180;
+  return K % 64 == 0 ? (M <= 16 ? 80 : 64) : (M <= 16 ? 100 : 88);
+}
 // The cheapest of the tiles and of one, two or four slices a workgroup by rounds_cost.  (us)
 // float32, from 33 rows on: 64 x 64 tiles, from nine workgroups for sixteen CUs on (48 x 1,024 x 2,048, eight, 7.1 by a wave a slice / 8.6), eight or
 // sixteen stages a workgroup (33 x 4,096 x 4,096 24.9 / 22.1, 160 x 10,240 x 768 31.7 / 36.4, 200 x 5,120 x 1,024 27.4 / 30.4); slices of sixteen
 // stages by themselves (56 x 8,192 x 8,192 83, two of them 98).
-// bfloat16, from 4 rows on: 32 x 64 or 64 x 64 tiles, two a CU.  What a wave a slice does instead grows with the rows that every block of 16 columns
-// reads again, and a tile's time hardly: the line is a number of products a CU, the same from 4 rows to 256 (a wave a slice / tiles: 17 x 1,024 x
-// 3,072 4.0 / 4.7, 17 x 2,048 x 3,072 7.1 / 5.5, 32 x 4,096 x 552 3.4 / 4.2, 32 x 16,384 x 768 11.7 / 8.4, 48 x 5,120 x 1,576 15.2 / 8.3, 16 x 1,024
-// x 4,096 4.2 / 4.8, 8 x 4,096 x 12,288 23.9 / 20.2, 8 x 4,096 x 4,096 9.6 / 8.0, 64 x 1,024 x 2,048 4.5 / 4.1, 256 x 512 x 512 3.3 / 3.8; one row
-// 5,120 x 8,192 17.9 / 18.7).  Sixteen stages a workgroup at most, eight with more than 64 rows, and beyond 32 rows slices of eight and more by
-// themselves (128 x 5,120 x 5,120 with one, two and four 27.6, 29.5, 30.7; 64 x 10,240 x 5,120 31.3, 33.6, 34.9).
+// bfloat16, from 4 rows on: 32 x 64 or 64 x 64 tiles, two a CU, beyond slices_line.  Sixteen stages a workgroup at most, eight with more than 64
+// rows, and beyond 32 rows slices of eight and more by themselves (128 x 5,120 x 5,120 with one, two and four 27.6, 29.5, 30.7; 64 x 10,240 x 5,120 31.3, 33.6, 34.9).
 // Up to 32 rows also two longer slices, where that is one nearly full round of one or of two a CU (one slice a workgroup / two: 8 x 1,280 x 14,472
 // 13.8 / 12.5, 6 x 1,472 x 9,576 10.9 / 9.9, 8 x 4,096 x 12,288 23.1 / 22.1), unless both the rows of weights and the workgroups' first columns lie a
 // multiple of 4 KB apart, so that all ask the same memory channels at once (18 x 2,240 x 14,336 14.2 / 17.0).
@@ -1445,7 +1452,7 @@ static SlicesPlan slices_plan(int dtype, int M, int N, int K) {
   const long cus = compute_units();
   const bool f32 = dtype == kF32;
   SlicesPlan best{kRing64x64, 0};
-  if (f32 ? M < 33 : M < 4 || (long)((N + 15) / 16) * std::max(K, 256) * M <= 72 * 256 * cus) return best;
+  if (f32 ? M < 33 : M < 4 || (long)((N + 15) / 16) * std::max(K, 256) * M <= slices_line(M, K) * 256 * cus) return best;
   constexpr float k32x64[2] = {0.18f, 0.39f}, k64x64[2] = {0.33f, 0.52f};
   const int most = f32 || M > 64 || (M > 32 && kslice > 256) ? 512 : 1024;  // elements of K a workgroup
   float least = 0.f;

@@ -399,14 +399,15 @@ def test_products_on_both_sides_of_the_lines_of_the_ring_kernel_have_the_same_bi
 
 
 # (rows, columns, K) of slice sums, and (rows of the tile, slices a workgroup) of the ring kernel that computes them in bfloat16 and in float32
-SLICES_PLANS = [(3, 4096, 4096, (0, 0), (0, 0)), (4, 4096, 4096, (0, 0), (0, 0)), (17, 1028, 1288, (0, 0), (0, 0)), (33, 1024, 8, (0, 0), (0, 0)),
-                (40, 260, 328, (0, 0), (0, 0)), (65, 508, 2048, (0, 0), (0, 0)), (32, 1020, 4424, (32, 1), (0, 0)), (64, 1024, 2048, (32, 1), (0, 0)),
+SLICES_PLANS = [(3, 4096, 4096, (0, 0), (0, 0)), (4, 4096, 4096, (32, 4), (0, 0)), (17, 1028, 1288, (0, 0), (0, 0)), (33, 1024, 8, (0, 0), (0, 0)),
+                (40, 260, 328, (0, 0), (0, 0)), (65, 508, 2048, (32, 1), (0, 0)), (32, 1020, 4424, (32, 1), (0, 0)), (64, 1024, 2048, (32, 1), (0, 0)),
                 (8, 5116, 8192, (32, 2), (0, 0)), (24, 8188, 1032, (32, 4), (0, 0)), (64, 4092, 1032, (64, 1), (64, 1)),
                 (64, 1020, 3072, (64, 1), (64, 1)), (128, 5116, 5120, (64, 1), (64, 1)), (56, 8188, 4424, (64, 1), (64, 1)),
                 (33, 4092, 4096, (64, 2), (64, 2)), (64, 4092, 4096, (64, 2), (64, 2)), (200, 1024, 3072, (64, 2), (64, 1)),
                 (256, 4096, 520, (64, 2), (64, 1)), (33, 12284, 3080, (64, 4), (64, 1)),
                 (8, 4092, 12288, (32, 2), (0, 0)), (6, 1468, 9576, (32, 2), (0, 0)), (18, 2236, 14336, (32, 1), (0, 0)), (32, 1020, 9576, (32, 1), (0, 0)),
-                (24, 3004, 9576, (32, 1), (0, 0))]
+                (24, 3004, 9576, (32, 1), (0, 0)), (6, 6656, 2304, (0, 0), (0, 0)), (10, 6784, 1128, (0, 0), (0, 0)), (17, 1404, 3072, (32, 2), (0, 0)),
+                (17, 1404, 3080, (0, 0), (0, 0)), (8, 4096, 2560, (0, 0), (0, 0)), (256, 512, 512, (0, 0), (0, 0))]
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
